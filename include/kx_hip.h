@@ -86,7 +86,7 @@ int kx_gemv_awq_bf16(const uint16_t* x, const int32_t* qweight, const uint16_t* 
                      int32_t group_size, void* workspace, size_t workspace_bytes, void* stream);
 
 /* Two kernels implement kx_gemv_awq_bf16, chosen by shape: one on the vector ALUs and one on the matrix
- * cores (MFMA; M >= 2 when the group size is a power of two and N a multiple of sixteen).  The library keeps no state about the choice. */
+ * cores (MFMA; M >= 2 and N >= 16).  The library keeps no state about the choice. */
 
 /* kx_gemv_awq_bf16 for callers that cannot allocate or hand over a workspace (code under HIP graph capture,
  * serving loops and harnesses that forbid hipMalloc): the split-K workspace is a static device array inside
@@ -189,7 +189,7 @@ int kx_gemv_awq_qkv_rope_bf16(const uint16_t* residual, const uint16_t* delta, c
  * norm_sumsq [rows, norm_parts, 4], sumsq_out [rows, ceil(N / 256), 4]); gate, up and norm_row may have their rows
  * act_ld elements apart.  That form runs on the matrix-core kernel and takes KX_IN_ROW / KX_IN_SWIGLU /
  * KX_IN_NORM with any output kind (KX_OUT_QKV_ROPE: q_out [rows, n_q * 128], pos [rows], one cache pair per
- * row, see cache_stride), a power-of-two group size, N a multiple of 16, act_ld a
+ * row, see cache_stride), N a multiple of 16, act_ld a
  * multiple of 8 and 16-byte aligned gate / up / norm_row / norm_gain; with SwiGLU input and residual output it
  * is bitwise kx_swiglu_bf16, kx_gemv_awq_bf16 and kx_add_bf16 back to back.
  * One row: always the vector kernel.  Replaces: the chain LayerMHA -> LayerMatmul -> LayerAdd -> LayerRMSNorm ->

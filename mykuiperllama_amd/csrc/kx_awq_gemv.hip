@@ -10,7 +10,8 @@ namespace kx {
 namespace {
 
 struct AwqPlan {
-    bool mfma;     // matrix-core kernel (any M) or the VALU kernel
+    bool mfma;     // matrix-core kernel or the VALU kernel
+    bool sliced;   // MFMA kernel: all workgroups of a column tile finish it together
     int waves;     // waves per workgroup stacked along K (4, 8 or 16)
     int rt;        // VALU kernel: consecutive rows per lane (8 or 16); MFMA kernel: 32-row steps per wave
     int mb;        // activation rows per workgroup (1, 2, 4 or 8)
@@ -26,16 +27,19 @@ inline int rows_per_block(int waves, int rt) {
 constexpr int kComputeUnits = 256;  // MI355X
 constexpr int kExchangeRows = 8;    // what a K tile's share of the split-K exchange costs, in rows of K streamed
 
-inline bool is_pow2(int v) {
-    return v > 0 && (v & (v - 1)) == 0;
-}
-
-// MFMA kernel: four waves per workgroup, each walking `ks` consecutive 32-row steps that must lie in
-// one quantisation group.  Measured on the Qwen3-8B shapes: two steps per wave (256 rows per
-// workgroup) are best up to M = 8, except that long K (down 12288 -> 4096, 48 K tiles) does better
-// with four steps from M = 5 (15.7 -> 14.4 us at M = 8); from M = 9 four steps (512 rows, half the
-// partial sums to exchange) win everywhere (M = 16: q 12.1 -> 10.5, gate 15.6 -> 13.7, down
-// 24.7 -> 18.0 us), even where they leave fewer workgroups than compute units.
+// MFMA kernel: four waves per workgroup, each walking `ks` consecutive 32-row steps that must lie in one quantisation
+// group.  What it costs besides the weights is the exchange of partial sums, M KB per K tile and column tile.
+//   M <= 4   one workgroup (or wave) of a column tile reads all of them back, sixteen K tiles in flight: two steps per
+//            wave, or four where that brings the K tiles down to one such batch (5120 -> 5120 at M = 4: 9.2 -> 8.1 us).
+//   M >= 5   every workgroup of a column tile finishes a share (splitk_exchange_sliced), provided that they are on the
+//            chip together: at most two per compute unit.  The shortest run of steps that leaves one workgroup per
+//            compute unit and sixteen K tiles (fewer workgroups idle against more partial sums: 1024 -> 2048 ks = 1, q ks
+//            = 2, q|k|v and down ks = 4).  Against the single reader, us per launch at M = 8 / 16: k 4096 -> 1024
+//            7.6 / 10.2 -> 6.9 / 8.1, q 4096 -> 4096 8.2 / 10.7 -> 7.5 / 8.9, q|k|v 9.2 / 11.0 -> 8.6 / 9.8, down
+//            12288 -> 4096 15.4 / 18.9 -> 12.6 / 14.7, gate 4096 -> 12288 12.1 / 14.3 -> 12.0 / 12.6, 5120 -> 10240
+//            17.4 / 17.4 -> 12.9 / 14.1.  Larger grids, whose workgroups come in rounds, keep the single reader: with
+//            shares the early ones would hold the places the late ones need (gate|up 4096 -> 24576 at M = 16: 19.7
+//            against 21.5 us), and so do their column-tile-fastest order and 256 / 512 rows per workgroup.
 inline AwqPlan make_mfma_plan(int M, int K, int N, int group) {
     AwqPlan p;
     p.mfma = true;
@@ -43,18 +47,31 @@ inline AwqPlan make_mfma_plan(int M, int K, int N, int group) {
     p.mb = M;
     p.mtiles = 1;
     p.waves = 4;
+    const auto ktiles_with = [&](int ks) { return (K + p.waves * ks * kStepRows - 1) / (p.waves * ks * kStepRows); };
+    const auto allowed = [&](int ks) { return group % (ks * kStepRows) == 0 && (ks == 1 || p.waves * ks * kStepRows <= K); };
     int ks = (M >= 9 || (M >= 5 && K >= 8192)) ? 4 : 2;
-    while (ks > 1 && ks * kStepRows > group) ks /= 2;
-    while (ks > 1 && p.waves * ks * kStepRows > K) ks /= 2;
+    if (M <= 4 && ktiles_with(2) > 16 && ktiles_with(2) <= 32) ks = 4;
+    while (!allowed(ks)) ks /= 2;
+    p.sliced = false;
+    if (M >= 5) {
+        int best = 0;  // the longest run that is allowed, or the shortest that is short enough
+        for (int c = 4; c >= 1; c /= 2) {
+            if (allowed(c) && (best == 0 || (p.coltiles * ktiles_with(c) <= kComputeUnits && ktiles_with(c) <= 16))) best = c;
+        }
+        const int kt = ktiles_with(best);
+        if (kt > 1 && kt <= kSliceMaxKTiles && p.coltiles * kt <= 2 * kComputeUnits) {
+            p.sliced = true;
+            ks = best;
+        }
+    }
     p.rt = ks;  // steps per wave
-    const int kb = p.waves * ks * kStepRows;
-    p.ktiles = (K + kb - 1) / kb;
+    p.ktiles = ktiles_with(ks);
     return p;
 }
 
 inline AwqPlan make_valu_plan(int M, int K, int N, bool allow_long_rows = true, bool allow_12_waves = true) {
     AwqPlan p;
-    p.mfma = false;
+    p.mfma = p.sliced = false;
     p.coltiles = (N / 8 + kWC - 1) / kWC;
     p.mb = M >= 8 ? 8 : (M >= 4 ? 4 : (M >= 2 ? 2 : 1));
     p.mtiles = (M + p.mb - 1) / p.mb;
@@ -116,7 +133,7 @@ constexpr int kFixedExchangeRows = 4;
 
 inline AwqPlan make_fixed_plan(int K, int N) {
     AwqPlan p{};
-    p.mfma = false;
+    p.mfma = p.sliced = false;
     p.coltiles = (N / 8 + kWC - 1) / kWC;
     p.mb = 1;
     p.mtiles = 1;
@@ -144,14 +161,27 @@ inline AwqPlan make_fixed_plan(int K, int N) {
 }
 
 inline AwqPlan make_plan(int M, int K, int N, int group, int mode) {
-    // The MFMA kernel needs quantisation groups that tile the workgroup's K range (powers of two)
-    // and loads two packed words at a time (N a multiple of sixteen).
-    const bool mfma_ok = is_pow2(group) && (N % 16) == 0;  // mfma_shape_ok() below
     // One activation row stays on the vector kernel: with the fixed-point exchange it is ahead of the MFMA kernel on
     // every measured shape (kx_gemv_awq_bf16_policy decides that before it comes here), and the launches with an
     // activation prologue or an epilogue live in it.
-    const bool mfma = mfma_ok && (mode == KX_POLICY_MFMA || (mode == KX_POLICY_BY_SHAPE && M >= 2));
+    const bool mfma = N >= 16 && (mode >= KX_POLICY_MFMA || (mode == KX_POLICY_BY_SHAPE && M >= 2));  // a lane loads two words
     return mfma ? make_mfma_plan(M, K, N, group) : make_valu_plan(M, K, N);
+}
+
+inline MfmaGrid mfma_grid(const AwqPlan& p, int group) {
+    const uint32_t gs = static_cast<uint32_t>(group / kStepRows);
+    MfmaGrid g{};
+    g.coltiles = p.coltiles;
+    g.ktiles = p.ktiles;
+    g.side = p.coltiles;
+    if (p.sliced) {  // the widest group that divides the tiles: no workgroup without a tile, no test for one
+        g.side = kTileGroup;
+        while (p.coltiles % g.side != 0) g.side--;
+    }
+    g.sliced = p.sliced;
+    g.wait_ticks = kSliceWaitTicks;
+    g.group_magic = gs == 1 ? 0u : static_cast<uint32_t>(((1ull << 32) + gs - 1) / gs);
+    return g;
 }
 
 template <int WAVES, int RT>
@@ -220,9 +250,8 @@ void launch_mfma_fused(const AwqPlan& p, const FusedInput& fi, const ResidualTar
                        const int32_t* qweight, const uint16_t* scales, const int32_t* qzeros, uint16_t* y,
                        float* partials, uint32_t* counters, int M, int K, int N, int group, hipStream_t stream,
                        const RopeTarget& rope = RopeTarget{}, size_t cache_stride = 0) {
-    int group_shift = 0;
-    while ((1 << group_shift) < group) group_shift++;
-#define KX_MARGS x, qweight, scales, qzeros, y, partials, counters, M, K, N, group_shift, p.coltiles, p.ktiles, stream, fi, res, rope, cache_stride
+    const MfmaGrid grid = mfma_grid(p, group);
+#define KX_MARGS x, qweight, scales, qzeros, y, partials, counters, M, K, N, grid, stream, fi, res, rope, cache_stride
 #define KX_MFMA_BY_M(KS)                                                             \
     do {                                                                             \
         if (M <= 2) launch_awq_gemv_mfma<4, KS, 2, 1, PRO, EPI>(KX_MARGS);           \
@@ -235,12 +264,6 @@ void launch_mfma_fused(const AwqPlan& p, const FusedInput& fi, const ResidualTar
     else KX_MFMA_BY_M(1);
 #undef KX_MFMA_BY_M
 #undef KX_MARGS
-}
-
-// What the matrix-core kernel asks of a shape: quantisation groups that tile the workgroup's K range
-// (powers of two) and two packed words per load (N a multiple of sixteen).
-inline bool mfma_shape_ok(int N, int group) {
-    return is_pow2(group) && (N % 16) == 0;
 }
 
 inline bool aligned_to(const void* p, size_t a) {
@@ -399,7 +422,7 @@ extern "C" int kx_gemv_awq_bf16_policy(const uint16_t* x, const int32_t* qweight
                                        const int32_t* qzeros, uint16_t* y, int32_t M, int32_t K, int32_t N,
                                        int32_t group_size, void* workspace, size_t workspace_bytes,
                                        void* stream, int32_t policy) {
-    if (policy < KX_POLICY_BY_SHAPE || policy > KX_POLICY_MFMA) return KX_ERR_BAD_SHAPE;
+    if (policy < KX_POLICY_BY_SHAPE || policy > KX_POLICY_MFMA_NO_WAIT) return KX_ERR_BAD_SHAPE;
     if (!x) return KX_ERR_NULL_POINTER;
     int rc = kx::check_awq_weights(qweight, scales, qzeros, y, M, K, N, group_size);
     if (rc != KX_OK) return rc;
@@ -426,20 +449,26 @@ extern "C" int kx_gemv_awq_bf16_policy(const uint16_t* x, const int32_t* qweight
     rc = kx::resolve_workspace(p, M, N, workspace, workspace_bytes, &partials, &counters);
     if (rc != KX_OK) return rc;
     if (p.mfma) {
-        int group_shift = 0;
-        while ((1 << group_shift) < group_size) group_shift++;
-#define KX_MARGS x, qweight, scales, qzeros, y, partials, counters, M, K, N, group_shift, p.coltiles, p.ktiles, s
-#define KX_MFMA_BY_M(KS)                                                        \
-    do {                                                                        \
-        if (M == 1) kx::launch_awq_gemv_mfma<4, KS, 1, 1>(KX_MARGS);            \
-        else if (M == 2) kx::launch_awq_gemv_mfma<4, KS, 2, 1>(KX_MARGS);       \
-        else if (M <= 4) kx::launch_awq_gemv_mfma<4, KS, 4, 1>(KX_MARGS);       \
-        else if (M <= 8) kx::launch_awq_gemv_mfma<4, KS, 8, 1>(KX_MARGS);       \
-        else kx::launch_awq_gemv_mfma<4, KS, 8, 2>(KX_MARGS);                   \
+        kx::MfmaGrid grid = kx::mfma_grid(p, group_size);
+        if (policy == KX_POLICY_MFMA_NO_WAIT) grid.wait_ticks = 0;
+#define KX_MARGS x, qweight, scales, qzeros, y, partials, counters, M, K, N, grid, s
+#define KX_MFMA_ROWS(KS, LONE)                                                                                \
+    do {                                                                                                       \
+        if (M == 1) kx::launch_awq_gemv_mfma<4, KS, 1, 1, kx::kProNone, kx::kEpiStore, LONE>(KX_MARGS);        \
+        else if (M == 2) kx::launch_awq_gemv_mfma<4, KS, 2, 1, kx::kProNone, kx::kEpiStore, LONE>(KX_MARGS);   \
+        else if (M <= 4) kx::launch_awq_gemv_mfma<4, KS, 4, 1, kx::kProNone, kx::kEpiStore, LONE>(KX_MARGS);   \
+        else if (M <= 8) kx::launch_awq_gemv_mfma<4, KS, 8, 1, kx::kProNone, kx::kEpiStore, LONE>(KX_MARGS);   \
+        else kx::launch_awq_gemv_mfma<4, KS, 8, 2, kx::kProNone, kx::kEpiStore, LONE>(KX_MARGS);               \
+    } while (0)
+#define KX_MFMA_BY_M(KS)                        \
+    do {                                        \
+        if (N % 16) KX_MFMA_ROWS(KS, true);     \
+        else KX_MFMA_ROWS(KS, false);           \
     } while (0)
         if (p.rt == 4) KX_MFMA_BY_M(4);
         else if (p.rt == 2) KX_MFMA_BY_M(2);
         else KX_MFMA_BY_M(1);
+#undef KX_MFMA_ROWS
 #undef KX_MFMA_BY_M
 #undef KX_MARGS
         return kx::launch_status();
@@ -477,7 +506,7 @@ extern "C" int kx_gemv_awq_swiglu_bf16(const uint16_t* gate, const uint16_t* up,
     fi.b = up;
     fi.ld = act_ld;
     // Several rows go to the matrix cores, as in kx_gemv_awq_bf16, when gate and up can be read 16 bytes at a time
-    if (M >= 2 && kx::mfma_shape_ok(N, group_size) && kx::aligned_to(gate, 16) && kx::aligned_to(up, 16) &&
+    if (M >= 2 && (N % 16) == 0 && kx::aligned_to(gate, 16) && kx::aligned_to(up, 16) &&
         (act_ld % 8) == 0) {
         const kx::AwqPlan mp = kx::make_mfma_plan(M, K, N, group_size);
         float* partials = nullptr;
@@ -689,7 +718,7 @@ extern "C" int kx_gemv_awq_chain_bf16(const kx_chain_desc* d, const int32_t* qwe
     if (rows > 1) {
         // several rows: the matrix-core kernel, which produces activations 16 bytes at a time
         if (d->in_kind == KX_IN_ATTN) return KX_ERR_BAD_SHAPE;
-        if (!kx::mfma_shape_ok(N, group_size) || (act_ld % 8) != 0) return KX_ERR_BAD_SHAPE;
+        if ((N % 16) != 0 || (act_ld % 8) != 0) return KX_ERR_BAD_SHAPE;
     }
 
     // where the activations come from

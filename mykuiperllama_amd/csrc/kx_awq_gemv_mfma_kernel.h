@@ -38,6 +38,7 @@
 namespace kx {
 
 constexpr int kStepRows = 32;  // rows of K per MFMA step
+constexpr int kTileGroup = 8;  // most column tiles whose workgroups start side by side when they finish together
 
 // Column (0..7) inside a word -> nibble that holds it (inverse of order_of).
 __host__ __device__ constexpr int nibble_of(int col) {
@@ -73,15 +74,40 @@ __device__ __forceinline__ uint4 f32_to_bf16x8(const float (&f)[8]) {
     return make_uint4(w[0], w[1], w[2], w[3]);
 }
 
+template <bool LONE>
+struct WordPair {
+    typedef u32x2 type;
+};
+template <>
+struct WordPair<true> {
+    typedef u32x2 __attribute__((aligned(4))) type;
+};
+
+// How a launch divides the matrix between workgroups.
+struct MfmaGrid {
+    int coltiles;
+    int ktiles;
+    int side;              // column tiles side by side in the grid (gridDim.x, whose own load is a trip to memory)
+    int sliced;            // all K tiles of a column tile finish it together (splitk_exchange_sliced)
+    uint32_t group_magic;  // ceil(2^32 / (G / 32)), 0 for groups of 32
+    uint32_t wait_ticks;   // how long a workgroup waits for the others of its tile
+};
+
+// Quantisation group of a 32-row step: step / (G / 32) for any number of steps a matrix can have.
+__device__ __forceinline__ int group_of_step(const MfmaGrid& g, int step) {
+    return g.group_magic ? static_cast<int>(__umulhi(static_cast<uint32_t>(step), g.group_magic)) : step;
+}
+
 // KS: consecutive 32-row steps per wave (they must share a quantisation group);
-// MC: activation rows a workgroup reduces per LDS round (1, 2, 4 or 8); ROUNDS: 2 for M > 8, else 1.
+// MC: activation rows a workgroup reduces per LDS round (1, 2, 4 or 8); ROUNDS: 2 for M > 8, else 1;
+// LONE: N is an odd multiple of eight (a template parameter: the moves cost 20 registers, an occupancy step).
 // With a prologue, `x` is not read: fi.a / fi.b (/ fi.gain) are 16-byte aligned, fi.ld a multiple of eight.
-template <int WAVES, int KS, int MC, int ROUNDS, int PRO = kProNone, int EPI = kEpiStore>
+template <int WAVES, int KS, int MC, int ROUNDS, int PRO = kProNone, int EPI = kEpiStore, bool LONE = false>
 __global__ __launch_bounds__(WAVES * kWave, 2) void awq_gemv_mfma_kernel(
     const uint16_t* __restrict__ x, const uint32_t* __restrict__ qweight,
     const uint16_t* __restrict__ scales, const uint32_t* __restrict__ qzeros,
     uint16_t* __restrict__ y, float* __restrict__ partials, uint32_t* __restrict__ counters,
-    int M, int K, int N, int group_shift, int ktiles, FusedInput fi, ResidualTarget res, RopeTarget rope,
+    int M, int K, int N, MfmaGrid grid, FusedInput fi, ResidualTarget res, RopeTarget rope,
     size_t cache_stride) {
     constexpr int WROWS = KS * kStepRows;  // rows of K per wave
     constexpr int KB = WAVES * WROWS;      // rows of K per workgroup
@@ -100,7 +126,7 @@ __global__ __launch_bounds__(WAVES * kWave, 2) void awq_gemv_mfma_kernel(
 
     __shared__ __attribute__((aligned(16))) float red[WAVES][MC][kTileCols];
     __shared__ float xs_red[WAVES][MC];
-    __shared__ uint32_t s_prev;
+    __shared__ uint32_t s_word[3];
     __shared__ __attribute__((aligned(16))) uint16_t s_x[STAGED ? ROWS : 1][STAGED ? XPITCH : 8];
     __shared__ float s_inv[PRO == kProPreNorm ? ROWS : 1];
 
@@ -109,34 +135,14 @@ __global__ __launch_bounds__(WAVES * kWave, 2) void awq_gemv_mfma_kernel(
     const int lane = tid % kWave;
     const int c = lane % 16;  // column slot: word pair c of the tile, MFMA column c
     const int b = lane / 16;  // k block inside the step, D row block
-    const int ct = blockIdx.x;  // column tile; x runs fastest, so neighbours in time are neighbours in N
+    // Column tiles run fastest, so neighbours in time are neighbours in N; where workgroups finish a tile together, in
+    // groups of at most eight, so that they start within 8 * ktiles of each other.
+    const int ct = blockIdx.z * grid.side + blockIdx.x;
     const int kt = blockIdx.y;
+    const int ktiles = grid.ktiles;
     const int nw = N >> 3;
 
     const int kwave = kt * KB + wave * WROWS;  // first row of this wave
-
-    // The rotary epilogue (row m of the result belongs to sequence m): the workgroup that finishes a column
-    // tile holds two heads of every row; wave w will take the (row, head) items w, w + WAVES, ...  Its
-    // positions and the heads' gains are requested now, long before the epilogue needs them.
-    constexpr int ROPE_ITEMS = (2 * ROWS + WAVES - 1) / WAVES;  // items per wave
-    int rope_pos[EPI == kEpiQkRope ? ROPE_ITEMS : 1];
-    uint16_t rope_ga[2], rope_gb[2];
-    if constexpr (EPI == kEpiQkRope) {
-#pragma unroll
-        for (int i = 0; i < ROPE_ITEMS; i++) {
-            const int r = (wave + i * WAVES) / 2;
-            rope_pos[i] = rope.pos[r < M ? r : M - 1];
-        }
-        // both gains, then a select of values (a select between pointers ends up as a table in private memory)
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-            const bool q_head = ct * (kTileCols / kHeadDim) + h < rope.n_q;
-            const uint16_t qa = rope.q_gain[lane], qb = rope.q_gain[lane + 64];
-            const uint16_t ka = rope.k_gain[lane], kb = rope.k_gain[lane + 64];
-            rope_ga[h] = q_head ? qa : ka;
-            rope_gb[h] = q_head ? qb : kb;
-        }
-    }
 
     // ---- operands of the activation prologue go out first: they are small, mostly cached, and the prologue
     // should run while the weights are still on their way ----
@@ -186,7 +192,7 @@ __global__ __launch_bounds__(WAVES * kWave, 2) void awq_gemv_mfma_kernel(
 #pragma unroll
     for (int wv = 0; wv < WAVES; wv++) {
         const int krow = kt * KB + wv * WROWS;
-        const int g = (krow < K ? krow : K - 1) >> group_shift;  // rows past K meet zero activations
+        const int g = group_of_step(grid, (krow < K ? krow : K - 1) / kStepRows);  // rows past K meet zero activations
         s_bits[wv] = scales[static_cast<size_t>(g) * N + own_ld];
         z_word[wv] = qzeros[static_cast<size_t>(g) * nw + (own_ld >> 3)];
     }
@@ -204,11 +210,13 @@ __global__ __launch_bounds__(WAVES * kWave, 2) void awq_gemv_mfma_kernel(
             xa[ks] = make_uint4(live ? got.x : 0u, live ? got.y : 0u, live ? got.z : 0u, live ? got.w : 0u);
         }
     }
-    // The lane's two word columns, eight rows per step, both words in one load: the host sends only
-    // N that are multiples of sixteen here, so word rows are 8-byte aligned.
+    // The lane's two word columns, eight rows per step, both words in one load, of four-byte alignment where the
+    // number of words is odd; the last lane's one word then comes as the second of its pair and is moved over.
+    using word_pair = typename WordPair<LONE>::type;
     uint32_t w[KS][8][2];
     const int wc_first = ct * 32 + 2 * c;
-    const int wc0 = wc_first < nw ? wc_first : nw - 2;
+    const int wc0 = max(0, min(wc_first, nw - 2));
+    const bool lone_word = wc_first == nw - 1;
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) {
         const int kstep = kwave + ks * kStepRows;
@@ -216,7 +224,7 @@ __global__ __launch_bounds__(WAVES * kWave, 2) void awq_gemv_mfma_kernel(
         const uint32_t* wp = qweight + static_cast<size_t>(k0) * nw + wc0;
 #pragma unroll
         for (int r = 0; r < 8; r++) {
-            const u32x2 v = __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(wp + static_cast<size_t>(r) * nw));
+            const u32x2 v = __builtin_nontemporal_load(reinterpret_cast<const word_pair*>(wp + static_cast<size_t>(r) * nw));
             w[ks][r][0] = v.x;
             w[ks][r][1] = v.y;
         }
@@ -293,6 +301,10 @@ __global__ __launch_bounds__(WAVES * kWave, 2) void awq_gemv_mfma_kernel(
     const uint32_t magic = opaque_bf16_128_pair();
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) {
+        if constexpr (LONE) {
+#pragma unroll
+            for (int r = 0; r < 8; r++) w[ks][r][0] = lone_word ? w[ks][r][1] : w[ks][r][0];
+        }
         const bf16x8 a_op = as_bf16x8(xa[ks].x, xa[ks].y, xa[ks].z, xa[ks].w);
         xs = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_op, ones, ks == 0 ? zero4 : xs, 0, 0, 0);
 #pragma unroll
@@ -378,118 +390,170 @@ __global__ __launch_bounds__(WAVES * kWave, 2) void awq_gemv_mfma_kernel(
         return;
     }
 #endif
-    if constexpr (EPI == kEpiResidual || EPI == kEpiQkRope) {
-        static_assert(THREADS == kTileCols, "these epilogues are laid out for 256 threads");
-        // Thread t ends up with the finished sums of tile column t, every row; the residual rows are
-        // requested as soon as the workgroup knows that it is the one to finish.
+    // ---- the finished rows, by slices: activation row m of half a tile (128 columns, one head of a q|k|v row);
+    // a lane holds columns lane and lane + 64 of the half ----
+    struct Operands {
+        uint16_t a, b, c, d;
+        int pos;
+    };
+    auto request = [&](int m, int half) {
+        Operands o{};
+        const int ca = ct * kTileCols + half * kSliceCols + lane;
+        if constexpr (EPI == kEpiResidual) {
+            const size_t row = static_cast<size_t>(m) * N;
+            o.a = res.in[row + (ca < N ? ca : N - 1)];
+            o.b = res.in[row + (ca + kWave < N ? ca + kWave : N - 1)];
+        }
+        if constexpr (EPI == kEpiQkRope) {
+            // both gains, then a select of values (a select between pointers ends up as a table in private memory)
+            o.pos = rope.pos[m];
+            o.a = rope.q_gain[lane];
+            o.b = rope.q_gain[lane + 64];
+            o.c = rope.k_gain[lane];
+            o.d = rope.k_gain[lane + 64];
+        }
+        return o;
+    };
+    auto finish = [&](int m, int half, float a, float b, const Operands& o) {
+        const int ca = ct * kTileCols + half * kSliceCols + lane;
+        const int cb = ca + kWave;
+        // the projection's output is a bf16 tensor, whatever follows
+        const uint16_t oa = f32_to_bf16(a), ob = f32_to_bf16(b);
+        if constexpr (EPI == kEpiStore) {
+            uint16_t* row = y + static_cast<size_t>(m) * N;
+            if (ca < N) row[ca] = oa;
+            if (cb < N) row[cb] = ob;
+        } else if constexpr (EPI == kEpiResidual) {
+            const uint16_t ra = f32_to_bf16(bf16_to_f32(o.a) + bf16_to_f32(oa));
+            const uint16_t rb = f32_to_bf16(bf16_to_f32(o.b) + bf16_to_f32(ob));
+            uint16_t* row = res.out + static_cast<size_t>(m) * N;
+            if (ca < N) row[ca] = ra;
+            if (cb < N) row[cb] = rb;
+            const float va = ca < N ? bf16_to_f32(ra) : 0.0f, vb = cb < N ? bf16_to_f32(rb) : 0.0f;
+            const float qa = wave_sum(va * va), qb = wave_sum(vb * vb);  // quarters of the tile; past N: 0
+            if (lane == 0) {
+                float* dst = res.sumsq + (static_cast<size_t>(m) * grid.coltiles + ct) * (kTileCols / kWave) + 2 * half;
+                dst[0] = qa;
+                dst[1] = qb;
+            }
+        } else {
+            const int head = ct * (kTileCols / kHeadDim) + half;
+            const bool q_head = head < rope.n_q;
+            RopeTarget t = rope;
+            t.q_out += static_cast<size_t>(m) * rope.n_q * kHeadDim;
+            t.k_cache += static_cast<size_t>(m) * cache_stride;
+            t.v_cache += static_cast<size_t>(m) * cache_stride;
+            qk_norm_rope_head_with(oa, ob, head, lane, t, o.pos, q_head ? o.a : o.c, q_head ? o.b : o.d);
+        }
+    };
+    static_assert(THREADS == kTileCols && kSliceCols == kHeadDim, "one thread per tile column, a slice is a head");
+    float* s_sum = &red[0][0][0];  // a tile of finished rows, where one workgroup holds them all: the reduction buffer, free again
+    static_assert(WAVES * MC >= ROWS, "the reduction buffer holds a tile of finished rows");
+    auto finish_from_lds = [&] {
+        __syncthreads();
+        for (int i = wave; i < 2 * M; i += WAVES) {
+            const int m = i >> 1, half = i & 1;
+            const float* src = s_sum + m * kTileCols + half * kSliceCols + lane;
+            finish(m, half, src[0], src[kWave], request(m, half));
+        }
+    };
+    if (ktiles == 1) {
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < ROWS; r++) s_sum[r * kTileCols + tid] = psum[r];
+        finish_from_lds();
+        return;
+    }
+    if constexpr (ROWS <= 2) {
         float sum[ROWS];
-        uint16_t rin[EPI == kEpiResidual ? ROWS : 1];
-        auto load_residual = [&] {
+        if constexpr (EPI == kEpiQkRope) {
+            if (!splitk_exchange_sum<ROWS>(psum, sum, 0, M, N, ct, kt, ktiles, ct, partials, counters, s_word)) return;
+#pragma unroll
+            for (int r = 0; r < ROWS; r++) s_sum[r * kTileCols + tid] = sum[r];
+            finish_from_lds();
+        } else {
+            // every wave of 64 columns finishes for itself: the epilogue needs nothing from the other waves
+            uint16_t rin[ROWS];
             if constexpr (EPI == kEpiResidual) {
 #pragma unroll
                 for (int r = 0; r < ROWS; r++) rin[r] = res.in[static_cast<size_t>(r < M ? r : M - 1) * N + own_ld];
             }
-        };
-        if constexpr (ROWS >= 4) {
-            // the wide read-back hands out two columns and half of the rows per thread: through LDS (the
-            // reduction buffer, free again) to one column and every row per thread
-            float* s_sum = &red[0][0][0];
-            static_assert(WAVES * MC >= ROWS, "the reduction buffer holds a tile of finished sums");
-            if (ktiles == 1) {
-                load_residual();
-#pragma unroll
-                for (int r = 0; r < ROWS; r++) sum[r] = psum[r];
-            } else {
-                constexpr int HALF = ROWS / 2;
-                float lo[HALF], hi[HALF];
-                if (!splitk_exchange_sum_wide<ROWS>(psum, lo, hi, M, N, ct, kt, ktiles, partials, counters, &s_prev,
-                                                    load_residual)) {
-                    return;
-                }
-                const int row0 = (tid / (kTileCols / 2)) * HALF;
-#pragma unroll
-                for (int i = 0; i < HALF; i++) {
-                    *reinterpret_cast<f32x2*>(&s_sum[(row0 + i) * kTileCols + 2 * (tid % (kTileCols / 2))]) = f32x2{lo[i], hi[i]};
-                }
-                __syncthreads();
-#pragma unroll
-                for (int r = 0; r < ROWS; r++) sum[r] = s_sum[r * kTileCols + tid];
-            }
-        } else if constexpr (EPI == kEpiResidual) {
-            // every wave of 64 columns finishes for itself: the epilogue below needs nothing from the other waves
-            load_residual();
             if (!splitk_exchange_sum_per_wave_rows<ROWS>(psum, sum, M, N, ct, kt, ktiles, partials, counters)) return;
-        } else {
-            if (!splitk_exchange_sum<ROWS>(psum, sum, 0, M, N, ct, kt, ktiles, ct, partials, counters, &s_prev)) return;
-        }
-        if constexpr (EPI == kEpiQkRope) {
-            // The finished rows, rounded to bf16 as a separate GEMV would store them, go through LDS so that a
-            // wave holds elements i and i + 64 of a head in lane i, the layout of the per-head routine.
-            __shared__ uint16_t s_rows[ROWS][kTileCols];
-#pragma unroll
-            for (int r = 0; r < ROWS; r++) s_rows[r][tid] = f32_to_bf16(sum[r]);
-            __syncthreads();
-#pragma unroll
-            for (int i = 0; i < ROPE_ITEMS; i++) {
-                const int item = wave + i * WAVES;
-                const int r = item / 2;
-                const int h = item % 2;
-                if (r < M) {  // the same in every lane of the wave
-                    RopeTarget t = rope;
-                    t.q_out += static_cast<size_t>(r) * rope.n_q * kHeadDim;
-                    t.k_cache += static_cast<size_t>(r) * cache_stride;
-                    t.v_cache += static_cast<size_t>(r) * cache_stride;
-                    qk_norm_rope_head_with(s_rows[r][h * kHeadDim + lane], s_rows[r][h * kHeadDim + lane + 64],
-                                           ct * (kTileCols / kHeadDim) + h, lane, t, rope_pos[i], rope_ga[h], rope_gb[h]);
-                }
-            }
-        } else {
-            // a wave is a quarter of the tile: its sum of squares of every row goes out as it is
             const bool col_ok = own_col < N;
 #pragma unroll
             for (int r = 0; r < ROWS; r++) {
-                float rv = 0.0f;
-                if (col_ok && r < M) {
-                    const float o = bf16_to_f32(f32_to_bf16(sum[r]));  // the projection's output is a bf16 tensor
-                    const uint16_t rbits = f32_to_bf16(bf16_to_f32(rin[r]) + o);
-                    res.out[static_cast<size_t>(r) * N + own_col] = rbits;
-                    rv = bf16_to_f32(rbits);
-                }
-                const float q = wave_sum(rv * rv);
-                if (lane == 0 && r < M) {
-                    res.sumsq[(static_cast<size_t>(r) * gridDim.x + ct) * (kTileCols / kWave) + wave] = q;
+                const uint16_t o = f32_to_bf16(sum[r]);
+                if constexpr (EPI == kEpiStore) {
+                    if (col_ok && r < M) y[static_cast<size_t>(r) * N + own_col] = o;
+                } else {
+                    const uint16_t rbits = f32_to_bf16(bf16_to_f32(rin[r]) + bf16_to_f32(o));
+                    if (col_ok && r < M) res.out[static_cast<size_t>(r) * N + own_col] = rbits;
+                    const float rv = col_ok ? bf16_to_f32(rbits) : 0.0f;
+                    const float q = wave_sum(rv * rv);
+                    if (lane == 0 && r < M) res.sumsq[(static_cast<size_t>(r) * grid.coltiles + ct) * (kTileCols / kWave) + wave] = q;
                 }
             }
         }
-    } else if constexpr (ROWS >= 4) {
-        static_assert(THREADS == kTileCols, "the wide exchange is laid out for 256 threads");
-        splitk_exchange_store_wide<ROWS>(psum, M, N, ct, kt, ktiles, partials, counters, y, &s_prev);
     } else {
-        // one or two activation rows: every wave of 64 columns is an exchange of its own
-        float sum[ROWS];
-        if (!splitk_exchange_sum_per_wave_rows<ROWS>(psum, sum, M, N, ct, kt, ktiles, partials, counters)) return;
-        if (own_col < N) {
+        if constexpr (ROWS >= 8) {
+            if (grid.sliced) {
+                splitk_exchange_sliced<ROWS>(psum, M, N, ct, kt, ktiles, partials, counters, s_word, grid.wait_ticks, request,
+                                             finish);
+                return;
+            }
+        }
+        // the wide read-back hands out two columns and half of the rows per thread
+        constexpr int HALF = ROWS / 2;
+        constexpr int PER_WAVE = 2 * ROWS / WAVES;  // slices a wave finishes below
+        Operands early[PER_WAVE];
+        auto request_all = [&] {
+            if constexpr (EPI != kEpiStore) {
 #pragma unroll
-            for (int r = 0; r < ROWS; r++) {
-                if (r < M) y[static_cast<size_t>(r) * N + own_col] = f32_to_bf16(sum[r]);
+                for (int j = 0; j < PER_WAVE; j++) {
+                    const int i = min(wave + j * WAVES, 2 * M - 1);
+                    early[j] = request(i >> 1, i & 1);
+                }
+            }
+        };
+        float lo[HALF], hi[HALF];
+        if (!splitk_exchange_sum_wide<ROWS>(psum, lo, hi, M, N, ct, kt, ktiles, partials, counters, s_word, request_all)) return;
+        const int row0 = (tid / (kTileCols / 2)) * HALF;
+        const int pair = 2 * (tid % (kTileCols / 2));
+        if constexpr (EPI == kEpiStore) {
+#pragma unroll
+            for (int i = 0; i < HALF; i++) {
+                if (row0 + i < M && ct * kTileCols + pair < N) {
+                    *reinterpret_cast<uint32_t*>(y + static_cast<size_t>(row0 + i) * N + ct * kTileCols + pair) = f32x2_to_bf16x2(lo[i], hi[i]);
+                }
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < HALF; i++) *reinterpret_cast<f32x2*>(&s_sum[(row0 + i) * kTileCols + pair]) = f32x2{lo[i], hi[i]};
+            __syncthreads();
+#pragma unroll
+            for (int j = 0; j < PER_WAVE; j++) {
+                const int i = wave + j * WAVES;
+                const float* src = s_sum + (i >> 1) * kTileCols + (i & 1) * kSliceCols + lane;
+                if (i < 2 * M) finish(i >> 1, i & 1, src[0], src[kWave], early[j]);
             }
         }
     }
 }
 
-template <int WAVES, int KS, int MC, int ROUNDS, int PRO = kProNone, int EPI = kEpiStore>
+template <int WAVES, int KS, int MC, int ROUNDS, int PRO = kProNone, int EPI = kEpiStore, bool LONE = false>
 inline void launch_awq_gemv_mfma(const uint16_t* x, const int32_t* qweight, const uint16_t* scales,
                                  const int32_t* qzeros, uint16_t* y, float* partials, uint32_t* counters,
-                                 int M, int K, int N, int group_shift, int coltiles, int ktiles,
+                                 int M, int K, int N, const MfmaGrid& split,
                                  hipStream_t stream, const FusedInput& fi = FusedInput{},
                                  const ResidualTarget& res = ResidualTarget{}, const RopeTarget& rope = RopeTarget{},
                                  size_t cache_stride = 0) {
-    dim3 grid(coltiles, ktiles, 1);
+
+    const dim3 grid(split.side, split.ktiles, split.coltiles / split.side);
     dim3 block(WAVES * kWave, 1, 1);
-    hipLaunchKernelGGL((awq_gemv_mfma_kernel<WAVES, KS, MC, ROUNDS, PRO, EPI>), grid, block, 0, stream, x,
+    hipLaunchKernelGGL((awq_gemv_mfma_kernel<WAVES, KS, MC, ROUNDS, PRO, EPI, LONE>), grid, block, 0, stream, x,
                        reinterpret_cast<const uint32_t*>(qweight), scales,
                        reinterpret_cast<const uint32_t*>(qzeros), y, partials, counters, M, K, N,
-                       group_shift, ktiles, fi, res, rope, cache_stride);
+                       split, fi, res, rope, cache_stride);
 }
 
 }  // namespace kx

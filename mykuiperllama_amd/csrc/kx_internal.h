@@ -17,7 +17,9 @@ extern "C" {
                                   wherever that applies, several rows on the MFMA kernel */
 #define KX_POLICY_VECTOR 1     /* the vector-ALU kernel with the ordered fp32 exchange (any accepted shape): the sums of
                                   the launches with a prologue or an epilogue, bit for bit */
-#define KX_POLICY_MFMA 2       /* the one-shot MFMA kernel where group size and N allow, else the vector kernel */
+#define KX_POLICY_MFMA 2       /* the one-shot MFMA kernel where N allows, else the vector kernel */
+#define KX_POLICY_MFMA_NO_WAIT 3  /* the same, and workgroups that finish a column tile together give up waiting at once:
+                                  the path a workgroup takes whose neighbours cannot start while it waits */
 
 /* kx_gemv_awq_bf16 with the kernel chosen by the caller. */
 int kx_gemv_awq_bf16_policy(const uint16_t* x, const int32_t* qweight, const uint16_t* scales,

@@ -615,37 +615,140 @@ __device__ __forceinline__ bool splitk_exchange_sum_wide(const float (&psum)[ROW
     return true;
 }
 
-// The wide exchange followed by the plain epilogue: y[m, col] = bf16(sum), two columns per store.
-template <int ROWS>
-__device__ __forceinline__ void splitk_exchange_store_wide(const float (&psum)[ROWS], int M, int N, int ct, int kt,
-                                                           int ktiles, float* __restrict__ partials,
-                                                           uint32_t* __restrict__ counters,
-                                                           uint16_t* __restrict__ y, uint32_t* s_prev) {
+// ---- Several activation rows (ROWS = 4, 8 or 16), a workgroup of 256 threads: the K tiles finish together ----
+//
+// With M rows a K tile leaves M * 1 KB of partial sums per column tile, and one workgroup that reads them all back is
+// the longest part of the launch (down 12288 -> 4096 at M = 16: 24 K tiles, 393 KB, about 8 us).  So every workgroup
+// of a column tile takes a share of the read-back: a slice is one activation row of one head-sized half of the tile
+// (128 columns), slice i goes to K tile i % ktiles, and a workgroup that has left its partial sums waits until all K
+// tiles have, then finishes its slices.  Measured: make_mfma_plan in kx_awq_gemv.hip.
+//
+// The counter word of a tile holds arrivals in its low half and departures in its high half; the last workgroup to
+// depart clears it.  Ordering as in the header: partial sums are acknowledged before the arrival, read after it.
+//
+// Waiting must not rest on the other workgroups being resident: another kernel may hold their place, or the grid may
+// be larger than the chip.  The wait is bounded (kSliceWaitTicks); a workgroup that gives up sets the bit of its K
+// tile in the tile's mask word and leaves, and the workgroup that arrives last takes over the marked slices.  Whoever
+// gives up looks at the arrivals once more after its mark is in memory, and whoever arrives last looks at the mask
+// after its arrival is: one of the two sees the other, and the bit, cleared by an atomic that returns it, decides who
+// finishes the slices.
+constexpr int kSliceCols = 128;
+constexpr int kSliceMaxKTiles = 64;           // bits of the mask word
+constexpr uint32_t kSliceDeparture = 0x10000u;
+constexpr uint32_t kSliceWaitTicks = 2000;    // of the 100 MHz clock: 20 us, ten times a launch's whole exchange
+
+// Columns col0 (lane) and col0 + 64 of activation row m, all K tiles in order; sixteen K tiles in flight.
+__device__ __forceinline__ void splitk_slice_sum(__amdgpu_buffer_rsrc_t rsrc, int M, int N, int ktiles, int m, int col_a,
+                                                 int col_b, float* a, float* b) {
+    constexpr int TB = 16;
+    const uint32_t tfloats = static_cast<uint32_t>(M) * static_cast<uint32_t>(N);
+    const uint32_t row = static_cast<uint32_t>(m) * static_cast<uint32_t>(N);
+    float sa = 0.0f, sb = 0.0f;
+    for (int t0 = 0; t0 < ktiles; t0 += TB) {
+        float va[TB], vb[TB];
+#pragma unroll
+        for (int u = 0; u < TB; u++) {
+            // clamped address, masked value: the loads of a batch are straight-line code
+            const int t = t0 + u;
+            const uint32_t at = static_cast<uint32_t>(t < ktiles ? t : ktiles - 1) * tfloats + row;
+            const float ga = load_partial(rsrc, col_a * static_cast<int>(sizeof(float)), at);
+            const float gb = load_partial(rsrc, col_b * static_cast<int>(sizeof(float)), at);
+            va[u] = t < ktiles ? ga : 0.0f;
+            vb[u] = t < ktiles ? gb : 0.0f;
+        }
+#pragma unroll
+        for (int u = 0; u < TB; u++) {
+            sa += va[u];
+            sb += vb[u];
+        }
+    }
+    *a = sa;
+    *b = sb;
+}
+
+// `psum[r]`: the thread's column (tid) of activation row r.  `finish(m, half, a, b, request(m, half))` is called by whole
+// waves, once per (row m < M, half of the tile) in the whole launch, with the finished sums of columns 128 half + lane
+// (`a`) and 64 further (`b`), and the loads that `request` issued ahead of the read-back; columns past N bring garbage.
+// More than one K tile.  `s_word`: three uint32 of LDS.
+template <int ROWS, class Request, class Finish>
+__device__ __forceinline__ void splitk_exchange_sliced(const float (&psum)[ROWS], int M, int N, int ct, int kt, int ktiles,
+                                                       float* __restrict__ partials, uint32_t* __restrict__ counters,
+                                                       uint32_t* s_word, uint32_t wait_ticks, Request&& request,
+                                                       Finish&& finish) {
     const int tid = threadIdx.x;
-    if (ktiles == 1) {
-        const int col = ct * kTileCols + tid;
-        if (col < N) {
+    const int lane = tid % kWave;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    constexpr int WAVES = kTileCols / kWave;
+    const int col = ct * kTileCols + tid;
+    const size_t tstride = static_cast<size_t>(M) * N;
+    if (col < N) {
 #pragma unroll
-            for (int r = 0; r < ROWS; r++) {
-                if (r < M) y[static_cast<size_t>(r) * N + col] = f32_to_bf16(psum[r]);
-            }
-        }
-        return;
-    }
-    constexpr int HALF = ROWS / 2;
-    float lo[HALF], hi[HALF];
-    if (!splitk_exchange_sum_wide<ROWS>(psum, lo, hi, M, N, ct, kt, ktiles, partials, counters, s_prev, [] {})) return;
-    const int row0 = __builtin_amdgcn_readfirstlane(tid / (kTileCols / 2)) * HALF;
-    const unsigned col2 = static_cast<unsigned>(ct * kTileCols + 2 * (tid % (kTileCols / 2)));
-    if (col2 < static_cast<unsigned>(N)) {
-#pragma unroll
-        for (int i = 0; i < HALF; i++) {
-            const int m = row0 + i;
-            if (m < M) {
-                *reinterpret_cast<uint32_t*>(y + static_cast<size_t>(m) * N + col2) = f32x2_to_bf16x2(lo[i], hi[i]);
-            }
+        for (int r = 0; r < ROWS; r++) {
+            if (r < M) store_agent(partials + static_cast<size_t>(kt) * tstride + static_cast<size_t>(r) * N + col, psum[r]);
         }
     }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    uint32_t* counter = counters + static_cast<size_t>(ct) * kCountersPerTile * kCounterStride;
+    unsigned long long* mask = reinterpret_cast<unsigned long long*>(counter + kCounterStride);  // on the tile's next line
+    const uint32_t all = static_cast<uint32_t>(ktiles);
+    const int slices = 2 * M;
+    const __amdgpu_buffer_rsrc_t rsrc = partials_buffer(partials, static_cast<size_t>(ktiles) * tstride);
+
+    auto finish_slices_of = [&](int owner) {
+        for (int i = wave; owner + i * ktiles < slices; i += WAVES) {
+            const int slice = owner + i * ktiles;
+            const int m = slice >> 1, half = slice & 1;
+            const int ca = ct * kTileCols + half * kSliceCols + lane;
+            const int cb = ca + kWave;
+            const auto operands = request(m, half);
+            float a, b;
+            splitk_slice_sum(rsrc, M, N, ktiles, m, ca < N ? ca : N - 1, cb < N ? cb : N - 1, &a, &b);
+            finish(m, half, a, b, operands);
+        }
+    };
+
+    if (tid == 0) {
+        // s_word[0]: whether this workgroup finishes its slices; s_word[1], [2]: K tiles whose slices it takes over
+        const uint32_t before = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) % kSliceDeparture;
+        const bool last = before == all - 1;
+        bool mine = kt < slices;
+        unsigned long long over = 0;
+        if (last) {
+            over = __hip_atomic_load(mask, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // usually nothing
+            if (over) over = __hip_atomic_exchange(mask, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        } else if (mine) {
+            auto arrived = [&] {
+                return __hip_atomic_load(counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) % kSliceDeparture == all;
+            };
+            const uint64_t began = __builtin_amdgcn_s_memrealtime();
+            mine = arrived();
+            while (!mine && __builtin_amdgcn_s_memrealtime() - began < wait_ticks) mine = arrived();
+            if (!mine) {
+                const unsigned long long bit = 1ull << kt;
+                const unsigned long long seen = __hip_atomic_fetch_or(mask, bit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                asm volatile("" ::"v"(seen));
+                __builtin_amdgcn_s_waitcnt(0);
+                compiler_fence();
+                if (arrived()) mine = (__hip_atomic_fetch_and(mask, ~bit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & bit) != 0;
+            }
+        }
+        s_word[0] = mine ? 1u : 0u;
+        s_word[1] = static_cast<uint32_t>(over);
+        s_word[2] = static_cast<uint32_t>(over >> 32);
+    }
+    __syncthreads();
+    compiler_fence();  // the read-back below stays behind the arrivals
+    // Departing before the read-back keeps the counter's trip out of the launch's tail; the last to depart leaves the
+    // counter ready for the next launch (nobody looks at it any more).
+    uint32_t departed = 0;
+    if (tid == 0) departed = __hip_atomic_fetch_add(counter, kSliceDeparture, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (s_word[0]) finish_slices_of(kt);
+    for (unsigned long long left = s_word[1] | (static_cast<unsigned long long>(s_word[2]) << 32); left; left &= left - 1) {
+        finish_slices_of(__ffsll(left) - 1);
+    }
+    if (tid == 0 && departed / kSliceDeparture == all - 1) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 }  // namespace kx
