@@ -3,8 +3,8 @@
 // One or two activation rows: one wave per output row, the 64 lanes walk the row in 16-byte pieces
 // (eight bf16 each), pairs along K go through the packed bf16 dot instruction with an fp32
 // accumulator, and the lanes meet in a wave-wide sum at the end.  Rows are contiguous, so every load
-// is a full 1 KiB per wave.  Three to sixteen rows: matrix cores, sixteen output rows per workgroup
-// (second kernel below).
+// is a full 1 KiB per wave.  Several rows: matrix cores, the activations held in registers while a workgroup walks over
+// blocks of output rows (third kernel below), or, for K > 8192, sixteen output rows per workgroup (second kernel).
 #include "kx_common.h"
 
 namespace kx {
@@ -186,6 +186,121 @@ __global__ __launch_bounds__(kMfmaWaves * kWave) void bf16_gemv_mfma_kernel(
     }
 }
 
+// Two to sixteen activation rows, K <= 1024 * UNITS: one workgroup per compute unit walks over blocks of sixteen output
+// columns, and its eight waves split K.  What bounded the kernel above was not W but everything round it: the
+// activation rows came out of L2 anew for every 64 columns, and an MFMA operand fetched straight from memory asks for
+// 64 bytes of sixteen rows at a time, which the memory system answers at three quarters of its rate.  Here the A operands
+// of a wave's part of K stay in registers for the life of the workgroup, and W goes through LDS: a unit is 128 elements
+// of the block's sixteen rows (4 KB, four loads of 4 rows x 256 bytes), loaded straight into the wave's own ring of
+// kRing units, so that no barrier and no register stands between the stream and the MFMAs and 128 KB per compute unit
+// are in flight.  The waves of a block meet in LDS, two buffers in turn, one barrier per block that leaves loads alone.
+// A row of a unit is stored with its 16-byte pieces permuted by the low bits of the row (the lane that loads piece j of
+// row r fetches piece j ^ (r & 7)), so that the sixteen rows that an operand read touches lie in different banks.
+// us at M = 3 / 8 / 16, kernel above -> this one: lm_head 151936 x 4096 273 / 308 / 297 -> 182 / 189 / 199 (W alone at the
+// read rate of a large buffer: 171), 151936 x 5120 382 / 447 / 405 -> 231 / 240 / 254, 4096 x 4096 11.4 / 12.1 / 26.3 ->
+// 9.1 / 9.2 / 10.5.
+// EXACT: K is 1024 * UNITS; otherwise what lies past K is zeroed in both operands.
+constexpr int kHeldWaves = 8;
+constexpr int kRing = 4;
+constexpr int kUnitBytes = 16 * 256;
+
+template <int UNITS, bool EXACT>
+__global__ __launch_bounds__(kHeldWaves * kWave, 2) void bf16_gemv_held_kernel(
+    const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, uint16_t* __restrict__ y, int M, int K, int N, int blocks) {
+    __shared__ __attribute__((aligned(1024))) char ring[kHeldWaves][kRing][kUnitBytes];
+    __shared__ __attribute__((aligned(16))) float red[2][kHeldWaves][4][kWave];
+    const int tid = threadIdx.x;
+    const int lane = tid % kWave;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int c = lane % 16;
+    const int b = lane / 16;
+    const int kw = wave * 128 * UNITS;  // the wave's first element of K
+    const int stride = gridDim.x;
+
+    bf16x8 held[UNITS][4];
+    const uint16_t* xrow = x + static_cast<size_t>(min(c, M - 1)) * K;
+#pragma unroll
+    for (int u = 0; u < UNITS; u++) {
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int k = kw + 128 * u + 32 * q + 8 * b;
+            const bool in = EXACT || k < K;
+            const u32x4 v = *reinterpret_cast<const u32x4*>(xrow + (in ? k : 0));
+            const bool live = in && c < M;
+            held[u][q] = as_bf16x8(live ? v.x : 0u, live ? v.y : 0u, live ? v.z : 0u, live ? v.w : 0u);
+        }
+    }
+
+    // Loads unit u of a block into a ring slot: load i brings rows 4 i + lane / 16.
+    auto fetch = [&](int block, int u, int slot) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int r = 4 * i + b;
+            const int k = kw + 128 * u + 8 * (c ^ (r & 7));
+            const uint16_t* src = w + static_cast<size_t>(min(16 * block + r, N - 1)) * K + (EXACT || k < K ? k : 0);
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                             (__attribute__((address_space(3))) void*)(&ring[wave][slot][i * 1024]), 16, 0, 2);
+        }
+    };
+    // Where the lane finds its operand of step q: row c, piece 4 q + b; steps 2 and 3 lie 128 bytes behind 0 and 1.
+    const uint32_t ring0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
+        (__attribute__((address_space(3))) char*)(&ring[wave][0][0])));
+    const uint32_t at0 = ring0 + c * 256 + ((b ^ (c & 7)) * 16);
+    const uint32_t at1 = ring0 + c * 256 + (((4 + b) ^ (c & 7)) * 16);
+
+    const int first = blockIdx.x;
+#pragma unroll
+    for (int j = 0; j < kRing; j++) {
+        const int block = first + (j / UNITS) * stride;
+        if (block < blocks) fetch(block, j % UNITS, j);
+    }
+    int slot = 0, turn = 0;
+    for (int block = first; block < blocks; block += stride, turn ^= 1) {
+        f32x4v acc[2];
+        acc[0] = acc[1] = f32x4v{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int u = 0; u < UNITS; u++) {
+            // The unit kRing places further on will take this slot.  Loads return in order: with it to come, kRing - 1
+            // units may still be on their way when this one has arrived; in the last ring, wait for everything.
+            const int next = block + ((u + kRing) / UNITS) * stride;
+            const int held_back = block + ((u + kRing - 1) / UNITS) * stride;
+            if (held_back < blocks) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(4 * (kRing - 1)) : "memory");
+            else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            u32x4 v[4];
+            const uint32_t s0 = at0 + slot * kUnitBytes, s1 = at1 + slot * kUnitBytes;
+            // in assembly, because the compiler would wait for every load in flight ahead of a read of the ring
+            asm volatile("ds_read_b128 %0, %4\n\tds_read_b128 %1, %5\n\tds_read_b128 %2, %4 offset:128\n\tds_read_b128 %3, %5 offset:128\n\ts_waitcnt lgkmcnt(0)"
+                         : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3])
+                         : "v"(s0), "v"(s1)
+                         : "memory");
+            if (next < blocks) fetch(next, (u + kRing) % UNITS, slot);
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                u32x4 p = v[q];
+                if constexpr (!EXACT) {
+                    const bool live = kw + 128 * u + 32 * q + 8 * b < K;
+                    p = u32x4{live ? p.x : 0u, live ? p.y : 0u, live ? p.z : 0u, live ? p.w : 0u};
+                }
+                acc[q & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(held[u][q], as_bf16x8(p.x, p.y, p.z, p.w), acc[q & 1], 0, 0, 0);
+            }
+            slot = (slot + 1) % kRing;
+        }
+#pragma unroll
+        for (int v = 0; v < 4; v++) red[turn][wave][v][lane] = acc[0][v] + acc[1][v];
+        lds_barrier();
+        if (tid < 4 * kWave) {  // thread (v, lane): row 4 (lane / 16) + v of column lane % 16
+            const float* src = &red[turn][0][0][0] + tid;
+            float part[kHeldWaves];
+#pragma unroll
+            for (int u = 0; u < kHeldWaves; u++) part[u] = src[u * 4 * kWave];
+            const float sum = ((part[0] + part[1]) + (part[2] + part[3])) + ((part[4] + part[5]) + (part[6] + part[7]));
+            const int m = 4 * b + tid / kWave;
+            const int n = 16 * block + c;
+            if (m < M && n < N) y[static_cast<size_t>(m) * N + n] = f32_to_bf16(sum);
+        }
+    }
+}
+
 }  // namespace
 }  // namespace kx
 
@@ -200,9 +315,33 @@ extern "C" int kx_gemv_bf16(const uint16_t* x, const uint16_t* w, uint16_t* y, i
         return KX_ERR_ALIGNMENT;
     }
     hipStream_t s = kx::as_stream(stream);
+    constexpr int kReach = 128 * kx::kHeldWaves;  // elements of K that a unit of every wave covers
+    // Two rows share the vector kernel's loads well enough where W is small (4096 x 4096: 8.4 against 9.0 us, 151936 x
+    // 1024: 52 against 57); with eight blocks per compute unit and rows of 8 KB its wave sums no longer hide (151936 x
+    // 4096: 202 against 182).
+    if ((M >= 3 || (M == 2 && K >= 4096 && N >= 32768)) && K <= 8 * kReach) {
+        const int blocks = (N + 15) / 16;
+        const dim3 grid(blocks < 256 ? blocks : 256), block(kx::kHeldWaves * kx::kWave);
+#define KX_HELD(U)                                                                                                      \
+    do {                                                                                                                \
+        if (K == U * kReach) hipLaunchKernelGGL((kx::bf16_gemv_held_kernel<U, true>), grid, block, 0, s, x, w, y, M, K, N, blocks); \
+        else hipLaunchKernelGGL((kx::bf16_gemv_held_kernel<U, false>), grid, block, 0, s, x, w, y, M, K, N, blocks);     \
+    } while (0)
+        switch ((K + kReach - 1) / kReach) {
+            case 1: KX_HELD(1); break;
+            case 2: KX_HELD(2); break;
+            case 3: KX_HELD(3); break;
+            case 4: KX_HELD(4); break;
+            case 5: KX_HELD(5); break;
+            case 6: KX_HELD(6); break;
+            case 7: KX_HELD(7); break;
+            default: KX_HELD(8); break;
+        }
+#undef KX_HELD
+        return kx::launch_status();
+    }
     if (M >= 3) {
-        // One pass on the matrix cores; the vector kernel, whose every wave reads the activation rows for
-        // itself, needs 310 us on lm_head 151936 x 4096 for four rows and a pass over W per four rows beyond that.
+        // K > 8192: the activations of a wave's part do not fit its registers
         if (M <= 8) {
             hipLaunchKernelGGL((kx::bf16_gemv_mfma_kernel<1, 8>), dim3((N + 15) / 16), dim3(kx::kMfmaWaves * kx::kWave), 0,
                                s, x, w, y, M, K, N);
