@@ -11,6 +11,7 @@ namespace {
 
 struct AwqPlan {
     bool mfma;     // matrix-core kernel or the VALU kernel
+    int walk;      // MFMA kernel: blocks of K that a workgroup walks over
     bool sliced;   // MFMA kernel: all workgroups of a column tile finish it together
     int waves;     // waves per workgroup stacked along K (4, 8 or 16)
     int rt;        // VALU kernel: consecutive rows per lane (8 or 16); MFMA kernel: 32-row steps per wave
@@ -40,7 +41,14 @@ constexpr int kExchangeRows = 8;    // what a K tile's share of the split-K exch
 //            17.4 / 17.4 -> 12.9 / 14.1.  Larger grids, whose workgroups come in rounds, keep the single reader: with
 //            shares the early ones would hold the places the late ones need (gate|up 4096 -> 24576 at M = 16: 19.7
 //            against 21.5 us), and so do their column-tile-fastest order and 256 / 512 rows per workgroup.
-inline AwqPlan make_mfma_plan(int M, int K, int N, int group) {
+//            Unless K is long as well, more than 16 blocks of 512 rows (32 up to eight rows, and behind a prologue,
+//            whose operands sixteen rows cannot load ahead): then the partial sums outweigh that, and a workgroup
+//            walks over as many blocks as bring the grid down to two per compute unit.  us per launch, single reader
+//            -> walk: 25600 -> 5120 (50 blocks) at M = 5 / 8 / 12 / 16 27.1 / 27.7 / 36.1 / 36.6 -> 22.2 / 22.4 / 24.1 /
+//            24.3, behind SwiGLU at M = 5 / 16 29.0 / 40.3 -> 22.2 / 34.2.  With fewer blocks the walk loses: 12288
+//            -> 8192 (24) at M = 5 / 16 20.3 / 24.7 -> 21.4 / 23.2, behind SwiGLU 21.1 / 27.5 -> 22.7 / 31.8; 4096 ->
+//            24576 (8) 17.8 / 19.9 -> 19.7 / 23.6; 5120 -> 51200 (10) 42.4 / 48.3 -> 43.4 / 50.6.
+inline AwqPlan make_mfma_plan(int M, int K, int N, int group, bool allow_walk = true, bool produced_x = false) {
     AwqPlan p;
     p.mfma = true;
     p.coltiles = (N / 8 + kWC - 1) / kWC;
@@ -53,6 +61,7 @@ inline AwqPlan make_mfma_plan(int M, int K, int N, int group) {
     if (M <= 4 && ktiles_with(2) > 16 && ktiles_with(2) <= 32) ks = 4;
     while (!allowed(ks)) ks /= 2;
     p.sliced = false;
+    p.walk = 1;
     if (M >= 5) {
         int best = 0;  // the longest run that is allowed, or the shortest that is short enough
         for (int c = 4; c >= 1; c /= 2) {
@@ -62,16 +71,27 @@ inline AwqPlan make_mfma_plan(int M, int K, int N, int group) {
         if (kt > 1 && kt <= kSliceMaxKTiles && p.coltiles * kt <= 2 * kComputeUnits) {
             p.sliced = true;
             ks = best;
+        } else if (allow_walk && allowed(4) && ktiles_with(4) > (M >= 9 && !produced_x ? 16 : 32)) {
+            const int blocks = ktiles_with(4);
+            int walk = 2;
+            while (walk < blocks && p.coltiles * ((blocks + walk - 1) / walk) > 2 * kComputeUnits) walk++;
+            const int left = (blocks + walk - 1) / walk;
+            if (left > 1 && left <= kSliceMaxKTiles && p.coltiles * left <= 2 * kComputeUnits) {
+                p.sliced = true;
+                p.walk = (blocks + left - 1) / left;
+                ks = 4;
+            }
         }
     }
     p.rt = ks;  // steps per wave
-    p.ktiles = ktiles_with(ks);
+    p.ktiles = (ktiles_with(ks) + p.walk - 1) / p.walk;
     return p;
 }
 
 inline AwqPlan make_valu_plan(int M, int K, int N, bool allow_long_rows = true, bool allow_12_waves = true) {
     AwqPlan p;
     p.mfma = p.sliced = false;
+    p.walk = 1;
     p.coltiles = (N / 8 + kWC - 1) / kWC;
     p.mb = M >= 8 ? 8 : (M >= 4 ? 4 : (M >= 2 ? 2 : 1));
     p.mtiles = (M + p.mb - 1) / p.mb;
@@ -134,6 +154,7 @@ constexpr int kFixedExchangeRows = 4;
 inline AwqPlan make_fixed_plan(int K, int N) {
     AwqPlan p{};
     p.mfma = p.sliced = false;
+    p.walk = 1;
     p.coltiles = (N / 8 + kWC - 1) / kWC;
     p.mb = 1;
     p.mtiles = 1;
@@ -179,6 +200,7 @@ inline MfmaGrid mfma_grid(const AwqPlan& p, int group) {
         while (p.coltiles % g.side != 0) g.side--;
     }
     g.sliced = p.sliced;
+    g.walk = p.walk;
     g.wait_ticks = kSliceWaitTicks;
     g.group_magic = gs == 1 ? 0u : static_cast<uint32_t>(((1ull << 32) + gs - 1) / gs);
     return g;
@@ -259,6 +281,13 @@ void launch_mfma_fused(const AwqPlan& p, const FusedInput& fi, const ResidualTar
         else if (M <= 8) launch_awq_gemv_mfma<4, KS, 8, 1, PRO, EPI>(KX_MARGS);      \
         else launch_awq_gemv_mfma<4, KS, 8, 2, PRO, EPI>(KX_MARGS);                  \
     } while (0)
+    if constexpr (PRO != kProPreNorm && EPI != kEpiQkRope) {
+        if (p.walk > 1) {
+            if (M <= 8) launch_awq_gemv_mfma<4, 4, 8, 1, PRO, EPI, false, true>(KX_MARGS);
+            else launch_awq_gemv_mfma<4, 4, 8, 2, PRO, EPI, false, true>(KX_MARGS);
+            return;
+        }
+    }
     if (p.rt == 4) KX_MFMA_BY_M(4);
     else if (p.rt == 2) KX_MFMA_BY_M(2);
     else KX_MFMA_BY_M(1);
@@ -452,6 +481,17 @@ extern "C" int kx_gemv_awq_bf16_policy(const uint16_t* x, const int32_t* qweight
         kx::MfmaGrid grid = kx::mfma_grid(p, group_size);
         if (policy == KX_POLICY_MFMA_NO_WAIT) grid.wait_ticks = 0;
 #define KX_MARGS x, qweight, scales, qzeros, y, partials, counters, M, K, N, grid, s
+#define KX_MFMA_WALK(LONE)                                                                                         \
+    do {                                                                                                            \
+        if (M <= 8) kx::launch_awq_gemv_mfma<4, 4, 8, 1, kx::kProNone, kx::kEpiStore, LONE, true>(KX_MARGS);        \
+        else kx::launch_awq_gemv_mfma<4, 4, 8, 2, kx::kProNone, kx::kEpiStore, LONE, true>(KX_MARGS);               \
+    } while (0)
+        if (p.walk > 1) {
+            if (N % 16) KX_MFMA_WALK(true);
+            else KX_MFMA_WALK(false);
+            return kx::launch_status();
+        }
+#undef KX_MFMA_WALK
 #define KX_MFMA_ROWS(KS, LONE)                                                                                \
     do {                                                                                                       \
         if (M == 1) kx::launch_awq_gemv_mfma<4, KS, 1, 1, kx::kProNone, kx::kEpiStore, LONE>(KX_MARGS);        \
@@ -508,7 +548,7 @@ extern "C" int kx_gemv_awq_swiglu_bf16(const uint16_t* gate, const uint16_t* up,
     // Several rows go to the matrix cores, as in kx_gemv_awq_bf16, when gate and up can be read 16 bytes at a time
     if (M >= 2 && (N % 16) == 0 && kx::aligned_to(gate, 16) && kx::aligned_to(up, 16) &&
         (act_ld % 8) == 0) {
-        const kx::AwqPlan mp = kx::make_mfma_plan(M, K, N, group_size);
+        const kx::AwqPlan mp = kx::make_mfma_plan(M, K, N, group_size, true, true);
         float* partials = nullptr;
         uint32_t* counters = nullptr;
         rc = kx::resolve_workspace(mp, M, N, workspace, workspace_bytes, &partials, &counters);
@@ -832,7 +872,9 @@ extern "C" int kx_gemv_awq_chain_bf16(const kx_chain_desc* d, const int32_t* qwe
     if (d->in_kind == KX_IN_ATTN && (K % kx::kHeadDim) != 0) return KX_ERR_BAD_SHAPE;
 
     if (rows > 1) {
-        const kx::AwqPlan mp = kx::make_mfma_plan(rows, K, N, group_size);
+        const kx::AwqPlan mp = kx::make_mfma_plan(rows, K, N, group_size,
+                                                   d->in_kind != KX_IN_NORM && d->out_kind != KX_OUT_QKV_ROPE,
+                                                   d->in_kind != KX_IN_ROW);
         float* partials = nullptr;
         uint32_t* counters = nullptr;
         rc = kx::resolve_workspace(mp, rows, N, workspace, workspace_bytes, &partials, &counters);

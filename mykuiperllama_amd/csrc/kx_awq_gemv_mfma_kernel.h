@@ -88,6 +88,7 @@ struct MfmaGrid {
     int coltiles;
     int ktiles;
     int side;              // column tiles side by side in the grid (gridDim.x, whose own load is a trip to memory)
+    int walk;              // blocks of K a workgroup walks over, one behind the other (WALK)
     int sliced;            // all K tiles of a column tile finish it together (splitk_exchange_sliced)
     uint32_t group_magic;  // ceil(2^32 / (G / 32)), 0 for groups of 32
     uint32_t wait_ticks;   // how long a workgroup waits for the others of its tile
@@ -100,9 +101,11 @@ __device__ __forceinline__ int group_of_step(const MfmaGrid& g, int step) {
 
 // KS: consecutive 32-row steps per wave (they must share a quantisation group);
 // MC: activation rows a workgroup reduces per LDS round (1, 2, 4 or 8); ROUNDS: 2 for M > 8, else 1;
+// WALK: a workgroup works through grid.walk blocks of KB rows of K, one behind the other, and adds their sums up in
+// registers (make_mfma_plan says when; carrying the loop costs the other launches up to a microsecond);
 // LONE: N is an odd multiple of eight (a template parameter: the moves cost 20 registers, an occupancy step).
 // With a prologue, `x` is not read: fi.a / fi.b (/ fi.gain) are 16-byte aligned, fi.ld a multiple of eight.
-template <int WAVES, int KS, int MC, int ROUNDS, int PRO = kProNone, int EPI = kEpiStore, bool LONE = false>
+template <int WAVES, int KS, int MC, int ROUNDS, int PRO = kProNone, int EPI = kEpiStore, bool LONE = false, bool WALK = false>
 __global__ __launch_bounds__(WAVES * kWave, 2) void awq_gemv_mfma_kernel(
     const uint16_t* __restrict__ x, const uint32_t* __restrict__ qweight,
     const uint16_t* __restrict__ scales, const uint32_t* __restrict__ qzeros,
@@ -112,11 +115,16 @@ __global__ __launch_bounds__(WAVES * kWave, 2) void awq_gemv_mfma_kernel(
     constexpr int WROWS = KS * kStepRows;  // rows of K per wave
     constexpr int KB = WAVES * WROWS;      // rows of K per workgroup
     constexpr int ROWS = MC * ROUNDS;      // activation rows this kernel carries (>= M)
+    static_assert(!WALK || (KS == 4 && ROWS >= 8), "the launches that walk");
     constexpr int THREADS = WAVES * kWave;
     static_assert(THREADS >= kTileCols, "one thread per tile column");
     static_assert(PRO == kProNone || PRO == kProSwiGLU || PRO == kProPreNorm, "prologues of the matrix-core kernel");
     static_assert(EPI == kEpiStore || EPI == kEpiResidual || EPI == kEpiQkRope, "epilogues of the matrix-core kernel");
     constexpr bool STAGED = PRO != kProNone;
+    // The loads of the next block go out while the waves of this one meet, except at sixteen rows behind a prologue, whose
+    // operands do not fit the registers beside the weights and the sums: there the other workgroup of the compute unit
+    // has to cover the gap.
+    constexpr bool AHEAD = PRO == kProNone || ROUNDS == 1;
     // A staged row is the workgroup's K range plus 16 bytes, so that the rows a wave reads together
     // start in different banks.
     constexpr int XPITCH = KB + 8;
@@ -142,41 +150,29 @@ __global__ __launch_bounds__(WAVES * kWave, 2) void awq_gemv_mfma_kernel(
     const int ktiles = grid.ktiles;
     const int nw = N >> 3;
 
-    const int kwave = kt * KB + wave * WROWS;  // first row of this wave
+    // first row of the block that is loaded next, and how many blocks the workgroup has
+    int kblock = kt * KB * (WALK ? grid.walk : 1);
+    const int blocks = WALK ? min(grid.walk, (K - kblock + KB - 1) / KB) : 1;
 
     // ---- operands of the activation prologue go out first: they are small, mostly cached, and the prologue
     // should run while the weights are still on their way ----
     // Piece e = tid + i * THREADS of the workgroup is (row e / KPIECES, elements 8 (e % KPIECES) .. + 7 of
-    // the K range); addresses are clamped, what a clamped load brings is replaced by zeros.
+    // the block); addresses are clamped, what a clamped load brings is replaced by zeros.
     uint4 pa[STAGED ? PPT : 1], pb[STAGED ? PPT : 1];
     float tile_ss[PRO == kProPreNorm ? (ROWS + WAVES - 1) / WAVES : 1];
-    if constexpr (STAGED) {
+    if constexpr (PRO == kProPreNorm) {
+        // wave w adds the tiles of rows w, w + WAVES, ...: lane = tile
 #pragma unroll
-        for (int i = 0; i < PPT; i++) {
-            const int e = tid + i * THREADS;
-            const int pm = e / KPIECES;
-            const int k = kt * KB + 8 * (e % KPIECES);
-            const int mc = pm < M ? pm : M - 1;
-            const int kc = k < K ? k : K - 8;
-            const size_t at = static_cast<size_t>(mc) * fi.ld + kc;
-            pa[i] = *reinterpret_cast<const uint4*>(fi.a + at);
-            if constexpr (PRO == kProSwiGLU) pb[i] = *reinterpret_cast<const uint4*>(fi.b + at);
-            else pb[i] = *reinterpret_cast<const uint4*>(fi.gain + kc);
-        }
-        if constexpr (PRO == kProPreNorm) {
-            // wave w adds the tiles of rows w, w + WAVES, ...: lane = tile
-#pragma unroll
-            for (int rr = 0; rr < (ROWS + WAVES - 1) / WAVES; rr++) {
-                const int m = wave + rr * WAVES;
-                const int mc = m < M ? m : M - 1;
-                const f32x4 qs = reinterpret_cast<const f32x4*>(fi.sumsq)[static_cast<size_t>(mc) * fi.sumsq_parts +
-                                                                          (lane < fi.sumsq_parts ? lane : fi.sumsq_parts - 1)];
-                tile_ss[rr] = ((qs.x + qs.y) + qs.z) + qs.w;  // the order that defines a tile's sum
-            }
+        for (int rr = 0; rr < (ROWS + WAVES - 1) / WAVES; rr++) {
+            const int m = wave + rr * WAVES;
+            const int mc = m < M ? m : M - 1;
+            const f32x4 qs = reinterpret_cast<const f32x4*>(fi.sumsq)[static_cast<size_t>(mc) * fi.sumsq_parts +
+                                                                      (lane < fi.sumsq_parts ? lane : fi.sumsq_parts - 1)];
+            tile_ss[rr] = ((qs.x + qs.y) + qs.z) + qs.w;  // the order that defines a tile's sum
         }
     }
 
-    // ---- loads, all issued before anything is consumed ----
+    // ---- loads of a block, all issued before anything is consumed ----
     // Every load is unconditional: an address that would fall outside is clamped to one inside, and
     // what it brings is either masked (activations) or lands in outputs that are never stored
     // (columns past N).  A load under a condition becomes a branch with a full wait behind it, and
@@ -189,27 +185,10 @@ __global__ __launch_bounds__(WAVES * kWave, 2) void awq_gemv_mfma_kernel(
     const int own_ld = own_col < N ? own_col : N - 1;
     uint16_t s_bits[WAVES];
     uint32_t z_word[WAVES];
-#pragma unroll
-    for (int wv = 0; wv < WAVES; wv++) {
-        const int krow = kt * KB + wv * WROWS;
-        const int g = group_of_step(grid, (krow < K ? krow : K - 1) / kStepRows);  // rows past K meet zero activations
-        s_bits[wv] = scales[static_cast<size_t>(g) * N + own_ld];
-        z_word[wv] = qzeros[static_cast<size_t>(g) * nw + (own_ld >> 3)];
-    }
     // The A operand: row c of the activations, whether or not column slot c holds weights.  Rows
     // past M and steps past K (K is a multiple of 32: a step is all in or all out) are zeros.
     uint4 xa[KS];
     const int x_row = c < M ? c : M - 1;
-    if constexpr (!STAGED) {
-#pragma unroll
-        for (int ks = 0; ks < KS; ks++) {
-            const int kstep = kwave + ks * kStepRows;
-            const int kld = kstep < K ? kstep : K - kStepRows;
-            const uint4 got = *reinterpret_cast<const uint4*>(x + static_cast<size_t>(x_row) * K + kld + 8 * b);
-            const bool live = c < M && kstep < K;
-            xa[ks] = make_uint4(live ? got.x : 0u, live ? got.y : 0u, live ? got.z : 0u, live ? got.w : 0u);
-        }
-    }
     // The lane's two word columns, eight rows per step, both words in one load, of four-byte alignment where the
     // number of words is odd; the last lane's one word then comes as the second of its pair and is moved over.
     using word_pair = typename WordPair<LONE>::type;
@@ -217,18 +196,55 @@ __global__ __launch_bounds__(WAVES * kWave, 2) void awq_gemv_mfma_kernel(
     const int wc_first = ct * 32 + 2 * c;
     const int wc0 = max(0, min(wc_first, nw - 2));
     const bool lone_word = wc_first == nw - 1;
+    auto load_operands = [&] {
+        if constexpr (STAGED) {
 #pragma unroll
-    for (int ks = 0; ks < KS; ks++) {
-        const int kstep = kwave + ks * kStepRows;
-        const int k0 = (kstep < K ? kstep : K - kStepRows) + 8 * b;  // first of the lane's eight rows
-        const uint32_t* wp = qweight + static_cast<size_t>(k0) * nw + wc0;
-#pragma unroll
-        for (int r = 0; r < 8; r++) {
-            const u32x2 v = __builtin_nontemporal_load(reinterpret_cast<const word_pair*>(wp + static_cast<size_t>(r) * nw));
-            w[ks][r][0] = v.x;
-            w[ks][r][1] = v.y;
+            for (int i = 0; i < PPT; i++) {
+                const int e = tid + i * THREADS;
+                const int pm = e / KPIECES;
+                const int k = kblock + 8 * (e % KPIECES);
+                const int mc = pm < M ? pm : M - 1;
+                const int kc = k < K ? k : K - 8;
+                const size_t at = static_cast<size_t>(mc) * fi.ld + kc;
+                pa[i] = *reinterpret_cast<const uint4*>(fi.a + at);
+                if constexpr (PRO == kProSwiGLU) pb[i] = *reinterpret_cast<const uint4*>(fi.b + at);
+                else pb[i] = *reinterpret_cast<const uint4*>(fi.gain + kc);
+            }
         }
-    }
+#pragma unroll
+        for (int wv = 0; wv < WAVES; wv++) {
+            const int krow = kblock + wv * WROWS;
+            const int g = group_of_step(grid, (krow < K ? krow : K - 1) / kStepRows);  // rows past K meet zero activations
+            s_bits[wv] = scales[static_cast<size_t>(g) * N + own_ld];
+            z_word[wv] = qzeros[static_cast<size_t>(g) * nw + (own_ld >> 3)];
+        }
+        if constexpr (!STAGED) {
+#pragma unroll
+            for (int ks = 0; ks < KS; ks++) {
+                const int kstep = kblock + wave * WROWS + ks * kStepRows;
+                const int kld = kstep < K ? kstep : K - kStepRows;
+                const uint4 got = *reinterpret_cast<const uint4*>(x + static_cast<size_t>(x_row) * K + kld + 8 * b);
+                const bool live = c < M && kstep < K;
+                xa[ks] = make_uint4(live ? got.x : 0u, live ? got.y : 0u, live ? got.z : 0u, live ? got.w : 0u);
+            }
+        }
+    };
+    auto load_weights = [&] {
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+            const int kstep = kblock + wave * WROWS + ks * kStepRows;
+            const int k0 = (kstep < K ? kstep : K - kStepRows) + 8 * b;  // first of the lane's eight rows
+            const uint32_t* wp = qweight + static_cast<size_t>(k0) * nw + wc0;
+#pragma unroll
+            for (int r = 0; r < 8; r++) {
+                const u32x2 v = __builtin_nontemporal_load(reinterpret_cast<const word_pair*>(wp + static_cast<size_t>(r) * nw));
+                w[ks][r][0] = v.x;
+                w[ks][r][1] = v.y;
+            }
+        }
+    };
+    load_operands();
+    load_weights();
     __builtin_amdgcn_sched_barrier(0);
 #if defined(KX_ABLATE) && KX_ABLATE == 2
     if (!STAGED && ktiles > 1) {  // profiling build: loads only - fold what arrived into one word and leave
@@ -246,142 +262,161 @@ __global__ __launch_bounds__(WAVES * kWave, 2) void awq_gemv_mfma_kernel(
     }
 #endif
 
-    // ---- the activation prologue: produce the staged rows, then read the A operand back ----
-    if constexpr (STAGED) {
-        if constexpr (PRO == kProPreNorm) {
+    if constexpr (PRO == kProPreNorm) {
 #pragma unroll
-            for (int rr = 0; rr < (ROWS + WAVES - 1) / WAVES; rr++) {
-                const int m = wave + rr * WAVES;
-                const float total = wave_sum(lane < fi.sumsq_parts ? tile_ss[rr] : 0.0f);
-                if (lane == 0 && m < ROWS) s_inv[m] = 1.0f / sqrtf(total / static_cast<float>(K) + fi.eps);
-            }
-            lds_barrier();
-        }
-#pragma unroll
-        for (int i = 0; i < PPT; i++) {
-            const int e = tid + i * THREADS;
-            const int pm = e / KPIECES;
-            const int kp = e % KPIECES;
-            if (pm < ROWS) {
-                float av[8], bv[8], out[8];
-                bf16x8_to_f32(pa[i], av);
-                bf16x8_to_f32(pb[i], bv);
-                const bool live = pm < M && kt * KB + 8 * kp < K;  // K is a multiple of eight: a piece is all in or all out
-                if constexpr (PRO == kProSwiGLU) {
-#pragma unroll
-                    for (int j = 0; j < 8; j++) {
-                        const float act = silu_rounded_to_bf16(av[j]);
-                        out[j] = live ? act * bv[j] : 0.0f;
-                    }
-                } else {
-                    const float inv = s_inv[pm];
-#pragma unroll
-                    for (int j = 0; j < 8; j++) {
-                        out[j] = live ? bv[j] * bf16_to_f32(f32_to_bf16(av[j] * inv)) : 0.0f;
-                    }
-                }
-                *reinterpret_cast<uint4*>(&s_x[pm][8 * kp]) = f32_to_bf16x8(out);
-            }
+        for (int rr = 0; rr < (ROWS + WAVES - 1) / WAVES; rr++) {
+            const int m = wave + rr * WAVES;
+            const float total = wave_sum(lane < fi.sumsq_parts ? tile_ss[rr] : 0.0f);
+            if (lane == 0 && m < ROWS) s_inv[m] = 1.0f / sqrtf(total / static_cast<float>(K) + fi.eps);
         }
         lds_barrier();
-        const int s_row = c < ROWS ? c : ROWS - 1;
+    }
+    float psum[ROWS];
+    for (int block = 0; block < blocks; block++) {
+        // ---- the activation prologue: produce the staged rows, then read the A operand back ----
+        if constexpr (STAGED) {
+#pragma unroll
+            for (int i = 0; i < PPT; i++) {
+                const int e = tid + i * THREADS;
+                const int pm = e / KPIECES;
+                const int kp = e % KPIECES;
+                if (pm < ROWS) {
+                    float av[8], bv[8], out[8];
+                    bf16x8_to_f32(pa[i], av);
+                    bf16x8_to_f32(pb[i], bv);
+                    const bool live = pm < M && kblock + 8 * kp < K;  // K is a multiple of eight: a piece is all in or all out
+                    if constexpr (PRO == kProSwiGLU) {
+#pragma unroll
+                        for (int j = 0; j < 8; j++) {
+                            const float act = silu_rounded_to_bf16(av[j]);
+                            out[j] = live ? act * bv[j] : 0.0f;
+                        }
+                    } else {
+                        const float inv = s_inv[pm];
+#pragma unroll
+                        for (int j = 0; j < 8; j++) {
+                            out[j] = live ? bv[j] * bf16_to_f32(f32_to_bf16(av[j] * inv)) : 0.0f;
+                        }
+                    }
+                    *reinterpret_cast<uint4*>(&s_x[pm][8 * kp]) = f32_to_bf16x8(out);
+                }
+            }
+            lds_barrier();
+            const int s_row = c < ROWS ? c : ROWS - 1;
+#pragma unroll
+            for (int ks = 0; ks < KS; ks++) {
+                const uint4 got = *reinterpret_cast<const uint4*>(&s_x[s_row][(wave * KS + ks) * kStepRows + 8 * b]);
+                const bool live = c < M;  // rows M .. ROWS-1 and elements past K were staged as zeros
+                xa[ks] = make_uint4(live ? got.x : 0u, live ? got.y : 0u, live ? got.z : 0u, live ? got.w : 0u);
+            }
+        }
+
+        // ---- matrix products ----
+        const bf16x8 ones = as_bf16x8(0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u);
+        const f32x4v zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
+        f32x4v xs;
+        f32x4v acc[2][8];  // [word h][nibble p]
+        const uint32_t magic = opaque_bf16_128_pair();
 #pragma unroll
         for (int ks = 0; ks < KS; ks++) {
-            const uint4 got = *reinterpret_cast<const uint4*>(&s_x[s_row][(wave * KS + ks) * kStepRows + 8 * b]);
-            const bool live = c < M;  // rows M .. ROWS-1 and elements past K were staged as zeros
-            xa[ks] = make_uint4(live ? got.x : 0u, live ? got.y : 0u, live ? got.z : 0u, live ? got.w : 0u);
+            if constexpr (LONE) {
+#pragma unroll
+                for (int r = 0; r < 8; r++) w[ks][r][0] = lone_word ? w[ks][r][1] : w[ks][r][0];
+            }
+            const bf16x8 a_op = as_bf16x8(xa[ks].x, xa[ks].y, xa[ks].z, xa[ks].w);
+            xs = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_op, ones, ks == 0 ? zero4 : xs, 0, 0, 0);
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                uint32_t bop[8][4];  // [nibble p][row pair]
+#pragma unroll
+                for (int rp = 0; rp < 4; rp++) {
+                    const uint32_t wa = w[ks][2 * rp][h];      // row 2rp   -> low half
+                    const uint32_t wb = w[ks][2 * rp + 1][h];  // row 2rp+1 -> high half
+                    const uint32_t lo = __builtin_amdgcn_perm(wb, wa, 0x05040100u);  // nibbles 0..3, both rows
+                    const uint32_t hi = __builtin_amdgcn_perm(wb, wa, 0x07060302u);  // nibbles 4..7
+#pragma unroll
+                    for (int p = 0; p < 4; p++) {
+                        bop[p][rp] = code_pair_to_bf16(p == 0 ? lo : lo >> (4 * p), magic);
+                        bop[4 + p][rp] = code_pair_to_bf16(p == 0 ? hi : hi >> (4 * p), magic);
+                    }
+                }
+#pragma unroll
+                for (int p = 0; p < 8; p++) {
+                    acc[h][p] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                        a_op, as_bf16x8(bop[p][0], bop[p][1], bop[p][2], bop[p][3]), ks == 0 ? zero4 : acc[h][p], 0, 0, 0);
+                }
+            }
+            // a step is worked through while the loads of the later steps are still in flight
+            __builtin_amdgcn_sched_barrier(0);
         }
-    }
 
-    // ---- matrix products ----
-    const bf16x8 ones = as_bf16x8(0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u);
-    const f32x4v zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
-    f32x4v xs;
-    f32x4v acc[2][8];  // [word h][nibble p]
-    const uint32_t magic = opaque_bf16_128_pair();
+        float sc[WAVES], zc[WAVES];
 #pragma unroll
-    for (int ks = 0; ks < KS; ks++) {
-        if constexpr (LONE) {
-#pragma unroll
-            for (int r = 0; r < 8; r++) w[ks][r][0] = lone_word ? w[ks][r][1] : w[ks][r][0];
+        for (int wv = 0; wv < WAVES; wv++) {
+            sc[wv] = f16_bits_to_f32(s_bits[wv]);
+            zc[wv] = -(128.0f + static_cast<float>((z_word[wv] >> (4 * nibble_of(own_col & 7))) & 0xFu));
         }
-        const bf16x8 a_op = as_bf16x8(xa[ks].x, xa[ks].y, xa[ks].z, xa[ks].w);
-        xs = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_op, ones, ks == 0 ? zero4 : xs, 0, 0, 0);
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-            uint32_t bop[8][4];  // [nibble p][row pair]
-#pragma unroll
-            for (int rp = 0; rp < 4; rp++) {
-                const uint32_t wa = w[ks][2 * rp][h];      // row 2rp   -> low half
-                const uint32_t wb = w[ks][2 * rp + 1][h];  // row 2rp+1 -> high half
-                const uint32_t lo = __builtin_amdgcn_perm(wb, wa, 0x05040100u);  // nibbles 0..3, both rows
-                const uint32_t hi = __builtin_amdgcn_perm(wb, wa, 0x07060302u);  // nibbles 4..7
-#pragma unroll
-                for (int p = 0; p < 4; p++) {
-                    bop[p][rp] = code_pair_to_bf16(p == 0 ? lo : lo >> (4 * p), magic);
-                    bop[4 + p][rp] = code_pair_to_bf16(p == 0 ? hi : hi >> (4 * p), magic);
-                }
+        auto load_next = [&] {
+            if (block + 1 < blocks) {
+                kblock += KB;
+                load_operands();
+                load_weights();
+                __builtin_amdgcn_sched_barrier(0);
             }
-#pragma unroll
-            for (int p = 0; p < 8; p++) {
-                acc[h][p] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                    a_op, as_bf16x8(bop[p][0], bop[p][1], bop[p][2], bop[p][3]), ks == 0 ? zero4 : acc[h][p], 0, 0, 0);
-            }
-        }
-        // a step is worked through while the loads of the later steps are still in flight
-        __builtin_amdgcn_sched_barrier(0);
-    }
+        };
+        if constexpr (WALK && AHEAD) load_next();
 
-    // ---- waves meet in LDS; thread t < 256 then owns tile column t ----
-    // A round carries MC activation rows; a lane holds D rows 4b .. 4b+3 and joins the round they fall in.
-    constexpr int VR = MC < 4 ? MC : 4;  // rows of the lane's four that exist at all
-    float psum[ROWS];
+        // ---- waves meet in LDS; thread t < 256 then owns tile column t ----
+        // A round carries MC activation rows; a lane holds D rows 4b .. 4b+3 and joins the round they fall in.
+        constexpr int VR = MC < 4 ? MC : 4;  // rows of the lane's four that exist at all
 #pragma unroll
-    for (int rd = 0; rd < ROUNDS; rd++) {
-        if (rd > 0) __syncthreads();  // the previous round has been read
-        const int local0 = 4 * b - rd * MC;  // the lane's first row inside this round
-        if (local0 >= 0 && local0 < MC) {
-            // the lane's sixteen columns are 16c .. 16c+15
+        for (int rd = 0; rd < ROUNDS; rd++) {
+            if (rd > 0 || block > 0) lds_barrier();  // the previous round has been read
+            const int local0 = 4 * b - rd * MC;  // the lane's first row inside this round
+            if (local0 >= 0 && local0 < MC) {
+                // the lane's sixteen columns are 16c .. 16c+15
 #pragma unroll
-            for (int v = 0; v < VR; v++) {
+                for (int v = 0; v < VR; v++) {
 #pragma unroll
-                for (int h = 0; h < 2; h++) {
-                    f32x4* dst = reinterpret_cast<f32x4*>(&red[wave][local0 + v][16 * c + 8 * h]);
-                    dst[0] = f32x4{acc[h][nibble_of(0)][v], acc[h][nibble_of(1)][v], acc[h][nibble_of(2)][v],
-                                   acc[h][nibble_of(3)][v]};
-                    dst[1] = f32x4{acc[h][nibble_of(4)][v], acc[h][nibble_of(5)][v], acc[h][nibble_of(6)][v],
-                                   acc[h][nibble_of(7)][v]};
+                    for (int h = 0; h < 2; h++) {
+                        f32x4* dst = reinterpret_cast<f32x4*>(&red[wave][local0 + v][16 * c + 8 * h]);
+                        dst[0] = f32x4{acc[h][nibble_of(0)][v], acc[h][nibble_of(1)][v], acc[h][nibble_of(2)][v],
+                                       acc[h][nibble_of(3)][v]};
+                        dst[1] = f32x4{acc[h][nibble_of(4)][v], acc[h][nibble_of(5)][v], acc[h][nibble_of(6)][v],
+                                       acc[h][nibble_of(7)][v]};
+                    }
+                    if (c == 0) xs_red[wave][local0 + v] = xs[v];
                 }
-                if (c == 0) xs_red[wave][local0 + v] = xs[v];
+            }
+            lds_barrier();
+            if (tid < kTileCols) {
+                constexpr int AT_ONCE = WALK ? 4 : MC;  // rows whose sums are read together: registers are short with a block in flight
+#pragma unroll
+                for (int v0 = 0; v0 < MC; v0 += AT_ONCE) {
+                    float qv[AT_ONCE][WAVES], xv[AT_ONCE][WAVES];
+#pragma unroll
+                    for (int v = 0; v < AT_ONCE; v++) {
+#pragma unroll
+                        for (int wv = 0; wv < WAVES; wv++) {
+                            qv[v][wv] = red[wv][v0 + v][tid];
+                            xv[v][wv] = xs_red[wv][v0 + v];
+                        }
+                    }
+#pragma unroll
+                    for (int v = 0; v < AT_ONCE; v++) {
+                        float total = 0.0f;
+#pragma unroll
+                        for (int wv = 0; wv < WAVES; wv++) {
+                            total += sc[wv] * __builtin_fmaf(zc[wv], xv[v][wv], qv[v][wv]);
+                        }
+                        float& sum = psum[rd * MC + v0 + v];
+                        sum = WALK && block > 0 ? sum + total : total;
+                    }
+                    if constexpr (WALK) __builtin_amdgcn_sched_barrier(0);
+                }
             }
         }
-        __syncthreads();
-        if (tid < kTileCols) {
-            float sc[WAVES], zc[WAVES];
-#pragma unroll
-            for (int wv = 0; wv < WAVES; wv++) {
-                sc[wv] = f16_bits_to_f32(s_bits[wv]);
-                zc[wv] = -(128.0f + static_cast<float>((z_word[wv] >> (4 * nibble_of(own_col & 7))) & 0xFu));
-            }
-            float qv[MC][WAVES], xv[MC][WAVES];
-#pragma unroll
-            for (int v = 0; v < MC; v++) {
-#pragma unroll
-                for (int wv = 0; wv < WAVES; wv++) {
-                    qv[v][wv] = red[wv][v][tid];
-                    xv[v][wv] = xs_red[wv][v];
-                }
-            }
-#pragma unroll
-            for (int v = 0; v < MC; v++) {
-                float total = 0.0f;
-#pragma unroll
-                for (int wv = 0; wv < WAVES; wv++) {
-                    total += sc[wv] * __builtin_fmaf(zc[wv], xv[v][wv], qv[v][wv]);
-                }
-                psum[rd * MC + v] = total;
-            }
-        }
+        if constexpr (WALK && !AHEAD) load_next();
     }
 
 #if defined(KX_ABLATE) && KX_ABLATE >= 1 && KX_ABLATE <= 3
@@ -540,7 +575,7 @@ __global__ __launch_bounds__(WAVES * kWave, 2) void awq_gemv_mfma_kernel(
     }
 }
 
-template <int WAVES, int KS, int MC, int ROUNDS, int PRO = kProNone, int EPI = kEpiStore, bool LONE = false>
+template <int WAVES, int KS, int MC, int ROUNDS, int PRO = kProNone, int EPI = kEpiStore, bool LONE = false, bool WALK = false>
 inline void launch_awq_gemv_mfma(const uint16_t* x, const int32_t* qweight, const uint16_t* scales,
                                  const int32_t* qzeros, uint16_t* y, float* partials, uint32_t* counters,
                                  int M, int K, int N, const MfmaGrid& split,
@@ -550,7 +585,7 @@ inline void launch_awq_gemv_mfma(const uint16_t* x, const int32_t* qweight, cons
 
     const dim3 grid(split.side, split.ktiles, split.coltiles / split.side);
     dim3 block(WAVES * kWave, 1, 1);
-    hipLaunchKernelGGL((awq_gemv_mfma_kernel<WAVES, KS, MC, ROUNDS, PRO, EPI, LONE>), grid, block, 0, stream, x,
+    hipLaunchKernelGGL((awq_gemv_mfma_kernel<WAVES, KS, MC, ROUNDS, PRO, EPI, LONE, WALK>), grid, block, 0, stream, x,
                        reinterpret_cast<const uint32_t*>(qweight), scales,
                        reinterpret_cast<const uint32_t*>(qzeros), y, partials, counters, M, K, N,
                        split, fi, res, rope, cache_stride);
