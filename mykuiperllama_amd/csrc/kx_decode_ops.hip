@@ -404,7 +404,7 @@ constexpr int kMergeDimsLong = 32;
 // flight, not the bytes: a chain of trips to memory where the chunks do not fit one, and a head's partial sums passing
 // through one compute unit (313 chunks of 32 heads are 5 MB).  Up to 128 chunks a workgroup takes a whole head; beyond,
 // a quarter of one (128-byte pieces of the partial sums), and the first flight covers 320 chunks.
-// us per launch at 32 heads and 313 chunks, a whole head and 128 chunks ahead -> a quarter and 320: 10.6 -> 5.0.
+// us per launch at 32 heads and 313 chunks, a whole head and 128 chunks ahead -> a quarter and 320: 10.6 -> 4.8.
 // Per dimension the additions run in the same order whatever DIMS and FRONT are.
 template <int DIMS, int FRONT>
 __global__ __launch_bounds__(DIMS * kMergeParts) void attn_decode_stage2(const float* __restrict__ part_out,
