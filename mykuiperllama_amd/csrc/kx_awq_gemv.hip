@@ -11,7 +11,8 @@ namespace {
 
 struct AwqPlan {
     bool mfma;     // matrix-core kernel or the VALU kernel
-    int walk;      // MFMA kernel: blocks of K that a workgroup walks over
+    int run;       // MFMA kernel: blocks of K whose sums are added up before they join the others'
+    bool walks;    // MFMA kernel: a workgroup walks over such a run; otherwise the read-back adds in that order
     bool sliced;   // MFMA kernel: all workgroups of a column tile finish it together
     int waves;     // waves per workgroup stacked along K (4, 8 or 16)
     int rt;        // VALU kernel: consecutive rows per lane (8 or 16); MFMA kernel: 32-row steps per wave
@@ -41,14 +42,23 @@ constexpr int kExchangeRows = 8;    // what a K tile's share of the split-K exch
 //            17.4 / 17.4 -> 12.9 / 14.1.  Larger grids, whose workgroups come in rounds, keep the single reader: with
 //            shares the early ones would hold the places the late ones need (gate|up 4096 -> 24576 at M = 16: 19.7
 //            against 21.5 us), and so do their column-tile-fastest order and 256 / 512 rows per workgroup.
-//            Unless K is long as well, more than 16 blocks of 512 rows (32 up to eight rows, and behind a prologue,
-//            whose operands sixteen rows cannot load ahead): then the partial sums outweigh that, and a workgroup
-//            walks over as many blocks as bring the grid down to two per compute unit.  us per launch, single reader
-//            -> walk: 25600 -> 5120 (50 blocks) at M = 5 / 8 / 12 / 16 27.1 / 27.7 / 36.1 / 36.6 -> 22.2 / 22.4 / 24.1 /
-//            24.3, behind SwiGLU at M = 5 / 16 29.0 / 40.3 -> 22.2 / 34.2.  With fewer blocks the walk loses: 12288
-//            -> 8192 (24) at M = 5 / 16 20.3 / 24.7 -> 21.4 / 23.2, behind SwiGLU 21.1 / 27.5 -> 22.7 / 31.8; 4096 ->
-//            24576 (8) 17.8 / 19.9 -> 19.7 / 23.6; 5120 -> 51200 (10) 42.4 / 48.3 -> 43.4 / 50.6.
-inline AwqPlan make_mfma_plan(int M, int K, int N, int group, bool allow_walk = true, bool produced_x = false) {
+//            Unless K is long as well, more than 16 blocks of 512 rows (32 up to eight rows): then the partial sums
+//            outweigh that, and a workgroup walks over as many blocks as bring the grid down to two per compute unit.  us
+//            per launch, single reader -> walk, M = 5 / 8 / 9 / 16: 14336 -> 5120 (28 blocks) 18.4 / 18.8 / 25.0 / 26.5
+//            -> 19.2 / 19.4 / 21.7 / 22.4, 16384 -> 5120 (32) 18.6 / 19.0 / 25.4 / 26.7 -> 20.1 / 20.2 / 22.1 / 22.7,
+//            18432 -> 5120 (36) 21.1 / 21.7 / 28.0 / 29.3 -> 21.1 / 20.8 / 22.8 / 23.6, 25600 -> 5120 (50) 27.1 / 27.7 /
+//            36.1 / 36.6 -> 22.2 / 22.4 / 24.1 / 24.3; M = 9 / 16: 8192 -> 10240 (16) 21.7 / 22.2 -> 22.5 / 23.7, 8704 ->
+//            10240 (17) 24.1 / 24.7 -> 23.2 / 24.1, 12288 -> 8192 (24) 24.1 / 25.0 -> 22.8 / 23.1.
+//            Behind SwiGLU nine and more rows cannot load the next block's operands ahead, and walk past 32 blocks only:
+//            M = 9 / 16 14336 -> 5120 27.3 / 28.9 -> 28.4 / 30.3, 16384 -> 5120 28.1 / 29.0 -> 29.4 / 30.9, 18432 -> 5120
+//            30.7 / 31.7 -> 30.3 / 31.9, 20480 -> 5120 (40) 34.2 / 35.5 -> 30.9 / 32.3.
+//
+// What a launch does to its activations and its result decides whether its workgroups walk, but not how the sums are
+// added: K tiles, steps per wave and the runs of blocks that are added up ahead of the others depend on M, K, N and the
+// group size alone, so that the launches of a shape return the same bits (one that does not walk leaves the runs to the
+// read-back, splitk_sum_runs: 14336 -> 5120 behind SwiGLU at M = 16 30.3 us with K tiles in order, 29.9 in runs).
+// `may_walk`: the kernel exists in a form that walks; `produced_x`: its activations are produced on the way in.
+inline AwqPlan make_mfma_plan(int M, int K, int N, int group, bool may_walk = true, bool produced_x = false) {
     AwqPlan p;
     p.mfma = true;
     p.coltiles = (N / 8 + kWC - 1) / kWC;
@@ -60,8 +70,8 @@ inline AwqPlan make_mfma_plan(int M, int K, int N, int group, bool allow_walk = 
     int ks = (M >= 9 || (M >= 5 && K >= 8192)) ? 4 : 2;
     if (M <= 4 && ktiles_with(2) > 16 && ktiles_with(2) <= 32) ks = 4;
     while (!allowed(ks)) ks /= 2;
-    p.sliced = false;
-    p.walk = 1;
+    p.sliced = p.walks = false;
+    p.run = 1;
     if (M >= 5) {
         int best = 0;  // the longest run that is allowed, or the shortest that is short enough
         for (int c = 4; c >= 1; c /= 2) {
@@ -71,27 +81,27 @@ inline AwqPlan make_mfma_plan(int M, int K, int N, int group, bool allow_walk = 
         if (kt > 1 && kt <= kSliceMaxKTiles && p.coltiles * kt <= 2 * kComputeUnits) {
             p.sliced = true;
             ks = best;
-        } else if (allow_walk && allowed(4) && ktiles_with(4) > (M >= 9 && !produced_x ? 16 : 32)) {
+        } else if (allowed(4) && ktiles_with(4) > (M >= 9 ? 16 : 32)) {
             const int blocks = ktiles_with(4);
             int walk = 2;
             while (walk < blocks && p.coltiles * ((blocks + walk - 1) / walk) > 2 * kComputeUnits) walk++;
             const int left = (blocks + walk - 1) / walk;
             if (left > 1 && left <= kSliceMaxKTiles && p.coltiles * left <= 2 * kComputeUnits) {
-                p.sliced = true;
-                p.walk = (blocks + left - 1) / left;
+                p.run = (blocks + left - 1) / left;
+                p.walks = p.sliced = may_walk && (M <= 8 || !produced_x || blocks > 32);
                 ks = 4;
             }
         }
     }
     p.rt = ks;  // steps per wave
-    p.ktiles = (ktiles_with(ks) + p.walk - 1) / p.walk;
+    p.ktiles = p.walks ? (ktiles_with(ks) + p.run - 1) / p.run : ktiles_with(ks);
     return p;
 }
 
 inline AwqPlan make_valu_plan(int M, int K, int N, bool allow_long_rows = true, bool allow_12_waves = true) {
     AwqPlan p;
-    p.mfma = p.sliced = false;
-    p.walk = 1;
+    p.mfma = p.sliced = p.walks = false;
+    p.run = 1;
     p.coltiles = (N / 8 + kWC - 1) / kWC;
     p.mb = M >= 8 ? 8 : (M >= 4 ? 4 : (M >= 2 ? 2 : 1));
     p.mtiles = (M + p.mb - 1) / p.mb;
@@ -153,8 +163,8 @@ constexpr int kFixedExchangeRows = 4;
 
 inline AwqPlan make_fixed_plan(int K, int N) {
     AwqPlan p{};
-    p.mfma = p.sliced = false;
-    p.walk = 1;
+    p.mfma = p.sliced = p.walks = false;
+    p.run = 1;
     p.coltiles = (N / 8 + kWC - 1) / kWC;
     p.mb = 1;
     p.mtiles = 1;
@@ -200,7 +210,7 @@ inline MfmaGrid mfma_grid(const AwqPlan& p, int group) {
         while (p.coltiles % g.side != 0) g.side--;
     }
     g.sliced = p.sliced;
-    g.walk = p.walk;
+    g.run = p.run;
     g.wait_ticks = kSliceWaitTicks;
     g.group_magic = gs == 1 ? 0u : static_cast<uint32_t>(((1ull << 32) + gs - 1) / gs);
     return g;
@@ -282,7 +292,7 @@ void launch_mfma_fused(const AwqPlan& p, const FusedInput& fi, const ResidualTar
         else launch_awq_gemv_mfma<4, KS, 8, 2, PRO, EPI>(KX_MARGS);                  \
     } while (0)
     if constexpr (PRO != kProPreNorm && EPI != kEpiQkRope) {
-        if (p.walk > 1) {
+        if (p.walks) {
             if (M <= 8) launch_awq_gemv_mfma<4, 4, 8, 1, PRO, EPI, false, true>(KX_MARGS);
             else launch_awq_gemv_mfma<4, 4, 8, 2, PRO, EPI, false, true>(KX_MARGS);
             return;
@@ -486,7 +496,7 @@ extern "C" int kx_gemv_awq_bf16_policy(const uint16_t* x, const int32_t* qweight
         if (M <= 8) kx::launch_awq_gemv_mfma<4, 4, 8, 1, kx::kProNone, kx::kEpiStore, LONE, true>(KX_MARGS);        \
         else kx::launch_awq_gemv_mfma<4, 4, 8, 2, kx::kProNone, kx::kEpiStore, LONE, true>(KX_MARGS);               \
     } while (0)
-        if (p.walk > 1) {
+        if (p.walks) {
             if (N % 16) KX_MFMA_WALK(true);
             else KX_MFMA_WALK(false);
             return kx::launch_status();

@@ -88,7 +88,8 @@ struct MfmaGrid {
     int coltiles;
     int ktiles;
     int side;              // column tiles side by side in the grid (gridDim.x, whose own load is a trip to memory)
-    int walk;              // blocks of K a workgroup walks over, one behind the other (WALK)
+    int run;               // blocks of K whose sums are added up first: by a workgroup that walks over them (WALK), or by
+                           // the one that reads the partial sums back, so that every launch of a shape adds alike
     int sliced;            // all K tiles of a column tile finish it together (splitk_exchange_sliced)
     uint32_t group_magic;  // ceil(2^32 / (G / 32)), 0 for groups of 32
     uint32_t wait_ticks;   // how long a workgroup waits for the others of its tile
@@ -101,7 +102,7 @@ __device__ __forceinline__ int group_of_step(const MfmaGrid& g, int step) {
 
 // KS: consecutive 32-row steps per wave (they must share a quantisation group);
 // MC: activation rows a workgroup reduces per LDS round (1, 2, 4 or 8); ROUNDS: 2 for M > 8, else 1;
-// WALK: a workgroup works through grid.walk blocks of KB rows of K, one behind the other, and adds their sums up in
+// WALK: a workgroup works through grid.run blocks of KB rows of K, one behind the other, and adds their sums up in
 // registers (make_mfma_plan says when; carrying the loop costs the other launches up to a microsecond);
 // LONE: N is an odd multiple of eight (a template parameter: the moves cost 20 registers, an occupancy step).
 // With a prologue, `x` is not read: fi.a / fi.b (/ fi.gain) are 16-byte aligned, fi.ld a multiple of eight.
@@ -125,6 +126,8 @@ __global__ __launch_bounds__(WAVES * kWave, 2) void awq_gemv_mfma_kernel(
     // operands do not fit the registers beside the weights and the sums: there the other workgroup of the compute unit
     // has to cover the gap.
     constexpr bool AHEAD = PRO == kProNone || ROUNDS == 1;
+    // Launches of a shape that walks elsewhere (make_mfma_plan): behind a prologue at sixteen rows, and the rotary epilogue.
+    constexpr bool RUNS = !WALK && KS == 4 && ((ROWS == 16 && PRO != kProNone) || (ROWS >= 8 && EPI == kEpiQkRope));
     // A staged row is the workgroup's K range plus 16 bytes, so that the rows a wave reads together
     // start in different banks.
     constexpr int XPITCH = KB + 8;
@@ -151,8 +154,8 @@ __global__ __launch_bounds__(WAVES * kWave, 2) void awq_gemv_mfma_kernel(
     const int nw = N >> 3;
 
     // first row of the block that is loaded next, and how many blocks the workgroup has
-    int kblock = kt * KB * (WALK ? grid.walk : 1);
-    const int blocks = WALK ? min(grid.walk, (K - kblock + KB - 1) / KB) : 1;
+    int kblock = kt * KB * (WALK ? grid.run : 1);
+    const int blocks = WALK ? min(grid.run, (K - kblock + KB - 1) / KB) : 1;
 
     // ---- operands of the activation prologue go out first: they are small, mostly cached, and the prologue
     // should run while the weights are still on their way ----
@@ -551,7 +554,9 @@ __global__ __launch_bounds__(WAVES * kWave, 2) void awq_gemv_mfma_kernel(
             }
         };
         float lo[HALF], hi[HALF];
-        if (!splitk_exchange_sum_wide<ROWS>(psum, lo, hi, M, N, ct, kt, ktiles, partials, counters, s_word, request_all)) return;
+        if (!splitk_exchange_sum_wide<ROWS, RUNS>(psum, lo, hi, M, N, ct, kt, ktiles, partials, counters, s_word, request_all, grid.run)) {
+            return;
+        }
         const int row0 = (tid / (kTileCols / 2)) * HALF;
         const int pair = 2 * (tid % (kTileCols / 2));
         if constexpr (EPI == kEpiStore) {

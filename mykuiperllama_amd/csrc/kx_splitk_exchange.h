@@ -523,22 +523,71 @@ __device__ __forceinline__ bool splitk_exchange_sum_per_head(float psum, float* 
     return true;
 }
 
+// Columns `lane_bytes` / 4 (`lo`) and the next one (`hi`) of rows row0 .. row0 + HALF-1: runs of `run` K tiles, each added
+// up on its own, then the runs in order.  TB K tiles in flight; rows past M bring row M-1.
+template <int HALF, int TB>
+__device__ __forceinline__ void splitk_sum_runs(__amdgpu_buffer_rsrc_t rsrc, int lane_bytes, int row0, int M, int N, int ktiles,
+                                                int run, float (&lo)[HALF], float (&hi)[HALF]) {
+    const uint32_t row_stride = static_cast<uint32_t>(N) * 4u;  // M * N and N are multiples of eight: rows start on 8 bytes
+    uint32_t row_bytes[HALF];
+    float run_lo[HALF] = {}, run_hi[HALF] = {};
+    auto take_run = [&] {
+#pragma unroll
+        for (int i = 0; i < HALF; i++) {
+            lo[i] += run_lo[i];
+            hi[i] += run_hi[i];
+            run_lo[i] = run_hi[i] = 0.0f;
+        }
+    };
+#pragma unroll
+    for (int i = 0; i < HALF; i++) row_bytes[i] = static_cast<uint32_t>(row0 + i < M ? row0 + i : M - 1) * row_stride;
+    int in_run = 0;
+    for (int t0 = 0; t0 < ktiles; t0 += TB) {
+        u32x2 got[TB][HALF];
+#pragma unroll
+        for (int u = 0; u < TB; u++) {
+            const uint32_t tile = static_cast<uint32_t>(t0 + u < ktiles ? t0 + u : ktiles - 1) * static_cast<uint32_t>(M) * row_stride;
+#pragma unroll
+            for (int i = 0; i < HALF; i++) {
+                got[u][i] = __builtin_amdgcn_raw_buffer_load_b64(rsrc, lane_bytes, static_cast<int>(tile + row_bytes[i]), 16);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);  // every load of the batch is out before the first is waited for
+#pragma unroll
+        for (int u = 0; u < TB; u++) {
+            if (t0 + u < ktiles) {  // the same in every lane
+                if (in_run == 0) take_run();  // the run before is complete
+#pragma unroll
+                for (int i = 0; i < HALF; i++) {
+                    // two scalars: a bit cast applied to one element of a vector (v.y) reads element 0 with this compiler
+                    const uint32_t bits_lo = got[u][i].x, bits_hi = got[u][i].y;
+                    run_lo[i] += __builtin_bit_cast(float, bits_lo);
+                    run_hi[i] += __builtin_bit_cast(float, bits_hi);
+                }
+                in_run = in_run + 1 == run ? 0 : in_run + 1;
+            }
+        }
+    }
+    take_run();  // the last one
+}
+
 // The exchange for several activation rows (ROWS = 4, 8 or 16) and a workgroup of exactly 256 threads, more
 // than one K tile.  Partial sums go out as above, one column per thread.  The last workgroup reads them back
 // two columns per load: threads 0..127 take rows 0 .. ROWS/2-1 of column pairs 0..127, threads 128..255 the
 // other rows, so a K tile costs a thread ROWS/2 eight-byte loads instead of ROWS four-byte ones and every
 // K tile of the usual shapes is in flight at once.  Per output the additions run t = 0, 1, 2, ... as in
-// the narrow exchange.
+// the narrow exchange, or, with RUNS and run > 1, over runs of `run` K tiles that are added up on their own first: the
+// order of the launches of the same shape whose workgroups walk over `run` blocks of K.
 // Returns true, the same in every thread, in the workgroup that ends up with the finished sums: thread tid
 // then holds rows (tid / 128) * ROWS/2 + i, i < ROWS/2, of columns 2 (tid % 128) (`lo`) and the next one
 // (`hi`) of the tile.  `before_read_back()` runs in that workgroup once it knows it is the last one, ahead
 // of the read-back: loads issued there return under the read-back's round trip.
-template <int ROWS, class Before>
+template <int ROWS, bool RUNS = false, class Before>
 __device__ __forceinline__ bool splitk_exchange_sum_wide(const float (&psum)[ROWS], float (&lo)[ROWS / 2],
                                                          float (&hi)[ROWS / 2], int M, int N, int ct, int kt,
                                                          int ktiles, float* __restrict__ partials,
                                                          uint32_t* __restrict__ counters, uint32_t* s_prev,
-                                                         Before&& before_read_back) {
+                                                         Before&& before_read_back, int run = 1) {
     static_assert(ROWS == 4 || ROWS == 8 || ROWS == 16, "row counts the wide read-back is laid out for");
     const int tid = threadIdx.x;
     const int col = ct * kTileCols + tid;
@@ -577,6 +626,10 @@ __device__ __forceinline__ bool splitk_exchange_sum_wide(const float (&psum)[ROW
     for (int i = 0; i < HALF; i++) lo[i] = hi[i] = 0.0f;
     if (col2 < static_cast<unsigned>(N)) {  // N is even: a pair is all in or all out
         const int lane_bytes = static_cast<int>(col2 * sizeof(float));
+        if (RUNS && run > 1) {
+            splitk_sum_runs<HALF, TB>(rsrc, lane_bytes, row0, M, N, ktiles, run, lo, hi);
+            ktiles = 0;
+        }
         for (int t0 = 0; t0 < ktiles; t0 += TB) {
             // two scalars per load: a bit cast applied to one element of a vector (v.y) reads
             // element 0 with this compiler
