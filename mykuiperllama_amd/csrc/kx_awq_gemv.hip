@@ -191,11 +191,16 @@ inline AwqPlan make_fixed_plan(int K, int N) {
     return p;
 }
 
+// Several activation rows go to the matrix cores, where a lane loads two words of a row.
+inline bool rows_on_mfma(int M, int N) {
+    return M >= 2 && N >= 16;
+}
+
 inline AwqPlan make_plan(int M, int K, int N, int group, int mode) {
     // One activation row stays on the vector kernel: with the fixed-point exchange it is ahead of the MFMA kernel on
     // every measured shape (kx_gemv_awq_bf16_policy decides that before it comes here), and the launches with an
     // activation prologue or an epilogue live in it.
-    const bool mfma = N >= 16 && (mode >= KX_POLICY_MFMA || (mode == KX_POLICY_BY_SHAPE && M >= 2));  // a lane loads two words
+    const bool mfma = mode >= KX_POLICY_MFMA ? N >= 16 : mode == KX_POLICY_BY_SHAPE && rows_on_mfma(M, N);
     return mfma ? make_mfma_plan(M, K, N, group) : make_valu_plan(M, K, N);
 }
 
@@ -277,7 +282,7 @@ void launch_fused(const AwqPlan& p, const FusedInput& fi, const int32_t* qweight
 }
 
 // The matrix-core kernel with an activation prologue and / or the residual epilogue, 2 <= M <= 16.
-template <int PRO, int EPI>
+template <int PRO, int EPI, bool LONE = false>
 void launch_mfma_fused(const AwqPlan& p, const FusedInput& fi, const ResidualTarget& res, const uint16_t* x,
                        const int32_t* qweight, const uint16_t* scales, const int32_t* qzeros, uint16_t* y,
                        float* partials, uint32_t* counters, int M, int K, int N, int group, hipStream_t stream,
@@ -286,12 +291,12 @@ void launch_mfma_fused(const AwqPlan& p, const FusedInput& fi, const ResidualTar
 #define KX_MARGS x, qweight, scales, qzeros, y, partials, counters, M, K, N, grid, stream, fi, res, rope, cache_stride
 #define KX_MFMA_BY_M(KS)                                                             \
     do {                                                                             \
-        if (M <= 2) launch_awq_gemv_mfma<4, KS, 2, 1, PRO, EPI>(KX_MARGS);           \
-        else if (M <= 4) launch_awq_gemv_mfma<4, KS, 4, 1, PRO, EPI>(KX_MARGS);      \
-        else if (M <= 8) launch_awq_gemv_mfma<4, KS, 8, 1, PRO, EPI>(KX_MARGS);      \
-        else launch_awq_gemv_mfma<4, KS, 8, 2, PRO, EPI>(KX_MARGS);                  \
+        if (M <= 2) launch_awq_gemv_mfma<4, KS, 2, 1, PRO, EPI, LONE>(KX_MARGS);     \
+        else if (M <= 4) launch_awq_gemv_mfma<4, KS, 4, 1, PRO, EPI, LONE>(KX_MARGS); \
+        else if (M <= 8) launch_awq_gemv_mfma<4, KS, 8, 1, PRO, EPI, LONE>(KX_MARGS); \
+        else launch_awq_gemv_mfma<4, KS, 8, 2, PRO, EPI, LONE>(KX_MARGS);            \
     } while (0)
-    if constexpr (PRO != kProPreNorm && EPI != kEpiQkRope) {
+    if constexpr (PRO != kProPreNorm && EPI != kEpiQkRope && !LONE) {
         if (p.walks) {
             if (M <= 8) launch_awq_gemv_mfma<4, 4, 8, 1, PRO, EPI, false, true>(KX_MARGS);
             else launch_awq_gemv_mfma<4, 4, 8, 2, PRO, EPI, false, true>(KX_MARGS);
@@ -555,17 +560,18 @@ extern "C" int kx_gemv_awq_swiglu_bf16(const uint16_t* gate, const uint16_t* up,
     fi.a = gate;
     fi.b = up;
     fi.ld = act_ld;
-    // Several rows go to the matrix cores, as in kx_gemv_awq_bf16, when gate and up can be read 16 bytes at a time
-    if (M >= 2 && (N % 16) == 0 && kx::aligned_to(gate, 16) && kx::aligned_to(up, 16) &&
-        (act_ld % 8) == 0) {
-        const kx::AwqPlan mp = kx::make_mfma_plan(M, K, N, group_size, true, true);
+    // Several rows go where kx_gemv_awq_bf16 takes them, when gate and up can be read 16 bytes at a time
+    if (kx::rows_on_mfma(M, N) && kx::aligned_to(gate, 16) && kx::aligned_to(up, 16) && (act_ld % 8) == 0) {
+        const bool lone = N % 16 != 0;
+        const kx::AwqPlan mp = kx::make_mfma_plan(M, K, N, group_size, !lone, true);
         float* partials = nullptr;
         uint32_t* counters = nullptr;
         rc = kx::resolve_workspace(mp, M, N, workspace, workspace_bytes, &partials, &counters);
         if (rc != KX_OK) return rc;
-        kx::launch_mfma_fused<kx::kProSwiGLU, kx::kEpiStore>(mp, fi, kx::ResidualTarget{}, nullptr, qweight, scales,
-                                                             qzeros, y, partials, counters, M, K, N, group_size,
-                                                             kx::as_stream(stream));
+#define KX_MARGS mp, fi, kx::ResidualTarget{}, nullptr, qweight, scales, qzeros, y, partials, counters, M, K, N, group_size, kx::as_stream(stream)
+        if (lone) kx::launch_mfma_fused<kx::kProSwiGLU, kx::kEpiStore, true>(KX_MARGS);
+        else kx::launch_mfma_fused<kx::kProSwiGLU, kx::kEpiStore>(KX_MARGS);
+#undef KX_MARGS
         return kx::launch_status();
     }
     const kx::AwqPlan p = kx::make_fused_plan(M, K, N, true);

@@ -126,8 +126,10 @@ __global__ __launch_bounds__(WAVES * kWave, 2) void awq_gemv_mfma_kernel(
     // operands do not fit the registers beside the weights and the sums: there the other workgroup of the compute unit
     // has to cover the gap.
     constexpr bool AHEAD = PRO == kProNone || ROUNDS == 1;
-    // Launches of a shape that walks elsewhere (make_mfma_plan): behind a prologue at sixteen rows, and the rotary epilogue.
-    constexpr bool RUNS = !WALK && KS == 4 && ((ROWS == 16 && PRO != kProNone) || (ROWS >= 8 && EPI == kEpiQkRope));
+    // Launches of a shape that walks elsewhere (make_mfma_plan): behind a prologue at sixteen rows or with an odd number
+    // of words, and the rotary epilogue.
+    constexpr bool RUNS = !WALK && KS == 4 &&
+                          ((ROWS == 16 && PRO != kProNone) || (ROWS >= 8 && (EPI == kEpiQkRope || (LONE && PRO != kProNone))));
     // A staged row is the workgroup's K range plus 16 bytes, so that the rows a wave reads together
     // start in different banks.
     constexpr int XPITCH = KB + 8;

@@ -49,6 +49,26 @@ def test_swiglu_and_residual_forms(M, K, N):
         assert torch.equal(out, added)
 
 
+# N an odd multiple of eight (one word of a row has no partner): three words in all, groups of 96 and 32, shapes whose plain
+# launch walks over two and three blocks; and eight columns, which stay on the vector kernel
+@pytest.mark.parametrize("K,N,group", [(256, 24, 128), (1152, 1000, 96), (5472, 9000, 32), (17408, 4360, 128),
+                                       (8704, 22024, 128), (512, 8, 128)])
+@pytest.mark.parametrize("M", [2, 3] + ROWS)
+def test_swiglu_form_of_odd_word_counts(M, K, N, group):
+    import torch
+    from mykuiperllama_amd import capi
+    w, rand = problem(torch, M, K, N, group)
+    both = rand(M, 2 * K)
+    act, plain, fused = empty(torch, M, K), empty(torch, M, N), empty(torch, M, N)
+    ws = capi.make_workspace(M, K, N)
+    gate, up = both[:, :K], both[:, K:]
+    capi.swiglu_bf16(gate.contiguous(), up.contiguous(), act)
+    capi.gemv_awq_bf16(act, *w, plain, group, ws)
+    capi.gemv_awq_swiglu_bf16(gate, up, *w, fused, group, ws)
+    torch.cuda.synchronize()
+    assert torch.equal(plain, fused)
+
+
 @pytest.mark.parametrize("K,N", [(8704, 8704), (13824, 5120), (16384, 4352), (17408, 4352), (25600, 2816)])
 @pytest.mark.parametrize("M", ROWS)
 def test_rotary_form(M, K, N):
