@@ -191,16 +191,22 @@ inline AwqPlan make_fixed_plan(int K, int N) {
     return p;
 }
 
-// Several activation rows go to the matrix cores, where a lane loads two words of a row.
-inline bool rows_on_mfma(int M, int N) {
-    return M >= 2 && N >= 16;
+// Several activation rows go to the matrix cores, where a lane loads two words of a row.  Groups that leave a wave one
+// step make one K tile of every 128 rows, and many of them meet slowly: with an odd number of words, which the vector kernel
+// used to serve, two rows past K = 2048 and narrow matrices past K = 8192 are still faster there.  us per launch, vector
+// kernel against this one, groups of 32: M = 2 6144 -> 5128 10.3 / 12.2, 12288 -> 10248 28.3 / 31.8 (1536 -> 1288 8.8 /
+// 5.9); M = 5 and 12 12288 -> 1288 18.4 / 22.4 and 35.7 / 42.4 (12288 -> 5128 43.0 / 32.8 and 66.3 / 55.7).
+inline bool rows_on_mfma(int M, int K, int N, int group) {
+    if (M < 2 || N < 16) return false;
+    const bool odd = N % 16 != 0, one_step = group % (2 * kStepRows) != 0;
+    return !(odd && one_step && (M == 2 ? K > 2048 : K > 8192 && N <= 2048));
 }
 
 inline AwqPlan make_plan(int M, int K, int N, int group, int mode) {
     // One activation row stays on the vector kernel: with the fixed-point exchange it is ahead of the MFMA kernel on
     // every measured shape (kx_gemv_awq_bf16_policy decides that before it comes here), and the launches with an
     // activation prologue or an epilogue live in it.
-    const bool mfma = mode >= KX_POLICY_MFMA ? N >= 16 : mode == KX_POLICY_BY_SHAPE && rows_on_mfma(M, N);
+    const bool mfma = mode >= KX_POLICY_MFMA ? N >= 16 : mode == KX_POLICY_BY_SHAPE && rows_on_mfma(M, K, N, group);
     return mfma ? make_mfma_plan(M, K, N, group) : make_valu_plan(M, K, N);
 }
 
@@ -561,7 +567,7 @@ extern "C" int kx_gemv_awq_swiglu_bf16(const uint16_t* gate, const uint16_t* up,
     fi.b = up;
     fi.ld = act_ld;
     // Several rows go where kx_gemv_awq_bf16 takes them, when gate and up can be read 16 bytes at a time
-    if (kx::rows_on_mfma(M, N) && kx::aligned_to(gate, 16) && kx::aligned_to(up, 16) && (act_ld % 8) == 0) {
+    if (kx::rows_on_mfma(M, K, N, group_size) && kx::aligned_to(gate, 16) && kx::aligned_to(up, 16) && (act_ld % 8) == 0) {
         const bool lone = N % 16 != 0;
         const kx::AwqPlan mp = kx::make_mfma_plan(M, K, N, group_size, !lone, true);
         float* partials = nullptr;

@@ -50,9 +50,10 @@ def test_swiglu_and_residual_forms(M, K, N):
 
 
 # N an odd multiple of eight (one word of a row has no partner): three words in all, groups of 96 and 32, shapes whose plain
-# launch walks over two and three blocks; and eight columns, which stay on the vector kernel
+# launch walks over two and three blocks; and what stays on the vector kernel: eight columns, many short K tiles
 @pytest.mark.parametrize("K,N,group", [(256, 24, 128), (1152, 1000, 96), (5472, 9000, 32), (17408, 4360, 128),
-                                       (8704, 22024, 128), (512, 8, 128)])
+                                       (8704, 22024, 128), (512, 8, 128),
+                                       (9216, 520, 32)])
 @pytest.mark.parametrize("M", [2, 3] + ROWS)
 def test_swiglu_form_of_odd_word_counts(M, K, N, group):
     import torch
