@@ -106,8 +106,12 @@ __device__ __forceinline__ int group_of_step(const MfmaGrid& g, int step) {
 // registers (make_mfma_plan says when; carrying the loop costs the other launches up to a microsecond);
 // LONE: N is an odd multiple of eight (a template parameter: the moves cost 20 registers, an occupancy step).
 // With a prologue, `x` is not read: fi.a / fi.b (/ fi.gain) are 16-byte aligned, fi.ld a multiple of eight.
+// Three workgroups per compute unit where the registers nearly allow it: left alone, one or two steps per wave at sixteen
+// rows take 169 to 185 of them, one occupancy step down.  us per launch, two -> three: groups of 32 3072 -> 23808 at M = 9 /
+// 16 33.8 / 35.8 -> 28.7 / 33.7, 9728 -> 18432 77.7 / 81.3 -> 67.4 / 71.7; groups of 64 11264 -> 24064 70.2 / 73.5 -> 62.8 /
+// 69.2, 4096 -> 14304 (896 workgroups) 22.7 / 23.7 -> 23.5 / 26.0; grids of up to 512 alike.
 template <int WAVES, int KS, int MC, int ROUNDS, int PRO = kProNone, int EPI = kEpiStore, bool LONE = false, bool WALK = false>
-__global__ __launch_bounds__(WAVES * kWave, 2) void awq_gemv_mfma_kernel(
+__global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEpiStore ? 3 : 2) void awq_gemv_mfma_kernel(
     const uint16_t* __restrict__ x, const uint32_t* __restrict__ qweight,
     const uint16_t* __restrict__ scales, const uint32_t* __restrict__ qzeros,
     uint16_t* __restrict__ y, float* __restrict__ partials, uint32_t* __restrict__ counters,
