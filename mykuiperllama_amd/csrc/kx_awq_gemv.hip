@@ -39,7 +39,8 @@ constexpr int kExchangeRows = 8;    // what a K tile's share of the split-K exch
 //            = 2, q|k|v and down ks = 4).  Against the single reader, us per launch at M = 8 / 16: k 4096 -> 1024
 //            7.6 / 10.2 -> 6.9 / 8.1, q 4096 -> 4096 8.2 / 10.7 -> 7.5 / 8.9, q|k|v 9.2 / 11.0 -> 8.6 / 9.8, down
 //            12288 -> 4096 15.4 / 18.9 -> 12.6 / 14.7, gate 4096 -> 12288 12.1 / 14.3 -> 12.0 / 12.6, 5120 -> 10240
-//            17.4 / 17.4 -> 12.9 / 14.1.  Larger grids, whose workgroups come in rounds, keep the single reader: with
+//            17.4 / 17.4 -> 12.9 / 14.1.  A K that one workgroup covers stays with one, which has nothing to exchange (512 ->
+//            17920 at M = 8 / 16 8.1 / 10.7 -> 6.1 / 7.3, 512 -> 1280 6.6 / 8.3 -> 5.5 / 6.7).  Larger grids, whose workgroups come in rounds, keep the single reader: with
 //            shares the early ones would hold the places the late ones need (gate|up 4096 -> 24576 at M = 16: 19.7
 //            against 21.5 us), and so do their column-tile-fastest order and 256 / 512 rows per workgroup.
 //            Unless K is long as well, more than 16 blocks of 512 rows (32 up to eight rows): then the partial sums
@@ -75,11 +76,12 @@ inline AwqPlan make_mfma_plan(int M, int K, int N, int group, bool may_walk = tr
     if (M >= 5) {
         int best = 0;  // the longest run that is allowed, or the shortest that is short enough
         for (int c = 4; c >= 1; c /= 2) {
+            if (best > 0 && ktiles_with(best) == 1) break;  // nothing to exchange
             if (allowed(c) && (best == 0 || (p.coltiles * ktiles_with(c) <= kComputeUnits && ktiles_with(c) <= 16))) best = c;
         }
         const int kt = ktiles_with(best);
-        if (kt > 1 && kt <= kSliceMaxKTiles && p.coltiles * kt <= 2 * kComputeUnits) {
-            p.sliced = true;
+        if (kt == 1 || (kt <= kSliceMaxKTiles && p.coltiles * kt <= 2 * kComputeUnits)) {
+            p.sliced = kt > 1;
             ks = best;
         } else if (allowed(4) && ktiles_with(4) > (M >= 9 ? 16 : 32)) {
             const int blocks = ktiles_with(4);

@@ -502,10 +502,17 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
         }
     };
     if (ktiles == 1) {
-        __syncthreads();
+        if constexpr (EPI == kEpiStore) {  // a thread stores its own column: nothing to hand over
 #pragma unroll
-        for (int r = 0; r < ROWS; r++) s_sum[r * kTileCols + tid] = psum[r];
-        finish_from_lds();
+            for (int r = 0; r < ROWS; r++) {
+                if (r < M && own_col < N) y[static_cast<size_t>(r) * N + own_col] = f32_to_bf16(psum[r]);
+            }
+        } else {
+            __syncthreads();
+#pragma unroll
+            for (int r = 0; r < ROWS; r++) s_sum[r * kTileCols + tid] = psum[r];
+            finish_from_lds();
+        }
         return;
     }
     if constexpr (ROWS <= 2) {
