@@ -427,15 +427,17 @@ __device__ __forceinline__ bool splitk_exchange_sum_per_wave_rows(const float (&
                 const int t = t0 + u;
                 const int tc = t < ktiles ? t : ktiles - 1;
                 const int rc = r < M ? r : M - 1;
-                const float got = load_partial(rsrc, lane_bytes, static_cast<uint32_t>(tc) * tfloats +
-                                                                     static_cast<uint32_t>(rc) * static_cast<uint32_t>(N));
-                v[r][u] = (t < ktiles && r < M) ? got : 0.0f;
+                v[r][u] = load_partial(rsrc, lane_bytes, static_cast<uint32_t>(tc) * tfloats +
+                                                             static_cast<uint32_t>(rc) * static_cast<uint32_t>(N));
             }
         }
+        // without this the compiler waits for each load in turn where registers are short (8192 -> 5120 into the residual
+        // stream at M = 2 with four steps per wave: 16.5 us instead of 10.5)
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int r = 0; r < ROWS; r++) {
 #pragma unroll
-            for (int u = 0; u < TB; u++) sum[r] += v[r][u];
+            for (int u = 0; u < TB; u++) sum[r] += (t0 + u < ktiles && r < M) ? v[r][u] : 0.0f;
         }
     }
     if (tid % kWave == 0) {
