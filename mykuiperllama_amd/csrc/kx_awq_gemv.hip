@@ -32,7 +32,14 @@ constexpr int kExchangeRows = 8;    // what a K tile's share of the split-K exch
 // MFMA kernel: four waves per workgroup, each walking `ks` consecutive 32-row steps that must lie in one quantisation
 // group.  What it costs besides the weights is the exchange of partial sums, M KB per K tile and column tile.
 //   M <= 4   one workgroup (or wave) of a column tile reads all of them back, sixteen K tiles in flight: two steps per
-//            wave, or four where that brings the K tiles down to one such batch (5120 -> 5120 at M = 4: 9.2 -> 8.1 us).
+//            wave, or four where that brings the K tiles down to one such batch and gives the busiest compute unit no
+//            more rows to stream (or saves three rows and more a nearly full second batch), on at most two workgroups per
+//            compute unit.  us per launch at M = 2 / 3 / 4, two steps -> four: 5120 -> 5120 (200 workgroups of four) 8.5 /
+//            9.6 / 9.6 -> 7.6 / 8.5 / 8.5, 5120 -> 10240 (400) 11.8 / 13.2 / 13.3 -> 11.0 / 11.8 / 11.8, 8192 -> 5120 (320)
+//            at M = 3 / 4 11.1 / 11.2 -> 10.8 / 11.0.  What the rule leaves out: 5120 -> 1024 (40) 6.8 / 7.8 / 7.9 -> 7.0 /
+//            7.8 / 7.9, 6400 -> 5120 (260) 8.6 / 9.8 / 9.8 -> 9.3 / 10.2 / 10.2, 5120 -> 8192 (320) 9.6 / 10.7 / 10.8 ->
+//            10.7 / 11.5 / 11.6, 6400 -> 10240 (520) 12.3 / 13.3 / 13.7 -> 14.0 / 14.8 / 14.9, 5120 -> 51200 (2000) behind a
+//            norm 31.9 / 33.9 / 34.4 -> 34.8 / 37.2 / 37.8.
 //   M >= 5   every workgroup of a column tile finishes a share (splitk_exchange_sliced), provided that they are on the
 //            chip together: at most two per compute unit.  The shortest run of steps that leaves one workgroup per
 //            compute unit and sixteen K tiles (fewer workgroups idle against more partial sums: 1024 -> 2048 ks = 1, q ks
@@ -40,9 +47,10 @@ constexpr int kExchangeRows = 8;    // what a K tile's share of the split-K exch
 //            7.6 / 10.2 -> 6.9 / 8.1, q 4096 -> 4096 8.2 / 10.7 -> 7.5 / 8.9, q|k|v 9.2 / 11.0 -> 8.6 / 9.8, down
 //            12288 -> 4096 15.4 / 18.9 -> 12.6 / 14.7, gate 4096 -> 12288 12.1 / 14.3 -> 12.0 / 12.6, 5120 -> 10240
 //            17.4 / 17.4 -> 12.9 / 14.1.  A K that one workgroup covers stays with one, which has nothing to exchange (512 ->
-//            17920 at M = 8 / 16 8.1 / 10.7 -> 6.1 / 7.3, 512 -> 1280 6.6 / 8.3 -> 5.5 / 6.7).  Larger grids, whose workgroups come in rounds, keep the single reader: with
-//            shares the early ones would hold the places the late ones need (gate|up 4096 -> 24576 at M = 16: 19.7
-//            against 21.5 us), and so do their column-tile-fastest order and 256 / 512 rows per workgroup.
+//            17920 at M = 8 / 16 8.1 / 10.7 -> 6.1 / 7.3, 512 -> 1280 6.6 / 8.3 -> 5.5 / 6.7).  Larger grids, whose workgroups
+//            come in rounds, keep the single reader: with shares the early ones would hold the places the late ones need
+//            (gate|up 4096 -> 24576 at M = 16: 19.7 against 21.5 us), and so do their column-tile-fastest order and 256 /
+//            512 rows per workgroup.
 //            Unless K is long as well, more than 16 blocks of 512 rows (32 up to eight rows): then the partial sums
 //            outweigh that, and a workgroup walks over as many blocks as bring the grid down to two per compute unit.  us
 //            per launch, single reader -> walk, M = 5 / 8 / 9 / 16: 14336 -> 5120 (28 blocks) 18.4 / 18.8 / 25.0 / 26.5
@@ -69,7 +77,11 @@ inline AwqPlan make_mfma_plan(int M, int K, int N, int group, bool may_walk = tr
     const auto ktiles_with = [&](int ks) { return (K + p.waves * ks * kStepRows - 1) / (p.waves * ks * kStepRows); };
     const auto allowed = [&](int ks) { return group % (ks * kStepRows) == 0 && (ks == 1 || p.waves * ks * kStepRows <= K); };
     int ks = (M >= 9 || (M >= 5 && K >= 8192)) ? 4 : 2;
-    if (M <= 4 && ktiles_with(2) > 16 && ktiles_with(2) <= 32) ks = 4;
+    const auto rounds_with = [&](int c) { return (p.coltiles * ktiles_with(c) + kComputeUnits - 1) / kComputeUnits; };
+    if (M <= 4 && ktiles_with(2) > 16 && ktiles_with(2) <= 32 && rounds_with(4) <= 2 &&
+        (2 * rounds_with(4) <= rounds_with(2) || (M >= 3 && ktiles_with(2) >= 30))) {
+        ks = 4;
+    }
     while (!allowed(ks)) ks /= 2;
     p.sliced = p.walks = false;
     p.run = 1;

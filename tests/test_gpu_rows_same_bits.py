@@ -49,6 +49,34 @@ def test_swiglu_and_residual_forms(M, K, N):
         assert torch.equal(out, added)
 
 
+# two to four rows at the edges of "four steps per wave": sixteen K tiles of two steps and one more; too few workgroups, one
+# and two per compute unit and just past either; thirty and thirty-two K tiles of two steps; one more than two batches
+@pytest.mark.parametrize("K,N", [(4096, 5120), (4352, 5120), (5120, 1024), (6400, 4864), (6400, 5120), (5120, 13056),
+                                 (7680, 5120), (8192, 8448), (8448, 5120)])
+@pytest.mark.parametrize("M", [2, 3, 4])
+def test_two_to_four_rows(M, K, N):
+    import torch
+    from mykuiperllama_amd import capi
+    w, rand = problem(torch, M, K, N)
+    x, res = rand(M, K), rand(M, N)
+    plain, out, added = empty(torch, M, N), empty(torch, M, N), empty(torch, M, N)
+    ssq = torch.empty((M, (N + 255) // 256, 4), dtype=torch.float32, device="cuda")
+    ws = capi.make_workspace(M, K, N)
+    capi.gemv_awq_bf16(x, *w, plain, 128, ws)
+    capi.add_bf16(res, plain, added)
+    capi.gemv_awq_chain_bf16({"in_kind": capi.IN_ROW, "x": x, "rows": M, "out_kind": capi.OUT_RESIDUAL, "residual_in": res,
+                              "residual_out": out, "sumsq_out": ssq}, *w, K, N, 128, ws)
+    torch.cuda.synchronize()
+    assert torch.equal(out, added)
+    qw, sc, qz = w
+    ref = torch.empty((M, N), dtype=torch.float64, device="cuda")
+    for i, col in enumerate((0, 2, 4, 6, 1, 3, 5, 7)):  # nibble i of a word holds column col of its eight
+        q, z = ((qw >> (4 * i)) & 15).double(), ((qz >> (4 * i)) & 15).double().repeat_interleave(128, 0)
+        ref[:, col::8] = x.double() @ ((q - z) * sc[:, col::8].double().repeat_interleave(128, 0))
+    rounded = ref.bfloat16().double()
+    assert ((plain.double() - rounded).norm() / rounded.norm()).item() <= 1e-3
+
+
 # N an odd multiple of eight (one word of a row has no partner): three words in all, groups of 96 and 32, shapes whose plain
 # launch walks over two and three blocks; and what stays on the vector kernel: eight columns, many short K tiles
 @pytest.mark.parametrize("K,N,group", [(256, 24, 128), (1152, 1000, 96), (5472, 9000, 32), (17408, 4360, 128),
