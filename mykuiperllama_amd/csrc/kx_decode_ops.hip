@@ -402,10 +402,22 @@ constexpr int kMergeDimsLong = 32;
 
 // DIMS dimensions of a head per workgroup, FRONT chunks per thread in the first flight of loads.  What bounds it is the
 // flight, not the bytes: a chain of trips to memory where the chunks do not fit one, and a head's partial sums passing
-// through one compute unit (313 chunks of 32 heads are 5 MB).  Up to 128 chunks a workgroup takes a whole head; beyond,
-// a quarter of one (128-byte pieces of the partial sums), and the first flight covers 320 chunks.
+// through one compute unit (313 chunks of 32 heads are 5 MB).  A workgroup takes a whole head, 128 chunks in the first
+// flight, or a quarter of one (128-byte pieces of the partial sums) with 320: merge_by_quarters.
 // us per launch at 32 heads and 313 chunks, a whole head and 128 chunks ahead -> a quarter and 320: 10.6 -> 4.8.
 // Per dimension the additions run in the same order whatever DIMS and FRONT are.
+// Whether the merge takes a head in quarters.  A quarter's 80 loads per thread go out whatever the number of chunks, so it
+// takes a good deal more than the 128 chunks that a whole head covers in one flight, and the more so the more workgroups
+// share a compute unit; with more than four each it gains nothing at any length.  Attention in all, whole heads ->
+// quarters, difference in us at 129 / 144 / 160 / 168 / 192 / 208 / 256 / 320 / 512 chunks: 32 heads of one sequence (128
+// workgroups) +0.5 / +0.3 / -0.1 / -0.9 / -1.2 / -2.1 / -3.4 / -5.5 / -5.6, of four (512) +1.7 / +1.2 / +1.3 / +0.2 / +0.1 /
+// -1.1 / -2.4 / -3.5 / -3.7, of eight (1024) +2.2 / +1.8 / +1.9 / +1.4 / +1.1 / +0.6 / -0.1 / -1.1 / -0.8, of sixteen (2048)
+// slower throughout.
+inline bool merge_by_quarters(int nchunks, int heads) {
+    const int per_cu = (heads * (kHeadDim / kMergeDimsLong) + 255) / 256;  // workgroups, of 256 compute units
+    return per_cu <= 4 && nchunks > kMergeParts * kMergeFront + 32 * per_cu;
+}
+
 template <int DIMS, int FRONT>
 __global__ __launch_bounds__(DIMS * kMergeParts) void attn_decode_stage2(const float* __restrict__ part_out,
                                                                          const float* __restrict__ part_ml,
@@ -750,7 +762,7 @@ int attn_decode(const uint16_t* q, const uint16_t* k_cache, const uint16_t* v_ca
     }
     if (out) {
         // slots per chunk subset: at least what the first flight of the merge covers
-        const bool long_merge = nchunks > kx::kMergeParts * kx::kMergeFront;
+        const bool long_merge = kx::merge_by_quarters(nchunks, n_q_heads * batch);
         int per_part = (nchunks + kx::kMergeParts - 1) / kx::kMergeParts;
         const int front = long_merge ? kx::kMergeFrontLong : kx::kMergeFront;
         if (per_part < front) per_part = front;
