@@ -58,9 +58,12 @@ constexpr int kExchangeRows = 8;    // what a K tile's share of the split-K exch
 //            18432 -> 5120 (36) 21.1 / 21.7 / 28.0 / 29.3 -> 21.1 / 20.8 / 22.8 / 23.6, 25600 -> 5120 (50) 27.1 / 27.7 /
 //            36.1 / 36.6 -> 22.2 / 22.4 / 24.1 / 24.3; M = 9 / 16: 8192 -> 10240 (16) 21.7 / 22.2 -> 22.5 / 23.7, 8704 ->
 //            10240 (17) 24.1 / 24.7 -> 23.2 / 24.1, 12288 -> 8192 (24) 24.1 / 25.0 -> 22.8 / 23.1.
-//            Behind SwiGLU nine and more rows cannot load the next block's operands ahead, and walk past 32 blocks only:
-//            M = 9 / 16 14336 -> 5120 27.3 / 28.9 -> 28.4 / 30.3, 16384 -> 5120 28.1 / 29.0 -> 29.4 / 30.9, 18432 -> 5120
-//            30.7 / 31.7 -> 30.3 / 31.9, 20480 -> 5120 (40) 34.2 / 35.5 -> 30.9 / 32.3.
+//            Behind SwiGLU nine and more rows cannot load the next block's operands ahead, and walk past 32 blocks only,
+//            over no more of them than there would be rounds of workgroups: M = 9 / 16 14336 -> 5120 27.3 / 28.9 -> 28.4 /
+//            30.3, 16384 -> 5120 28.1 / 29.0 -> 29.4 / 30.9, 18432 -> 5120 30.7 / 31.7 -> 30.3 / 31.9, 20480 -> 5120 (40)
+//            34.2 / 35.5 -> 30.9 / 32.3; 24576 -> 16384 (six, for six rounds) 72.2 / 77.4 -> 69.7 / 73.4, 17408 -> 8192 (three,
+//            for three) 38.0 / 40.2 -> 35.2 / 38.0, 20096 -> 9616 (four, for three) 51.7 / 54.1 -> 58.7 / 61.9, 17920 -> 14592
+//            (five, for four) 50.7 / 53.0 -> 55.6 / 59.4.
 //
 // What a launch does to its activations and its result decides whether its workgroups walk, but not how the sums are
 // added: K tiles, steps per wave and the runs of blocks that are added up ahead of the others depend on M, K, N and the
@@ -102,7 +105,8 @@ inline AwqPlan make_mfma_plan(int M, int K, int N, int group, bool may_walk = tr
             const int left = (blocks + walk - 1) / walk;
             if (left > 1 && left <= kSliceMaxKTiles && p.coltiles * left <= 2 * kComputeUnits) {
                 p.run = (blocks + left - 1) / left;
-                p.walks = p.sliced = may_walk && (M <= 8 || !produced_x || blocks > 32);
+                const int rounds = (p.coltiles * blocks + 2 * kComputeUnits - 1) / (2 * kComputeUnits);  // without the walk
+                p.walks = p.sliced = may_walk && (M <= 8 || !produced_x || (blocks > 32 && p.run <= rounds));
                 ks = 4;
             }
         }

@@ -7,9 +7,10 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 # K, N: 27 and 24 blocks; a last block half past K; runs of three blocks whose last is shorter; 32 blocks and 33, where
-# the SwiGLU form walks as well; 34 in whole tiles of heads; 43 blocks in runs of three
+# the SwiGLU form walks as well; 34 in whole tiles of heads; 43 blocks in runs of three, 40 in runs of four, over which the
+# SwiGLU form at nine rows does not walk
 SHAPES = [(13824, 5120), (12288, 8192), (8960, 10240), (10240, 16384), (16384, 4352), (16896, 4352), (17408, 4352),
-          (22016, 8192)]
+          (22016, 8192), (20096, 9616)]
 ROWS = [5, 8, 9, 16]
 
 
