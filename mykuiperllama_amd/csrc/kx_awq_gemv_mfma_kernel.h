@@ -109,7 +109,8 @@ __device__ __forceinline__ int group_of_step(const MfmaGrid& g, int step) {
 // Three workgroups per compute unit where the registers nearly allow it: left alone, one or two steps per wave at sixteen
 // rows take 169 to 185 of them, one occupancy step down.  us per launch, two -> three: groups of 32 3072 -> 23808 at M = 9 /
 // 16 33.8 / 35.8 -> 28.7 / 33.7, 9728 -> 18432 77.7 / 81.3 -> 67.4 / 71.7; groups of 64 11264 -> 24064 70.2 / 73.5 -> 62.8 /
-// 69.2, 4096 -> 14304 (896 workgroups) 22.7 / 23.7 -> 23.5 / 26.0; grids of up to 512 alike.
+// 69.2.  Over 540 to 2600 workgroups 0.92 times as long on average, 1.00 to 1.11 between 1150 and 1270; grids of up to 512
+// alike.
 template <int WAVES, int KS, int MC, int ROUNDS, int PRO = kProNone, int EPI = kEpiStore, bool LONE = false, bool WALK = false>
 __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEpiStore ? 3 : 2) void awq_gemv_mfma_kernel(
     const uint16_t* __restrict__ x, const uint32_t* __restrict__ qweight,
