@@ -494,12 +494,25 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
     static_assert(THREADS == kTileCols && kSliceCols == kHeadDim, "one thread per tile column, a slice is a head");
     float* s_sum = &red[0][0][0];  // a tile of finished rows, where one workgroup holds them all: the reduction buffer, free again
     static_assert(WAVES * MC >= ROWS, "the reduction buffer holds a tile of finished rows");
+    // Wave w finishes slices w, w + WAVES, ...; what they need besides the sums is asked for together, ahead of the barrier.
+    constexpr int PER_WAVE = (2 * ROWS + WAVES - 1) / WAVES;
+    Operands early[PER_WAVE];
+    auto request_all = [&] {
+        if constexpr (EPI != kEpiStore) {
+#pragma unroll
+            for (int j = 0; j < PER_WAVE; j++) {
+                const int i = min(wave + j * WAVES, 2 * M - 1);
+                early[j] = request(i >> 1, i & 1);
+            }
+        }
+    };
     auto finish_from_lds = [&] {
         __syncthreads();
-        for (int i = wave; i < 2 * M; i += WAVES) {
-            const int m = i >> 1, half = i & 1;
-            const float* src = s_sum + m * kTileCols + half * kSliceCols + lane;
-            finish(m, half, src[0], src[kWave], request(m, half));
+#pragma unroll
+        for (int j = 0; j < PER_WAVE; j++) {
+            const int i = wave + j * WAVES;
+            const float* src = s_sum + (i >> 1) * kTileCols + (i & 1) * kSliceCols + lane;
+            if (i < 2 * M) finish(i >> 1, i & 1, src[0], src[kWave], early[j]);
         }
     };
     if (ktiles == 1) {
@@ -509,6 +522,7 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
                 if (r < M && own_col < N) y[static_cast<size_t>(r) * N + own_col] = f32_to_bf16(psum[r]);
             }
         } else {
+            request_all();
             __syncthreads();
 #pragma unroll
             for (int r = 0; r < ROWS; r++) s_sum[r * kTileCols + tid] = psum[r];
@@ -520,6 +534,7 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
         float sum[ROWS];
         if constexpr (EPI == kEpiQkRope) {
             if (!splitk_exchange_sum<ROWS>(psum, sum, 0, M, N, ct, kt, ktiles, ct, partials, counters, s_word)) return;
+            request_all();
 #pragma unroll
             for (int r = 0; r < ROWS; r++) s_sum[r * kTileCols + tid] = sum[r];
             finish_from_lds();
@@ -556,17 +571,6 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
         }
         // the wide read-back hands out two columns and half of the rows per thread
         constexpr int HALF = ROWS / 2;
-        constexpr int PER_WAVE = 2 * ROWS / WAVES;  // slices a wave finishes below
-        Operands early[PER_WAVE];
-        auto request_all = [&] {
-            if constexpr (EPI != kEpiStore) {
-#pragma unroll
-                for (int j = 0; j < PER_WAVE; j++) {
-                    const int i = min(wave + j * WAVES, 2 * M - 1);
-                    early[j] = request(i >> 1, i & 1);
-                }
-            }
-        };
         float lo[HALF], hi[HALF];
         if (!splitk_exchange_sum_wide<ROWS, RUNS>(psum, lo, hi, M, N, ct, kt, ktiles, partials, counters, s_word, request_all, grid.run)) {
             return;
@@ -583,13 +587,7 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
         } else {
 #pragma unroll
             for (int i = 0; i < HALF; i++) *reinterpret_cast<f32x2*>(&s_sum[(row0 + i) * kTileCols + pair]) = f32x2{lo[i], hi[i]};
-            __syncthreads();
-#pragma unroll
-            for (int j = 0; j < PER_WAVE; j++) {
-                const int i = wave + j * WAVES;
-                const float* src = s_sum + (i >> 1) * kTileCols + (i & 1) * kSliceCols + lane;
-                if (i < 2 * M) finish(i >> 1, i & 1, src[0], src[kWave], early[j]);
-            }
+            finish_from_lds();
         }
     }
 }
