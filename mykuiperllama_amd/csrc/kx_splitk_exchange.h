@@ -26,7 +26,8 @@
 // In the language's memory model this is weaker than a release/acquire pair at agent scope; with such a pair
 // the compiler adds a write-back and invalidation of the whole L2 per workgroup (measured: 3 us more on a
 // 256-workgroup launch, 27 us on 2000 workgroups).  Because the argument is about this chip, other targets
-// are refused below, and tests/test_gpu_exchange_soak.py replays thousands of launches on one workspace.
+// are refused below, and tests/test_gpu_exchange_soak.py replays thousands of launches on one workspace, of one row and of
+// several.
 #ifndef KX_SPLITK_EXCHANGE_H
 #define KX_SPLITK_EXCHANGE_H
 
@@ -686,7 +687,7 @@ __device__ __forceinline__ bool splitk_exchange_sum_wide(const float (&psum)[ROW
 // tile in the tile's mask word and leaves, and the workgroup that arrives last takes over the marked slices.  Whoever
 // gives up looks at the arrivals once more after its mark is in memory, and whoever arrives last looks at the mask
 // after its arrival is: one of the two sees the other, and the bit, cleared by an atomic that returns it, decides who
-// finishes the slices.
+// finishes the slices.  tests/test_slice_handover.py goes through every interleaving of these steps.
 constexpr int kSliceCols = 128;
 constexpr int kSliceMaxKTiles = 64;           // bits of the mask word
 constexpr uint32_t kSliceDeparture = 0x10000u;

@@ -144,3 +144,113 @@ def test_chained_launches_on_one_workspace_repeat_their_first_results():
                     same = torch.equal(got.view(torch.int32) if got.dtype == torch.float32 else got.view(torch.int16),
                                        ref.view(torch.int32) if ref.dtype == torch.float32 else ref.view(torch.int16))
                     assert same, f"round {r}, set {i}: a {kind} launch differs from the first one"
+
+
+def _rows_problem(torch, gen, M, K, N):
+    codes = lambda rows: torch.randint(-2**31, 2**31, (rows, N // 8), dtype=torch.int32, device="cuda", generator=gen)
+    w = codes(K), (torch.rand((K // 128, N), device="cuda", generator=gen) * 0.019 + 0.001).half(), codes(K // 128)
+    return w, torch.randn((M, K), device="cuda", generator=gen).bfloat16()
+
+
+@pytest.mark.parametrize("M", [2, 3, 8, 16])
+def test_several_row_launches_on_one_workspace_repeat_their_first_results(M):
+    """Two and more rows: counters per wave, per workgroup and, from five rows on, arrivals, departures and masks of column
+    tiles that are finished together, all in the same area of one workspace.  About a thousand launches cycle over
+    shapes that finish together with few and with many K tiles, that have one reader, and that walk over blocks of K;
+    over the residual, rotary and norm forms; and over launches whose workgroups do not wait for each other."""
+    import torch
+    from mykuiperllama_amd import capi
+    lib = capi.load()
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(synth.BASE_SEED + 20 + M)
+    H, n_q, n_kv, positions = 4096, 32, 8, 32
+    wide = (n_q + 2 * n_kv) * 128
+    shapes = {"narrow": (H, 1024), "square": (H, H), "long": (12288, H), "wide": (H, 24576), "walk": (8704, 8192),
+              "longest": (25600, 2816), "qkv": (H, wide)}
+    probs = {name: _rows_problem(torch, gen, M, K, N) for name, (K, N) in shapes.items()}
+    ws = capi.make_workspace(M, 25600, 24576)
+    resid = torch.randn((M, H), device="cuda", generator=gen).bfloat16()
+    gains = [1 + 0.1 * torch.randn((n,), device="cuda", generator=gen) for n in (128, 128, H)]
+    q_gain, k_gain, norm_gain = (g.bfloat16() for g in gains)
+    pos = torch.arange(M, dtype=torch.int32, device="cuda") + 3
+    sums = torch.rand((M, H // 256, 4), device="cuda", generator=gen) * 64 + 1
+
+    def bf16(*shape):
+        return torch.zeros(shape, dtype=torch.bfloat16, device="cuda")
+
+    def plain(name, policy):
+        (K, N), (w, x) = shapes[name], probs[name]
+        y = bf16(M, N)
+        assert lib.kx_gemv_awq_bf16_policy(x.data_ptr(), *(t.data_ptr() for t in w), y.data_ptr(), M, K, N, 128,
+                                           ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream, policy) == 0
+        return (y,)
+
+    def residual(name):
+        (K, N), (w, x) = shapes[name], probs[name]
+        out, ssq = bf16(M, N), torch.zeros((M, N // 256, 4), dtype=torch.float32, device="cuda")
+        capi.gemv_awq_chain_bf16({"in_kind": capi.IN_ROW, "x": x, "rows": M, "out_kind": capi.OUT_RESIDUAL,
+                                  "residual_in": resid, "residual_out": out, "sumsq_out": ssq}, *w, K, N, 128, ws)
+        return out, ssq
+
+    def rotary():
+        w, x = probs["qkv"]
+        q, kc, vc = bf16(M, n_q * 128), bf16(M, positions, n_kv, 128), bf16(M, positions, n_kv, 128)
+        capi.gemv_awq_chain_bf16({"in_kind": capi.IN_ROW, "x": x, "rows": M, "out_kind": capi.OUT_QKV_ROPE, "q_gain": q_gain,
+                                  "k_gain": k_gain, "q_out": q, "k_cache": kc, "v_cache": vc, "pos": pos,
+                                  "rope_n_q_heads": n_q, "rope_n_kv_heads": n_kv, "cache_positions": positions,
+                                  "rope_theta": 1e6, "qk_eps": 1e-6, "cache_stride": positions * n_kv * 128}, *w, H, wide, 128, ws)
+        return q, kc, vc
+
+    def norm():
+        w, x = probs["wide"]
+        y = bf16(M, shapes["wide"][1])
+        capi.gemv_awq_chain_bf16({"in_kind": capi.IN_NORM, "norm_row": x, "norm_sumsq": sums, "norm_parts": H // 256,
+                                  "norm_gain": norm_gain, "norm_eps": 1e-6, "rows": M, "out_kind": capi.OUT_ROW, "y": y},
+                                 *w, H, shapes["wide"][1], 128, ws)
+        return (y,)
+
+    launches = [lambda n=n, p=p: plain(n, p) for p in (0, 3) for n in ("narrow", "square", "long", "wide", "walk", "longest")]
+    launches += [lambda: residual("square"), lambda: residual("long"), rotary, norm]
+    first = [launch() for launch in launches]
+    torch.cuda.synchronize()
+    for r in range(16):
+        sets = [[launch() for launch in launches] for _ in range(4)]  # no synchronisation in between
+        torch.cuda.synchronize()
+        for got in sets:
+            for i, (a, b) in enumerate(zip(got, first)):
+                assert all(torch.equal(x, y) for x, y in zip(a, b)), f"round {r}: launch {i} differs from its first result"
+    for i in range(6):  # waiting or not, the same sums
+        assert torch.equal(first[i][0], first[i + 6][0])
+
+
+@pytest.mark.parametrize("M", [5, 16])
+def test_two_streams_with_a_workspace_each(M):
+    """Grids that fill the chip on two streams at once, so that workgroups hold the places their neighbours need: the wait of
+    the shared finishing is bounded for this, whoever gives up hands its share on, and every launch still returns its bits."""
+    import torch
+    from mykuiperllama_amd import capi
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(synth.BASE_SEED + 40 + M)
+    shapes = [(4096, 16384), (25600, 2816), (12288, 4096), (1024, 2048)]  # 512 and 550 workgroups (walking), 384, small ones
+    probs = [_rows_problem(torch, gen, M, K, N) for K, N in shapes]
+    spaces = [capi.make_workspace(M, 25600, 16384) for _ in range(2)]
+
+    def launch(i, ws):
+        (w, x), y = probs[i], torch.zeros((M, shapes[i][1]), dtype=torch.bfloat16, device="cuda")
+        capi.gemv_awq_bf16(x, *w, y, 128, ws)
+        return y
+
+    first = [launch(i, spaces[0]) for i in range(len(shapes))]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in spaces]
+    for r in range(12):
+        got = [[], []]
+        for j in range(12):
+            for s, stream in enumerate(streams):
+                with torch.cuda.stream(stream):
+                    i = (j + s * (r % 4)) % len(shapes)  # the same shapes side by side, and different ones
+                    got[s].append((i, launch(i, spaces[s])))
+        torch.cuda.synchronize()
+        for s in range(2):
+            for i, y in got[s]:
+                assert torch.equal(y, first[i]), f"round {r}, stream {s}: {shapes[i]} differs"
