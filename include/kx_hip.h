@@ -86,7 +86,8 @@ int kx_gemv_awq_bf16(const uint16_t* x, const int32_t* qweight, const uint16_t* 
                      int32_t group_size, void* workspace, size_t workspace_bytes, void* stream);
 
 /* Two kernels implement kx_gemv_awq_bf16, chosen by shape: one on the vector ALUs and one on the matrix
- * cores (MFMA; M >= 2 and N >= 16).  The library keeps no state about the choice. */
+ * cores (MFMA; M >= 2 and N >= 16, except for some shapes with N an odd multiple of eight and groups that are no
+ * multiple of 64).  The library keeps no state about the choice. */
 
 /* kx_gemv_awq_bf16 for callers that cannot allocate or hand over a workspace (code under HIP graph capture,
  * serving loops and harnesses that forbid hipMalloc): the split-K workspace is a static device array inside
@@ -112,7 +113,8 @@ int kx_gemv_awq_bf16_static(const uint16_t* x, const int32_t* qweight, const uin
  * instead of two; M <= KX_MAX_BATCH).  Rounding points are those of the stand-alone kernels further
  * down; the K ranges of a column are added as fp32 in a fixed order here, so at M = 1 a call agrees with the two
  * separate calls to the rounding of that sum (kx_gemv_awq_bf16 adds them in fixed point there), at M >= 2 bit
- * for bit.
+ * for bit where both run on the same kernel (SwiGLU: see below; the norm form stays on the vector kernel and
+ * agrees to that rounding).
  *
  *   kx_gemv_awq_swiglu_bf16:  x[m,k] = bf16( bf16(silu(gate[m,k])) * up[m,k] ),  y = x W
  *       gate, up bf16, rows act_ld elements apart (act_ld >= K; halves of one [M, 2K] tensor or two
@@ -160,9 +162,9 @@ int kx_gemv_awq_qkv_rope_bf16(const uint16_t* residual, const uint16_t* delta, c
 
 /* ------------------------------------------------------------------------------------------
  * Chained GEMV: one launch whose activations come from the previous operator of a decoder
- * layer and whose result goes straight into the next one.  One activation row unless `rows` says otherwise.  `in_kind` selects where the activation
- * row x [K] comes from, `out_kind` what happens to the finished row o [N]; only the fields of the
- * selected kinds are read.
+ * layer and whose result goes straight into the next one.  One activation row unless `rows` says
+ * otherwise.  `in_kind` selects where the activation row x [K] comes from, `out_kind` what happens to the
+ * finished row o [N]; only the fields of the selected kinds are read.
  *
  *   KX_IN_ROW       x                                    bf16 [K], 16-byte aligned
  *   KX_IN_SWIGLU    gate, up                             x = bf16(bf16(silu(gate)) * up)

@@ -17,8 +17,10 @@
 //
 // and sum_k x comes out of one more MFMA against a B operand of ones, in the same register layout.
 // Raw sums of the waves of a workgroup meet in LDS; the thread that owns a column applies zero
-// point and scale once per wave (a wave never straddles a quantisation group: groups are powers of
-// two here and the host picks KS so that KS*32 divides the group) and takes part in the split-K exchange.
+// point and scale once per wave (a wave never straddles a quantisation group: groups are multiples of
+// 32 and the host picks KS so that KS*32 divides the group) and takes part in the split-K exchange.
+// The offset that cancels is 128 where the vector kernel has 16, which shows in the last bits of the fp32 sum only: against
+// float64 the bf16 outputs of both are 1.63e-3 to 1.70e-3 off, equal to six digits (K 512 to 25600, x of mean 0 and 1).
 //
 // Cost per weight: one VALU operation to build the operand (two byte permutes, three shifts and
 // eight and/or pairs per sixteen weights) and 1/512 of an MFMA, whatever M is.

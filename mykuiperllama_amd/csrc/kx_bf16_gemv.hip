@@ -98,16 +98,17 @@ __global__ __launch_bounds__(kRowsPerBlock * kWave) void bf16_gemv_kernel(
     }
 }
 
-// Three to sixteen activation rows: matrix cores, one pass over W whatever M is.
+// Three to sixteen activation rows, K > 8192 (up to there bf16_gemv_held_kernel serves): matrix cores, one pass over W
+// whatever M is.
 // v_mfma_f32_16x16x32_bf16 with A = the activations (row m = lane % 16, zero rows past M) and
 // B = sixteen rows of W (column n = lane % 16): lane (c, b) supplies x[c][32 s + 8 b .. + 7] and
 // W[n0 + c][32 s + 8 b .. + 7], sixteen contiguous bytes each, and receives y[4 b + v][n0 + c].
-// A workgroup owns BLOCKS blocks of sixteen output columns, which share every A operand.  One block
-// with eight steps in flight serves up to eight rows (lm_head 151936 x 4096: 270 us at M = 3..5, 300 at
-// 8); from nine rows on four blocks with four steps in flight each, so that the activation rows come out
-// of L2 once per 64 columns instead of once per 16 - at sixteen rows they are as many bytes as the sixteen
-// rows of W they meet, and with one block the L2 traffic for x equalled the HBM traffic for W (370 us at
-// M = 16, 299 with four blocks; at M = 3 four blocks are the slower choice, 297 us).  Its four waves take the
+// A workgroup owns kMfmaBlocks blocks of sixteen output columns, which share every A operand.  One block
+// with eight steps in flight serves up to eight rows (12288 -> 151936 925 / 930 / 1004 us at M = 3 / 5 / 8, 4.0 to 3.7 TB/s;
+// 12288 -> 4096 27.8 / 29.2 / 32.3); from nine rows on four blocks with four steps in flight each (924 / 947 us at M = 9 /
+// 16; 74 / 80), so that the activation rows come out of L2 once per 64 columns instead of once per 16 - at sixteen rows they
+// are as many bytes as the sixteen rows of W they meet, and with one block the L2 traffic for x equals the HBM traffic for
+// W (4096 -> 151936, one block against four: 370 / 299 us at M = 16, 270 / 297 at M = 3).  Its four waves take the
 // 32-element steps of K in turn (step s goes to wave s % 4; runs of consecutive steps per wave measured
 // slower) in sweeps of UNROLL steps with all loads of a sweep in flight together, and meet in LDS.  Addresses are clamped, what lies past K or M is zeroed
 // in both operands; per output the additions run in the same order whatever kMfmaBlocks is.
@@ -316,9 +317,11 @@ extern "C" int kx_gemv_bf16(const uint16_t* x, const uint16_t* w, uint16_t* y, i
     }
     hipStream_t s = kx::as_stream(stream);
     constexpr int kReach = 128 * kx::kHeldWaves;  // elements of K that a unit of every wave covers
-    // Two rows share the vector kernel's loads well enough where W is small (4096 x 4096: 8.4 against 9.0 us, 151936 x
-    // 1024: 52 against 57); with eight blocks per compute unit and rows of 8 KB its wave sums no longer hide (151936 x
-    // 4096: 202 against 182).
+    // Two rows share the vector kernel's loads well enough where W is small; with eight blocks per compute unit and rows of
+    // 8 KB its wave sums no longer hide.  us, vector -> held, 151936 outputs: K = 1024 50.9 -> 56.1, 2048 99 -> 99, 4096 204
+    // -> 187, 5120 269 -> 230, 8192 439 -> 380; 32768 outputs: 1024 13.4 -> 15.2, 2048 24.1 -> 25.8, 4096 46.4 -> 44.0, 8192
+    // 97.8 -> 85.2; 4096 outputs: 4096 9.0 -> 9.4, 8192 15.4 -> 15.5.  The line is on the safe side: K = 1536, 2560, 3072 and
+    // 3584 (6 to 15 % ahead from 32768 outputs on) and 16384 outputs from K = 4096 on (5 to 12 %) stay with the vector kernel.
     if ((M >= 3 || (M == 2 && K >= 4096 && N >= 32768)) && K <= 8 * kReach) {
         const int blocks = (N + 15) / 16;
         const dim3 grid(blocks < 256 ? blocks : 256), block(kx::kHeldWaves * kx::kWave);

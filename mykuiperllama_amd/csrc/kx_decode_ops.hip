@@ -397,7 +397,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_stage1(
 }
 
 constexpr int kMergeFront = 32;      // chunks per thread in the first flight: 128 chunks of the context
-constexpr int kMergeFrontLong = 80;  // 320 chunks
+constexpr int kMergeFrontLong = 80;  // 320 chunks: 40960 positions, the longest context that Qwen3 models are trained for
 constexpr int kMergeDimsLong = 32;
 
 // DIMS dimensions of a head per workgroup, FRONT chunks per thread in the first flight of loads.  What bounds it is the

@@ -272,9 +272,10 @@ class BatchDecodeModel:
     sequence ([B, positions, n_kv, 128] per layer) and activations of B rows.  The GEMVs run on the matrix-core
     kernel (2 <= B <= 16 rows), rotation and attention take the sequence as a grid dimension.
 
-    fused=True   six or seven launches per layer: q|k|v with the RMSNorm on the way in and rotation + cache append
-                 on the way out (a launch of its own with rope_in_qkv=False), attention (two stages), o with the residual add on the way out, gate|up with the RMSNorm on the way in,
-                 down with SwiGLU on the way in and the residual add on the way out
+    fused=True   six launches per layer: q|k|v with the RMSNorm on the way in and rotation + cache append on the way
+                 out (seven launches with rope_in_qkv=False), attention (two stages), o with the residual add on the way
+                 out, gate|up with the RMSNorm on the way in, down with SwiGLU on the way in and the residual add on
+                 the way out
     fused=False  every operator a launch of its own (SwiGLU one per sequence)
     The two agree to the rounding of the RMSNorm's sum of squares (added per 256 columns when fused).
     """

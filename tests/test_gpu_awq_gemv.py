@@ -147,8 +147,8 @@ def test_ragged_and_small_shapes(capi, torch, oracle, K, N, G):
                                    (1536, 784, 256), (384, 264, 128), (8192, 512, 128)])
 def test_ragged_shapes_with_many_rows(capi, torch, oracle, M, K, N, G):
     """Five to sixteen activation rows on column counts that end inside a tile (and, for the MFMA kernel's
-    two-column read-back, inside a pair of threads), on K that one workgroup covers, and on N that only
-    the vector kernel takes (not a multiple of sixteen)."""
+    two-column read-back, inside a pair of threads), on K that one workgroup covers, and on N that is an
+    odd multiple of eight, where the MFMA kernel's last word has no partner."""
     p = synth.make_awq_problem(f"ragged_rows_{M}_{K}x{N}", M, K, N, group=G)
     y, _ = run_awq(capi, torch, p)
     check_against_oracle(oracle, p, y)
