@@ -46,7 +46,12 @@ constexpr int kExchangeRows = 8;    // what a K tile's share of the split-K exch
 //            = 2, q|k|v and down ks = 4).  Against the single reader, us per launch at M = 8 / 16: k 4096 -> 1024
 //            7.6 / 10.2 -> 6.9 / 8.1, q 4096 -> 4096 8.2 / 10.7 -> 7.5 / 8.9, q|k|v 9.2 / 11.0 -> 8.6 / 9.8, down
 //            12288 -> 4096 15.4 / 18.9 -> 12.6 / 14.7, gate 4096 -> 12288 12.1 / 14.3 -> 12.0 / 12.6, 5120 -> 10240
-//            17.4 / 17.4 -> 12.9 / 14.1.  A K that one workgroup covers stays with one, which has nothing to exchange (512 ->
+//            17.4 / 17.4 -> 12.9 / 14.1.  Where that leaves two per compute unit and K ends in the first half of a block,
+//            half the run may need no more of them: behind a norm at M = 5 / 8 / 9 / 16 1152 -> 23040 (270 workgroups of
+//            four steps, 450 of two) 12.3 / 13.0 / 15.8 / 16.9 -> 10.0 / 10.2 / 12.4 / 13.8, 2304 -> 13824 (270, 486) 12.7 /
+//            12.6 / 15.5 / 16.5 -> 10.1 / 10.4 / 12.9 / 13.7, 3328 -> 9984 (273, 507) 12.7 / 12.9 / 15.6 / 16.6 -> 10.8 / 11.0 /
+//            13.4 / 14.6; with K a multiple of 512 there is no such case, and
+//            from two steps to one (groups of 64, 1664 -> 9344 at M = 11 / 16 10.7 / 11.3 -> 11.2 / 11.9) it loses.  A K that one workgroup covers stays with one, which has nothing to exchange (512 ->
 //            17920 at M = 8 / 16 8.1 / 10.7 -> 6.1 / 7.3, 512 -> 1280 6.6 / 8.3 -> 5.5 / 6.7).  Larger grids, whose workgroups
 //            come in rounds, keep the single reader: with shares the early ones would hold the places the late ones need
 //            (gate|up 4096 -> 24576 at M = 16: 19.7 against 21.5 us), and so do their column-tile-fastest order and 256 /
@@ -89,10 +94,12 @@ inline AwqPlan make_mfma_plan(int M, int K, int N, int group, bool may_walk = tr
     p.sliced = p.walks = false;
     p.run = 1;
     if (M >= 5) {
-        int best = 0;  // the longest run that is allowed, or the shortest that is short enough
+        int best = 0;  // the longest run that is allowed, or a shorter one that is short enough
         for (int c = 4; c >= 1; c /= 2) {
             if (best > 0 && ktiles_with(best) == 1) break;  // nothing to exchange
-            if (allowed(c) && (best == 0 || (p.coltiles * ktiles_with(c) <= kComputeUnits && ktiles_with(c) <= 16))) best = c;
+            if (!allowed(c) || (best > 0 && ktiles_with(c) > 16)) continue;
+            // one workgroup per compute unit, or two where twice the run leaves two as well (its last block mostly idle)
+            if (best == 0 || rounds_with(c) == 1 || (best == 4 && rounds_with(c) == 2 && rounds_with(best) == 2)) best = c;
         }
         const int kt = ktiles_with(best);
         if (kt == 1 || (kt <= kSliceMaxKTiles && p.coltiles * kt <= 2 * kComputeUnits)) {
