@@ -50,9 +50,10 @@ constexpr int kExchangeRows = 8;    // what a K tile's share of the split-K exch
 //            half the run may need no more of them: behind a norm at M = 5 / 8 / 9 / 16 1152 -> 23040 (270 workgroups of
 //            four steps, 450 of two) 12.3 / 13.0 / 15.8 / 16.9 -> 10.0 / 10.2 / 12.4 / 13.8, 2304 -> 13824 (270, 486) 12.7 /
 //            12.6 / 15.5 / 16.5 -> 10.1 / 10.4 / 12.9 / 13.7, 3328 -> 9984 (273, 507) 12.7 / 12.9 / 15.6 / 16.6 -> 10.8 / 11.0 /
-//            13.4 / 14.6; with K a multiple of 512 there is no such case, and
-//            from two steps to one (groups of 64, 1664 -> 9344 at M = 11 / 16 10.7 / 11.3 -> 11.2 / 11.9) it loses.  A K that one workgroup covers stays with one, which has nothing to exchange (512 ->
-//            17920 at M = 8 / 16 8.1 / 10.7 -> 6.1 / 7.3, 512 -> 1280 6.6 / 8.3 -> 5.5 / 6.7).  Larger grids, whose workgroups
+//            13.4 / 14.6; with K a multiple of 512 there is no such case, and from two steps to one (groups of 64, 1664 ->
+//            9344 at M = 11 / 16 10.7 / 11.3 -> 11.2 / 11.9) it loses.  A K that one workgroup covers stays with one, which
+//            has nothing to exchange (512 -> 17920 at M = 8 / 16 8.1 / 10.7 -> 6.1 / 7.3, 512 -> 1280 6.6 / 8.3 -> 5.5 /
+//            6.7; into the residual stream 512 -> 4096 6.6 / 8.6 -> 7.1 / 9.0).  Larger grids, whose workgroups
 //            come in rounds, keep the single reader: with shares the early ones would hold the places the late ones need
 //            (gate|up 4096 -> 24576 at M = 16: 19.7 against 21.5 us), and so do their column-tile-fastest order and 256 /
 //            512 rows per workgroup.
