@@ -76,6 +76,43 @@ __device__ __forceinline__ uint4 f32_to_bf16x8(const float (&f)[8]) {
     return make_uint4(w[0], w[1], w[2], w[3]);
 }
 
+// Sums of the waves in LDS, [wave][word half h][row][128 columns 16 c + 8 h + j], c < 16, j < 8: lane (c, b) writes two 16-byte
+// pieces per row.  The two change places in every other group of four lanes, so that eight lanes side by side write to all
+// banks.  What bounds this phase is the number of LDS writes: a ds_write_b128 takes the compute unit 13.5 cycles however many
+// of its lanes are active (22 to 33 where they meet in a quarter of the banks), a ds_read_b128 4.5.  So from four rows on the
+// lanes without a row of their own take over a part of the others' (v_permlane32_swap, v_permlane16_swap), which leaves
+// 16 / 8 / 4 writes per wave at 16 / 8 / 4 rows instead of 32 / 16 / 16, and a thread reads and stores four columns at a time.
+// us per launch, before -> now, M = 4 / 8 / 16: 4096 -> 1024 6.6 / 7.1 / 8.3 -> 6.4 / 6.9 / 7.5, 4096 -> 4096 into the residual
+// stream 7.8 / 8.2 / 9.5 -> 7.6 / 7.8 / 8.8, 12288 -> 4096 behind SwiGLU 13.5 / 15.1 / 17.8 -> 13.5 / 14.4 / 16.5,
+// 4096 -> 24576 behind a norm 16.9 / 21.1 / 24.3 -> 16.8 / 20.2 / 23.0; one and two rows alike.
+constexpr int kHalfCols = 128;
+__device__ __forceinline__ int red_piece(int piece) {  // 16-byte piece 0 .. 31 of a row of 128 columns -> where it lies
+    return piece ^ ((piece >> 3) & 1);
+}
+
+// Half `which` of the lanes of `a`, then of `b`; lanes 0 .. 15 of `a`, then of `b` (and the same of lanes 32 .. 63).
+__device__ __forceinline__ float half_wave_pack(float a, float b, int which) {
+    return __uint_as_float(__builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false)[which]);
+}
+__device__ __forceinline__ float quarter_wave_pack(float a, float b) {
+    return __uint_as_float(__builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false)[0]);
+}
+
+// A thread's columns: their sums, and the scales as loaded.
+template <int COLS>
+struct alignas(4 * COLS) FloatsOf {
+    float v[COLS];
+    __device__ __forceinline__ float& operator[](int i) { return v[i]; }
+    __device__ __forceinline__ float operator[](int i) const { return v[i]; }
+};
+template <int COLS>
+struct ScaleBits {
+    struct alignas(2 * COLS) type {
+        uint16_t v[COLS];
+        __device__ __forceinline__ uint16_t operator[](int i) const { return v[i]; }
+    };
+};
+
 template <bool LONE>
 struct WordPair {
     typedef u32x2 type;
@@ -111,7 +148,7 @@ __device__ __forceinline__ int group_of_step(const MfmaGrid& g, int step) {
 // Three workgroups per compute unit where the registers nearly allow it: left alone, one or two steps per wave at sixteen
 // rows take 169 to 185 of them, one occupancy step down.  us per launch, two -> three: groups of 32 3072 -> 23808 at M = 9 /
 // 16 33.8 / 35.8 -> 28.7 / 33.7, 9728 -> 18432 77.7 / 81.3 -> 67.4 / 71.7; groups of 64 11264 -> 24064 70.2 / 73.5 -> 62.8 /
-// 69.2.  Over 540 to 2600 workgroups 0.92 times as long on average, 1.00 to 1.11 between 1150 and 1270; grids of up to 512
+// 69.2 (with the sums' phase of that day).  Over 540 to 2600 workgroups 0.92 times as long on average, 1.00 to 1.11 between 1150 and 1270; grids of up to 512
 // alike.
 template <int WAVES, int KS, int MC, int ROUNDS, int PRO = kProNone, int EPI = kEpiStore, bool LONE = false, bool WALK = false>
 __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEpiStore ? 3 : 2) void awq_gemv_mfma_kernel(
@@ -144,8 +181,17 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
     constexpr int PIECES = ROWS * KPIECES;
     constexpr int PPT = (PIECES + THREADS - 1) / THREADS;  // pieces a thread produces
 
-    __shared__ __attribute__((aligned(16))) float red[WAVES][MC][kTileCols];
-    __shared__ float xs_red[WAVES][MC];
+    // From eight rows on a thread owns pieces of four columns, so that the sums are read, multiplied and stored sixteen bytes at
+    // a time: word half tid / 128, piece tid % 32 of its 128 columns, rows tid / 32 % 4 + 4 i.  Up to four rows a thread owns
+    // one column of each (four columns' scales and zero points cost a step of occupancy there).
+    constexpr bool QUADS = ROWS >= 8;
+    constexpr int OWN = QUADS ? 4 : 1;                 // columns of a thread
+    constexpr int RROWS = ROWS < 8 ? ROWS : 8;         // activation rows per LDS round
+    constexpr int RSUMS = QUADS ? RROWS / 4 : ROWS;    // rows of a thread per round
+    constexpr int PSUMS = QUADS ? ROWS / 4 : ROWS;     // rows of a thread
+
+    __shared__ __attribute__((aligned(16))) float red[WAVES][2][RROWS][kHalfCols];
+    __shared__ __attribute__((aligned(16))) float xs_red[WAVES][ROWS < 4 ? 4 : ROWS];
     __shared__ uint32_t s_word[3];
     __shared__ __attribute__((aligned(16))) uint16_t s_x[STAGED ? ROWS : 1][STAGED ? XPITCH : 8];
     __shared__ float s_inv[PRO == kProPreNorm ? ROWS : 1];
@@ -190,12 +236,15 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
     // (columns past N).  A load under a condition becomes a branch with a full wait behind it, and
     // a chain of those is a chain of memory round trips.
     //
-    // Scale and zero point of the column this thread will own after the LDS round, one pair per
+    // Scales and zero points of the columns this thread will own after the LDS round, one set per
     // wave of the workgroup (a wave never straddles a quantisation group; waves that share a group
     // read the same address).
-    const int own_col = ct * kTileCols + tid;
-    const int own_ld = own_col < N ? own_col : N - 1;
-    uint16_t s_bits[WAVES];
+    const int own_piece = tid % 32;
+    const int own_half = tid / 128;
+    const int own_row = tid / 32 % 4;
+    const int own_col = ct * kTileCols + (QUADS ? 16 * (own_piece / 2) + 8 * own_half + 4 * (own_piece % 2) : tid);  // the first
+    const int own_ld = own_col < N ? own_col : N - OWN;
+    typename ScaleBits<OWN>::type s_bits[WAVES];
     uint32_t z_word[WAVES];
     // The A operand: row c of the activations, whether or not column slot c holds weights.  Rows
     // past M and steps past K (K is a multiple of 32: a step is all in or all out) are zeros.
@@ -223,13 +272,6 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
                 else pb[i] = *reinterpret_cast<const uint4*>(fi.gain + kc);
             }
         }
-#pragma unroll
-        for (int wv = 0; wv < WAVES; wv++) {
-            const int krow = kblock + wv * WROWS;
-            const int g = group_of_step(grid, (krow < K ? krow : K - 1) / kStepRows);  // rows past K meet zero activations
-            s_bits[wv] = scales[static_cast<size_t>(g) * N + own_ld];
-            z_word[wv] = qzeros[static_cast<size_t>(g) * nw + (own_ld >> 3)];
-        }
         if constexpr (!STAGED) {
 #pragma unroll
             for (int ks = 0; ks < KS; ks++) {
@@ -255,7 +297,18 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
             }
         }
     };
+    auto load_scales = [&] {
+#pragma unroll
+        for (int wv = 0; wv < WAVES; wv++) {
+            const int krow = kblock + wv * WROWS;
+            const int g = group_of_step(grid, (krow < K ? krow : K - 1) / kStepRows);  // rows past K meet zero activations
+            s_bits[wv] = *reinterpret_cast<const typename ScaleBits<OWN>::type*>(scales + static_cast<size_t>(g) * N + own_ld);
+            z_word[wv] = qzeros[static_cast<size_t>(g) * nw + (own_ld >> 3)];
+        }
+    };
+    if constexpr (!STAGED) load_scales();
     load_operands();
+    if constexpr (STAGED) load_scales();
     load_weights();
     __builtin_amdgcn_sched_barrier(0);
 #if defined(KX_ABLATE) && KX_ABLATE == 2
@@ -268,7 +321,7 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
             for (int r = 0; r < 8; r++) f ^= w[ks][r][0] ^ w[ks][r][1];
         }
 #pragma unroll
-        for (int wv = 0; wv < WAVES; wv++) f ^= s_bits[wv] ^ z_word[wv];
+        for (int wv = 0; wv < WAVES; wv++) f ^= s_bits[wv][0] ^ z_word[wv];
         if (f == 0x9E3779B9u) partials[tid] = 1.0f;
         return;
     }
@@ -283,7 +336,7 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
         }
         lds_barrier();
     }
-    float psum[ROWS];
+    FloatsOf<OWN> psum[PSUMS];
     for (int block = 0; block < blocks; block++) {
         // ---- the activation prologue: produce the staged rows, then read the A operand back ----
         if constexpr (STAGED) {
@@ -362,78 +415,100 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
             __builtin_amdgcn_sched_barrier(0);
         }
 
-        float sc[WAVES], zc[WAVES];
+        // scales, and 128 + zero point, of the columns of the thread's pieces: nibbles 0, 4, 1, 5 of a word, or one byte up
+        FloatsOf<OWN> sc[WAVES], zc[WAVES];
 #pragma unroll
         for (int wv = 0; wv < WAVES; wv++) {
-            sc[wv] = f16_bits_to_f32(s_bits[wv]);
-            zc[wv] = -(128.0f + static_cast<float>((z_word[wv] >> (4 * nibble_of(own_col & 7))) & 0xFu));
+            const uint32_t zeros = z_word[wv] >> (QUADS ? 8 * (own_piece % 2) : 4 * nibble_of(own_col & 7));
+            const uint32_t even = (zeros & 0x000F000Fu) | 0x00800080u, odd = ((zeros >> 4) & 0x000F000Fu) | 0x00800080u;
+#pragma unroll
+            for (int j = 0; j < OWN; j++) {
+                sc[wv][j] = f16_bits_to_f32(s_bits[wv][j]);
+                const uint32_t both = j < 2 ? even : odd;
+                zc[wv][j] = static_cast<float>(j % 2 ? (both >> 16) & 0xFFu : both & 0xFFu);
+            }
         }
         auto load_next = [&] {
             if (block + 1 < blocks) {
                 kblock += KB;
                 load_operands();
+                if constexpr (STAGED) load_scales();
                 load_weights();
                 __builtin_amdgcn_sched_barrier(0);
             }
         };
         if constexpr (WALK && AHEAD) load_next();
 
-        // ---- waves meet in LDS; thread t < 256 then owns tile column t ----
-        // A round carries MC activation rows; a lane holds D rows 4b .. 4b+3 and joins the round they fall in.
-        constexpr int VR = MC < 4 ? MC : 4;  // rows of the lane's four that exist at all
+        // ---- waves meet in LDS; every thread then owns its columns ----
+        // D rows 4b .. 4b+3 of the lane; its sixteen columns are 16c .. 16c+15, those of word h eight of them.  A round writes
+        // with all lanes: eight rows fill half of them, and the word halves are packed side by side.
+        const int piece0 = 4 * red_piece(2 * c), piece1 = 4 * red_piece(2 * c + 1);
 #pragma unroll
-        for (int rd = 0; rd < ROUNDS; rd++) {
+        for (int rd = 0; rd < ROWS / RROWS; rd++) {
             if (rd > 0 || block > 0) lds_barrier();  // the previous round has been read
-            const int local0 = 4 * b - rd * MC;  // the lane's first row inside this round
-            if (local0 >= 0 && local0 < MC) {
-                // the lane's sixteen columns are 16c .. 16c+15
+            if (rd == 0 && c == 0 && 4 * b < ROWS) *reinterpret_cast<f32x4v*>(&xs_red[wave][4 * b]) = xs;
 #pragma unroll
-                for (int v = 0; v < VR; v++) {
+            for (int v = 0; v < (ROWS < 4 ? ROWS : 4); v++) {
+                if constexpr (ROWS >= 8) {
+                    float m[8];
+#pragma unroll
+                    for (int q = 0; q < 8; q++) m[q] = half_wave_pack(acc[0][q][v], acc[1][q][v], rd);
+                    float* dst = &red[wave][b / 2][4 * (b % 2) + v][0];
+                    *reinterpret_cast<f32x4*>(dst + piece0) = f32x4{m[0], m[4], m[1], m[5]};
+                    *reinterpret_cast<f32x4*>(dst + piece1) = f32x4{m[2], m[6], m[3], m[7]};
+                } else if constexpr (ROWS == 4) {  // a quarter of the lanes: every lane takes one of the four pieces of sixteen columns
+                    float m[4];
+#pragma unroll
+                    for (int q = 0; q < 4; q++) {
+                        const int e = q / 2 + 4 * (q % 2);  // nibble of the piece's column q; two further up in the second piece
+                        m[q] = half_wave_pack(quarter_wave_pack(acc[0][e][v], acc[0][e + 2][v]), quarter_wave_pack(acc[1][e][v], acc[1][e + 2][v]), 0);
+                    }
+                    *reinterpret_cast<f32x4*>(&red[wave][b / 2][v][b % 2 ? piece1 : piece0]) = f32x4{m[0], m[1], m[2], m[3]};
+                } else if (b == 0) {
 #pragma unroll
                     for (int h = 0; h < 2; h++) {
-                        f32x4* dst = reinterpret_cast<f32x4*>(&red[wave][local0 + v][16 * c + 8 * h]);
-                        dst[0] = f32x4{acc[h][nibble_of(0)][v], acc[h][nibble_of(1)][v], acc[h][nibble_of(2)][v],
-                                       acc[h][nibble_of(3)][v]};
-                        dst[1] = f32x4{acc[h][nibble_of(4)][v], acc[h][nibble_of(5)][v], acc[h][nibble_of(6)][v],
-                                       acc[h][nibble_of(7)][v]};
+                        float* dst = &red[wave][h][v][0];
+                        *reinterpret_cast<f32x4*>(dst + piece0) = f32x4{acc[h][0][v], acc[h][4][v], acc[h][1][v], acc[h][5][v]};
+                        *reinterpret_cast<f32x4*>(dst + piece1) = f32x4{acc[h][2][v], acc[h][6][v], acc[h][3][v], acc[h][7][v]};
                     }
-                    if (c == 0) xs_red[wave][local0 + v] = xs[v];
                 }
             }
             lds_barrier();
-            if (tid < kTileCols) {
-                constexpr int AT_ONCE = WALK ? 4 : MC;  // rows whose sums are read together: registers are short with a block in flight
+            FloatsOf<OWN> qv[RSUMS][WAVES];
+            float xv[RSUMS][WAVES];
 #pragma unroll
-                for (int v0 = 0; v0 < MC; v0 += AT_ONCE) {
-                    float qv[AT_ONCE][WAVES], xv[AT_ONCE][WAVES];
+            for (int i = 0; i < RSUMS; i++) {
+                const int row = QUADS ? own_row + 4 * i : i;
+                const int at = QUADS ? 4 * red_piece(own_piece) : 4 * red_piece(tid / 16 * 2 + tid / 4 % 2) + tid % 4;
 #pragma unroll
-                    for (int v = 0; v < AT_ONCE; v++) {
+                for (int wv = 0; wv < WAVES; wv++) {
+                    qv[i][wv] = *reinterpret_cast<const FloatsOf<OWN>*>(&red[wv][QUADS ? own_half : tid / 8 % 2][row][at]);
+                    xv[i][wv] = xs_red[wv][rd * RROWS + row];
+                }
+            }
 #pragma unroll
-                        for (int wv = 0; wv < WAVES; wv++) {
-                            qv[v][wv] = red[wv][v0 + v][tid];
-                            xv[v][wv] = xs_red[wv][v0 + v];
-                        }
+            for (int i = 0; i < RSUMS; i++) {
+#pragma unroll
+                for (int j = 0; j < OWN; j++) {
+                    float total = 0.0f;
+#pragma unroll
+                    for (int wv = 0; wv < WAVES; wv++) {
+                        total += sc[wv][j] * __builtin_fmaf(-zc[wv][j], xv[i][wv], qv[i][wv][j]);
                     }
-#pragma unroll
-                    for (int v = 0; v < AT_ONCE; v++) {
-                        float total = 0.0f;
-#pragma unroll
-                        for (int wv = 0; wv < WAVES; wv++) {
-                            total += sc[wv] * __builtin_fmaf(zc[wv], xv[v][wv], qv[v][wv]);
-                        }
-                        float& sum = psum[rd * MC + v0 + v];
-                        sum = WALK && block > 0 ? sum + total : total;
-                    }
-                    if constexpr (WALK) __builtin_amdgcn_sched_barrier(0);
+                    float& sum = psum[rd * RSUMS + i].v[j];
+                    sum = WALK && block > 0 ? sum + total : total;
                 }
             }
         }
         if constexpr (WALK && !AHEAD) load_next();
+        if constexpr (WALK && !STAGED) {  // the next block's operands are out: what its sums need comes last, where registers are free
+            if (block + 1 < blocks) load_scales();
+        }
     }
 
 #if defined(KX_ABLATE) && KX_ABLATE >= 1 && KX_ABLATE <= 3
     if (ktiles > 1) {  // profiling build: no exchange - every workgroup leaves its partial sums and is done
-        if (tid < kTileCols && own_col < N) partials[static_cast<size_t>(kt) * M * N + own_col] = psum[0];
+        if (own_col < N) partials[static_cast<size_t>(kt) * M * N + own_col] = psum[0][0];
         return;
     }
 #endif
@@ -494,8 +569,8 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
         }
     };
     static_assert(THREADS == kTileCols && kSliceCols == kHeadDim, "one thread per tile column, a slice is a head");
-    float* s_sum = &red[0][0][0];  // a tile of finished rows, where one workgroup holds them all: the reduction buffer, free again
-    static_assert(WAVES * MC >= ROWS, "the reduction buffer holds a tile of finished rows");
+    float* s_sum = &red[0][0][0][0];  // a tile of finished rows, where one workgroup holds them all: the reduction buffer, free again
+    static_assert(WAVES * 2 * RROWS * kHalfCols >= ROWS * kTileCols, "the reduction buffer holds a tile of finished rows");
     // Wave w finishes slices w, w + WAVES, ...; what they need besides the sums is asked for together, ahead of the barrier.
     constexpr int PER_WAVE = (2 * ROWS + WAVES - 1) / WAVES;
     Operands early[PER_WAVE];
@@ -517,25 +592,36 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
             if (i < 2 * M) finish(i >> 1, i & 1, src[0], src[kWave], early[j]);
         }
     };
+    const auto row_of = [&](int i) { return QUADS ? own_row + 4 * i : i; };  // row of psum[i]
     if (ktiles == 1) {
-        if constexpr (EPI == kEpiStore) {  // a thread stores its own column: nothing to hand over
+        if constexpr (EPI == kEpiStore) {  // a thread stores its own columns: nothing to hand over
 #pragma unroll
-            for (int r = 0; r < ROWS; r++) {
-                if (r < M && own_col < N) y[static_cast<size_t>(r) * N + own_col] = f32_to_bf16(psum[r]);
+            for (int i = 0; i < PSUMS; i++) {
+                const int r = row_of(i);
+                if (r < M && own_col < N) {
+                    uint16_t* dst = y + static_cast<size_t>(r) * N + own_col;
+                    if constexpr (QUADS) {
+                        *reinterpret_cast<u32x2*>(dst) = u32x2{f32x2_to_bf16x2(psum[i][0], psum[i][1]), f32x2_to_bf16x2(psum[i][2], psum[i][3])};
+                    } else {
+                        *dst = f32_to_bf16(psum[i][0]);
+                    }
+                }
             }
         } else {
             request_all();
             __syncthreads();
 #pragma unroll
-            for (int r = 0; r < ROWS; r++) s_sum[r * kTileCols + tid] = psum[r];
+            for (int i = 0; i < PSUMS; i++) *reinterpret_cast<FloatsOf<OWN>*>(&s_sum[row_of(i) * kTileCols + own_col - ct * kTileCols]) = psum[i];
             finish_from_lds();
         }
         return;
     }
     if constexpr (ROWS <= 2) {
-        float sum[ROWS];
+        float own[ROWS], sum[ROWS];
+#pragma unroll
+        for (int r = 0; r < ROWS; r++) own[r] = psum[r][0];
         if constexpr (EPI == kEpiQkRope) {
-            if (!splitk_exchange_sum<ROWS>(psum, sum, 0, M, N, ct, kt, ktiles, ct, partials, counters, s_word)) return;
+            if (!splitk_exchange_sum<ROWS>(own, sum, 0, M, N, ct, kt, ktiles, ct, partials, counters, s_word)) return;
             request_all();
 #pragma unroll
             for (int r = 0; r < ROWS; r++) s_sum[r * kTileCols + tid] = sum[r];
@@ -545,9 +631,9 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
             uint16_t rin[ROWS];
             if constexpr (EPI == kEpiResidual) {
 #pragma unroll
-                for (int r = 0; r < ROWS; r++) rin[r] = res.in[static_cast<size_t>(r < M ? r : M - 1) * N + own_ld];
+                for (int r = 0; r < ROWS; r++) rin[r] = res.in[static_cast<size_t>(r < M ? r : M - 1) * N + (own_col < N ? own_col : N - 1)];
             }
-            if (!splitk_exchange_sum_per_wave_rows<ROWS>(psum, sum, M, N, ct, kt, ktiles, partials, counters)) return;
+            if (!splitk_exchange_sum_per_wave_rows<ROWS>(own, sum, M, N, ct, kt, ktiles, partials, counters)) return;
             const bool col_ok = own_col < N;
 #pragma unroll
             for (int r = 0; r < ROWS; r++) {
@@ -564,9 +650,19 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
             }
         }
     } else {
+        // this workgroup's partial sums, sixteen bytes per lane and a row's 128 columns of a word half side by side
+        const __amdgpu_buffer_rsrc_t rsrc = partials_buffer(partials, static_cast<size_t>(ktiles) * M * N);
+#pragma unroll
+        for (int i = 0; i < PSUMS; i++) {
+            const int r = row_of(i);
+            if (r < M && own_col < N) {
+                if constexpr (!QUADS) store_agent(partials + (static_cast<size_t>(kt) * M + r) * N + own_col, psum[i][0]);
+                else store_partial_quad(rsrc, partial_column(own_col, N) + r * N, static_cast<uint32_t>(kt) * M * static_cast<uint32_t>(N), psum[i].v);
+            }
+        }
         if constexpr (ROWS >= 8) {
             if (grid.sliced) {
-                splitk_exchange_sliced<ROWS>(psum, M, N, ct, kt, ktiles, partials, counters, s_word, grid.wait_ticks, request,
+                splitk_exchange_sliced<ROWS>(M, N, ct, kt, ktiles, partials, counters, s_word, grid.wait_ticks, request,
                                              finish);
                 return;
             }
@@ -574,7 +670,7 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
         // the wide read-back hands out two columns and half of the rows per thread
         constexpr int HALF = ROWS / 2;
         float lo[HALF], hi[HALF];
-        if (!splitk_exchange_sum_wide<ROWS, RUNS>(psum, lo, hi, M, N, ct, kt, ktiles, partials, counters, s_word, request_all, grid.run)) {
+        if (!splitk_exchange_sum_wide<ROWS, RUNS>(lo, hi, M, N, ct, ktiles, partials, counters, s_word, request_all, grid.run)) {
             return;
         }
         const int row0 = (tid / (kTileCols / 2)) * HALF;

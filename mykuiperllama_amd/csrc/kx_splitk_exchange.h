@@ -71,6 +71,20 @@ __device__ __forceinline__ float load_partial(__amdgpu_buffer_rsrc_t rsrc, int l
                                                                           static_cast<int>(tile_floats * 4u), 16));
 }
 
+// Partial sums of eight and more rows (ROWS >= 8): where column `col` of a row lies.  The matrix-core kernel holds the columns of a tile
+// by word halves (columns 16 c + 8 h + j together for each h), and leaves them in that order; a last tile of fewer than 256
+// columns stays in column order, so that a row takes N floats either way.
+__device__ __forceinline__ int partial_column(int col, int N) {
+    const int x = col % kTileCols;
+    return col - x + kTileCols > N ? col : col - x + 128 * ((x >> 3) & 1) + 8 * (x >> 4) + (x & 7);
+}
+// Four neighbouring columns of a partial sum, written through like store_agent's, `at` floats (a multiple of
+// four) into the K tile that starts `tile_floats` floats into the buffer.
+__device__ __forceinline__ void store_partial_quad(__amdgpu_buffer_rsrc_t rsrc, int at, uint32_t tile_floats, const float (&v)[4]) {
+    const u32x4 bits = {__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3])};
+    __builtin_amdgcn_raw_buffer_store_b128(bits, rsrc, at * 4, static_cast<int>(tile_floats * 4u), 16);
+}
+
 // Called by every thread of the workgroup (it contains barriers).  Thread tid < 256 owns tile column
 // tid and brings psum[r], its partial sum for activation row m0 + r.  `s_prev` is one uint32 of LDS.
 // Returns true, the same in every thread, in the workgroup that ends up with the finished sums
@@ -575,7 +589,7 @@ __device__ __forceinline__ void splitk_sum_runs(__amdgpu_buffer_rsrc_t rsrc, int
 }
 
 // The exchange for several activation rows (ROWS = 4, 8 or 16) and a workgroup of exactly 256 threads, more
-// than one K tile.  Partial sums go out as above, one column per thread.  The last workgroup reads them back
+// than one K tile.  The caller has stored the workgroup's partial sums (store_partial_quad).  The last workgroup reads them back
 // two columns per load: threads 0..127 take rows 0 .. ROWS/2-1 of column pairs 0..127, threads 128..255 the
 // other rows, so a K tile costs a thread ROWS/2 eight-byte loads instead of ROWS four-byte ones and every
 // K tile of the usual shapes is in flight at once.  Per output the additions run t = 0, 1, 2, ... as in
@@ -586,21 +600,13 @@ __device__ __forceinline__ void splitk_sum_runs(__amdgpu_buffer_rsrc_t rsrc, int
 // (`hi`) of the tile.  `before_read_back()` runs in that workgroup once it knows it is the last one, ahead
 // of the read-back: loads issued there return under the read-back's round trip.
 template <int ROWS, bool RUNS = false, class Before>
-__device__ __forceinline__ bool splitk_exchange_sum_wide(const float (&psum)[ROWS], float (&lo)[ROWS / 2],
-                                                         float (&hi)[ROWS / 2], int M, int N, int ct, int kt,
+__device__ __forceinline__ bool splitk_exchange_sum_wide(float (&lo)[ROWS / 2], float (&hi)[ROWS / 2], int M, int N, int ct,
                                                          int ktiles, float* __restrict__ partials,
                                                          uint32_t* __restrict__ counters, uint32_t* s_prev,
                                                          Before&& before_read_back, int run = 1) {
     static_assert(ROWS == 4 || ROWS == 8 || ROWS == 16, "row counts the wide read-back is laid out for");
     const int tid = threadIdx.x;
-    const int col = ct * kTileCols + tid;
     const size_t tstride = static_cast<size_t>(M) * N;
-    if (col < N) {
-#pragma unroll
-        for (int r = 0; r < ROWS; r++) {
-            if (r < M) store_agent(partials + static_cast<size_t>(kt) * tstride + static_cast<size_t>(r) * N + col, psum[r]);
-        }
-    }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
@@ -628,7 +634,7 @@ __device__ __forceinline__ bool splitk_exchange_sum_wide(const float (&psum)[ROW
 #pragma unroll
     for (int i = 0; i < HALF; i++) lo[i] = hi[i] = 0.0f;
     if (col2 < static_cast<unsigned>(N)) {  // N is even: a pair is all in or all out
-        const int lane_bytes = static_cast<int>(col2 * sizeof(float));
+        const int lane_bytes = (ROWS >= 8 ? partial_column(static_cast<int>(col2), N) : static_cast<int>(col2)) * static_cast<int>(sizeof(float));
         if (RUNS && run > 1) {
             splitk_sum_runs<HALF, TB>(rsrc, lane_bytes, row0, M, N, ktiles, run, lo, hi);
             ktiles = 0;
@@ -722,12 +728,12 @@ __device__ __forceinline__ void splitk_slice_sum(__amdgpu_buffer_rsrc_t rsrc, in
     *b = sb;
 }
 
-// `psum[r]`: the thread's column (tid) of activation row r.  `finish(m, half, a, b, request(m, half))` is called by whole
+// The caller has stored the workgroup's partial sums.  `finish(m, half, a, b, request(m, half))` is called by whole
 // waves, once per (row m < M, half of the tile) in the whole launch, with the finished sums of columns 128 half + lane
 // (`a`) and 64 further (`b`), and the loads that `request` issued ahead of the read-back; columns past N bring garbage.
 // More than one K tile.  `s_word`: three uint32 of LDS.
 template <int ROWS, class Request, class Finish>
-__device__ __forceinline__ void splitk_exchange_sliced(const float (&psum)[ROWS], int M, int N, int ct, int kt, int ktiles,
+__device__ __forceinline__ void splitk_exchange_sliced(int M, int N, int ct, int kt, int ktiles,
                                                        float* __restrict__ partials, uint32_t* __restrict__ counters,
                                                        uint32_t* s_word, uint32_t wait_ticks, Request&& request,
                                                        Finish&& finish) {
@@ -735,14 +741,7 @@ __device__ __forceinline__ void splitk_exchange_sliced(const float (&psum)[ROWS]
     const int lane = tid % kWave;
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
     constexpr int WAVES = kTileCols / kWave;
-    const int col = ct * kTileCols + tid;
     const size_t tstride = static_cast<size_t>(M) * N;
-    if (col < N) {
-#pragma unroll
-        for (int r = 0; r < ROWS; r++) {
-            if (r < M) store_agent(partials + static_cast<size_t>(kt) * tstride + static_cast<size_t>(r) * N + col, psum[r]);
-        }
-    }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
@@ -760,7 +759,7 @@ __device__ __forceinline__ void splitk_exchange_sliced(const float (&psum)[ROWS]
             const int cb = ca + kWave;
             const auto operands = request(m, half);
             float a, b;
-            splitk_slice_sum(rsrc, M, N, ktiles, m, ca < N ? ca : N - 1, cb < N ? cb : N - 1, &a, &b);
+            splitk_slice_sum(rsrc, M, N, ktiles, m, partial_column(ca < N ? ca : N - 1, N), partial_column(cb < N ? cb : N - 1, N), &a, &b);
             finish(m, half, a, b, operands);
         }
     };
