@@ -61,20 +61,9 @@ __device__ __forceinline__ uint32_t code_pair_to_bf16(uint32_t v, uint32_t magic
     return (v & 0x000F000Fu) | magic;
 }
 
-// Eight consecutive bf16 of a 16-byte piece as floats, and back (round to nearest even).
-__device__ __forceinline__ void bf16x8_to_f32(const uint4& v, float (&f)[8]) {
-    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-    for (int i = 0; i < 8; i++) f[i] = __uint_as_float((i & 1) ? (w[i >> 1] & 0xffff0000u) : (w[i >> 1] << 16));
-}
-__device__ __forceinline__ uint4 f32_to_bf16x8(const float (&f)[8]) {
-    uint32_t w[4];
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        w[i] = static_cast<uint32_t>(f32_to_bf16(f[2 * i])) | (static_cast<uint32_t>(f32_to_bf16(f[2 * i + 1])) << 16);
-    }
-    return make_uint4(w[0], w[1], w[2], w[3]);
-}
+// Two neighbouring bf16 as floats.
+__device__ __forceinline__ float low_bf16(uint32_t w) { return __uint_as_float(w << 16); }
+__device__ __forceinline__ float high_bf16(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
 
 // Sums of the waves in LDS, [wave][word half h][row][128 columns 16 c + 8 h + j], c < 16, j < 8: lane (c, b) writes two 16-byte
 // pieces per row.  The two change places in every other group of four lanes, so that eight lanes side by side write to all
@@ -179,7 +168,8 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
     constexpr int XPITCH = KB + 8;
     constexpr int KPIECES = KB / 8;             // 16-byte pieces per staged row
     constexpr int PIECES = ROWS * KPIECES;
-    constexpr int PPT = (PIECES + THREADS - 1) / THREADS;  // pieces a thread produces
+    constexpr int PPT = (PIECES + THREADS - 1) / THREADS;  // pieces a thread produces, of the same k in every THREADS / KPIECES-th row
+    static_assert(THREADS % KPIECES == 0, "a thread's pieces share their k");
 
     // From eight rows on a thread owns pieces of four columns, so that the sums are read, multiplied and stored sixteen bytes at
     // a time: word half tid / 128, piece tid % 32 of its 128 columns, rows tid / 32 % 4 + 4 i.  Up to four rows a thread owns
@@ -216,7 +206,7 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
     // should run while the weights are still on their way ----
     // Piece e = tid + i * THREADS of the workgroup is (row e / KPIECES, elements 8 (e % KPIECES) .. + 7 of
     // the block); addresses are clamped, what a clamped load brings is replaced by zeros.
-    uint4 pa[STAGED ? PPT : 1], pb[STAGED ? PPT : 1];
+    uint4 pa[STAGED ? PPT : 1], pb[PRO == kProSwiGLU ? PPT : 1];  // gate or row; up, or the norm's gain, which all rows share
     float tile_ss[PRO == kProPreNorm ? (ROWS + WAVES - 1) / WAVES : 1];
     if constexpr (PRO == kProPreNorm) {
         // wave w adds the tiles of rows w, w + WAVES, ...: lane = tile
@@ -269,7 +259,7 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
                 const size_t at = static_cast<size_t>(mc) * fi.ld + kc;
                 pa[i] = *reinterpret_cast<const uint4*>(fi.a + at);
                 if constexpr (PRO == kProSwiGLU) pb[i] = *reinterpret_cast<const uint4*>(fi.b + at);
-                else pb[i] = *reinterpret_cast<const uint4*>(fi.gain + kc);
+                else if (i == 0) pb[0] = *reinterpret_cast<const uint4*>(fi.gain + kc);
             }
         }
         if constexpr (!STAGED) {
@@ -328,12 +318,16 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
 #endif
 
     if constexpr (PRO == kProPreNorm) {
+        // lane rr takes the total of row wave + rr * WAVES: one square root and division for all rows of the wave
+        constexpr int NORM_ROWS = (ROWS + WAVES - 1) / WAVES;
+        float mine = 0.0f;
 #pragma unroll
-        for (int rr = 0; rr < (ROWS + WAVES - 1) / WAVES; rr++) {
-            const int m = wave + rr * WAVES;
+        for (int rr = 0; rr < NORM_ROWS; rr++) {
             const float total = wave_sum(lane < fi.sumsq_parts ? tile_ss[rr] : 0.0f);
-            if (lane == 0 && m < ROWS) s_inv[m] = 1.0f / sqrtf(total / static_cast<float>(K) + fi.eps);
+            mine = lane == rr ? total : mine;
         }
+        const float inv = 1.0f / sqrtf(mine / static_cast<float>(K) + fi.eps);
+        if (lane < NORM_ROWS && wave + lane * WAVES < ROWS) s_inv[wave + lane * WAVES] = inv;
         lds_barrier();
     }
     FloatsOf<OWN> psum[PSUMS];
@@ -345,25 +339,24 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
                 const int e = tid + i * THREADS;
                 const int pm = e / KPIECES;
                 const int kp = e % KPIECES;
-                if (pm < ROWS) {
-                    float av[8], bv[8], out[8];
-                    bf16x8_to_f32(pa[i], av);
-                    bf16x8_to_f32(pb[i], bv);
-                    const bool live = pm < M && kblock + 8 * kp < K;  // K is a multiple of eight: a piece is all in or all out
-                    if constexpr (PRO == kProSwiGLU) {
+                if (PIECES % THREADS == 0 || pm < ROWS) {
+                    // Vector instructions bound the prologue (every column tile produces its rows anew), so two elements share a
+                    // conversion, the norm's gain is loaded and the inverse worked out once, and the words of a dead piece are
+                    // masked at the end: a select per element had become a branch per element.  us per launch at M = 8 / 16:
+                    // 4096 -> 24576 behind a norm 20.2 / 23.0 -> 19.6 / 21.0, q|k|v 10.1 / 12.0 -> 10.0 / 11.3.
+                    const uint32_t aw[4] = {pa[i].x, pa[i].y, pa[i].z, pa[i].w};
+                    const uint4 second = pb[PRO == kProSwiGLU ? i : 0];
+                    const uint32_t bw[4] = {second.x, second.y, second.z, second.w};
+                    const uint32_t keep = pm < M && kblock + 8 * kp < K ? 0xffffffffu : 0u;  // K is a multiple of eight: all in or all out
+                    const float inv = PRO == kProPreNorm ? s_inv[pm] : 0.0f;
+                    uint32_t out[4];
 #pragma unroll
-                        for (int j = 0; j < 8; j++) {
-                            const float act = silu_rounded_to_bf16(av[j]);
-                            out[j] = live ? act * bv[j] : 0.0f;
-                        }
-                    } else {
-                        const float inv = s_inv[pm];
-#pragma unroll
-                        for (int j = 0; j < 8; j++) {
-                            out[j] = live ? bv[j] * bf16_to_f32(f32_to_bf16(av[j] * inv)) : 0.0f;
-                        }
+                    for (int j = 0; j < 4; j++) {
+                        const float lo = low_bf16(aw[j]), hi = high_bf16(aw[j]);
+                        const uint32_t act = PRO == kProSwiGLU ? f32x2_to_bf16x2(silu(lo), silu(hi)) : f32x2_to_bf16x2(lo * inv, hi * inv);
+                        out[j] = f32x2_to_bf16x2(low_bf16(act) * low_bf16(bw[j]), high_bf16(act) * high_bf16(bw[j])) & keep;
                     }
-                    *reinterpret_cast<uint4*>(&s_x[pm][8 * kp]) = f32_to_bf16x8(out);
+                    *reinterpret_cast<uint4*>(&s_x[pm][8 * kp]) = make_uint4(out[0], out[1], out[2], out[3]);
                 }
             }
             lds_barrier();

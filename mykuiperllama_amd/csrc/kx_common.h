@@ -70,14 +70,17 @@ __device__ __forceinline__ void store_result(T* p, T v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// bf16(silu(g)), g / (1 + exp(-g)), as every SwiGLU of the library computes it: the hardware's exponential and
+// silu(g), g / (1 + exp(-g)), as every SwiGLU of the library computes it, ahead of its rounding to bf16: the hardware's exponential and
 // reciprocal (v_exp_f32, v_rcp_f32: each good to about one unit in the last place of fp32, the product
 // -g * log2(e) to a few more for large |g|), far inside the bf16 rounding that follows.  The library expf and a
 // true division cost some 35 instructions per element against 8, which a launch that produces sixteen rows of
 // activations in its prologue feels (down projection at sixteen rows: 26.0 -> 23.5 us).
-__device__ __forceinline__ float silu_rounded_to_bf16(float g) {
+__device__ __forceinline__ float silu(float g) {
     const float e = __builtin_amdgcn_exp2f(-g * 1.44269504088896341f);
-    return bf16_to_f32(f32_to_bf16(g * __builtin_amdgcn_rcpf(1.0f + e)));
+    return g * __builtin_amdgcn_rcpf(1.0f + e);
+}
+__device__ __forceinline__ float silu_rounded_to_bf16(float g) {
+    return bf16_to_f32(f32_to_bf16(silu(g)));
 }
 
 // Operand and result types of v_mfma_f32_16x16x32_bf16: lane l supplies eight consecutive k
