@@ -4,6 +4,7 @@ Device memory comes from torch tensors (plumbing only): the binding passes `tens
 and torch's current HIP stream.  There is no fallback: if libkx_hip.so is missing, loading
 raises, and every entry point turns a non-zero return code into an exception.
 """
+import array
 import ctypes
 import os
 
@@ -56,9 +57,10 @@ SIGNATURES = {
 }
 
 
-# entry points outside the drop-in boundary (csrc/kx_internal.h): tests and the benchmark only
+# entry points outside the drop-in boundary (csrc/kx_internal.h): tests, the benchmark and the decode step of decode.py
 INTERNAL_SIGNATURES = {
     "kx_gemv_awq_bf16_policy": (ctypes.c_int, [_P, _P, _P, _P, _P, _I32, _I32, _I32, _I32, _P, _SZ, _P, _I32]),
+    "kx_decode_step_bf16": (ctypes.c_int, [_P, _P, _P]),
 }
 
 
@@ -79,6 +81,18 @@ class ChainDesc(ctypes.Structure):
         ("rows", _I32), ("act_ld", _I32), ("cache_stride", _SZ),
     ]
 
+
+class StepDesc(ctypes.Structure):
+    """Mirror of kx_step_desc (csrc/kx_internal.h), field for field."""
+    _fields_ = [(n, _P) for n in ("embed", "token", "pos", "final_norm", "lm_head", "x", "h", "q", "attn", "gate_up",
+                                  "logits", "sumsq", "next_token")] + [
+        ("gemv_workspace", _P), ("gemv_workspace_bytes", _SZ), ("attn_workspace", _P), ("attn_workspace_bytes", _SZ)] + [
+        (n, _I32) for n in ("layers", "hidden", "intermediate", "n_q", "n_kv", "group", "max_positions", "norm_parts",
+                            "merge_in_o", "embed_rows", "head_rows", "logits_n")] + [
+        ("rope_theta", ctypes.c_float), ("eps", ctypes.c_float)]
+
+
+STEP_LAYER_WORDS = 19  # eight-byte words of a kx_step_layer
 
 IN_ROW, IN_SWIGLU, IN_ATTN, IN_NORM = 0, 1, 2, 3
 OUT_ROW, OUT_RESIDUAL, OUT_QKV_ROPE = 0, 1, 2
@@ -116,6 +130,11 @@ def load(path=None):
     if built_as != ABI_VERSION:
         raise RuntimeError(f"{lib_path} was built as ABI version {built_as}, this binding mirrors version "
                            f"{ABI_VERSION} of include/kx_hip.h (ChainDesc would not match kx_chain_desc)")
+    global _raw_stream, _get_device
+    raw, device = getattr(torch._C, "_cuda_getCurrentRawStream", None), getattr(torch._C, "_cuda_getDevice", None)
+    if raw is not None and device is not None:
+        _get_device = device
+        _raw_stream = raw
     _lib = lib
     return lib
 
@@ -162,9 +181,21 @@ def _check(code):
         raise KxError(code, load().kx_error_string(code).decode())
 
 
-def _stream():
+def _current_stream():
     import torch
     return torch.cuda.current_stream().cuda_stream
+
+
+def _stream():
+    """Handle of torch's current stream on the current device."""
+    if _raw_stream is None:
+        return _current_stream()
+    return _raw_stream(_get_device())
+
+
+# torch's own bindings behind current_stream(): a tenth of its time, which was a third of a small launch on the host.
+# Looked up once the library is loaded; without them the public call serves.
+_raw_stream = _get_device = None
 
 
 def _ptr(t):
@@ -195,9 +226,11 @@ def gemv_awq_bf16(x, qweight, scales, qzeros, y, group_size, workspace):
                                               M, K, N, group_size, _ptr(workspace),
                                               0 if workspace is None else workspace.numel(), _stream(), _policy))
         return
-    _check(load().kx_gemv_awq_bf16(_ptr(x), _ptr(qweight), _ptr(scales), _ptr(qzeros), _ptr(y),
-                                   M, K, N, group_size, _ptr(workspace),
-                                   0 if workspace is None else workspace.numel(), _stream()))
+    code = (_lib or load()).kx_gemv_awq_bf16(_ptr(x), _ptr(qweight), _ptr(scales), _ptr(qzeros), _ptr(y),
+                                             M, K, N, group_size, _ptr(workspace),
+                                             0 if workspace is None else workspace.numel(), _stream())
+    if code:
+        _check(code)
 
 
 def gemv_awq_bf16_static(x, qweight, scales, qzeros, y, group_size):
@@ -338,6 +371,16 @@ def gemv_awq_chain_bf16(desc, qweight, scales, qzeros, K, N, group_size, workspa
         setattr(d, name, value.data_ptr() if hasattr(value, "data_ptr") else value)
     _check(load().kx_gemv_awq_chain_bf16(ctypes.byref(d), _ptr(qweight), _ptr(scales), _ptr(qzeros), K, N, group_size,
                                          _ptr(workspace), 0 if workspace is None else workspace.numel(), _stream()))
+
+
+def decode_step_bf16(fields, layer_words):
+    """One decode step in one call: see kx_decode_step_bf16.  `fields` maps the fields of StepDesc to tensors, None or
+    scalars (the number of layers aside); `layer_words` holds STEP_LAYER_WORDS integers per layer."""
+    layers = array.array("q", layer_words)
+    d = StepDesc(layers=len(layer_words) // STEP_LAYER_WORDS)
+    for name, value in fields.items():
+        setattr(d, name, value.data_ptr() if hasattr(value, "data_ptr") else value)
+    _check(load().kx_decode_step_bf16(ctypes.addressof(d), layers.buffer_info()[0], _stream()))
 
 
 FUSED_MERGE_MAX_POSITIONS = 80 * 128  # the o projection merges at most 80 chunks (of 128 positions past 5120)

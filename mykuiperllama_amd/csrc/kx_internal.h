@@ -1,7 +1,7 @@
 /*
  * Entry points of libkx_hip.so that are not part of the drop-in boundary (include/kx_hip.h): what the
- * tests and the benchmark need to put one particular kernel under a shape.  No state is kept: the
- * choice travels with the call.
+ * tests and the benchmark need to put one particular kernel under a shape, and the decode step of the Python
+ * driver in one call.  No state is kept: everything travels with the call.
  */
 #ifndef KX_INTERNAL_H
 #define KX_INTERNAL_H
@@ -26,6 +26,44 @@ int kx_gemv_awq_bf16_policy(const uint16_t* x, const int32_t* qweight, const uin
                             const int32_t* qzeros, uint16_t* y, int32_t M, int32_t K, int32_t N,
                             int32_t group_size, void* workspace, size_t workspace_bytes, void* stream,
                             int32_t policy);
+
+/* One decode step of one sequence (mykuiperllama_amd.decode, the chained form): the same calls of include/kx_hip.h in the
+ * same order as the Python driver would make, from native code.  Through ctypes a call costs the host 9 us, more than
+ * most of the launches take on the GPU: a step of 28 layers of 1024 hidden that is not captured in a graph took 1380 us,
+ * and takes 800 this way.  Stops at the first call that is refused and returns its code; the pointers are read during
+ * the call only.  A layer is nineteen eight-byte words. */
+typedef struct kx_step_matrix {
+    const int32_t* qweight;
+    const uint16_t* scales;
+    const int32_t* qzeros;
+} kx_step_matrix;
+
+typedef struct kx_step_layer {
+    kx_step_matrix qkv, o, gate_up, down;
+    const uint16_t *in_norm, *post_norm, *q_norm, *k_norm;
+    uint16_t *k_cache, *v_cache;
+    int64_t cache_positions;
+} kx_step_layer;
+
+typedef struct kx_step_desc {
+    const uint16_t* embed;
+    const int32_t* token;
+    const int32_t* pos;
+    const uint16_t* final_norm;
+    const uint16_t* lm_head; /* null: the step ends with the normalised row */
+    uint16_t *x, *h, *q, *attn, *gate_up, *logits;
+    float* sumsq;
+    int32_t* next_token;
+    void* gemv_workspace;
+    size_t gemv_workspace_bytes;
+    void* attn_workspace;
+    size_t attn_workspace_bytes;
+    int32_t layers, hidden, intermediate, n_q, n_kv, group, max_positions, norm_parts, merge_in_o;
+    int32_t embed_rows, head_rows, logits_n;
+    float rope_theta, eps;
+} kx_step_desc;
+
+int kx_decode_step_bf16(const kx_step_desc* desc, const kx_step_layer* layers, void* stream);
 
 #ifdef __cplusplus
 }

@@ -216,49 +216,23 @@ class DecodeModel:
 
     def _step_chain(self, with_lm_head):
         c = self.cfg
-        g, ws = c.group, self.gemv_ws
-        H, I = c.hidden, c.intermediate
-        merge_in_o = self.merge_in_o
-        capi.embedding_bf16(self.embed, self.token, self.x)
-        x, ssq = self.x, self.ssq
-        rope = {"out_kind": capi.OUT_QKV_ROPE, "q_out": self.q, "pos": self.pos, "rope_n_q_heads": c.n_q,
-                "rope_n_kv_heads": c.n_kv, "rope_theta": c.rope_theta, "qk_eps": c.eps}
-        into_residual = {"out_kind": capi.OUT_RESIDUAL, "residual_in": x, "residual_out": x, "sumsq_out": ssq}
-        for li, L in enumerate(self.layers):
-            qw, sc, qz = L["qkv"]
-            if li == 0:  # the embedding row comes without its sums of squares
-                capi.gemv_awq_qkv_rope_bf16(x, None, L["in_norm"], c.eps, None, qw, sc, qz, L["q_norm"], L["k_norm"],
-                                            self.q, self.k_cache[li], self.v_cache[li], c.n_q, c.n_kv, self.pos,
-                                            c.rope_theta, c.eps, g, ws)
-            else:
-                capi.gemv_awq_chain_bf16(dict(rope, in_kind=capi.IN_NORM, norm_row=x, norm_sumsq=ssq,
-                                              norm_parts=ssq.shape[0], norm_gain=L["in_norm"], norm_eps=c.eps,
-                                              q_gain=L["q_norm"], k_gain=L["k_norm"], k_cache=self.k_cache[li],
-                                              v_cache=self.v_cache[li]), qw, sc, qz, H, c.qkv_out, g, ws)
-            qw, sc, qz = L["o"]
-            if merge_in_o:
-                capi.attn_decode_partial_bf16(self.q, self.k_cache[li], self.v_cache[li], c.n_q, c.n_kv, self.pos,
-                                              self.max_positions, self.attn_ws)
-                capi.gemv_awq_chain_bf16(dict(into_residual, in_kind=capi.IN_ATTN, attn_workspace=self.attn_ws,
-                                              attn_workspace_bytes=self.attn_ws.numel(), n_q_heads=c.n_q,
-                                              n_kv_heads=c.n_kv, max_positions=self.max_positions),
-                                         qw, sc, qz, c.n_q * c.head_dim, H, g, ws)
-            else:
-                capi.attn_decode_bf16(self.q, self.k_cache[li], self.v_cache[li], self.attn, c.n_q, c.n_kv,
-                                      self.pos, self.max_positions, self.attn_ws)
-                capi.gemv_awq_chain_bf16(dict(into_residual, in_kind=capi.IN_ROW, x=self.attn),
-                                         qw, sc, qz, c.n_q * c.head_dim, H, g, ws)
-            qw, sc, qz = L["gateup"]
-            capi.gemv_awq_chain_bf16({"in_kind": capi.IN_NORM, "norm_row": x, "norm_sumsq": ssq,
-                                      "norm_parts": ssq.shape[0], "norm_gain": L["post_norm"], "norm_eps": c.eps,
-                                      "out_kind": capi.OUT_ROW, "y": self.gu}, qw, sc, qz, H, 2 * I, g, ws)
-            qw, sc, qz = L["down"]
-            capi.gemv_awq_chain_bf16(dict(into_residual, in_kind=capi.IN_SWIGLU, gate=self.gu[:, :I],
-                                          up=self.gu[:, I:]), qw, sc, qz, I, H, g, ws)
-        capi.rmsnorm_bf16(x, self.final_norm, self.h, c.eps)
-        if with_lm_head:
-            capi.gemv_bf16(self.h, self.lm_head, self.logits)
-            capi.argmax_bf16(self.logits, self.next_token)
+        # One native call for all launches; the addresses are looked up anew in every step, so that tensors may be replaced
+        # between steps as with any other form.
+        words = []
+        for L, kc, vc in zip(self.layers, self.k_cache, self.v_cache):
+            words += [t.data_ptr() for t in (*L["qkv"], *L["o"], *L["gateup"], *L["down"], L["in_norm"], L["post_norm"],
+                                             L["q_norm"], L["k_norm"], kc, vc)]
+            words.append(min(kc.shape[0], vc.shape[0]))
+        capi.decode_step_bf16({
+            "embed": self.embed, "token": self.token, "pos": self.pos, "final_norm": self.final_norm,
+            "lm_head": self.lm_head if with_lm_head else None, "x": self.x, "h": self.h, "q": self.q, "attn": self.attn,
+            "gate_up": self.gu, "logits": self.logits, "sumsq": self.ssq, "next_token": self.next_token,
+            "gemv_workspace": self.gemv_ws, "gemv_workspace_bytes": self.gemv_ws.numel(),
+            "attn_workspace": self.attn_ws, "attn_workspace_bytes": self.attn_ws.numel(),
+            "hidden": c.hidden, "intermediate": c.intermediate, "n_q": c.n_q, "n_kv": c.n_kv, "group": c.group,
+            "max_positions": self.max_positions, "norm_parts": self.ssq.shape[0], "merge_in_o": bool(self.merge_in_o),
+            "embed_rows": self.embed.shape[0], "head_rows": self.lm_head.shape[0], "logits_n": self.logits.numel(),
+            "rope_theta": c.rope_theta, "eps": c.eps}, words)
 
     def launches_per_step(self, with_lm_head=True, fused=True):
         per_layer = 10
