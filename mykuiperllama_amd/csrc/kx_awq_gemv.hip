@@ -13,6 +13,7 @@ struct AwqPlan {
     bool mfma;     // matrix-core kernel or the VALU kernel
     int run;       // MFMA kernel: blocks of K whose sums are added up before they join the others'
     bool walks;    // MFMA kernel: a workgroup walks over such a run; otherwise the read-back adds in that order
+    bool fine;     // MFMA kernel: the steps of a wave lie in groups of their own
     bool sliced;   // MFMA kernel: all workgroups of a column tile finish it together
     int waves;     // waves per workgroup stacked along K (4, 8 or 16)
     int rt;        // VALU kernel: consecutive rows per lane (8 or 16); MFMA kernel: 32-row steps per wave
@@ -29,8 +30,8 @@ inline int rows_per_block(int waves, int rt) {
 constexpr int kComputeUnits = 256;  // MI355X
 constexpr int kExchangeRows = 8;    // what a K tile's share of the split-K exchange costs, in rows of K streamed
 
-// MFMA kernel: four waves per workgroup, each walking `ks` consecutive 32-row steps that must lie in one quantisation
-// group.  What it costs besides the weights is the exchange of partial sums, M KB per K tile and column tile.
+// MFMA kernel: four waves per workgroup, each walking `ks` consecutive 32-row steps, in one quantisation group or (below) across
+// them.  What it costs besides the weights is the exchange of partial sums, M KB per K tile and column tile.
 //   M <= 4   one workgroup (or wave) of a column tile reads all of them back, sixteen K tiles in flight: two steps per
 //            wave, or four where that brings the K tiles down to one such batch and gives the busiest compute unit no
 //            more rows to stream (or saves three rows and more a nearly full second batch), on at most two workgroups per
@@ -76,9 +77,11 @@ constexpr int kExchangeRows = 8;    // what a K tile's share of the split-K exch
 // group size alone, so that the launches of a shape return the same bits (one that does not walk leaves the runs to the
 // read-back, splitk_sum_runs: 14336 -> 5120 behind SwiGLU at M = 16 30.3 us with K tiles in order, 29.9 in runs).
 // `may_walk`: the kernel exists in a form that walks; `produced_x`: its activations are produced on the way in.
-inline AwqPlan make_mfma_plan(int M, int K, int N, int group, bool may_walk = true, bool produced_x = false) {
+inline AwqPlan make_mfma_plan(int M, int K, int N, int group, bool may_walk = true, bool produced_x = false,
+                              bool may_cross_groups = true) {
     AwqPlan p;
     p.mfma = true;
+    p.fine = false;
     p.coltiles = (N / 8 + kWC - 1) / kWC;
     p.mb = M;
     p.mtiles = 1;
@@ -91,14 +94,31 @@ inline AwqPlan make_mfma_plan(int M, int K, int N, int group, bool may_walk = tr
         (2 * rounds_with(4) <= rounds_with(2) || (M >= 3 && ktiles_with(2) >= 30))) {
         ks = 4;
     }
-    while (!allowed(ks)) ks /= 2;
+    // Groups that leave a wave one or two steps make a K tile of every 128 or 256 rows.  Where there are many of them, four
+    // steps across groups, scaled step by step, cost less than the exchange; few of them are better met by the shorter
+    // run.  us per launch, inside a group -> across: groups of 32 5472 -> 9000 (43 tiles) at M = 4 / 6 / 11 / 16 19.0 / 24.0 /
+    // 32 / 34 -> 15.9 / 16.8 / 17.1 / 17.9, 12288 -> 4096 behind SwiGLU at M = 2 / 4 / 6 / 16 14.5 / 17.9 / 26.5 / 45 -> 13.2 /
+    // 15.0 / 15.9 / 17.8, 4096 -> 12288 (32) at M = 6 / 16 16.5 / 24.5 -> 12.6 / 13.7, 1536 -> 17920 (groups of 96, 12) 11.9 /
+    // 18.7 -> 10.7 / 13.6, 3072 -> 5120 (24, 480 workgroups) 10.2 / 12.0 -> 9.6 / 11.3; groups of 64 16384 -> 4096 (64) at
+    // M = 2 / 4 / 6 / 16 13.5 / 15.2 / 21.8 / 33.5 -> 12.3 / 14.0 / 14.9 / 16.2, 5120 -> 5120 (20, 400) at M = 6 / 16 11.5 / 12.7
+    // -> 10.5 / 12.1.  What the rule leaves out: groups of 32 at M = 2 / 4 3072 -> 5120 7.5 / 8.5 -> 7.9 / 9.1; 2560 -> 4096
+    // (20, 320) at M = 6 / 11 9.9 / 10.1 -> 10.2 / 12.1, 3072 -> 1024 (24, 96) 7.4 / 7.7 -> 8.8 / 9.6, 1280 -> 10240 (10, 400)
+    // at M = 6 / 16 8.9 / 11.2 -> 10.3 / 12.7; groups of 64 4096 -> 12288 (16) at M = 2 / 4 / 8 9.5 / 10.2 / 12.2 -> 11.0 /
+    // 12.3 / 13.3, 9728 -> 512 (38, 76) at M = 6 9.0 -> 9.8.
+    const int inside = allowed(2) ? 2 : 1;
+    const int inside_kt = ktiles_with(inside);
+    const int line = inside == 2 ? (M <= 2 ? 60 : (M <= 4 ? 52 : (M <= 8 ? 16 : 8))) : (M <= 2 ? 48 : (M <= 4 ? 32 : 8));
+    const bool crosses = may_cross_groups && !allowed(4) && p.waves * 4 * kStepRows <= K && inside_kt > line &&
+                         (inside_kt > 48 || 8 * p.coltiles * inside_kt > (inside_kt < 20 ? 16 : 11) * kComputeUnits);
+    if (crosses) ks = 4;
+    else while (!allowed(ks)) ks /= 2;
     p.sliced = p.walks = false;
     p.run = 1;
     if (M >= 5) {
         int best = 0;  // the longest run that is allowed, or a shorter one that is short enough
         for (int c = 4; c >= 1; c /= 2) {
             if (best > 0 && ktiles_with(best) == 1) break;  // nothing to exchange
-            if (!allowed(c) || (best > 0 && ktiles_with(c) > 16)) continue;
+            if ((!allowed(c) && !(crosses && c == 4)) || (best > 0 && ktiles_with(c) > 16)) continue;
             // one workgroup per compute unit, or two where twice the run leaves two as well (its last block mostly idle)
             if (best == 0 || rounds_with(c) == 1 || (best == 4 && rounds_with(c) == 2 && rounds_with(best) == 2)) best = c;
         }
@@ -120,13 +140,14 @@ inline AwqPlan make_mfma_plan(int M, int K, int N, int group, bool may_walk = tr
         }
     }
     p.rt = ks;  // steps per wave
+    p.fine = group % (ks * kStepRows) != 0;
     p.ktiles = p.walks ? (ktiles_with(ks) + p.run - 1) / p.run : ktiles_with(ks);
     return p;
 }
 
 inline AwqPlan make_valu_plan(int M, int K, int N, bool allow_long_rows = true, bool allow_12_waves = true) {
     AwqPlan p;
-    p.mfma = p.sliced = p.walks = false;
+    p.mfma = p.sliced = p.walks = p.fine = false;
     p.run = 1;
     p.coltiles = (N / 8 + kWC - 1) / kWC;
     p.mb = M >= 8 ? 8 : (M >= 4 ? 4 : (M >= 2 ? 2 : 1));
@@ -189,7 +210,7 @@ constexpr int kFixedExchangeRows = 4;
 
 inline AwqPlan make_fixed_plan(int K, int N) {
     AwqPlan p{};
-    p.mfma = p.sliced = p.walks = false;
+    p.mfma = p.sliced = p.walks = p.fine = false;
     p.run = 1;
     p.coltiles = (N / 8 + kWC - 1) / kWC;
     p.mb = 1;
@@ -335,6 +356,13 @@ void launch_mfma_fused(const AwqPlan& p, const FusedInput& fi, const ResidualTar
             return;
         }
     }
+    if (p.fine) {
+        if (M <= 2) launch_awq_gemv_mfma<4, 4, 2, 1, PRO, EPI, LONE, false, true>(KX_MARGS);
+        else if (M <= 4) launch_awq_gemv_mfma<4, 4, 4, 1, PRO, EPI, LONE, false, true>(KX_MARGS);
+        else if (M <= 8) launch_awq_gemv_mfma<4, 4, 8, 1, PRO, EPI, LONE, false, true>(KX_MARGS);
+        else launch_awq_gemv_mfma<4, 4, 8, 2, PRO, EPI, LONE, false, true>(KX_MARGS);
+        return;
+    }
     if (p.rt == 4) KX_MFMA_BY_M(4);
     else if (p.rt == 2) KX_MFMA_BY_M(2);
     else KX_MFMA_BY_M(1);
@@ -401,7 +429,7 @@ extern "C" size_t kx_gemv_workspace_bytes(int32_t M, int32_t K, int32_t N) {
     if (M < 1 || M > KX_MAX_BATCH || K < 1 || N < 8) return 0;
     // Either kernel may serve a shape (the group size and M decide); size for the larger exchange.
     const int kt_valu = kx::make_valu_plan(M, K, N, true, false).ktiles;  // the entry points that keep 8 waves exchange more
-    const int kt_mfma = kx::make_mfma_plan(M, K, N, 32).ktiles;  // the smallest group gives the most K tiles
+    const int kt_mfma = kx::make_mfma_plan(M, K, N, 32, true, false, false).ktiles;  // one step per wave gives the most K tiles
     size_t ktiles = static_cast<size_t>(kt_valu > kt_mfma ? kt_valu : kt_mfma);
     if (M == 1) {
         const size_t kt_fixed = static_cast<size_t>(kx::make_fixed_plan(K, N).ktiles);  // its slow path parks partial sums there
@@ -539,6 +567,20 @@ extern "C" int kx_gemv_awq_bf16_policy(const uint16_t* x, const int32_t* qweight
             return kx::launch_status();
         }
 #undef KX_MFMA_WALK
+#define KX_MFMA_FINE(LONE)                                                                                          \
+    do {                                                                                                             \
+        if (M == 1) kx::launch_awq_gemv_mfma<4, 4, 1, 1, kx::kProNone, kx::kEpiStore, LONE, false, true>(KX_MARGS);  \
+        else if (M == 2) kx::launch_awq_gemv_mfma<4, 4, 2, 1, kx::kProNone, kx::kEpiStore, LONE, false, true>(KX_MARGS); \
+        else if (M <= 4) kx::launch_awq_gemv_mfma<4, 4, 4, 1, kx::kProNone, kx::kEpiStore, LONE, false, true>(KX_MARGS); \
+        else if (M <= 8) kx::launch_awq_gemv_mfma<4, 4, 8, 1, kx::kProNone, kx::kEpiStore, LONE, false, true>(KX_MARGS); \
+        else kx::launch_awq_gemv_mfma<4, 4, 8, 2, kx::kProNone, kx::kEpiStore, LONE, false, true>(KX_MARGS);         \
+    } while (0)
+        if (p.fine) {
+            if (N % 16) KX_MFMA_FINE(true);
+            else KX_MFMA_FINE(false);
+            return kx::launch_status();
+        }
+#undef KX_MFMA_FINE
 #define KX_MFMA_ROWS(KS, LONE)                                                                                \
     do {                                                                                                       \
         if (M == 1) kx::launch_awq_gemv_mfma<4, KS, 1, 1, kx::kProNone, kx::kEpiStore, LONE>(KX_MARGS);        \

@@ -79,6 +79,13 @@ __device__ __forceinline__ int red_piece(int piece) {  // 16-byte piece 0 .. 31 
     return piece ^ ((piece >> 3) & 1);
 }
 
+// 128 + zero point, indexed by nibble.
+__device__ __forceinline__ void zero_offsets(uint32_t zeros, float (&out)[8]) {
+    const uint32_t even = (zeros & 0x0F0F0F0Fu) | 0x80808080u, odd = ((zeros >> 4) & 0x0F0F0F0Fu) | 0x80808080u;
+#pragma unroll
+    for (int i = 0; i < 8; i++) out[i] = static_cast<float>(((i % 2 ? odd : even) >> (8 * (i / 2))) & 0xFFu);
+}
+
 // Half `which` of the lanes of `a`, then of `b`; lanes 0 .. 15 of `a`, then of `b` (and the same of lanes 32 .. 63).
 __device__ __forceinline__ float half_wave_pack(float a, float b, int which) {
     return __uint_as_float(__builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false)[which]);
@@ -128,10 +135,13 @@ __device__ __forceinline__ int group_of_step(const MfmaGrid& g, int step) {
     return g.group_magic ? static_cast<int>(__umulhi(static_cast<uint32_t>(step), g.group_magic)) : step;
 }
 
-// KS: consecutive 32-row steps per wave (they must share a quantisation group);
+// KS: consecutive 32-row steps per wave (they share a quantisation group, or FINE);
 // MC: activation rows a workgroup reduces per LDS round (1, 2, 4 or 8); ROUNDS: 2 for M > 8, else 1;
 // WALK: a workgroup works through grid.run blocks of KB rows of K, one behind the other, and adds their sums up in
 // registers (make_mfma_plan says when; carrying the loop costs the other launches up to a microsecond);
+// FINE: a wave's steps lie in groups of their own, and scale and zero point are applied per step, to the sums in registers:
+// groups that are no multiple of 128 with four steps per wave (make_mfma_plan says what that is worth).  The scales go through
+// LDS, each loaded once per workgroup (a lane's own take as many loads as the weights); the waves' sums then only add up;
 // LONE: N is an odd multiple of eight (a template parameter: the moves cost 20 registers, an occupancy step).
 // With a prologue, `x` is not read: fi.a / fi.b (/ fi.gain) are 16-byte aligned, fi.ld a multiple of eight.
 // Three workgroups per compute unit where the registers nearly allow it: left alone, one or two steps per wave at sixteen
@@ -139,7 +149,7 @@ __device__ __forceinline__ int group_of_step(const MfmaGrid& g, int step) {
 // 16 33.8 / 35.8 -> 28.7 / 33.7, 9728 -> 18432 77.7 / 81.3 -> 67.4 / 71.7; groups of 64 11264 -> 24064 70.2 / 73.5 -> 62.8 /
 // 69.2 (with the sums' phase of that day).  Over 540 to 2600 workgroups 0.92 times as long on average, 1.00 to 1.11 between 1150 and 1270; grids of up to 512
 // alike.
-template <int WAVES, int KS, int MC, int ROUNDS, int PRO = kProNone, int EPI = kEpiStore, bool LONE = false, bool WALK = false>
+template <int WAVES, int KS, int MC, int ROUNDS, int PRO = kProNone, int EPI = kEpiStore, bool LONE = false, bool WALK = false, bool FINE = false>
 __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEpiStore ? 3 : 2) void awq_gemv_mfma_kernel(
     const uint16_t* __restrict__ x, const uint32_t* __restrict__ qweight,
     const uint16_t* __restrict__ scales, const uint32_t* __restrict__ qzeros,
@@ -150,6 +160,7 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
     constexpr int KB = WAVES * WROWS;      // rows of K per workgroup
     constexpr int ROWS = MC * ROUNDS;      // activation rows this kernel carries (>= M)
     static_assert(!WALK || (KS == 4 && ROWS >= 8), "the launches that walk");
+    static_assert(!FINE || (KS == 4 && !WALK), "the launches whose waves cross groups");
     constexpr int THREADS = WAVES * kWave;
     static_assert(THREADS >= kTileCols, "one thread per tile column");
     static_assert(PRO == kProNone || PRO == kProSwiGLU || PRO == kProPreNorm, "prologues of the matrix-core kernel");
@@ -161,7 +172,7 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
     constexpr bool AHEAD = PRO == kProNone || ROUNDS == 1;
     // Launches of a shape that walks elsewhere (make_mfma_plan): behind a prologue at sixteen rows or with an odd number
     // of words, and the rotary epilogue.
-    constexpr bool RUNS = !WALK && KS == 4 &&
+    constexpr bool RUNS = !WALK && !FINE && KS == 4 &&
                           ((ROWS == 16 && PRO != kProNone) || (ROWS >= 8 && (EPI == kEpiQkRope || (LONE && PRO != kProNone))));
     // A staged row is the workgroup's K range plus 16 bytes, so that the rows a wave reads together
     // start in different banks.
@@ -183,11 +194,13 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
     __shared__ __attribute__((aligned(16))) float red[WAVES][2][RROWS][kHalfCols];
     __shared__ __attribute__((aligned(16))) float xs_red[WAVES][ROWS < 4 ? 4 : ROWS];
     __shared__ uint32_t s_word[3];
+    __shared__ __attribute__((aligned(16))) uint16_t s_fscale[FINE ? WAVES * KS : 1][FINE ? kTileCols : 8];
+    __shared__ uint32_t s_fzero[FINE ? WAVES * KS : 1][FINE ? kTileCols / 8 : 1];
     __shared__ __attribute__((aligned(16))) uint16_t s_x[STAGED ? ROWS : 1][STAGED ? XPITCH : 8];
     __shared__ float s_inv[PRO == kProPreNorm ? ROWS : 1];
 
     const int tid = threadIdx.x;
-    const int wave = tid / kWave;
+    const int wave = FINE ? __builtin_amdgcn_readfirstlane(tid / kWave) : tid / kWave;
     const int lane = tid % kWave;
     const int c = lane % 16;  // column slot: word pair c of the tile, MFMA column c
     const int b = lane / 16;  // k block inside the step, D row block
@@ -236,6 +249,14 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
     const int own_ld = own_col < N ? own_col : N - OWN;
     typename ScaleBits<OWN>::type s_bits[WAVES];
     uint32_t z_word[WAVES];
+    // FINE: the scales and zero points of the workgroup's steps go through LDS, eight columns (a word) of a step per piece; a lane
+    // reads those of the columns whose sums it keeps, packed as they go to LDS: its sixteen columns at sixteen rows, eight
+    // (word half b / 2) at eight, four (piece b % 2 of it) below.
+    constexpr int FSTEPS = WAVES * KS;
+    constexpr int FPIECES = FSTEPS * 32 / THREADS;  // pieces a thread stages
+    constexpr int FCOLS = ROWS >= 8 ? 8 : 4;
+    u32x4 f_scale[FINE ? FPIECES : 1];
+    uint32_t f_zero[FINE ? FPIECES : 1];
     // The A operand: row c of the activations, whether or not column slot c holds weights.  Rows
     // past M and steps past K (K is a multiple of 32: a step is all in or all out) are zeros.
     uint4 xa[KS];
@@ -268,7 +289,7 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
                 const int kstep = kblock + wave * WROWS + ks * kStepRows;
                 const int kld = kstep < K ? kstep : K - kStepRows;
                 const uint4 got = *reinterpret_cast<const uint4*>(x + static_cast<size_t>(x_row) * K + kld + 8 * b);
-                const bool live = c < M && kstep < K;
+                const bool live = FINE || (c < M && kstep < K);  // FINE masks at the product: here it waited in front of the weights' loads
                 xa[ks] = make_uint4(live ? got.x : 0u, live ? got.y : 0u, live ? got.z : 0u, live ? got.w : 0u);
             }
         }
@@ -288,6 +309,20 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
         }
     };
     auto load_scales = [&] {
+        if constexpr (FINE) {
+#pragma unroll
+            for (int i = 0; i < FPIECES; i++) {
+                const int e = tid + i * THREADS;
+                const int kstep = kblock + e / 32 * kStepRows;
+                const int step = (kstep < K ? kstep : K - 1) / kStepRows;  // rows past K meet zero activations
+                const int quotient = static_cast<int>(__umulhi(static_cast<uint32_t>(step), grid.group_magic));
+                const int g = grid.group_magic ? quotient : step;  // as group_of_step(), without a branch between the loads
+                const int word = ct * 32 + e % 32 < nw ? ct * 32 + e % 32 : nw - 1;
+                f_scale[i] = *reinterpret_cast<const u32x4*>(scales + static_cast<size_t>(g) * N + 8 * word);
+                f_zero[i] = qzeros[static_cast<size_t>(g) * nw + word];
+            }
+            return;
+        }
 #pragma unroll
         for (int wv = 0; wv < WAVES; wv++) {
             const int krow = kblock + wv * WROWS;
@@ -311,7 +346,7 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
             for (int r = 0; r < 8; r++) f ^= w[ks][r][0] ^ w[ks][r][1];
         }
 #pragma unroll
-        for (int wv = 0; wv < WAVES; wv++) f ^= s_bits[wv][0] ^ z_word[wv];
+        for (int wv = 0; wv < WAVES; wv++) f ^= FINE ? f_zero[0] : s_bits[wv][0] ^ z_word[wv];
         if (f == 0x9E3779B9u) partials[tid] = 1.0f;
         return;
     }
@@ -329,6 +364,15 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
         const float inv = 1.0f / sqrtf(mine / static_cast<float>(K) + fi.eps);
         if (lane < NORM_ROWS && wave + lane * WAVES < ROWS) s_inv[wave + lane * WAVES] = inv;
         lds_barrier();
+    }
+    if constexpr (FINE) {
+#pragma unroll
+        for (int i = 0; i < FPIECES; i++) {
+            const int e = tid + i * THREADS;
+            *reinterpret_cast<u32x4*>(&s_fscale[e / 32][8 * (e % 32)]) = f_scale[i];
+            s_fzero[e / 32][e % 32] = f_zero[i];
+        }
+        if constexpr (!STAGED) lds_barrier();  // otherwise the barrier behind the produced activations serves
     }
     FloatsOf<OWN> psum[PSUMS];
     for (int block = 0; block < blocks; block++) {
@@ -374,17 +418,27 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
         const f32x4v zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
         f32x4v xs;
         f32x4v acc[2][8];  // [word h][nibble p]
+        // FINE: scaled sums, [word h][nibble p] at sixteen rows, [nibble p] of word b / 2 at eight (rows 4 (b % 2) + v), and
+        // [column of the piece] below (rows v)
+        f32x4v fine[FINE ? (ROWS == 16 ? 16 : FCOLS) : 1];
         const uint32_t magic = opaque_bf16_128_pair();
+        // sixteen rows that are scaled per step take the word halves one after the other: both at once spill 80 registers
+        constexpr int PASSES = FINE && ROWS == 16 ? 2 : 1;
 #pragma unroll
-        for (int ks = 0; ks < KS; ks++) {
+        for (int i = 0; i < KS * PASSES; i++) {
+            const int ks = i % KS, h0 = PASSES == 2 ? i / KS : 0, h1 = PASSES == 2 ? h0 + 1 : 2;
             if constexpr (LONE) {
 #pragma unroll
-                for (int r = 0; r < 8; r++) w[ks][r][0] = lone_word ? w[ks][r][1] : w[ks][r][0];
+                for (int r = 0; r < 8 && i < KS; r++) w[ks][r][0] = lone_word ? w[ks][r][1] : w[ks][r][0];
+            }
+            if constexpr (FINE && !STAGED) {
+                const uint32_t keep = c < M && kblock + wave * WROWS + ks * kStepRows < K ? 0xffffffffu : 0u;
+                xa[ks] = make_uint4(xa[ks].x & keep, xa[ks].y & keep, xa[ks].z & keep, xa[ks].w & keep);
             }
             const bf16x8 a_op = as_bf16x8(xa[ks].x, xa[ks].y, xa[ks].z, xa[ks].w);
-            xs = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_op, ones, ks == 0 ? zero4 : xs, 0, 0, 0);
+            xs = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_op, ones, ks == 0 || FINE ? zero4 : xs, 0, 0, 0);
 #pragma unroll
-            for (int h = 0; h < 2; h++) {
+            for (int h = h0; h < h1; h++) {
                 uint32_t bop[8][4];  // [nibble p][row pair]
 #pragma unroll
                 for (int rp = 0; rp < 4; rp++) {
@@ -401,8 +455,63 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
 #pragma unroll
                 for (int p = 0; p < 8; p++) {
                     acc[h][p] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                        a_op, as_bf16x8(bop[p][0], bop[p][1], bop[p][2], bop[p][3]), ks == 0 ? zero4 : acc[h][p], 0, 0, 0);
+                        a_op, as_bf16x8(bop[p][0], bop[p][1], bop[p][2], bop[p][3]), ks == 0 || FINE ? zero4 : acc[h][p], 0, 0, 0);
                 }
+                if constexpr (FINE && ROWS == 16) {
+                    float zoff[8];
+                    zero_offsets(s_fzero[wave * KS + ks][2 * c + h], zoff);
+                    const auto scale = *reinterpret_cast<const typename ScaleBits<8>::type*>(&s_fscale[wave * KS + ks][16 * c + 8 * h]);
+#pragma unroll
+                    for (int p = 0; p < 8; p++) {
+                        const float sc = f16_bits_to_f32(scale[order_of(p)]);
+#pragma unroll
+                        for (int v = 0; v < 4; v++) {
+                            const float part = __builtin_fmaf(-zoff[p], xs[v], acc[h][p][v]);
+                            fine[8 * h + p][v] = ks == 0 ? sc * part : __builtin_fmaf(sc, part, fine[8 * h + p][v]);
+                        }
+                    }
+                }
+            }
+            if constexpr (FINE && ROWS == 8) {
+                float zoff[8], row_sum[4];
+                zero_offsets(s_fzero[wave * KS + ks][2 * c + b / 2], zoff);
+                const auto scale = *reinterpret_cast<const typename ScaleBits<8>::type*>(&s_fscale[wave * KS + ks][16 * c + 8 * (b / 2)]);
+#pragma unroll
+                for (int v = 0; v < 4; v++) row_sum[v] = half_wave_pack(xs[v], xs[v], 0);
+#pragma unroll
+                for (int p = 0; p < 8; p++) {
+                    const float sc = f16_bits_to_f32(scale[order_of(p)]);
+#pragma unroll
+                    for (int v = 0; v < 4; v++) {
+                        const float part = __builtin_fmaf(-zoff[p], row_sum[v], half_wave_pack(acc[0][p][v], acc[1][p][v], 0));
+                        fine[p][v] = ks == 0 ? sc * part : __builtin_fmaf(sc, part, fine[p][v]);
+                    }
+                }
+            }
+            if constexpr (FINE && ROWS <= 4) {
+                float zoff[8];
+                zero_offsets(s_fzero[wave * KS + ks][2 * c + b / 2] >> (8 * (b % 2)), zoff);
+                const auto scale = *reinterpret_cast<const typename ScaleBits<4>::type*>(&s_fscale[wave * KS + ks][16 * c + 4 * b]);
+#pragma unroll
+                for (int v = 0; v < ROWS; v++) {
+                    const float twice = quarter_wave_pack(xs[v], xs[v]);
+                    const float row_sum = half_wave_pack(twice, twice, 0);
+#pragma unroll
+                    for (int q = 0; q < 4; q++) {
+                        const int e = nibble_of(q);  // of the piece's column q; two further up in the second piece
+                        const float part = __builtin_fmaf(-zoff[e], row_sum,
+                                                          half_wave_pack(quarter_wave_pack(acc[0][e][v], acc[0][e + 2][v]),
+                                                                         quarter_wave_pack(acc[1][e][v], acc[1][e + 2][v]), 0));
+                        const float sc = f16_bits_to_f32(scale[q]);
+                        fine[q][v] = ks == 0 ? sc * part : __builtin_fmaf(sc, part, fine[q][v]);
+                    }
+                }
+            }
+            if constexpr (FINE) {
+                // A step's sums are scaled in the step; the compiler had put that off until all steps' sums were there, which
+                // took the registers of all of them (at sixteen rows 76 were spilled, and 5472 -> 9000 took 30.3 us, not 18.0).
+#pragma unroll
+                for (int q = PASSES == 2 ? 8 * h0 : 0; q < (PASSES == 2 ? 8 * h1 : FCOLS); q++) asm volatile("" : "+v"(fine[q]));
             }
             // a step is worked through while the loads of the later steps are still in flight
             __builtin_amdgcn_sched_barrier(0);
@@ -445,10 +554,16 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
                 if constexpr (ROWS >= 8) {
                     float m[8];
 #pragma unroll
-                    for (int q = 0; q < 8; q++) m[q] = half_wave_pack(acc[0][q][v], acc[1][q][v], rd);
+                    for (int q = 0; q < 8; q++) {
+                        if constexpr (!FINE) m[q] = half_wave_pack(acc[0][q][v], acc[1][q][v], rd);
+                        else if constexpr (ROWS == 16) m[q] = half_wave_pack(fine[q][v], fine[8 + q][v], rd);
+                        else m[q] = fine[q][v];
+                    }
                     float* dst = &red[wave][b / 2][4 * (b % 2) + v][0];
                     *reinterpret_cast<f32x4*>(dst + piece0) = f32x4{m[0], m[4], m[1], m[5]};
                     *reinterpret_cast<f32x4*>(dst + piece1) = f32x4{m[2], m[6], m[3], m[7]};
+                } else if constexpr (FINE) {
+                    *reinterpret_cast<f32x4*>(&red[wave][b / 2][v][b % 2 ? piece1 : piece0]) = f32x4{fine[0][v], fine[1][v], fine[2][v], fine[3][v]};
                 } else if constexpr (ROWS == 4) {  // a quarter of the lanes: every lane takes one of the four pieces of sixteen columns
                     float m[4];
 #pragma unroll
@@ -486,7 +601,7 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
                     float total = 0.0f;
 #pragma unroll
                     for (int wv = 0; wv < WAVES; wv++) {
-                        total += sc[wv][j] * __builtin_fmaf(-zc[wv][j], xv[i][wv], qv[i][wv][j]);
+                        total += FINE ? qv[i][wv][j] : sc[wv][j] * __builtin_fmaf(-zc[wv][j], xv[i][wv], qv[i][wv][j]);
                     }
                     float& sum = psum[rd * RSUMS + i].v[j];
                     sum = WALK && block > 0 ? sum + total : total;
@@ -683,7 +798,7 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
     }
 }
 
-template <int WAVES, int KS, int MC, int ROUNDS, int PRO = kProNone, int EPI = kEpiStore, bool LONE = false, bool WALK = false>
+template <int WAVES, int KS, int MC, int ROUNDS, int PRO = kProNone, int EPI = kEpiStore, bool LONE = false, bool WALK = false, bool FINE = false>
 inline void launch_awq_gemv_mfma(const uint16_t* x, const int32_t* qweight, const uint16_t* scales,
                                  const int32_t* qzeros, uint16_t* y, float* partials, uint32_t* counters,
                                  int M, int K, int N, const MfmaGrid& split,
@@ -693,7 +808,7 @@ inline void launch_awq_gemv_mfma(const uint16_t* x, const int32_t* qweight, cons
 
     const dim3 grid(split.side, split.ktiles, split.coltiles / split.side);
     dim3 block(WAVES * kWave, 1, 1);
-    hipLaunchKernelGGL((awq_gemv_mfma_kernel<WAVES, KS, MC, ROUNDS, PRO, EPI, LONE, WALK>), grid, block, 0, stream, x,
+    hipLaunchKernelGGL((awq_gemv_mfma_kernel<WAVES, KS, MC, ROUNDS, PRO, EPI, LONE, WALK, FINE>), grid, block, 0, stream, x,
                        reinterpret_cast<const uint32_t*>(qweight), scales,
                        reinterpret_cast<const uint32_t*>(qzeros), y, partials, counters, M, K, N,
                        split, fi, res, rope, cache_stride);
