@@ -223,16 +223,18 @@ class DecodeModel:
             words += [t.data_ptr() for t in (*L["qkv"], *L["o"], *L["gateup"], *L["down"], L["in_norm"], L["post_norm"],
                                              L["q_norm"], L["k_norm"], kc, vc)]
             words.append(min(kc.shape[0], vc.shape[0]))
+        head = {}  # without it the model needs no lm_head
+        if with_lm_head:
+            head = {"lm_head": self.lm_head, "head_rows": self.lm_head.shape[0], "logits": self.logits,
+                    "logits_n": self.logits.numel(), "next_token": self.next_token}
         capi.decode_step_bf16({
             "embed": self.embed, "token": self.token, "pos": self.pos, "final_norm": self.final_norm,
-            "lm_head": self.lm_head if with_lm_head else None, "x": self.x, "h": self.h, "q": self.q, "attn": self.attn,
-            "gate_up": self.gu, "logits": self.logits, "sumsq": self.ssq, "next_token": self.next_token,
+            "x": self.x, "h": self.h, "q": self.q, "attn": self.attn, "gate_up": self.gu, "sumsq": self.ssq,
             "gemv_workspace": self.gemv_ws, "gemv_workspace_bytes": self.gemv_ws.numel(),
             "attn_workspace": self.attn_ws, "attn_workspace_bytes": self.attn_ws.numel(),
             "hidden": c.hidden, "intermediate": c.intermediate, "n_q": c.n_q, "n_kv": c.n_kv, "group": c.group,
             "max_positions": self.max_positions, "norm_parts": self.ssq.shape[0], "merge_in_o": bool(self.merge_in_o),
-            "embed_rows": self.embed.shape[0], "head_rows": self.lm_head.shape[0], "logits_n": self.logits.numel(),
-            "rope_theta": c.rope_theta, "eps": c.eps}, words)
+            "embed_rows": self.embed.shape[0], "rope_theta": c.rope_theta, "eps": c.eps, **head}, words)
 
     def launches_per_step(self, with_lm_head=True, fused=True):
         per_layer = 10

@@ -26,3 +26,34 @@ def test_structures_match_the_header(capi):
     # thirteen pointers, two workspaces with their sizes, twelve 32-bit integers, two floats
     assert ctypes.sizeof(capi.StepDesc) == 17 * 8 + 14 * 4
     assert capi.STEP_LAYER_WORDS == 4 * 3 + 4 + 2 + 1
+
+
+def stubbed_model(monkeypatch, **changes):
+    """A two-layer model on the CPU whose native call only records what it was given."""
+    import torch
+    from mykuiperllama_amd import capi, decode
+    cfg = decode.ModelConfig(layers=2, hidden=256, intermediate=512, n_q=2, n_kv=1, vocab=64)
+    row = lambda n=1: torch.zeros((1, n), dtype=torch.bfloat16)
+    matrix = lambda: tuple(torch.zeros(4) for _ in range(3))
+    model = decode.DecodeModel.__new__(decode.DecodeModel)
+    model.__dict__.update(
+        torch=torch, cfg=cfg, max_positions=8, merge_in_o=True,
+        layers=[dict({m: matrix() for m in ("qkv", "o", "gateup", "down")},
+                     **{n: row() for n in ("in_norm", "post_norm", "q_norm", "k_norm")}) for _ in range(2)],
+        embed=row(256), lm_head=torch.zeros((64, 256)), final_norm=row(256), logits=row(64), ssq=torch.zeros((1, 4)),
+        k_cache=[torch.zeros((8, 1, 128)) for _ in range(2)], v_cache=[torch.zeros((8, 1, 128)) for _ in range(2)],
+        **{n: row() for n in ("x", "h", "q", "attn", "gu", "token", "pos", "next_token", "gemv_ws", "attn_ws")})
+    model.__dict__.update(changes)
+    calls = []
+    monkeypatch.setattr(capi, "decode_step_bf16", lambda fields, words: calls.append((fields, words)))
+    return model, calls
+
+
+def test_a_step_without_the_head_needs_no_lm_head(monkeypatch):
+    model, calls = stubbed_model(monkeypatch, lm_head=None)
+    model.step(with_lm_head=False)
+    (fields, _), = calls
+    assert fields.get("lm_head") is None
+    with pytest.raises(AttributeError):  # with the head it is asked for its shape, and nothing is launched
+        model.step(with_lm_head=True)
+    assert len(calls) == 1
