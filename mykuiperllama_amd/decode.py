@@ -219,7 +219,8 @@ class DecodeModel:
         # One native call for all launches; the addresses are looked up anew in every step, so that tensors may be replaced
         # between steps as with any other form.
         words = []
-        for L, kc, vc in zip(self.layers, self.k_cache, self.v_cache):
+        for li, L in enumerate(self.layers):
+            kc, vc = self.k_cache[li], self.v_cache[li]  # a layer without a cache is an error, not the end of the model
             words += [t.data_ptr() for t in (*L["qkv"], *L["o"], *L["gateup"], *L["down"], L["in_norm"], L["post_norm"],
                                              L["q_norm"], L["k_norm"], kc, vc)]
             words.append(min(kc.shape[0], vc.shape[0]))

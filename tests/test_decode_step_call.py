@@ -57,3 +57,22 @@ def test_a_step_without_the_head_needs_no_lm_head(monkeypatch):
     with pytest.raises(AttributeError):  # with the head it is asked for its shape, and nothing is launched
         model.step(with_lm_head=True)
     assert len(calls) == 1
+
+
+@pytest.mark.parametrize("caches", ["k_cache", "v_cache"])
+def test_a_missing_cache_is_refused(monkeypatch, caches):
+    import torch
+    model, calls = stubbed_model(monkeypatch, **{caches: [torch.zeros((8, 1, 128))]})  # of two layers
+    with pytest.raises(IndexError):
+        model.step()
+    assert not calls
+
+
+def test_caches_are_taken_by_layer(monkeypatch):
+    import torch
+    model, calls = stubbed_model(monkeypatch)
+    model.step()
+    by_number = {1: model.k_cache[1], 0: model.k_cache[0], 2: torch.zeros((8, 1, 128))}  # more caches than layers, in any order
+    model.k_cache = by_number
+    model.step()
+    assert calls[0][1] == calls[1][1] and len(calls[0][1]) == 2 * 19
