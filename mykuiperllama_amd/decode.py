@@ -221,8 +221,10 @@ class DecodeModel:
         words = []
         for li, L in enumerate(self.layers):
             kc, vc = self.k_cache[li], self.v_cache[li]  # a layer without a cache is an error, not the end of the model
-            words += [t.data_ptr() for t in (*L["qkv"], *L["o"], *L["gateup"], *L["down"], L["in_norm"], L["post_norm"],
-                                             L["q_norm"], L["k_norm"], kc, vc)]
+            for name in ("qkv", "o", "gateup", "down"):
+                qw, sc, qz = L[name]
+                words += (qw.data_ptr(), sc.data_ptr(), qz.data_ptr())
+            words += [t.data_ptr() for t in (L["in_norm"], L["post_norm"], L["q_norm"], L["k_norm"], kc, vc)]
             words.append(min(kc.shape[0], vc.shape[0]))
         head = {}  # without it the model needs no lm_head
         if with_lm_head:

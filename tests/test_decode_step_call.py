@@ -76,3 +76,14 @@ def test_caches_are_taken_by_layer(monkeypatch):
     model.k_cache = by_number
     model.step()
     assert calls[0][1] == calls[1][1] and len(calls[0][1]) == 2 * 19
+
+
+@pytest.mark.parametrize("matrix", ["qkv", "o", "gateup", "down"])
+@pytest.mark.parametrize("parts", [2, 4])
+def test_a_matrix_has_three_parts(monkeypatch, matrix, parts):
+    import torch
+    model, calls = stubbed_model(monkeypatch)
+    model.layers[0][matrix] = tuple(torch.zeros(4) for _ in range(parts))
+    with pytest.raises(ValueError):  # anything else would move every address behind it
+        model.step()
+    assert not calls
