@@ -781,8 +781,13 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
         if (!splitk_exchange_sum_wide<ROWS, RUNS>(lo, hi, M, N, ct, ktiles, partials, counters, s_word, request_all, grid.run)) {
             return;
         }
-        const int row0 = (tid / (kTileCols / 2)) * HALF;
-        const int pair = 2 * (tid % (kTileCols / 2));
+        // Where they go is worked out anew: kept over the read-back it took the registers of sixteen rows past three workgroups
+        // per compute unit, and 19 were spilled.  us per launch, spilled -> anew, 2048 -> 24584 behind SwiGLU, groups of 64, M = 9 /
+        // 16: 20.5 / 22.4 -> 19.0 / 20.8.
+        int thread = tid;
+        asm volatile("" : "+v"(thread));
+        const int row0 = (thread / (kTileCols / 2)) * HALF;
+        const int pair = 2 * (thread % (kTileCols / 2));
         if constexpr (EPI == kEpiStore) {
 #pragma unroll
             for (int i = 0; i < HALF; i++) {

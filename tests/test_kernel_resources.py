@@ -1,0 +1,55 @@
+"""What the compiler made of the matrix-core kernels, read from the code objects in libkx_hip.so (no GPU needed): scratch
+memory and registers where they decide how a launch runs."""
+import os
+import re
+import struct
+import subprocess
+
+import pytest
+
+READELF = "/opt/rocm/llvm/bin/llvm-readelf"
+MAGIC = b"__CLANG_OFFLOAD_BUNDLE__"
+
+
+def code_objects(data):
+    """The gfx950 code objects of a host library's offload bundles."""
+    at = data.find(MAGIC)
+    while at >= 0:
+        entry = at + len(MAGIC) + 8
+        for _ in range(struct.unpack_from("<Q", data, at + len(MAGIC))[0]):
+            offset, size, name = struct.unpack_from("<QQQ", data, entry)
+            if size and data[entry + 24:entry + 24 + name].endswith(b"gfx950"):
+                yield data[at + offset:at + offset + size]
+            entry += 24 + name
+        at = data.find(MAGIC, at + 1)
+
+
+@pytest.fixture(scope="module")
+def kernels(tmp_path_factory):
+    """Template arguments of each awq_gemv_mfma_kernel (waves, steps, rows per round, rounds, prologue, epilogue, odd words,
+    walks, crosses groups) -> its bytes of scratch memory and its vector registers."""
+    from mykuiperllama_amd.build import KX_LIB
+    if not os.path.exists(READELF):
+        pytest.skip("llvm-readelf is not installed")
+    found = {}
+    path = tmp_path_factory.mktemp("code") / "object"
+    with open(KX_LIB, "rb") as f:
+        data = f.read()
+    for code in code_objects(data):
+        path.write_bytes(code)
+        notes = subprocess.run([READELF, "--notes", str(path)], capture_output=True, text=True, check=True).stdout
+        for block in re.split(r"\n *- \.agpr_count", notes)[1:]:
+            field = lambda name: re.search(r"\." + name + r": +(\S+)", block).group(1)
+            m = re.search(r"awq_gemv_mfma_kernelI(.*?)EEv", field("name"))
+            if m:
+                args = tuple(int(v) for v in re.findall(r"L[ib](\d+)E", m.group(1) + "E"))
+                found[args] = int(field("private_segment_fixed_size")), int(field("vgpr_count"))
+    assert found, "no matrix-core kernel in the library"
+    return found
+
+
+def test_two_step_kernels_behind_a_prologue_do_not_spill(kernels):
+    # three workgroups per compute unit leave 168 registers; what does not fit goes to memory and back in the workgroup that
+    # finishes a column tile
+    spilled = {args: scratch for args, (scratch, _) in kernels.items() if args[1] <= 2 and args[2] * args[3] == 16 and args[4] and scratch}
+    assert not spilled
