@@ -66,7 +66,8 @@ constexpr int kExchangeRows = 8;    // what a K tile's share of the split-K exch
 //            36.1 / 36.6 -> 22.2 / 22.4 / 24.1 / 24.3; M = 9 / 16: 8192 -> 10240 (16) 21.7 / 22.2 -> 22.5 / 23.7, 8704 ->
 //            10240 (17) 24.1 / 24.7 -> 23.2 / 24.1, 12288 -> 8192 (24) 24.1 / 25.0 -> 22.8 / 23.1.
 //            Behind SwiGLU nine and more rows cannot load the next block's operands ahead, and walk past 32 blocks only,
-//            over no more of them than there would be rounds of workgroups: M = 9 / 16 14336 -> 5120 27.3 / 28.9 -> 28.4 /
+//            over no more of them than there would be rounds of workgroups (a line drawn while a walking block still waited
+//            for spilled addresses; without them 18432 -> 5120 takes 24.1 / 24.5): M = 9 / 16 14336 -> 5120 27.3 / 28.9 -> 28.4 /
 //            30.3, 16384 -> 5120 28.1 / 29.0 -> 29.4 / 30.9, 18432 -> 5120 30.7 / 31.7 -> 30.3 / 31.9, 20480 -> 5120 (40)
 //            34.2 / 35.5 -> 30.9 / 32.3; 24576 -> 16384 (six, for six rounds) 72.2 / 77.4 -> 69.7 / 73.4, 17408 -> 8192 (three,
 //            for three) 38.0 / 40.2 -> 35.2 / 38.0, 20096 -> 9616 (four, for three) 51.7 / 54.1 -> 58.7 / 61.9, 17920 -> 14592

@@ -170,6 +170,11 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
     // operands do not fit the registers beside the weights and the sums: there the other workgroup of the compute unit
     // has to cover the gap.
     constexpr bool AHEAD = PRO == kProNone || ROUNDS == 1;
+    // Those launches are short of registers.  What is cheap to work out is worked out per block (the addresses of the rows) or per
+    // round (the scales as floats) instead of kept: spilled addresses came back behind the weights, so that a block waited for
+    // them before it produced its activations.  us per launch behind SwiGLU, kept -> worked out, M = 9 / 16: 18432 -> 5120
+    // 29.9 / 30.7 -> 24.1 / 24.5, 25600 -> 5120 34.5 / 35.8 -> 26.7 / 27.2.
+    constexpr bool SHORT_OF_REGISTERS = WALK && !AHEAD;
     // Launches of a shape that walks elsewhere (make_mfma_plan): behind a prologue at sixteen rows or with an odd number
     // of words, and the rotary epilogue.
     constexpr bool RUNS = !WALK && !FINE && KS == 4 &&
@@ -270,11 +275,12 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
     const bool lone_word = wc_first == nw - 1;
     auto load_operands = [&] {
         if constexpr (STAGED) {
+            int thread = tid;
+            if constexpr (SHORT_OF_REGISTERS) asm volatile("" : "+v"(thread));
 #pragma unroll
             for (int i = 0; i < PPT; i++) {
-                const int e = tid + i * THREADS;
-                const int pm = e / KPIECES;
-                const int k = kblock + 8 * (e % KPIECES);
+                const int pm = thread / KPIECES + i * (THREADS / KPIECES);
+                const int k = kblock + 8 * (thread % KPIECES);
                 const int mc = pm < M ? pm : M - 1;
                 const int kc = k < K ? k : K - 8;
                 const size_t at = static_cast<size_t>(mc) * fi.ld + kc;
@@ -380,9 +386,8 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
         if constexpr (STAGED) {
 #pragma unroll
             for (int i = 0; i < PPT; i++) {
-                const int e = tid + i * THREADS;
-                const int pm = e / KPIECES;
-                const int kp = e % KPIECES;
+                const int pm = tid / KPIECES + i * (THREADS / KPIECES);  // a row's distance from the first is known when compiling
+                const int kp = tid % KPIECES;
                 if (PIECES % THREADS == 0 || pm < ROWS) {
                     // Vector instructions bound the prologue (every column tile produces its rows anew), so two elements share a
                     // conversion, the norm's gain is loaded and the inverse worked out once, and the words of a dead piece are
@@ -519,8 +524,7 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
 
         // scales, and 128 + zero point, of the columns of the thread's pieces: nibbles 0, 4, 1, 5 of a word, or one byte up
         FloatsOf<OWN> sc[WAVES], zc[WAVES];
-#pragma unroll
-        for (int wv = 0; wv < WAVES; wv++) {
+        auto convert_scales = [&](int wv) {
             const uint32_t zeros = z_word[wv] >> (QUADS ? 8 * (own_piece % 2) : 4 * nibble_of(own_col & 7));
             const uint32_t even = (zeros & 0x000F000Fu) | 0x00800080u, odd = ((zeros >> 4) & 0x000F000Fu) | 0x00800080u;
 #pragma unroll
@@ -529,6 +533,10 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
                 const uint32_t both = j < 2 ? even : odd;
                 zc[wv][j] = static_cast<float>(j % 2 ? (both >> 16) & 0xFFu : both & 0xFFu);
             }
+        };
+        if constexpr (!FINE && !SHORT_OF_REGISTERS) {
+#pragma unroll
+            for (int wv = 0; wv < WAVES; wv++) convert_scales(wv);
         }
         auto load_next = [&] {
             if (block + 1 < blocks) {
@@ -592,6 +600,13 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
                 for (int wv = 0; wv < WAVES; wv++) {
                     qv[i][wv] = *reinterpret_cast<const FloatsOf<OWN>*>(&red[wv][QUADS ? own_half : tid / 8 % 2][row][at]);
                     xv[i][wv] = xs_red[wv][rd * RROWS + row];
+                }
+            }
+            if constexpr (SHORT_OF_REGISTERS) {
+#pragma unroll
+                for (int wv = 0; wv < WAVES; wv++) {
+                    asm volatile("" : "+v"(z_word[wv]));
+                    convert_scales(wv);
                 }
             }
 #pragma unroll

@@ -53,3 +53,11 @@ def test_two_step_kernels_behind_a_prologue_do_not_spill(kernels):
     # finishes a column tile
     spilled = {args: scratch for args, (scratch, _) in kernels.items() if args[1] <= 2 and args[2] * args[3] == 16 and args[4] and scratch}
     assert not spilled
+
+
+def test_walking_kernels_keep_their_addresses(kernels):
+    # A few words of a walking launch at sixteen rows behind SwiGLU still go to memory; with the addresses of the staged rows
+    # among them every block waited for its weights before it could produce its activations.
+    walking = {args: scratch for args, (scratch, _) in kernels.items() if args[7]}
+    assert max(walking.values()) <= 40
+    assert not [args for args, scratch in walking.items() if scratch and not (args[4] and args[2] * args[3] == 16)]
