@@ -195,6 +195,11 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
     constexpr int RROWS = ROWS < 8 ? ROWS : 8;         // activation rows per LDS round
     constexpr int RSUMS = QUADS ? RROWS / 4 : ROWS;    // rows of a thread per round
     constexpr int PSUMS = QUADS ? ROWS / 4 : ROWS;     // rows of a thread
+    // One and two rows that are stored or added meet column by column: the few lanes that write leave the banks free either way,
+    // and the order of the pieces below cost a step of occupancy with one step per wave.  us per launch at M = 2, by pieces -> by
+    // columns, groups of 32: 4096 -> 24576 behind SwiGLU into the residual stream 18.2 -> 17.4.  (The rotary launches take fewer
+    // registers by pieces, and those behind a norm lose 0.1 to 0.2 us by columns and the test below.)
+    constexpr bool BY_COLUMNS = ROWS <= 2 && PRO != kProPreNorm && EPI != kEpiQkRope && !FINE;
 
     __shared__ __attribute__((aligned(16))) float red[WAVES][2][RROWS][kHalfCols];
     __shared__ __attribute__((aligned(16))) float xs_red[WAVES][ROWS < 4 ? 4 : ROWS];
@@ -552,11 +557,13 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
         // ---- waves meet in LDS; every thread then owns its columns ----
         // D rows 4b .. 4b+3 of the lane; its sixteen columns are 16c .. 16c+15, those of word h eight of them.  A round writes
         // with all lanes: eight rows fill half of them, and the word halves are packed side by side.
-        const int piece0 = 4 * red_piece(2 * c), piece1 = 4 * red_piece(2 * c + 1);
+        const int piece0 = BY_COLUMNS ? 8 * c : 4 * red_piece(2 * c), piece1 = BY_COLUMNS ? 8 * c + 4 : 4 * red_piece(2 * c + 1);
 #pragma unroll
         for (int rd = 0; rd < ROWS / RROWS; rd++) {
             if (rd > 0 || block > 0) lds_barrier();  // the previous round has been read
-            if (rd == 0 && c == 0 && 4 * b < ROWS) *reinterpret_cast<f32x4v*>(&xs_red[wave][4 * b]) = xs;
+            if constexpr (!BY_COLUMNS) {
+                if (rd == 0 && c == 0 && 4 * b < ROWS) *reinterpret_cast<f32x4v*>(&xs_red[wave][4 * b]) = xs;
+            }
 #pragma unroll
             for (int v = 0; v < (ROWS < 4 ? ROWS : 4); v++) {
                 if constexpr (ROWS >= 8) {
@@ -581,6 +588,7 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
                     }
                     *reinterpret_cast<f32x4*>(&red[wave][b / 2][v][b % 2 ? piece1 : piece0]) = f32x4{m[0], m[1], m[2], m[3]};
                 } else if (b == 0) {
+                    if (BY_COLUMNS && c == 0) xs_red[wave][v] = xs[v];
 #pragma unroll
                     for (int h = 0; h < 2; h++) {
                         float* dst = &red[wave][h][v][0];
@@ -595,7 +603,8 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
 #pragma unroll
             for (int i = 0; i < RSUMS; i++) {
                 const int row = QUADS ? own_row + 4 * i : i;
-                const int at = QUADS ? 4 * red_piece(own_piece) : 4 * red_piece(tid / 16 * 2 + tid / 4 % 2) + tid % 4;
+                const int at = QUADS ? 4 * red_piece(own_piece)
+                                     : (BY_COLUMNS ? tid / 16 * 8 + tid % 8 : 4 * red_piece(tid / 16 * 2 + tid / 4 % 2) + tid % 4);
 #pragma unroll
                 for (int wv = 0; wv < WAVES; wv++) {
                     qv[i][wv] = *reinterpret_cast<const FloatsOf<OWN>*>(&red[wv][QUADS ? own_half : tid / 8 % 2][row][at]);
@@ -716,6 +725,7 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
         }
     };
     const auto row_of = [&](int i) { return QUADS ? own_row + 4 * i : i; };  // row of psum[i]
+    constexpr bool STORES_FEW = ROWS <= 2 && PRO != kProPreNorm && EPI == kEpiStore;
     if (ktiles == 1) {
         if constexpr (EPI == kEpiStore) {  // a thread stores its own columns: nothing to hand over
 #pragma unroll
@@ -737,7 +747,15 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
             for (int i = 0; i < PSUMS; i++) *reinterpret_cast<FloatsOf<OWN>*>(&s_sum[row_of(i) * kTileCols + own_col - ct * kTileCols]) = psum[i];
             finish_from_lds();
         }
-        return;
+        if constexpr (!STORES_FEW) return;
+    }
+    // One and two stored rows: a test of its own rather than the other branch of the one above, whose values the compiler would
+    // carry through the exchange.  us per launch at M = 2, branch -> test: 12288 -> 4096 11.28 -> 11.02, behind SwiGLU 11.30 -> 11.01,
+    // 3072 -> 1024 with groups of 32 6.43 -> 6.26.  More rows lose by it (1536 -> 4096 at M = 16 7.45 -> 7.65).
+    if constexpr (STORES_FEW) {
+        int tiles = ktiles;
+        asm volatile("" : "+s"(tiles));
+        if (tiles == 1) return;
     }
     if constexpr (ROWS <= 2) {
         float own[ROWS], sum[ROWS];

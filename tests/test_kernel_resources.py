@@ -61,3 +61,9 @@ def test_walking_kernels_keep_their_addresses(kernels):
     walking = {args: scratch for args, (scratch, _) in kernels.items() if args[7]}
     assert max(walking.values()) <= 40
     assert not [args for args, scratch in walking.items() if scratch and not (args[4] and args[2] * args[3] == 16)]
+
+
+def test_two_rows_into_the_residual_stream_leave_room_for_six_workgroups(kernels):
+    # one step per wave: 512 registers a lane and six waves per SIMD are 80 registers a wave
+    few = {args: registers for args, (_, registers) in kernels.items() if args[1:4] == (1, 2, 1) and args[5] == 2 and not args[8]}
+    assert few and max(few.values()) <= 80
