@@ -239,16 +239,17 @@ inline AwqPlan make_fixed_plan(int K, int N) {
     return p;
 }
 
-// Several activation rows go to the matrix cores, where a lane loads two words of a row.  With an odd number of words and
-// groups that leave a wave one step, which the vector kernel used to serve, two rows past K = 2048 and three rows of narrow
-// matrices past K = 8192 are still faster there.  us per launch, vector kernel against this one, groups of 32: M = 2 8224 ->
-// 1288 8.9 / 9.5, 9216 -> 520 8.6 / 9.3 (1536 -> 1288 8.8 / 5.9, with sums of an earlier day); M = 3 9216 -> 520 9.2 / 10.7
-// (12288 -> 1288 13.6 / 11.4); M = 4 / 5 / 8 / 16 8224 -> 1288 12.3 / 16.1 / 18.8 / 27.0 against 11.8 / 11.9 / 11.8 / 12.7, 9216
-// -> 520 11.9 / 12.2 / 18.0 / 18.9 against 11.0 / 11.2 / 11.2 / 12.0.
+// Several activation rows go to the matrix cores, where a lane loads two words of a row.  With an odd number of words and groups
+// that leave a wave one step, two rows past K = 2048 and narrow matrices past K = 8192 stay on the vector kernel, which served
+// them first and whose sums are the more exact ones (its codes carry an offset of 16, not 128, that cancels in fp32: the error
+// of the sum against float64 is 1.3 to 4 times as large on the matrix cores, 12288 -> 1288 with groups of 32 and x of mean 0 and
+// 1).  us per launch, groups of 32, vector kernel / matrix cores: M = 2 8224 -> 1288 8.9 / 9.5, 9216 -> 520 8.6 / 9.3, wide matrices
+// not measured since waves cross groups; M = 3 9216 -> 520 9.2 / 10.7, 12288 -> 1288 13.6 / 11.4; M = 4 / 8 / 16 12288 -> 1288 13.7 /
+// 20.1 / 34.9 against 12.2 / 12.5 / 13.1: what the exactness costs.  Behind SwiGLU 10240 -> 24 at M = 6 / 16 8.8 / 9.6 against 9.9 / 10.9.
 inline bool rows_on_mfma(int M, int K, int N, int group) {
     if (M < 2 || N < 16) return false;
     const bool odd = N % 16 != 0, one_step = group % (2 * kStepRows) != 0;
-    return !(odd && one_step && (M == 2 ? K > 2048 : M == 3 && K > 8192 && N <= 1024));
+    return !(odd && one_step && (M == 2 ? K > 2048 : K > 8192 && N <= 2048));
 }
 
 inline AwqPlan make_plan(int M, int K, int N, int group, int mode) {
