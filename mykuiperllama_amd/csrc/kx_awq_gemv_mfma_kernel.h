@@ -345,6 +345,7 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
     if constexpr (!STAGED) load_scales();
     load_operands();
     if constexpr (STAGED) load_scales();
+    if constexpr (FINE && PRO == kProPreNorm) __builtin_amdgcn_sched_barrier(1);  // no load of them moves behind the weights
     load_weights();
     __builtin_amdgcn_sched_barrier(0);
 #if defined(KX_ABLATE) && KX_ABLATE == 2
@@ -380,7 +381,9 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
 #pragma unroll
         for (int i = 0; i < FPIECES; i++) {
             const int e = tid + i * THREADS;
-            *reinterpret_cast<u32x4*>(&s_fscale[e / 32][8 * (e % 32)]) = f_scale[i];
+            // a step past K adds nothing: its sums are zeros, but zero times an infinite scale is not
+            const uint32_t keep = kblock + e / 32 * kStepRows < K ? 0xffffffffu : 0u;
+            *reinterpret_cast<u32x4*>(&s_fscale[e / 32][8 * (e % 32)]) = f_scale[i] & keep;
             s_fzero[e / 32][e % 32] = f_zero[i];
         }
         if constexpr (!STAGED) lds_barrier();  // otherwise the barrier behind the produced activations serves
