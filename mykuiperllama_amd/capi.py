@@ -61,6 +61,8 @@ SIGNATURES = {
 INTERNAL_SIGNATURES = {
     "kx_gemv_awq_bf16_policy": (ctypes.c_int, [_P, _P, _P, _P, _P, _I32, _I32, _I32, _I32, _P, _SZ, _P, _I32]),
     "kx_decode_step_bf16": (ctypes.c_int, [_P, _P, _P]),
+    "kx_step_desc_bytes": (_SZ, []),
+    "kx_step_layer_bytes": (_SZ, []),
 }
 
 
@@ -130,6 +132,9 @@ def load(path=None):
     if built_as != ABI_VERSION:
         raise RuntimeError(f"{lib_path} was built as ABI version {built_as}, this binding mirrors version "
                            f"{ABI_VERSION} of include/kx_hip.h (ChainDesc would not match kx_chain_desc)")
+    mirrored, compiled = (ctypes.sizeof(StepDesc), 8 * STEP_LAYER_WORDS), (lib.kx_step_desc_bytes(), lib.kx_step_layer_bytes())
+    if mirrored != compiled:
+        raise RuntimeError(f"{lib_path} has a decode step of {compiled} bytes (step, layer), this binding mirrors {mirrored}")
     global _raw_stream, _get_device
     raw, device = getattr(torch._C, "_cuda_getCurrentRawStream", None), getattr(torch._C, "_cuda_getDevice", None)
     if raw is not None and device is not None:

@@ -358,7 +358,10 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
             for (int r = 0; r < 8; r++) f ^= w[ks][r][0] ^ w[ks][r][1];
         }
 #pragma unroll
-        for (int wv = 0; wv < WAVES; wv++) f ^= FINE ? f_zero[0] : s_bits[wv][0] ^ z_word[wv];
+        for (int wv = 0; wv < WAVES; wv++) {
+            if constexpr (FINE) f ^= f_zero[0];
+            else f ^= s_bits[wv][0] ^ z_word[wv];
+        }
         if (f == 0x9E3779B9u) partials[tid] = 1.0f;
         return;
     }

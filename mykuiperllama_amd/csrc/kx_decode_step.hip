@@ -17,6 +17,16 @@ struct Enqueue {
 
 }  // namespace
 
+static_assert(sizeof(kx_step_layer) == 19 * 8, "nineteen eight-byte words");
+
+extern "C" size_t kx_step_desc_bytes(void) {
+    return sizeof(kx_step_desc);
+}
+
+extern "C" size_t kx_step_layer_bytes(void) {
+    return sizeof(kx_step_layer);
+}
+
 extern "C" int kx_decode_step_bf16(const kx_step_desc* d, const kx_step_layer* layers, void* stream) {
     if (!d || (!layers && d->layers > 0)) return KX_ERR_NULL_POINTER;
     Enqueue run;

@@ -65,6 +65,10 @@ typedef struct kx_step_desc {
 
 int kx_decode_step_bf16(const kx_step_desc* desc, const kx_step_layer* layers, void* stream);
 
+/* Bytes of a kx_step_desc and of a kx_step_layer as the library was compiled: a binding that mirrors them compares. */
+size_t kx_step_desc_bytes(void);
+size_t kx_step_layer_bytes(void);
+
 #ifdef __cplusplus
 }
 #endif

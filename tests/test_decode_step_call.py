@@ -2,6 +2,8 @@
 structures have the sizes the library was compiled with."""
 import array
 import ctypes
+import os
+import re
 
 import pytest
 
@@ -26,6 +28,20 @@ def test_structures_match_the_header(capi):
     # thirteen pointers, two workspaces with their sizes, twelve 32-bit integers, two floats
     assert ctypes.sizeof(capi.StepDesc) == 17 * 8 + 14 * 4
     assert capi.STEP_LAYER_WORDS == 4 * 3 + 4 + 2 + 1
+
+
+def test_structures_match_the_library(capi):
+    lib = capi.load()
+    assert ctypes.sizeof(capi.StepDesc) == lib.kx_step_desc_bytes()
+    assert 8 * capi.STEP_LAYER_WORDS == lib.kx_step_layer_bytes()
+    # the fields in the order, and of the kind, in which the header declares them
+    with open(os.path.join(os.path.dirname(capi.__file__), "csrc", "kx_internal.h")) as f:
+        body = re.search(r"typedef struct kx_step_desc \{(.*?)\} kx_step_desc;", f.read(), re.S).group(1)
+    kinds = {"float": ctypes.c_float, "int32_t": ctypes.c_int32, "size_t": ctypes.c_size_t}
+    declared = []
+    for kind, names in re.findall(r"(?:const )?(\w+)([^;]*);", re.sub(r"/\*.*?\*/", "", body)):
+        declared += [(name.strip(" *"), ctypes.c_void_p if "*" in name else kinds[kind]) for name in names.split(",")]
+    assert declared == list(capi.StepDesc._fields_)
 
 
 def stubbed_model(monkeypatch, **changes):

@@ -299,3 +299,21 @@ def test_step_is_capturable_in_a_graph_and_replays_identically(torch, fused):
             side.synchronize()
             assert torch.equal(model.logits, eager)
     torch.cuda.synchronize()
+
+
+def test_a_step_without_the_head_leaves_logits_and_token_alone(torch):
+    from mykuiperllama_amd import decode
+    cfg = decode.ModelConfig(**CFG)
+    model = decode.DecodeModel(cfg, MAXPOS)
+    model.prefill_cache_random(CTX)
+    model.set_input(5, CTX)
+    model.step()
+    want = model.h.clone()
+    model.h.fill_(7)
+    model.logits.fill_(3)
+    model.next_token.fill_(-2)
+    model.lm_head = None
+    model.step(with_lm_head=False)
+    torch.cuda.synchronize()
+    assert torch.equal(model.h, want)
+    assert bool((model.logits == 3).all()) and model.next_token.item() == -2
