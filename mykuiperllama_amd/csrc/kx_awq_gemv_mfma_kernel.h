@@ -144,13 +144,13 @@ __device__ __forceinline__ int group_of_step(const MfmaGrid& g, int step) {
 // LDS, each loaded once per workgroup (a lane's own take as many loads as the weights); the waves' sums then only add up;
 // LONE: N is an odd multiple of eight (a template parameter: the moves cost 20 registers, an occupancy step).
 // With a prologue, `x` is not read: fi.a / fi.b (/ fi.gain) are 16-byte aligned, fi.ld a multiple of eight.
-// Three workgroups per compute unit where the registers nearly allow it: left alone, one or two steps per wave at sixteen
-// rows take 169 to 185 of them, one occupancy step down.  us per launch, two -> three: groups of 32 3072 -> 23808 at M = 9 /
-// 16 33.8 / 35.8 -> 28.7 / 33.7, 9728 -> 18432 77.7 / 81.3 -> 67.4 / 71.7; groups of 64 11264 -> 24064 70.2 / 73.5 -> 62.8 /
-// 69.2 (with the sums' phase of that day).  Over 540 to 2600 workgroups 0.92 times as long on average, 1.00 to 1.11 between 1150 and 1270; grids of up to 512
-// alike.
+// Three workgroups per compute unit (168 registers) at sixteen rows with one or two steps per wave.  One step is held to it: us
+// per launch, two -> three, groups of 32, M = 9 / 16: 1024 -> 34816 15.9 / 16.7 -> 15.4 / 16.5, behind a norm 16.8 / 17.7 -> 16.0 /
+// 17.1, 1024 -> 24576 11.4 / 11.8 -> 11.2 / 11.7.  Two steps take 167 by themselves; held to it, the plain launch spilled 19: spilled
+// -> left alone, groups of 64, 2048 -> 24576 14.7 / 15.9 -> 13.7 / 14.9, 2048 -> 16896 15.2 / 16.9 -> 13.4 / 15.1, 2048 -> 51200 24.3 /
+// 28.2 -> 23.0 / 26.6; grids of up to 512 workgroups alike.
 template <int WAVES, int KS, int MC, int ROUNDS, int PRO = kProNone, int EPI = kEpiStore, bool LONE = false, bool WALK = false, bool FINE = false>
-__global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEpiStore ? 3 : 2) void awq_gemv_mfma_kernel(
+__global__ __launch_bounds__(WAVES * kWave, KS == 1 && ROUNDS == 2 && EPI == kEpiStore ? 3 : 2) void awq_gemv_mfma_kernel(
     const uint16_t* __restrict__ x, const uint32_t* __restrict__ qweight,
     const uint16_t* __restrict__ scales, const uint32_t* __restrict__ qzeros,
     uint16_t* __restrict__ y, float* __restrict__ partials, uint32_t* __restrict__ counters,
@@ -821,8 +821,8 @@ __global__ __launch_bounds__(WAVES * kWave, KS <= 2 && ROUNDS == 2 && EPI == kEp
             return;
         }
         // Where they go is worked out anew: kept over the read-back it took the registers of sixteen rows past three workgroups
-        // per compute unit, and 19 were spilled.  us per launch, spilled -> anew, 2048 -> 24584 behind SwiGLU, groups of 64, M = 9 /
-        // 16: 20.5 / 22.4 -> 19.0 / 20.8.
+        // per compute unit (185 with two steps per wave).  us per launch, kept, at two workgroups -> anew, groups of 64, M = 9 / 16:
+        // 2048 -> 24576 behind SwiGLU 14.9 / 15.5 -> 13.8 / 14.3, behind a norm 15.2 / 16.0 -> 13.9 / 14.6.
         int thread = tid;
         asm volatile("" : "+v"(thread));
         const int row0 = (thread / (kTileCols / 2)) * HALF;

@@ -48,11 +48,10 @@ def kernels(tmp_path_factory):
     return found
 
 
-def test_two_step_kernels_behind_a_prologue_do_not_spill(kernels):
-    # three workgroups per compute unit leave 168 registers; what does not fit goes to memory and back in the workgroup that
-    # finishes a column tile
-    spilled = {args: scratch for args, (scratch, _) in kernels.items() if args[1] <= 2 and args[2] * args[3] == 16 and args[4] and scratch}
-    assert not spilled
+def test_short_waves_at_sixteen_rows_fit_three_to_a_compute_unit(kernels):
+    # three workgroups leave 168 registers; what does not fit goes to memory and back in the workgroup that finishes a column tile
+    short = {args: found for args, found in kernels.items() if args[1] <= 2 and args[2] * args[3] == 16 and args[5] == 0}
+    assert short and not [args for args, (scratch, registers) in short.items() if scratch or registers > 168]
 
 
 def test_walking_kernels_keep_their_addresses(kernels):
