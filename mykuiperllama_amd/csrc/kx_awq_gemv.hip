@@ -243,9 +243,11 @@ inline AwqPlan make_fixed_plan(int K, int N) {
 // that leave a wave one step, two rows past K = 2048 and narrow matrices past K = 8192 stay on the vector kernel, which served
 // them first and whose sums are the more exact ones (its codes carry an offset of 16, not 128, that cancels in fp32: the error
 // of the sum against float64 is 1.3 to 4 times as large on the matrix cores, 12288 -> 1288 with groups of 32 and x of mean 0 and
-// 1).  us per launch, groups of 32, vector kernel / matrix cores: M = 2 8224 -> 1288 8.9 / 9.5, 9216 -> 520 8.6 / 9.3, wide matrices
-// not measured since waves cross groups; M = 3 9216 -> 520 9.2 / 10.7, 12288 -> 1288 13.6 / 11.4; M = 4 / 8 / 16 12288 -> 1288 13.7 /
-// 20.1 / 34.9 against 12.2 / 12.5 / 13.1: what the exactness costs.  Behind SwiGLU 10240 -> 24 at M = 6 / 16 8.8 / 9.6 against 9.9 / 10.9.
+// 1: of 20608 outputs at M = 16 and mean 1, 1 against 9 are not the correctly rounded sum).  us per launch, vector kernel / matrix
+// cores, groups of 32: M = 2 3072 -> 5128 7.8 / 8.7, 5472 -> 9000 15.0 / 15.7, 8224 -> 1288 9.1 / 10.1, -> 5128 14.5 / 14.9, 12288 ->
+// 10248 28.9 / 26.7 (2080 -> 3000 6.9 / 6.9); M = 3 9216 -> 520 9.6 / 10.8, 12288 -> 1032 10.0 / 11.3, -> 1288 13.5 / 11.5; M = 4 / 16
+// 9216 -> 520 12.0 / 19.5 against 11.0 / 12.0, 12288 -> 1288 13.6 / 35.0 against 11.7 / 13.3, groups of 96 16512 -> 824 at M = 10 39.0
+// against 13.8: what the exactness costs.  Behind SwiGLU 10240 -> 24 at M = 6 / 16 8.8 / 9.6 against 9.9 / 10.9.
 inline bool rows_on_mfma(int M, int K, int N, int group) {
     if (M < 2 || N < 16) return false;
     const bool odd = N % 16 != 0, one_step = group % (2 * kStepRows) != 0;

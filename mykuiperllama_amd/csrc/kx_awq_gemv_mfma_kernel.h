@@ -16,11 +16,14 @@
 //   sum_k x*(q - z) = sum_k x*(128 + q)  -  (128 + z) * sum_k x
 //
 // and sum_k x comes out of one more MFMA against a B operand of ones, in the same register layout.
-// Raw sums of the waves of a workgroup meet in LDS; the thread that owns a column applies zero
-// point and scale once per wave (a wave never straddles a quantisation group: groups are multiples of
-// 32 and the host picks KS so that KS*32 divides the group) and takes part in the split-K exchange.
-// The offset that cancels is 128 where the vector kernel has 16, which shows in the last bits of the fp32 sum only: against
-// float64 the bf16 outputs of both are 1.63e-3 to 1.70e-3 off, equal to six digits (K 512 to 25600, x of mean 0 and 1).
+// Raw sums of the waves of a workgroup meet in LDS; the thread that owns a column applies zero point and scale once per
+// wave, whose steps lie in one quantisation group (groups are multiples of 32, and the host picks KS so that KS*32 divides
+// the group), and takes part in the split-K exchange.  With FINE the steps of a wave lie in groups of their own: zero point
+// and scale are applied per step in registers, and what meets in LDS are scaled sums.
+// The offset that cancels is 128 where the vector kernel has 16, which shows in the last bits of the fp32 sum: its error against
+// float64 is 1.3 to 4 times as large, and up to 1 in 1000 bf16 outputs is not the correctly rounded sum where on the vector
+// kernel next to none are (groups of 32, K 9216 and 12288).  The rounding itself is the larger part by far: the bf16 outputs
+// of both are 1.63e-3 to 1.70e-3 off, equal to six digits (K 512 to 25600, x of mean 0 and 1).
 //
 // Cost per weight: one VALU operation to build the operand (two byte permutes, three shifts and
 // eight and/or pairs per sixteen weights) and 1/512 of an MFMA, whatever M is.
@@ -249,9 +252,8 @@ __global__ __launch_bounds__(WAVES * kWave, KS == 1 && ROUNDS == 2 && EPI == kEp
     // (columns past N).  A load under a condition becomes a branch with a full wait behind it, and
     // a chain of those is a chain of memory round trips.
     //
-    // Scales and zero points of the columns this thread will own after the LDS round, one set per
-    // wave of the workgroup (a wave never straddles a quantisation group; waves that share a group
-    // read the same address).
+    // Scales and zero points of the columns this thread will own after the LDS round, one set per wave of the workgroup (whose
+    // steps share a quantisation group, FINE aside; waves that share one read the same address).
     const int own_piece = tid % 32;
     const int own_half = tid / 128;
     const int own_row = tid / 32 % 4;

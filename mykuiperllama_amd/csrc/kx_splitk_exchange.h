@@ -589,7 +589,8 @@ __device__ __forceinline__ void splitk_sum_runs(__amdgpu_buffer_rsrc_t rsrc, int
 }
 
 // The exchange for several activation rows (ROWS = 4, 8 or 16) and a workgroup of exactly 256 threads, more
-// than one K tile.  The caller has stored the workgroup's partial sums (store_partial_quad).  The last workgroup reads them back
+// than one K tile.  The caller has stored the workgroup's partial sums: from eight rows on in the order of partial_column
+// (store_partial_quad), with four rows column by column (store_agent).  The last workgroup reads them back
 // two columns per load: threads 0..127 take rows 0 .. ROWS/2-1 of column pairs 0..127, threads 128..255 the
 // other rows, so a K tile costs a thread ROWS/2 eight-byte loads instead of ROWS four-byte ones and every
 // K tile of the usual shapes is in flight at once.  Per output the additions run t = 0, 1, 2, ... as in
