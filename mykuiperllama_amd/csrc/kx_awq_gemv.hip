@@ -443,6 +443,15 @@ extern "C" size_t kx_gemv_workspace_bytes(int32_t M, int32_t K, int32_t N) {
     return kx::kCounterBytes + ktiles * M * static_cast<size_t>(N) * sizeof(float);
 }
 
+extern "C" int kx_shared_line_tile(int32_t coltiles, int32_t ktiles, int32_t id, int32_t* ct, int32_t* kt) {
+    const kx::TileOrder order = kx::tile_order_of(static_cast<uint32_t>(coltiles), static_cast<uint32_t>(ktiles));
+    if (!order.run) return 0;
+    const kx::Tile tile = kx::tile_of_workgroup(order, static_cast<uint32_t>(id), static_cast<uint32_t>(ktiles));
+    *ct = tile.ct;
+    *kt = tile.kt;
+    return 1;
+}
+
 extern "C" int kx_workspace_init(void* workspace, size_t workspace_bytes, void* stream) {
     if (!workspace) return KX_ERR_NULL_POINTER;
     if (workspace_bytes < kx::kCounterBytes) return KX_ERR_WORKSPACE;

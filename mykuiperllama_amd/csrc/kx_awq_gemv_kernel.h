@@ -91,8 +91,8 @@ __global__ __launch_bounds__(WAVES * kWave) void awq_gemv_kernel(
     const uint16_t* __restrict__ x, const uint32_t* __restrict__ qweight,
     const uint16_t* __restrict__ scales, const uint32_t* __restrict__ qzeros,
     uint16_t* __restrict__ y, float* __restrict__ partials, uint32_t* __restrict__ counters,
-    int M, int K, int N, int group, int group_shift, int coltiles, int ktiles, FusedInput fi, RopeTarget rope,
-    ResidualTarget res) {
+    int M, int K, int N, int group, int group_shift, int coltiles, int ktiles, TileOrder order, FusedInput fi,
+    RopeTarget rope, ResidualTarget res) {
     constexpr int SLOTS = WAVES * kSlotsPerWave;
     constexpr int KB = SLOTS * RT;
     constexpr int THREADS = WAVES * kWave;
@@ -122,8 +122,10 @@ __global__ __launch_bounds__(WAVES * kWave) void awq_gemv_kernel(
     const int tid = threadIdx.x;
     // grid = (column tiles, K tiles, activation-row tiles): x runs fastest, so workgroups that start together read
     // neighbouring 128-byte pieces of the same rows, and no division stands in front of the first load
-    const int ct = blockIdx.x;
-    const int kt = blockIdx.y;
+    Tile tile{static_cast<int>(blockIdx.x), static_cast<int>(blockIdx.y)};
+    if (order.run) tile = tile_of_workgroup(order, static_cast<uint32_t>(tile.kt * coltiles + tile.ct), static_cast<uint32_t>(ktiles));
+    const int ct = tile.ct;
+    const int kt = tile.kt;
     const int m0 = blockIdx.z * MB;
     const int nw = N >> 3;
 
@@ -671,7 +673,7 @@ inline void launch_awq_gemv(const uint16_t* x, const int32_t* qweight, const uin
     hipLaunchKernelGGL((awq_gemv_kernel<WAVES, RT, MB, PRO, EPI>), grid, block, 0, stream, x,
                        reinterpret_cast<const uint32_t*>(qweight), scales,
                        reinterpret_cast<const uint32_t*>(qzeros), y, partials, counters, M, K, N,
-                       group, group_shift, coltiles, ktiles, fi, rope, res);
+                       group, group_shift, coltiles, ktiles, packed_tile_order(qweight, N, coltiles, ktiles), fi, rope, res);
 }
 
 }  // namespace kx

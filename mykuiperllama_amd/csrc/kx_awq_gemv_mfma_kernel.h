@@ -131,6 +131,7 @@ struct MfmaGrid {
     int sliced;            // all K tiles of a column tile finish it together (splitk_exchange_sliced)
     uint32_t group_magic;  // ceil(2^32 / (G / 32)), 0 for groups of 32
     uint32_t wait_ticks;   // how long a workgroup waits for the others of its tile
+    TileOrder order;       // which tile a workgroup takes where not that of its own number
 };
 
 // Quantisation group of a 32-row step: step / (G / 32) for any number of steps a matrix can have.
@@ -219,9 +220,11 @@ __global__ __launch_bounds__(WAVES * kWave, KS == 1 && ROUNDS == 2 && EPI == kEp
     const int b = lane / 16;  // k block inside the step, D row block
     // Column tiles run fastest, so neighbours in time are neighbours in N; where workgroups finish a tile together, in
     // groups of at most eight, so that they start within 8 * ktiles of each other.
-    const int ct = blockIdx.z * grid.side + blockIdx.x;
-    const int kt = blockIdx.y;
+    Tile tile{static_cast<int>(blockIdx.z * grid.side + blockIdx.x), static_cast<int>(blockIdx.y)};
     const int ktiles = grid.ktiles;
+    if (grid.order.run) tile = tile_of_workgroup(grid.order, (blockIdx.z * ktiles + blockIdx.y) * grid.side + blockIdx.x, static_cast<uint32_t>(ktiles));
+    const int ct = tile.ct;
+    const int kt = tile.kt;
     const int nw = N >> 3;
 
     // first row of the block that is loaded next, and how many blocks the workgroup has
@@ -854,10 +857,12 @@ inline void launch_awq_gemv_mfma(const uint16_t* x, const int32_t* qweight, cons
 
     const dim3 grid(split.side, split.ktiles, split.coltiles / split.side);
     dim3 block(WAVES * kWave, 1, 1);
+    MfmaGrid ordered = split;
+    ordered.order = packed_tile_order(qweight, N, split.coltiles, split.ktiles);
     hipLaunchKernelGGL((awq_gemv_mfma_kernel<WAVES, KS, MC, ROUNDS, PRO, EPI, LONE, WALK, FINE>), grid, block, 0, stream, x,
                        reinterpret_cast<const uint32_t*>(qweight), scales,
                        reinterpret_cast<const uint32_t*>(qzeros), y, partials, counters, M, K, N,
-                       split, fi, res, rope, cache_stride);
+                       ordered, fi, res, rope, cache_stride);
 }
 
 }  // namespace kx

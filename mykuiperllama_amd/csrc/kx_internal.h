@@ -65,6 +65,10 @@ typedef struct kx_step_desc {
 
 int kx_decode_step_bf16(const kx_step_desc* desc, const kx_step_layer* layers, void* stream);
 
+/* Column tile and K tile of workgroup `id` of a grid whose neighbouring column tiles share memory lines (csrc/kx_tile_order.h):
+ * 1, or 0 where such a grid is too small or too large for it and a workgroup takes the tile of its own number. */
+int kx_shared_line_tile(int32_t coltiles, int32_t ktiles, int32_t id, int32_t* ct, int32_t* kt);
+
 /* Bytes of a kx_step_desc and of a kx_step_layer as the library was compiled: a binding that mirrors them compares. */
 size_t kx_step_desc_bytes(void);
 size_t kx_step_layer_bytes(void);

@@ -32,6 +32,7 @@
 #define KX_SPLITK_EXCHANGE_H
 
 #include "kx_common.h"
+#include "kx_tile_order.h"
 
 #if defined(__HIP_DEVICE_COMPILE__) && !defined(__gfx950__)
 #error "kx_splitk_exchange.h orders its memory operations by gfx950's write-through stores and vmcnt acknowledgements; other targets need release/acquire orderings"
@@ -39,8 +40,7 @@
 
 namespace kx {
 
-constexpr int kTileCols = 256;     // output columns per column tile, one thread each in the exchange
-constexpr int kCounterStride = 16; // uint32 slots between counters: one 64-byte line each
+constexpr int kCounterStride = 16;  // uint32 slots between counters: one 64-byte line each
 
 // Nothing in the language orders the relaxed loads of a read-back behind the relaxed atomic whose result decides
 // that they run; the hardware does (the loads sit behind a branch on that result).  This keeps the compiler from

@@ -1,0 +1,82 @@
+// Which part of the packed matrix a workgroup of the GEMV kernels takes.
+#ifndef KX_TILE_ORDER_H
+#define KX_TILE_ORDER_H
+
+#include "kx_common.h"
+
+namespace kx {
+
+constexpr int kTileCols = 256;  // output columns per column tile: 128 bytes of a packed row
+
+// Which tile of a (column tiles x K tiles) grid a workgroup takes when neighbouring column tiles are to run on one XCD.
+// Workgroups go to the eight XCDs in turn; the tiles, counted in groups of kTilesSideBySide columns with the columns of a
+// group fastest, are cut into eight runs, one per XCD.  (One group of all columns would give an XCD few K tiles of many
+// columns, and where the workgroup that comes last finishes a column alone, the XCD that is last would finish them all:
+// 1024 -> 17704, groups of 32, M = 16 12.9 -> 17.0 us; groups of eight columns have a boundary more often, 15872 -> 18064 at
+// M = 1 38.8 -> 40.4.)
+struct TileOrder {
+    uint32_t run = 0;          // tiles per XCD, 0: a workgroup takes the tile of its own number
+    uint32_t extra = 0;        // the first `extra` XCDs take one more
+    uint32_t whole = 0;        // columns in whole groups
+    uint32_t in_whole = 0;     // tiles of those
+    uint32_t group_magic = 0;  // divides by the tiles of a group
+    uint32_t rest = 0;         // columns behind the whole groups
+    uint32_t rest_magic = 0;   // divides by them; 0 for none and one
+};
+constexpr uint32_t kXcds = 8;
+constexpr uint32_t kTilesSideBySide = 32;
+
+// n / divisor = n * magic >> 32 where n * divisor < 2^32; divisor > 1
+inline uint32_t magic_of(uint32_t divisor) {
+    return static_cast<uint32_t>(((1ull << 32) + divisor - 1) / divisor);
+}
+__host__ __device__ inline uint32_t divide_by_magic(uint32_t n, uint32_t magic) {
+    return static_cast<uint32_t>((static_cast<uint64_t>(n) * magic) >> 32);
+}
+
+inline TileOrder tile_order_of(uint32_t coltiles, uint32_t ktiles) {
+    TileOrder o;
+    const uint64_t tiles = static_cast<uint64_t>(coltiles) * ktiles, group = static_cast<uint64_t>(kTilesSideBySide) * ktiles;
+    if (coltiles < 2 || tiles < 2 * kXcds || (tiles * group) >> 32) return o;
+    o.run = static_cast<uint32_t>(tiles / kXcds);
+    o.extra = static_cast<uint32_t>(tiles % kXcds);
+    o.rest = coltiles % kTilesSideBySide;
+    o.whole = coltiles - o.rest;
+    o.in_whole = o.whole * ktiles;
+    o.group_magic = magic_of(static_cast<uint32_t>(group));
+    o.rest_magic = o.rest > 1 ? magic_of(o.rest) : 0u;
+    return o;
+}
+
+struct Tile {
+    int ct, kt;
+};
+// `id` counts the workgroups of the grid as they are dispatched.
+__host__ __device__ __forceinline__ Tile tile_of_workgroup(const TileOrder& o, uint32_t id, uint32_t ktiles) {
+    const uint32_t xcd = id % kXcds;
+    uint32_t tile = xcd * o.run + (xcd < o.extra ? xcd : o.extra) + id / kXcds;
+    if (tile < o.in_whole) {
+        const uint32_t group = divide_by_magic(tile, o.group_magic);
+        tile -= group * ktiles * kTilesSideBySide;
+        return {static_cast<int>(group * kTilesSideBySide + tile % kTilesSideBySide), static_cast<int>(tile / kTilesSideBySide)};
+    }
+    tile -= o.in_whole;
+    const uint32_t kt = o.rest_magic ? divide_by_magic(tile, o.rest_magic) : tile;
+    return {static_cast<int>(o.whole + tile - kt * o.rest), static_cast<int>(kt)};
+}
+
+// Neighbouring column tiles share a memory line in every row whose 128-byte pieces do not start on a line: in the order of the
+// numbers they lie on different XCDs, each of which fetches the line into its own L2.  us per launch at M = 1 / 2 / 4 / 8 / 16, by
+// number -> by XCD: 4480 -> 20328 21.5 / 22.0 / 23.7 / 28.1 / 28.1 -> 15.6 / 17.3 / 18.6 / 23.4 / 23.9, 5472 -> 9000 with groups of 32
+// 12.4 / 14.7 / 16.0 / 16.7 / 17.9 -> 10.1 / 13.5 / 13.3 / 13.9 / 15.5, 15872 -> 18064 with groups of 64 49.4 / 51.4 / 54.1 / 60.7 / 70.2 ->
+// 38.8 / 41.8 / 43.3 / 50.3 / 61.5, 2176 -> 17792 (half a line) 8.3 / 10.0 / 11.0 / 12.8 / 14.9 -> 7.6 / 9.0 / 10.0 / 12.0 / 13.9.
+// Where the pieces are whole lines nothing is shared, and neighbours on different XCDs are up to 15 % faster: 4096 -> 24576
+// 13.9 / 15.3 / 16.6 / 19.3 / 20.3 by number against 14.6 / 15.8 / 17.7 / 21.1 / 21.2.
+inline TileOrder packed_tile_order(const void* qweight, int N, int coltiles, int ktiles) {
+    const bool whole_lines = N % kTileCols == 0 && reinterpret_cast<uintptr_t>(qweight) % 128 == 0;
+    return whole_lines ? TileOrder{} : tile_order_of(static_cast<uint32_t>(coltiles), static_cast<uint32_t>(ktiles));
+}
+
+}  // namespace kx
+
+#endif  // KX_TILE_ORDER_H

@@ -1,0 +1,42 @@
+"""Packed rows whose 128-byte pieces do not start on a memory line: column tiles taken in another order, the same sums."""
+import numpy as np
+import pytest
+
+from mykuiperllama_amd import synth
+from tests import helpers as H
+
+pytestmark = pytest.mark.gpu
+
+
+def run(torch, capi, M, K, N, group, shift):
+    p = synth.make_awq_problem(f"order_{M}_{K}_{N}", M, K, N, group)
+    words = torch.zeros(K * N // 8 + 64, dtype=torch.int32, device="cuda")
+    qw = words[shift:shift + K * N // 8].view(K, N // 8)
+    qw.copy_(H.to_dev_i32(p["qweight"], torch))
+    y = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda")
+    capi.gemv_awq_bf16(H.to_dev_bf16(p["x"], torch), qw, H.to_dev_f16(p["scales"], torch), H.to_dev_i32(p["qzeros"], torch), y,
+                       group, capi.make_workspace(M, K, N))
+    torch.cuda.synchronize()
+    return p, H.bf16_bits(y, torch)
+
+
+# one column short of, at and past groups of 32 column tiles, with one and several K tiles; fewer tiles than it takes
+@pytest.mark.parametrize("M", [1, 2, 5, 16])
+@pytest.mark.parametrize("K,N,group", [(512, 31 * 256 - 8, 128), (512, 32 * 256 + 128, 32), (640, 33 * 256 + 16, 64), (2048, 1048, 32),
+                                       (1024, 264, 128)])
+def test_against_the_oracle(oracle, M, K, N, group):
+    import torch
+    from mykuiperllama_amd import capi
+    p, bits = run(torch, capi, M, K, N, group, 0)
+    ref = oracle.gemv_awq_f64(p["x"], p["qweight"], p["scales"], p["qzeros"], group)
+    ref = H.bf16_to_f64(oracle.f32_to_bf16(ref.astype(np.float32)))
+    assert H.rel_l2(H.bf16_to_f64(bits), ref) <= 1e-3
+
+
+@pytest.mark.parametrize("M", [1, 3, 9])
+def test_weights_off_a_line_return_the_same_bits(M):
+    import torch
+    from mykuiperllama_amd import capi
+    on = run(torch, capi, M, 1024, 33 * 256, 128, 0)[1]
+    off = run(torch, capi, M, 1024, 33 * 256, 128, 1)[1]
+    assert np.array_equal(on, off)
