@@ -187,58 +187,75 @@ __global__ __launch_bounds__(kMfmaWaves * kWave) void bf16_gemv_mfma_kernel(
     }
 }
 
-// Two to sixteen activation rows, K <= 1024 * UNITS: one workgroup per compute unit walks over blocks of sixteen output
-// columns, and its eight waves split K.  What bounded the kernel above was not W but everything round it: the
-// activation rows came out of L2 anew for every 64 columns, and an MFMA operand fetched straight from memory asks for
-// 64 bytes of sixteen rows at a time, which the memory system answers at three quarters of its rate.  Here the A operands
-// of a wave's part of K stay in registers for the life of the workgroup, and W goes through LDS: a unit is 128 elements
-// of the block's sixteen rows (4 KB, four loads of 4 rows x 256 bytes), loaded straight into the wave's own ring of
-// kRing units, so that no barrier and no register stands between the stream and the MFMAs and 128 KB per compute unit
-// are in flight.  The waves of a block meet in LDS, two buffers in turn, one barrier per block that leaves loads alone.
+// Two to sixteen activation rows, K <= 8192: one workgroup per compute unit walks over blocks of sixteen output columns, and
+// PARTS of its waves split K between them (the others take further blocks side by side).  What bounded the kernel above was
+// not W but everything round it: the activation rows came out of L2 anew for every 64 columns, and an MFMA operand fetched
+// straight from memory asks for 64 bytes of sixteen rows at a time, which the memory system answers at three quarters of its
+// rate.  Here the A operands of a wave's part of K stay in registers for the life of the workgroup, and W goes through LDS: a
+// unit is UNIT elements of the block's sixteen rows, loaded straight into the wave's own ring, so that no barrier and no
+// register stands between the stream and the MFMAs and 128 KB per compute unit are in flight.  The waves of a block meet in
+// LDS, two buffers in turn, one barrier per block that leaves loads alone.  K is cut into whole units, as evenly as they go: a
+// part has UNITS of them or one less.
 // A row of a unit is stored with its 16-byte pieces permuted by the low bits of the row (the lane that loads piece j of
 // row r fetches piece j ^ (r & 7)), so that the sixteen rows that an operand read touches lie in different banks.
-// us at M = 3 / 8 / 16, kernel above -> this one: lm_head 151936 x 4096 273 / 308 / 297 -> 182 / 189 / 199 (W alone at the
-// read rate of a large buffer: 171), 151936 x 5120 382 / 447 / 405 -> 231 / 240 / 254, 4096 x 4096 11.4 / 12.1 / 26.3 ->
-// 9.1 / 9.2 / 10.5.
-// EXACT: K is 1024 * UNITS; otherwise what lies past K is zeroed in both operands.
-constexpr int kHeldWaves = 8;
-constexpr int kRing = 4;
-constexpr int kUnitBytes = 16 * 256;
+// Two shapes.  Where rows start on memory lines, eight waves and units of 128 elements, 256 bytes of a row, which are two lines.
+// Rows that do not start on lines would have such a piece touch three: four waves and units of 512 elements, nine lines for
+// eight.  us per launch at M = 3 / 8 / 16, eight waves of equal parts of K rounded up to 1024 -> now: rows on lines 151936 x 4096
+// 195 / 202 / 215 -> 194 / 199 / 204, 151936 x 5120 238 / 247 / 263 -> 239 / 242 / 250, 32000 x 768 12.9 / 13.2 / 13.4 -> 10.9 /
+// 11.1 / 11.8; others 144453 x 3144 180 / 192 / 210 -> 160 / 166 / 174, 101754 x 2336 92 / 96 / 106 -> 83 / 86 / 89, 79438 x 1240
+// 48.6 / 50.0 / 53.4 -> 38.8 / 39.6 / 41.7, 69572 x 4688 123 / 126 / 133 -> 110 / 113 / 116 (W alone at the read rate of a large
+// buffer: 173, 216, 6.8; 126, 66, 27, 91).  Cached loads instead of streaming ones lose 10 % on lines and win 2 % off them.
+constexpr int kRingBytes = 131072;
 
-template <int UNITS, bool EXACT>
-__global__ __launch_bounds__(kHeldWaves * kWave, 2) void bf16_gemv_held_kernel(
+template <int WAVES, int UNIT, int UNITS, int PARTS, bool RUNS>
+__global__ __launch_bounds__(WAVES * kWave, WAVES / 4) void bf16_gemv_held_kernel(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, uint16_t* __restrict__ y, int M, int K, int N, int blocks) {
-    __shared__ __attribute__((aligned(1024))) char ring[kHeldWaves][kRing][kUnitBytes];
-    __shared__ __attribute__((aligned(16))) float red[2][kHeldWaves][4][kWave];
+    constexpr int SIDE = WAVES / PARTS;          // blocks a workgroup works on side by side
+    constexpr int STEPS = UNIT / 32;
+    constexpr int PIECES = UNIT / 8;             // 16-byte pieces of a row of a unit
+    constexpr int ROWS = kWave / PIECES;         // rows a load brings
+    constexpr int LOADS = 16 / ROWS;
+    constexpr int RING = kRingBytes / WAVES / (32 * UNIT);
+    __shared__ __attribute__((aligned(1024))) char ring[WAVES][RING][32 * UNIT];
+    __shared__ __attribute__((aligned(16))) float red[2][WAVES][4][kWave];
     const int tid = threadIdx.x;
     const int lane = tid % kWave;
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int part = wave % PARTS;
     const int c = lane % 16;
     const int b = lane / 16;
-    const int kw = wave * 128 * UNITS;  // the wave's first element of K
-    const int stride = gridDim.x;
+    const int units = (K + UNIT - 1) / UNIT;
+    const int unit0 = part * units / PARTS;                // the wave's first unit of K
+    const int mine = (part + 1) * units / PARTS - unit0;   // UNITS, or one less
+    const int kw = UNIT * unit0;
+    // RUNS: a workgroup takes four blocks in a row as long as there are whole rounds of that, so that the 64 outputs of a line of
+    // y come from one XCD; the rest, and without RUNS all, go round one by one.
+    constexpr int RUN = RUNS && SIDE < 4 ? 4 / SIDE : 1;
+    const int wgs = gridDim.x, wg = blockIdx.x;
+    const int in_runs = (blocks + SIDE - 1) / SIDE / (RUN * wgs) * RUN;
+    auto block_of = [&](int turn) { return SIDE * (turn < in_runs ? turn / RUN * RUN * wgs + wg * RUN + turn % RUN : turn * wgs + wg); };
 
-    bf16x8 held[UNITS][4];
+    bf16x8 held[UNITS][STEPS];
     const uint16_t* xrow = x + static_cast<size_t>(min(c, M - 1)) * K;
 #pragma unroll
     for (int u = 0; u < UNITS; u++) {
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const int k = kw + 128 * u + 32 * q + 8 * b;
-            const bool in = EXACT || k < K;
+        for (int q = 0; q < STEPS; q++) {
+            const int k = kw + UNIT * u + 32 * q + 8 * b;
+            const bool in = k < K;
             const u32x4 v = *reinterpret_cast<const u32x4*>(xrow + (in ? k : 0));
             const bool live = in && c < M;
             held[u][q] = as_bf16x8(live ? v.x : 0u, live ? v.y : 0u, live ? v.z : 0u, live ? v.w : 0u);
         }
     }
 
-    // Loads unit u of a block into a ring slot: load i brings rows 4 i + lane / 16.
+    // Loads unit u of a block into a ring slot: load i brings rows ROWS * i + lane / PIECES.
     auto fetch = [&](int block, int u, int slot) {
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int r = 4 * i + b;
-            const int k = kw + 128 * u + 8 * (c ^ (r & 7));
-            const uint16_t* src = w + static_cast<size_t>(min(16 * block + r, N - 1)) * K + (EXACT || k < K ? k : 0);
+        for (int i = 0; i < LOADS; i++) {
+            const int r = ROWS * i + lane / PIECES;
+            const int k = kw + UNIT * u + 8 * (lane % PIECES ^ (r & 7));
+            const uint16_t* src = w + static_cast<size_t>(min(16 * block + r, N - 1)) * K + min(k, K - 8);
             __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
                                              (__attribute__((address_space(3))) void*)(&ring[wave][slot][i * 1024]), 16, 0, 2);
         }
@@ -246,60 +263,162 @@ __global__ __launch_bounds__(kHeldWaves * kWave, 2) void bf16_gemv_held_kernel(
     // Where the lane finds its operand of step q: row c, piece 4 q + b; steps 2 and 3 lie 128 bytes behind 0 and 1.
     const uint32_t ring0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
         (__attribute__((address_space(3))) char*)(&ring[wave][0][0])));
-    const uint32_t at0 = ring0 + c * 256 + ((b ^ (c & 7)) * 16);
-    const uint32_t at1 = ring0 + c * 256 + (((4 + b) ^ (c & 7)) * 16);
+    const uint32_t at0 = ring0 + c * (2 * UNIT) + ((b ^ (c & 7)) * 16);
+    const uint32_t at1 = ring0 + c * (2 * UNIT) + (((4 + b) ^ (c & 7)) * 16);
 
-    const int first = blockIdx.x;
+    // the unit that is fetched next, and how many are on their way or waiting in the ring
+    const int side_of_wave = wave / PARTS;
+    int fetch_turn = 0, fetch_block = block_of(0) + side_of_wave, fetch_unit = 0, ahead = 0;
+    auto fetch_next = [&](int slot) {
+        if (mine == 0 || fetch_block >= blocks) return;
+        fetch(fetch_block, fetch_unit, slot);
+        ahead++;
+        if (++fetch_unit == mine) {
+            fetch_unit = 0;
+            fetch_block = block_of(++fetch_turn) + side_of_wave;
+        }
+    };
 #pragma unroll
-    for (int j = 0; j < kRing; j++) {
-        const int block = first + (j / UNITS) * stride;
-        if (block < blocks) fetch(block, j % UNITS, j);
-    }
-    int slot = 0, turn = 0;
-    for (int block = first; block < blocks; block += stride, turn ^= 1) {
+    for (int j = 0; j < RING; j++) fetch_next(j);
+    int slot = 0;
+    for (int turn = 0, row; row = block_of(turn), row < blocks; turn++) {
+        const int block = row + side_of_wave;
         f32x4v acc[2];
         acc[0] = acc[1] = f32x4v{0.0f, 0.0f, 0.0f, 0.0f};
+        if (SIDE == 1 || block < blocks) {
 #pragma unroll
-        for (int u = 0; u < UNITS; u++) {
-            // The unit kRing places further on will take this slot.  Loads return in order: with it to come, kRing - 1
-            // units may still be on their way when this one has arrived; in the last ring, wait for everything.
-            const int next = block + ((u + kRing) / UNITS) * stride;
-            const int held_back = block + ((u + kRing - 1) / UNITS) * stride;
-            if (held_back < blocks) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(4 * (kRing - 1)) : "memory");
-            else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-            u32x4 v[4];
-            const uint32_t s0 = at0 + slot * kUnitBytes, s1 = at1 + slot * kUnitBytes;
-            // in assembly, because the compiler would wait for every load in flight ahead of a read of the ring
-            asm volatile("ds_read_b128 %0, %4\n\tds_read_b128 %1, %5\n\tds_read_b128 %2, %4 offset:128\n\tds_read_b128 %3, %5 offset:128\n\ts_waitcnt lgkmcnt(0)"
-                         : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3])
-                         : "v"(s0), "v"(s1)
-                         : "memory");
-            if (next < blocks) fetch(next, (u + kRing) % UNITS, slot);
+            for (int u = 0; u < UNITS; u++) {
+                if (u < mine) {
+                    // Loads return in order: with the ring full, RING - 1 units may still be on their way when this one has arrived.
+                    if (ahead == RING) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS * (RING - 1)) : "memory");
+                    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                    u32x4 v[STEPS];
+                    const uint32_t s0 = at0 + slot * (32 * UNIT), s1 = at1 + slot * (32 * UNIT);
+                    // in assembly, because the compiler would wait for every load in flight ahead of a read of the ring
 #pragma unroll
-            for (int q = 0; q < 4; q++) {
-                u32x4 p = v[q];
-                if constexpr (!EXACT) {
-                    const bool live = kw + 128 * u + 32 * q + 8 * b < K;
-                    p = u32x4{live ? p.x : 0u, live ? p.y : 0u, live ? p.z : 0u, live ? p.w : 0u};
+                    for (int q = 0; q < STEPS; q += 4) {
+                        asm volatile("ds_read_b128 %0, %4 offset:%6\n\tds_read_b128 %1, %5 offset:%6\n\tds_read_b128 %2, %4 offset:%7\n\t"
+                                     "ds_read_b128 %3, %5 offset:%7\n\ts_waitcnt lgkmcnt(0)"
+                                     : "=&v"(v[q]), "=&v"(v[q + 1]), "=&v"(v[q + 2]), "=&v"(v[q + 3])
+                                     : "v"(s0), "v"(s1), "n"(64 * q), "n"(64 * q + 128)
+                                     : "memory");
+                    }
+                    ahead--;
+                    fetch_next(slot);
+                    if (kw + UNIT * u + UNIT > K) {  // the last unit of a K that is no multiple of a unit
+#pragma unroll
+                        for (int q = 0; q < STEPS; q++) {
+                            const bool live = kw + UNIT * u + 32 * q + 8 * b < K;
+                            v[q] = u32x4{live ? v[q].x : 0u, live ? v[q].y : 0u, live ? v[q].z : 0u, live ? v[q].w : 0u};
+                        }
+                    }
+#pragma unroll
+                    for (int q = 0; q < STEPS; q++) {
+                        acc[q & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(held[u][q], as_bf16x8(v[q].x, v[q].y, v[q].z, v[q].w), acc[q & 1], 0, 0, 0);
+                    }
+                    slot = (slot + 1) % RING;
                 }
-                acc[q & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(held[u][q], as_bf16x8(p.x, p.y, p.z, p.w), acc[q & 1], 0, 0, 0);
             }
-            slot = (slot + 1) % kRing;
+        }
+        if constexpr (PARTS == 1) {
+            const int n = 16 * block + c;
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int m = 4 * b + v;
+                if (m < M && n < N && block < blocks) y[static_cast<size_t>(m) * N + n] = f32_to_bf16(acc[0][v] + acc[1][v]);
+            }
+            continue;
         }
 #pragma unroll
-        for (int v = 0; v < 4; v++) red[turn][wave][v][lane] = acc[0][v] + acc[1][v];
+        for (int v = 0; v < 4; v++) red[turn % 2][wave][v][lane] = acc[0][v] + acc[1][v];
         lds_barrier();
-        if (tid < 4 * kWave) {  // thread (v, lane): row 4 (lane / 16) + v of column lane % 16
-            const float* src = &red[turn][0][0][0] + tid;
-            float part[kHeldWaves];
+        // thread (v, lane): row 4 (lane / 16) + v of column lane % 16
 #pragma unroll
-            for (int u = 0; u < kHeldWaves; u++) part[u] = src[u * 4 * kWave];
-            const float sum = ((part[0] + part[1]) + (part[2] + part[3])) + ((part[4] + part[5]) + (part[6] + part[7]));
-            const int m = 4 * b + tid / kWave;
-            const int n = 16 * block + c;
-            if (m < M && n < N) y[static_cast<size_t>(m) * N + n] = f32_to_bf16(sum);
+        for (int e = 0; e < SIDE; e += WAVES / 4) {
+            const int side = e + tid / (4 * kWave);
+            if (SIDE % (WAVES / 4) != 0 && side >= SIDE) break;
+            const float* src = &red[turn % 2][side * PARTS][0][0] + tid % (4 * kWave);
+            float sum[PARTS];
+#pragma unroll
+            for (int u = 0; u < PARTS; u++) sum[u] = src[u * 4 * kWave];
+#pragma unroll
+            for (int d = 1; d < PARTS; d *= 2) {
+#pragma unroll
+                for (int u = 0; u < PARTS; u += 2 * d) sum[u] += sum[u + d];
+            }
+            const int m = 4 * b + wave % 4;
+            const int n = 16 * (row + side) + c;
+            if (m < M && n < N) y[static_cast<size_t>(m) * N + n] = f32_to_bf16(sum[0]);
         }
     }
+}
+
+constexpr int kHeldMostK = 8192;
+constexpr int kComputeUnits = 256;
+
+template <int WAVES, int UNIT, int PARTS, bool RUNS>
+int launch_held_parts(const uint16_t* x, const uint16_t* w, uint16_t* y, int M, int K, int N, hipStream_t s) {
+    constexpr int SIDE = WAVES / PARTS;
+    const int blocks = (N + 15) / 16, sides = (blocks + SIDE - 1) / SIDE;
+    const dim3 grid(sides < kComputeUnits ? sides : kComputeUnits), block(WAVES * kWave);
+#define KX_HELD(U)                                                                                                                   \
+    case U:                                                                                                                          \
+        if constexpr (UNIT * PARTS * (U - 1) < kHeldMostK && (PARTS > 1 || U <= 3)) {                                                \
+            hipLaunchKernelGGL((bf16_gemv_held_kernel<WAVES, UNIT, U, PARTS, RUNS>), grid, block, 0, s, x, w, y, M, K, N, blocks);   \
+        }                                                                                                                            \
+        break
+    switch (((K + UNIT - 1) / UNIT + PARTS - 1) / PARTS) {
+        KX_HELD(1);
+        KX_HELD(2);
+        KX_HELD(3);
+        KX_HELD(4);
+        KX_HELD(5);
+        KX_HELD(6);
+        KX_HELD(7);
+        KX_HELD(8);
+    }
+#undef KX_HELD
+    return launch_status();
+}
+
+// Runs of four blocks pay with the rows of y that are written and are lost among long rows of W: us per launch, one by one -> in
+// runs, M = 16 151936 x 4096 214 -> 204, 151936 x 5120 266 -> 250, 144453 x 3144 184 -> 174; M = 8 151936 x 4096 203 -> 199; M = 3
+// 144453 x 3144 160 -> 162; 40000 x 8192 at M = 8 / 16 110 / 114 -> 115 / 118.
+template <int WAVES, int UNIT, int PARTS>
+int launch_held_parts(const uint16_t* x, const uint16_t* w, uint16_t* y, int M, int K, int N, hipStream_t s) {
+    if (M >= 6 && K <= 6144) return launch_held_parts<WAVES, UNIT, PARTS, true>(x, w, y, M, K, N, s);
+    return launch_held_parts<WAVES, UNIT, PARTS, false>(x, w, y, M, K, N, s);
+}
+
+// The fewest parts whose A operands fit the registers and whose last round of blocks is not emptier for it by more than it gains:
+// a barrier for every PARTS-th of the blocks.  us per launch at M = 3, parts of K 8 / 4 / 2 on lines: 32000 x 768 12.0 / 11.6 / 10.9,
+// 60000 x 2048 44.8 / 42.9 / 42.0, 151936 x 4096 198 / 196 / -; 4 / 2 / 1 off lines: 67290 x 912 30.2 / 27.1 / 25.8, 98237 x 1232 49.6 /
+// 47.8 / 46.0, 91208 x 1568 54.1 / 54.3 / 54.7.  Few rounds leave compute units idle: up to four, all waves split K (4764 x 4032 at M = 16
+// 17.6 with four parts, 13.1 with eight).
+int launch_held(const uint16_t* x, const uint16_t* w, uint16_t* y, int M, int K, int N, hipStream_t s) {
+    const bool whole_lines = K % 64 == 0 && reinterpret_cast<uintptr_t>(w) % 128 == 0;
+    const int waves = whole_lines ? 8 : 4;
+    const int blocks = (N + 15) / 16;
+    const int least = blocks <= 4 * kComputeUnits ? waves : (whole_lines ? (K <= 2048 ? 2 : (K <= 4096 ? 4 : 8)) : (K <= 1536 ? 1 : 4));
+    int parts = waves;
+    long best = 0;
+    for (int p = waves, weight = 100 + (waves == 8 ? 9 : 6); p >= least; p /= 2, weight -= 3) {
+        const int side = waves / p;
+        const long rounds = ((blocks + side - 1) / side + kComputeUnits - 1) / kComputeUnits;
+        const long cost = rounds * side * weight;
+        if (best == 0 || cost < best) {
+            best = cost;
+            parts = p;
+        }
+    }
+    if (whole_lines) {
+        if (parts == 8) return launch_held_parts<8, 128, 8>(x, w, y, M, K, N, s);
+        if (parts == 4) return launch_held_parts<8, 128, 4>(x, w, y, M, K, N, s);
+        return launch_held_parts<8, 128, 2>(x, w, y, M, K, N, s);
+    }
+    if (parts == 4) return launch_held_parts<4, 512, 4>(x, w, y, M, K, N, s);
+    if (parts == 2) return launch_held_parts<4, 512, 2>(x, w, y, M, K, N, s);
+    return launch_held_parts<4, 512, 1>(x, w, y, M, K, N, s);
 }
 
 }  // namespace
@@ -316,33 +435,13 @@ extern "C" int kx_gemv_bf16(const uint16_t* x, const uint16_t* w, uint16_t* y, i
         return KX_ERR_ALIGNMENT;
     }
     hipStream_t s = kx::as_stream(stream);
-    constexpr int kReach = 128 * kx::kHeldWaves;  // elements of K that a unit of every wave covers
-    // Two rows share the vector kernel's loads well enough where W is small; with eight blocks per compute unit and rows of
-    // 8 KB its wave sums no longer hide.  us, vector -> held, 151936 outputs: K = 1024 50.9 -> 56.1, 2048 99 -> 99, 4096 204
-    // -> 187, 5120 269 -> 230, 8192 439 -> 380; 32768 outputs: 1024 13.4 -> 15.2, 2048 24.1 -> 25.8, 4096 46.4 -> 44.0, 8192
-    // 97.8 -> 85.2; 4096 outputs: 4096 9.0 -> 9.4, 8192 15.4 -> 15.5.  The line is on the safe side: K = 1536, 2560, 3072 and
-    // 3584 (6 to 15 % ahead from 32768 outputs on) and 16384 outputs from K = 4096 on (5 to 12 %) stay with the vector kernel.
-    if ((M >= 3 || (M == 2 && K >= 4096 && N >= 32768)) && K <= 8 * kReach) {
-        const int blocks = (N + 15) / 16;
-        const dim3 grid(blocks < 256 ? blocks : 256), block(kx::kHeldWaves * kx::kWave);
-#define KX_HELD(U)                                                                                                      \
-    do {                                                                                                                \
-        if (K == U * kReach) hipLaunchKernelGGL((kx::bf16_gemv_held_kernel<U, true>), grid, block, 0, s, x, w, y, M, K, N, blocks); \
-        else hipLaunchKernelGGL((kx::bf16_gemv_held_kernel<U, false>), grid, block, 0, s, x, w, y, M, K, N, blocks);     \
-    } while (0)
-        switch ((K + kReach - 1) / kReach) {
-            case 1: KX_HELD(1); break;
-            case 2: KX_HELD(2); break;
-            case 3: KX_HELD(3); break;
-            case 4: KX_HELD(4); break;
-            case 5: KX_HELD(5); break;
-            case 6: KX_HELD(6); break;
-            case 7: KX_HELD(7); break;
-            default: KX_HELD(8); break;
-        }
-#undef KX_HELD
-        return kx::launch_status();
-    }
+    // Two rows share the vector kernel's loads well enough where N is small or its sweeps of 128 pieces fit a short row.  us, vector
+    // -> held: 47090 x 776 17.2 -> 16.6, 53553 x 1176 33.5 -> 28.2, 101754 x 2336 96.7 -> 82.8, 46389 x 3912 71.6 -> 64.7, 69572 x 4688
+    // 122 -> 110, 151936 x 4096 195 -> 193, 17672 x 7064 53.4 -> 50.8; what the line leaves out: 32000 x 1024 13.2 -> 13.8, 28732 x 2696
+    // 31.7 -> 32.9, 83762 x 896 29.4 -> 29.4, 4361 x 1080 5.1 -> 5.7, 5573 x 3736 11.0 -> 12.7.
+    const int pieces = K / 8, swept = (pieces + 127) / 128 * 128;
+    const bool two_rows = M == 2 && N >= 6500 && (K >= 3072 || 5 * swept >= 6 * pieces);
+    if ((M >= 3 || two_rows) && K <= kx::kHeldMostK) return kx::launch_held(x, w, y, M, K, N, s);
     if (M >= 3) {
         // K > 8192: the activations of a wave's part do not fit its registers
         if (M <= 8) {

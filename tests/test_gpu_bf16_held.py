@@ -1,0 +1,61 @@
+"""BF16 GEMV of several rows: K at the edges of the units that a wave takes (128 elements where rows start on memory lines, 512
+elsewhere) and of the number of waves that split it, outputs at the edges of runs of four blocks and of a round of 256, against
+float64."""
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def check(torch, capi, w, K, N, Ms):
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(K * 31 + N)
+    for M in Ms:
+        x = torch.randn((M, K), device="cuda", generator=gen).bfloat16()
+        y = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda")
+        capi.gemv_bf16(x, w, y)
+        ref = (x.double() @ w.double().t().contiguous()).to(torch.bfloat16).double()
+        torch.cuda.synchronize()
+        # fp32 sums of bf16 products, rounded once: they differ from the rounded reference by flips of the last bit alone
+        assert ((y.double() - ref).norm() / ref.norm()).item() <= 1e-3, (M, K, N)
+
+
+@pytest.mark.parametrize("K", [16, 64, 128, 192, 504, 520, 896, 1032, 1088, 1536, 1544, 2048, 2056, 4032, 4104, 6144, 6152, 8184])
+@pytest.mark.parametrize("N", [4099, 16399])
+def test_units_and_parts(K, N):
+    import torch
+    from mykuiperllama_amd import capi
+    w = torch.randn((N, K), device="cuda").bfloat16()
+    check(torch, capi, w, K, N, (2, 3, 6, 16))
+
+
+@pytest.mark.parametrize("K", [520, 1024])
+@pytest.mark.parametrize("blocks", [255, 257, 1023, 1024, 1025, 1027, 2051, 2309])
+def test_rounds_and_runs(K, blocks):
+    import torch
+    from mykuiperllama_amd import capi
+    N = 16 * blocks - 5
+    w = torch.randn((N, K), device="cuda").bfloat16()
+    check(torch, capi, w, K, N, (3, 7))
+
+
+def test_weights_off_a_line():
+    import torch
+    from mykuiperllama_amd import capi
+    K, N = 1024, 17000
+    flat = torch.randn(N * K + 64, device="cuda").bfloat16()
+    check(torch, capi, flat[8:8 + N * K].view(N, K), K, N, (3, 16))
+
+
+@pytest.mark.parametrize("K", [136, 520, 1000])
+def test_what_lies_past_a_row_takes_no_part(K):
+    """The last unit of a row is read past K's end within W: an infinity there meets no zero."""
+    import torch
+    from mykuiperllama_amd import capi
+    N, M = 40, 5
+    w = torch.ones((N, K), device="cuda").bfloat16()
+    w[7, K - 1] = float("inf")
+    x = torch.ones((M, K), device="cuda").bfloat16()
+    y = torch.empty((M, N), dtype=torch.bfloat16, device="cuda")
+    capi.gemv_bf16(x, w, y)
+    torch.cuda.synchronize()
+    assert torch.isinf(y[:, 7]).all() and torch.isfinite(y[:, :7]).all() and torch.isfinite(y[:, 8:]).all()
