@@ -139,7 +139,6 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(const uint16_t* __res
 // ------------------------------------------------------------------------------------------------
 constexpr int kAttnThreads = 256;
 constexpr int kMaxGroup = 16;  // query heads per KV head: the rows of one MFMA tile
-
 template <int CHUNK>
 __global__ __launch_bounds__(kAttnThreads) void attn_decode_stage1(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k_cache, const uint16_t* __restrict__ v_cache,
@@ -152,7 +151,11 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_stage1(
     // neighbouring dims) of eight positions per lane, and with 66 dwords per row the four blocks of eight
     // positions that a read instruction touches fall on different banks.
     constexpr int kVRow = kHeadDim / 2 + 2;
-    __shared__ __attribute__((aligned(8))) uint32_t s_v[CHUNK][kVRow];
+    // Before that it holds the K rows, four dwords of padding per row (a lane reads sixteen bytes of its own row).
+    constexpr int kKRow = kHeadDim / 2 + 4;
+    __shared__ __attribute__((aligned(16))) uint32_t s_rows[CHUNK * kKRow];
+    uint32_t(*s_v)[kVRow] = reinterpret_cast<uint32_t(*)[kVRow]>(s_rows);
+    uint32_t(*s_k)[kKRow] = reinterpret_cast<uint32_t(*)[kKRow]>(s_rows);
 
     const int kvh = blockIdx.y;
     const int chunk = blockIdx.x;
@@ -197,14 +200,19 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_stage1(
         qraw[ks] = *reinterpret_cast<const u32x4*>(q + (static_cast<size_t>(kvh) * G + q_head) * kHeadDim + 32 * ks + 8 * mb);
     }
     u32x4 kraw[TPW][4], vraw[ITERS];
+    // K rows are loaded as the V rows are, sixteen lanes to a row of 256 bytes, and pass through LDS to the lanes whose operands
+    // they are.  Loaded as operands (four lanes to a row, 64 bytes of it per load) every memory line was asked for twice, and
+    // with more loads in flight than L1 holds it was fetched twice.  us per launch, as operands -> by rows, merge included: 16
+    // sequences at context 4096 55.0 -> 52.9, one at 40001 37.7 -> 35.7, four of 64 heads at 3000 17.7 -> 16.9; the first stage
+    // alone at 4096 6.55 -> 6.37, at 8192 with 64 heads 10.6 -> 9.85, 16 heads at 700 4.17 -> 4.03.  Same bits.
 #pragma unroll
     for (int t = 0; t < TPW; t++) {
-        const int p = p0 + (wave * TPW + t) * 16 + mc;
-        const int pc = p < max_positions ? p : max_positions - 1;
 #pragma unroll
-        for (int ks = 0; ks < 4; ks++) {
-            kraw[t][ks] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(
-                k_cache + pc * row_stride + static_cast<size_t>(kvh) * kHeadDim + 32 * ks + 8 * mb));
+        for (int j = 0; j < 4; j++) {
+            const int p = p0 + (wave * TPW + t) * 16 + 4 * j + mb;
+            const int pc = p < max_positions ? p : max_positions - 1;
+            kraw[t][j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(
+                k_cache + pc * row_stride + static_cast<size_t>(kvh) * kHeadDim + 8 * mc));
         }
     }
 #pragma unroll
@@ -245,12 +253,22 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_stage1(
     const bool q_live = mc < G;
 #pragma unroll
     for (int t = 0; t < TPW; t++) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) *reinterpret_cast<u32x4*>(&s_k[(wave * TPW + t) * 16 + 4 * j + mb][4 * mc]) = kraw[t][j];
+    }
+    // a wave reads only rows that it wrote itself, and its LDS instructions run in order
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+    for (int t = 0; t < TPW; t++) {
         f32x4v d = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int ks = 0; ks < 4; ks++) {
             const bf16x8 a_op = as_bf16x8(q_live ? qraw[ks].x : 0u, q_live ? qraw[ks].y : 0u,
                                           q_live ? qraw[ks].z : 0u, q_live ? qraw[ks].w : 0u);
-            const bf16x8 b_op = as_bf16x8(kraw[t][ks].x, kraw[t][ks].y, kraw[t][ks].z, kraw[t][ks].w);
+            const u32x4 k_row = *reinterpret_cast<const u32x4*>(&s_k[(wave * TPW + t) * 16 + mc][16 * ks + 4 * mb]);
+            const bf16x8 b_op = as_bf16x8(k_row.x, k_row.y, k_row.z, k_row.w);
             d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_op, b_op, d, 0, 0, 0);
         }
         // the lane holds heads 4 mb .. 4 mb + 3 of position mc of the tile
