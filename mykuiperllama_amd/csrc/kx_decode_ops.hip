@@ -139,7 +139,16 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(const uint16_t* __res
 // ------------------------------------------------------------------------------------------------
 constexpr int kAttnThreads = 256;
 constexpr int kMaxGroup = 16;  // query heads per KV head: the rows of one MFMA tile
-template <int CHUNK>
+// ASKS: the position is asked for before anything else, a chunk behind it is left alone and of the last one no row past it is
+// read; otherwise the loads do not wait for it, and a cache with room to spare is read to its end.  The trip for the position
+// takes 0.1 us where a launch's workgroups all start together, and is hidden where they do not or where there are several
+// sequences, which seldom end in the same chunk.  us per launch, not asking -> asking, merge included: 16 sequences at 4096 of
+// 4224 positions (4224 workgroups) 52.9 -> 51.5, three at 2050 of 2304 11.8 -> 11.5, eight at 500 of 1000 12.4 -> 11.5, one at
+// 40001 of 40960 (2560 workgroups) 35.7 -> 35.5; one at 15000 of 15500 (976) 16.9 -> 17.1, at 4096 of 4224 (528, first stage
+// alone) 6.38 -> 6.50, at 700 of 1024 (128) 4.03 -> 3.97.
+constexpr int kAsksFrom = 2048;  // workgroups of one sequence: eight for each compute unit
+
+template <int CHUNK, bool ASKS>
 __global__ __launch_bounds__(kAttnThreads) void attn_decode_stage1(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k_cache, const uint16_t* __restrict__ v_cache,
     float* __restrict__ part_out, float* __restrict__ part_ml, int n_kv, int G, const int32_t* __restrict__ pos_ptr,
@@ -173,10 +182,24 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_stage1(
         part_out += seq * nchunks * heads * kHeadDim;
         part_ml += seq * nchunks * heads * 2;
     }
+    const bool one_sequence = gridDim.z == 1;  // write-through results for the one-row step only (store_result)
+    float* out_base = part_out + (static_cast<size_t>(kvh) * nchunks + chunk) * G * kHeadDim;
+    float* ml_base = part_ml + (static_cast<size_t>(kvh) * nchunks + chunk) * G * 2;
+    int end = max_positions;  // the rows that are read
+    if constexpr (ASKS) {
+        end = min(pos_ptr[0] + 1, max_positions);
+        if (p0 >= end) {  // the merge does not look at the vectors of a chunk whose sum is zero
+            for (int i = tid; i < G; i += kAttnThreads) {
+                ml_base[2 * i] = -INFINITY;
+                ml_base[2 * i + 1] = 0.0f;
+            }
+            return;
+        }
+    }
     const int sub = tid % 16;    // which eight dims of the row
     const int slot = tid / 16;   // position slot inside the workgroup: 16 slots
 
-    // Every K and V row of this lane is requested before anything is consumed, and the addresses do
+    // Every K and V row of this lane is requested before anything is consumed, and (ASKS aside) the addresses do
     // not depend on *pos: any row below max_positions exists, rows past the context are masked once
     // the position has arrived.  The chunk then costs one memory round trip.
     const size_t row_stride = static_cast<size_t>(n_kv) * kHeadDim;  // elements between positions
@@ -210,7 +233,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_stage1(
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             const int p = p0 + (wave * TPW + t) * 16 + 4 * j + mb;
-            const int pc = p < max_positions ? p : max_positions - 1;
+            const int pc = p < end ? p : end - 1;
             kraw[t][j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(
                 k_cache + pc * row_stride + static_cast<size_t>(kvh) * kHeadDim + 8 * mc));
         }
@@ -218,17 +241,14 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_stage1(
 #pragma unroll
     for (int it = 0; it < ITERS; it++) {
         const int p = p0 + it * 16 + slot;
-        const int pc = p < max_positions ? p : max_positions - 1;
+        const int pc = p < end ? p : end - 1;
         vraw[it] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(
             v_cache + pc * row_stride + static_cast<size_t>(kvh) * kHeadDim + 8 * sub));
     }
     const int ctx = pos_ptr[0] + 1;  // positions 0 .. pos are valid (pos was appended just before)
     __builtin_amdgcn_sched_barrier(0);
 
-    const bool one_sequence = gridDim.z == 1;  // write-through results for the one-row step only (store_result)
-    float* out_base = part_out + (static_cast<size_t>(kvh) * nchunks + chunk) * G * kHeadDim;
-    float* ml_base = part_ml + (static_cast<size_t>(kvh) * nchunks + chunk) * G * 2;
-    // No early exit for a chunk past the end of the context: a branch on *pos ahead of the loads
+    // Without ASKS there is no early exit for a chunk past the end of the context: a branch on *pos ahead of the loads
     // lets the compiler sink every K and V load below it, and the chunk then costs the round trip
     // for *pos and the round trip for the rows one after the other.  Such a chunk runs through with
     // everything masked and reports max = -inf, sum = 0.
@@ -771,13 +791,15 @@ int attn_decode(const uint16_t* q, const uint16_t* k_cache, const uint16_t* v_ca
     const float scale = 1.0f / sqrtf(static_cast<float>(kx::kHeadDim));
     hipStream_t s = kx::as_stream(stream);
     dim3 grid1(nchunks, n_kv_heads, batch);
-    if (long_chunks) {
-        hipLaunchKernelGGL((kx::attn_decode_stage1<kx::kAttnChunkLong>), grid1, dim3(kx::kAttnThreads), 0, s, q, k_cache,
-                           v_cache, part_out, part_ml, n_kv_heads, G, pos, nchunks, max_positions, scale, cache_stride);
-    } else {
-        hipLaunchKernelGGL((kx::attn_decode_stage1<kx::kAttnChunkShort>), grid1, dim3(kx::kAttnThreads), 0, s, q, k_cache,
-                           v_cache, part_out, part_ml, n_kv_heads, G, pos, nchunks, max_positions, scale, cache_stride);
-    }
+    const bool asks = batch > 1 || nchunks * n_kv_heads > kx::kAsksFrom;
+#define KX_STAGE1(CHUNK, ASKS)                                                                                                     \
+    hipLaunchKernelGGL((kx::attn_decode_stage1<CHUNK, ASKS>), grid1, dim3(kx::kAttnThreads), 0, s, q, k_cache, v_cache, part_out, \
+                       part_ml, n_kv_heads, G, pos, nchunks, max_positions, scale, cache_stride)
+    if (long_chunks && asks) KX_STAGE1(kx::kAttnChunkLong, true);
+    else if (long_chunks) KX_STAGE1(kx::kAttnChunkLong, false);
+    else if (asks) KX_STAGE1(kx::kAttnChunkShort, true);
+    else KX_STAGE1(kx::kAttnChunkShort, false);
+#undef KX_STAGE1
     if (out) {
         // slots per chunk subset: at least what the first flight of the merge covers
         const bool long_merge = kx::merge_by_quarters(nchunks, n_q_heads * batch);

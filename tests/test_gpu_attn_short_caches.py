@@ -1,0 +1,62 @@
+"""Attention over caches that are not full: chunks behind the last position, at every form of the first stage (asking for the
+position first or not, chunks of 64 and 128) and of the merge (chunks covered by its first flight)."""
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def reference(torch, q, k, v, n_q, n_kv, last):
+    """Softmax attention of one sequence in float64: [n_q * 128]."""
+    k, v = (t[:last + 1].double().repeat_interleave(n_q // n_kv, dim=1) for t in (k, v))  # [positions, n_q, 128]
+    w = torch.softmax((k * q.double().view(1, n_q, 128)).sum(-1) / 128 ** 0.5, 0)
+    return (w.unsqueeze(-1) * v).sum(0).reshape(-1)
+
+
+# (query heads, KV heads, cache positions, last positions of the sequences); the merge's first flight covers 32, 48, 80 or 128 chunks
+CASES = [(4, 2, 64, [0, 63]), (4, 2, 200, [0, 62, 63, 64, 127, 128, 199]), (6, 2, 2048, [700, 2047]), (6, 2, 2049, [2048, 64]),
+         (6, 2, 3072, [3071, 1]), (6, 2, 3073, [3072, 1000]), (8, 1, 5120, [5119, 5]), (4, 4, 4097, [4096, 4095, 127, 128, 255]),
+         (16, 1, 130, [129, 127, 128, 0]),
+         (8, 8, 1000, [999]), (8, 8, 32768, [32767]), (8, 8, 32769, [32768]), (8, 8, 32769, [700]), (8, 8, 32769, [0])]
+
+
+@pytest.mark.parametrize("n_q,n_kv,positions,last", CASES)
+def test_chunks_behind_the_context(n_q, n_kv, positions, last):
+    torch = pytest.importorskip("torch")
+    from mykuiperllama_amd import capi
+    batch = len(last)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(positions + n_q)
+    rand = lambda *shape: torch.randn(shape, device="cuda", generator=g).bfloat16()
+    q, kc, vc = rand(batch, n_q * 128), rand(batch, positions, n_kv, 128), rand(batch, positions, n_kv, 128)
+    for b, p in enumerate(last):  # what lies behind the context may be anything
+        kc[b, p + 1:] = float("nan")
+        vc[b, p + 1:] = float("inf")
+    pos = torch.tensor(last, dtype=torch.int32, device="cuda")
+    ws = capi.attn_decode_batch_workspace(batch, n_q, positions)
+    ws.fill_(255)  # NaN: nothing that was not written may be used
+    out = torch.full((batch, n_q * 128), float("nan"), dtype=torch.bfloat16, device="cuda")
+    capi.attn_decode_batch_bf16(q, kc, vc, out, n_q, n_kv, pos, positions, ws)
+    one = torch.full_like(out, float("nan"))
+    for b in range(batch):
+        capi.attn_decode_bf16(q[b], kc[b], vc[b], one[b], n_q, n_kv, pos[b:b + 1], positions, ws)
+    torch.cuda.synchronize()
+    for b, p in enumerate(last):
+        ref = reference(torch, q[b], kc[b], vc[b], n_q, n_kv, p)
+        for got in (out[b], one[b]):
+            assert (got.double() - ref).norm() <= 2.0 ** -8 * ref.norm(), f"sequence {b}"  # one rounding to bf16: at most 2^-9
+    if batch < 4:  # the same chunks for one sequence as for several
+        assert torch.equal(out.view(torch.int16), one.view(torch.int16))
+
+
+def test_no_position_to_attend_to():
+    torch = pytest.importorskip("torch")
+    from mykuiperllama_amd import capi
+    n_q, n_kv, positions = 8, 2, 300
+    kc, vc = (torch.full((2, positions, n_kv, 128), float("nan"), dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    q = torch.ones((2, n_q * 128), dtype=torch.bfloat16, device="cuda")
+    out = torch.full_like(q, float("nan"))
+    ws = capi.attn_decode_batch_workspace(2, n_q, positions)
+    ws.fill_(255)
+    capi.attn_decode_batch_bf16(q, kc, vc, out, n_q, n_kv, torch.tensor([-1, -1], dtype=torch.int32, device="cuda"), positions, ws)
+    torch.cuda.synchronize()
+    assert not out.any()
