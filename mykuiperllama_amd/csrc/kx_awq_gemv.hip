@@ -810,7 +810,9 @@ extern "C" int kx_gemv_awq_attn_merge_bf16(const void* attn_workspace, size_t at
     fi.heads_per_kv = n_q_heads / n_kv_heads;
     hipStream_t s = kx::as_stream(stream);
 #define KX_ARGS nullptr, qweight, scales, qzeros, y, partials, counters, 1, K, N, group_size, p.coltiles, p.ktiles, 1, s, fi
-    if (p.waves == 8) kx::launch_awq_gemv<8, 16, 1, kx::kProAttnMerge>(KX_ARGS);
+    const bool few = nchunks <= kx::kMergeParts * kx::kMergeHoldShort;
+    if (p.waves == 8 && few) kx::launch_awq_gemv<8, 16, 1, kx::kProAttnMergeShort>(KX_ARGS);
+    else if (p.waves == 8) kx::launch_awq_gemv<8, 16, 1, kx::kProAttnMerge>(KX_ARGS);
     else kx::launch_awq_gemv<4, 16, 1, kx::kProAttnMerge>(KX_ARGS);  // K = 128: one head
 #undef KX_ARGS
     return kx::launch_status();
@@ -824,7 +826,8 @@ void launch_chain(const AwqPlan& p, const FusedInput& fi, const RopeTarget& rope
                   const uint16_t* x, const int32_t* qweight, const uint16_t* scales, const int32_t* qzeros,
                   uint16_t* y, float* partials, uint32_t* counters, int K, int N, int group, hipStream_t stream) {
 #define KX_ARGS x, qweight, scales, qzeros, y, partials, counters, 1, K, N, group, p.coltiles, p.ktiles, 1, stream, fi, rope, res
-    if constexpr (PRO != kProAttnMerge) {
+    constexpr bool MERGE = PRO == kProAttnMerge || PRO == kProAttnMergeShort;
+    if constexpr (!MERGE) {
         if (p.rt == 32) {
             launch_awq_gemv<8, 32, 1, PRO, EPI>(KX_ARGS);
             return;
@@ -838,7 +841,7 @@ void launch_chain(const AwqPlan& p, const FusedInput& fi, const RopeTarget& rope
     }
     if (p.waves == 8) launch_awq_gemv<8, 16, 1, PRO, EPI>(KX_ARGS);
     else if (p.rt == 16) launch_awq_gemv<4, 16, 1, PRO, EPI>(KX_ARGS);
-    else if constexpr (PRO != kProAttnMerge) launch_awq_gemv<4, 8, 1, PRO, EPI>(KX_ARGS);
+    else if constexpr (!MERGE) launch_awq_gemv<4, 8, 1, PRO, EPI>(KX_ARGS);
 #undef KX_ARGS
 }
 
@@ -1022,7 +1025,10 @@ extern "C" int kx_gemv_awq_chain_bf16(const kx_chain_desc* d, const int32_t* qwe
     switch (d->in_kind) {
         case KX_IN_ROW: KX_BY_OUT(kx::kProNone); break;
         case KX_IN_SWIGLU: KX_BY_OUT(kx::kProSwiGLU); break;
-        case KX_IN_ATTN: KX_BY_OUT(kx::kProAttnMerge); break;
+        case KX_IN_ATTN:
+            if (fi.nchunks <= kx::kMergeParts * kx::kMergeHoldShort) KX_BY_OUT(kx::kProAttnMergeShort);
+            else KX_BY_OUT(kx::kProAttnMerge);
+            break;
         default: KX_BY_OUT(kx::kProPreNorm); break;
     }
 #undef KX_BY_OUT

@@ -99,7 +99,10 @@ __global__ __launch_bounds__(WAVES * kWave) void awq_gemv_kernel(
     constexpr bool STAGED = PRO != kProNone;
     constexpr bool NORM = PRO == kProAddNorm || PRO == kProAddNormLong;
     constexpr int NCH = PRO == kProAddNormLong ? kNormChunks : 1;
-    constexpr bool MERGE = PRO == kProAttnMerge;
+    constexpr bool MERGE = PRO == kProAttnMerge || PRO == kProAttnMergeShort;
+    constexpr int HOLD = PRO == kProAttnMergeShort ? kMergeHoldShort : kMergeHold;
+    constexpr int STATS = PRO == kProAttnMergeShort ? 1 : kMergeStatsPerLane;
+    static_assert(kMergeParts * HOLD <= STATS * kWave, "the wave that prepares the factors sees every chunk");
     constexpr bool PRENORM = PRO == kProPreNorm;
     static_assert(!PRENORM || MB == 1, "the pre-reduced norm serves one activation row");
     constexpr int HB = KB / kHeadDim > 0 ? KB / kHeadDim : 1;     // heads in the workgroup's K range
@@ -112,7 +115,7 @@ __global__ __launch_bounds__(WAVES * kWave) void awq_gemv_kernel(
     __shared__ __attribute__((aligned(16))) float red[WAVES * kSlotsPerWave][kTileCols];
     __shared__ __attribute__((aligned(16))) uint16_t s_x[STAGED ? MB : 1][STAGED ? KB : 8];  // staged activations, bf16
     __shared__ float s_ss[NORM ? MB : 1][WAVES];
-    __shared__ __attribute__((aligned(16))) float s_factor[MERGE ? HB : 1][MERGE ? kMergeParts * kMergeHold : 4];
+    __shared__ __attribute__((aligned(16))) float s_factor[MERGE ? HB : 1][MERGE ? kMergeParts * HOLD : 4];
     __shared__ float s_norm[MERGE ? HB : 1];
     __shared__ float s_mpart[MERGE ? kMergeParts : 1][MERGE ? KB : 1];
 
@@ -180,8 +183,8 @@ __global__ __launch_bounds__(WAVES * kWave) void awq_gemv_kernel(
     const uint16_t* b_src = has_b ? fi.b : fi.a;  // without a delta the second operand is read and ignored
     uint16_t own_a[MB], own_b[MB], own_gain = 0;
     uint4 row_a[NORM ? MB : 1][NCH], row_b[NORM ? MB : 1][NCH];
-    float held[MERGE ? EPT : 1][MERGE ? kMergeHold : 1];
-    MergeStats<kMergeStatsPerLane> stats;
+    float held[MERGE ? EPT : 1][MERGE ? HOLD : 1];
+    MergeStats<STATS> stats;
     if constexpr (MERGE) {
         // element e of the workgroup = (part, row): row of the K range, chunks part, part + 4, ...
         const int G = fi.heads_per_kv;
@@ -196,7 +199,7 @@ __global__ __launch_bounds__(WAVES * kWave) void awq_gemv_kernel(
             const float* po = fi.part_out + (static_cast<size_t>(hq / G) * fi.nchunks * G + hq % G) * kHeadDim +
                               row_c % kHeadDim;
 #pragma unroll
-            for (int j = 0; j < kMergeHold; j++) {
+            for (int j = 0; j < HOLD; j++) {
                 const int c = part + j * kMergeParts;
                 held[i][j] = po[(c < fi.nchunks ? c : fi.nchunks - 1) * cstride];
             }
@@ -206,7 +209,7 @@ __global__ __launch_bounds__(WAVES * kWave) void awq_gemv_kernel(
         if (wave_id < HB) {
             const int hq0 = kt * HB + wave_id;
             const int hq = hq0 * kHeadDim < K ? hq0 : K / kHeadDim - 1;
-            stats = attn_merge_load<kMergeStatsPerLane>(fi.part_ml + static_cast<size_t>(hq / G) * fi.nchunks * G * 2,
+            stats = attn_merge_load<STATS>(fi.part_ml + static_cast<size_t>(hq / G) * fi.nchunks * G * 2,
                                                         hq % G, G, fi.nchunks, tid % kWave);
         }
     }
@@ -359,7 +362,7 @@ __global__ __launch_bounds__(WAVES * kWave) void awq_gemv_kernel(
     if constexpr (MERGE) {
         const int wave_id = tid / kWave;
         if (wave_id < HB) {
-            const float l = attn_merge_finish<kMergeStatsPerLane>(stats, s_factor[wave_id], kMergeHold, tid % kWave);
+            const float l = attn_merge_finish<STATS>(stats, s_factor[wave_id], HOLD, tid % kWave);
             if (tid % kWave == 0) s_norm[wave_id] = l;
         }
         lds_barrier();
@@ -368,14 +371,14 @@ __global__ __launch_bounds__(WAVES * kWave) void awq_gemv_kernel(
             const int e = tid + i * THREADS;
             const int part = e / KB;
             const int row = e % KB;
-            // The thread's kMergeHold factors lie side by side and chunks that do not exist carry factor 0, so
+            // The thread's HOLD factors lie side by side and chunks that do not exist carry factor 0, so
             // the sum is straight-line code: a test on the chunk count per step had been compiled to a branch
             // and an LDS read with a full wait per chunk, forty dependent LDS round trips per thread.
-            static_assert(kMergeHold % 4 == 0, "the factors are read four at a time");
-            const f32x4* f4 = reinterpret_cast<const f32x4*>(&s_factor[row / kHeadDim][part * kMergeHold]);
-            float f[kMergeHold];
+            static_assert(HOLD % 4 == 0, "the factors are read four at a time");
+            const f32x4* f4 = reinterpret_cast<const f32x4*>(&s_factor[row / kHeadDim][part * HOLD]);
+            float f[HOLD];
 #pragma unroll
-            for (int j4 = 0; j4 < kMergeHold / 4; j4++) {
+            for (int j4 = 0; j4 < HOLD / 4; j4++) {
                 const f32x4 v = f4[j4];
                 f[4 * j4] = v.x;
                 f[4 * j4 + 1] = v.y;
@@ -384,7 +387,7 @@ __global__ __launch_bounds__(WAVES * kWave) void awq_gemv_kernel(
             }
             float acc_m = 0.0f;
 #pragma unroll
-            for (int j = 0; j < kMergeHold; j++) acc_m = attn_merge_step(acc_m, held[i][j], f[j]);
+            for (int j = 0; j < HOLD; j++) acc_m = attn_merge_step(acc_m, held[i][j], f[j]);
             s_mpart[part][row] = acc_m;
         }
         lds_barrier();

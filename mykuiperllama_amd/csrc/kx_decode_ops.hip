@@ -444,6 +444,14 @@ constexpr int kMergeDimsLong = 32;
 // flight, or a quarter of one (128-byte pieces of the partial sums) with 320: merge_by_quarters.
 // us per launch at 32 heads and 313 chunks, a whole head and 128 chunks ahead -> a quarter and 320: 10.6 -> 4.8.
 // Per dimension the additions run in the same order whatever DIMS and FRONT are.
+// Whole heads of a shorter cache take the first flight that covers it (merge_front): the loads go out whatever the number of
+// chunks, and so do those of the statistics (LANES chunks per lane).  us per launch with the first stage, 32 chunks per thread and
+// eight per lane -> what is needed: 16 sequences of 32 heads, 33 chunks 51.5 -> 49.8; three, 36 chunks 11.5 -> 10.6; eight, 16
+// chunks 11.5 -> 10.5; two of 40 heads, ten chunks 7.4 -> 6.35.
+inline int merge_front(int nchunks) {
+    const int per_part = (nchunks + kMergeParts - 1) / kMergeParts;
+    return per_part <= 8 ? 8 : (per_part <= 12 ? 12 : (per_part <= 20 ? 20 : kMergeFront));
+}
 // Whether the merge takes a head in quarters.  A quarter's 80 loads per thread go out whatever the number of chunks, so it
 // takes a good deal more than the 128 chunks that a whole head covers in one flight, and the more so the more workgroups
 // share a compute unit; with more than four each it gains nothing at any length.  Attention in all, whole heads ->
@@ -456,11 +464,12 @@ inline bool merge_by_quarters(int nchunks, int heads) {
     return per_cu <= 4 && nchunks > kMergeParts * kMergeFront + 32 * per_cu;
 }
 
-template <int DIMS, int FRONT>
+template <int DIMS, int FRONT, int LANES>  // LANES: chunks per lane of the wave that prepares the factors
 __global__ __launch_bounds__(DIMS * kMergeParts) void attn_decode_stage2(const float* __restrict__ part_out,
                                                                          const float* __restrict__ part_ml,
                                                                          uint16_t* __restrict__ out, int G, int nchunks,
                                                                          int per_part) {
+    static_assert(kMergeParts * FRONT <= LANES * kWave || LANES == kMergeLanesLong, "the statistics cover the first flight");
     // rescaling factors exp(m_c - m), per_part slots for each of the four chunk subsets (attn_factor_slot);
     // slots of chunks that do not exist hold 0
     extern __shared__ __attribute__((aligned(16))) float s_factor[];
@@ -495,9 +504,9 @@ __global__ __launch_bounds__(DIMS * kMergeParts) void attn_decode_stage2(const f
     }
     __builtin_amdgcn_sched_barrier(0);
     if (tid < kWave) {
-        const MergeStats<kMergeLanesLong> st =
-            attn_merge_load<kMergeLanesLong>(part_ml + static_cast<size_t>(kvh) * nchunks * G * 2, g, G, nchunks, tid);
-        const float l = attn_merge_finish<kMergeLanesLong>(st, s_factor, per_part, tid);
+        const MergeStats<LANES> st =
+            attn_merge_load<LANES>(part_ml + static_cast<size_t>(kvh) * nchunks * G * 2, g, G, nchunks, tid);
+        const float l = attn_merge_finish<LANES>(st, s_factor, per_part, tid);
         if (tid == 0) s_norm = l;
     }
     __syncthreads();
@@ -804,18 +813,19 @@ int attn_decode(const uint16_t* q, const uint16_t* k_cache, const uint16_t* v_ca
         // slots per chunk subset: at least what the first flight of the merge covers
         const bool long_merge = kx::merge_by_quarters(nchunks, n_q_heads * batch);
         int per_part = (nchunks + kx::kMergeParts - 1) / kx::kMergeParts;
-        const int front = long_merge ? kx::kMergeFrontLong : kx::kMergeFront;
+        const int front = long_merge ? kx::kMergeFrontLong : kx::merge_front(nchunks);
         if (per_part < front) per_part = front;
         per_part = (per_part + 3) / 4 * 4;
         const size_t lds = kx::kMergeParts * per_part * sizeof(float);
-        if (long_merge) {
-            hipLaunchKernelGGL((kx::attn_decode_stage2<kx::kMergeDimsLong, kx::kMergeFrontLong>),
-                               dim3(n_q_heads, kx::kHeadDim / kx::kMergeDimsLong, batch), dim3(kx::kMergeDimsLong * kx::kMergeParts),
-                               lds, s, part_out, part_ml, out, G, nchunks, per_part);
-        } else {
-            hipLaunchKernelGGL((kx::attn_decode_stage2<kx::kHeadDim, kx::kMergeFront>), dim3(n_q_heads, 1, batch),
-                               dim3(kx::kHeadDim * kx::kMergeParts), lds, s, part_out, part_ml, out, G, nchunks, per_part);
-        }
+        const dim3 whole(n_q_heads, 1, batch);
+#define KX_MERGE(DIMS, FRONT, LANES, GRID) \
+    hipLaunchKernelGGL((kx::attn_decode_stage2<DIMS, FRONT, LANES>), GRID, dim3(DIMS * kx::kMergeParts), lds, s, part_out, part_ml, out, G, nchunks, per_part)
+        if (long_merge) KX_MERGE(kx::kMergeDimsLong, kx::kMergeFrontLong, kx::kMergeLanesLong, dim3(n_q_heads, kx::kHeadDim / kx::kMergeDimsLong, batch));
+        else if (front == 8) KX_MERGE(kx::kHeadDim, 8, 1, whole);
+        else if (front == 12) KX_MERGE(kx::kHeadDim, 12, 1, whole);
+        else if (front == 20) KX_MERGE(kx::kHeadDim, 20, 2, whole);
+        else KX_MERGE(kx::kHeadDim, kx::kMergeFront, kx::kMergeLanesLong, whole);
+#undef KX_MERGE
     }
     return kx::launch_status();
 }

@@ -60,3 +60,38 @@ def test_no_position_to_attend_to():
     capi.attn_decode_batch_bf16(q, kc, vc, out, n_q, n_kv, torch.tensor([-1, -1], dtype=torch.int32, device="cuda"), positions, ws)
     torch.cuda.synchronize()
     assert not out.any()
+
+
+@pytest.mark.parametrize("positions,last", [(64, 63), (300, 5), (2048, 2047), (2049, 2048), (2049, 63), (5120, 5119)])
+def test_merge_on_the_way_into_a_projection(positions, last):
+    """With up to 32 chunks, or more, the projection returns the bits of the merge followed by the projection."""
+    torch = pytest.importorskip("torch")
+    from mykuiperllama_amd import capi
+    n_q, n_kv, N, group = 4, 2, 512, 128
+    K = n_q * 128
+    g = torch.Generator(device="cuda")
+    g.manual_seed(positions)
+    rand = lambda *shape: torch.randn(shape, device="cuda", generator=g).bfloat16()
+    q, kc, vc = rand(1, K), rand(positions, n_kv, 128), rand(positions, n_kv, 128)
+    qw = torch.randint(-2**31, 2**31, (K, N // 8), dtype=torch.int32, device="cuda", generator=g)
+    qz = torch.randint(-2**31, 2**31, (K // group, N // 8), dtype=torch.int32, device="cuda", generator=g)
+    sc = torch.rand((K // group, N), device="cuda", generator=g).half()
+    pos = torch.tensor([last], dtype=torch.int32, device="cuda")
+    ws, attn_ws = capi.make_workspace(1, K, N), capi.attn_decode_workspace(n_q, positions)
+    attn, residual = torch.empty((1, K), dtype=torch.bfloat16, device="cuda"), rand(1, N)
+    capi.attn_decode_bf16(q, kc, vc, attn, n_q, n_kv, pos, positions, attn_ws)
+    outs = []
+    for inputs in ({"in_kind": capi.IN_ROW, "x": attn},
+                   {"in_kind": capi.IN_ATTN, "attn_workspace": attn_ws, "attn_workspace_bytes": attn_ws.numel(),
+                    "n_q_heads": n_q, "n_kv_heads": n_kv, "max_positions": positions}):
+        if "x" not in inputs:
+            attn_ws.fill_(255)
+            capi.attn_decode_partial_bf16(q, kc, vc, n_q, n_kv, pos, positions, attn_ws)
+        out = torch.full_like(residual, float("nan"))
+        sums = torch.empty((N // 256, 4), dtype=torch.float32, device="cuda")
+        capi.gemv_awq_chain_bf16({**inputs, "out_kind": capi.OUT_RESIDUAL, "residual_in": residual, "residual_out": out,
+                                  "sumsq_out": sums}, qw, sc, qz, K, N, group, ws)
+        outs.append((out, sums))
+    torch.cuda.synchronize()
+    assert torch.isfinite(outs[0][0]).all()
+    assert all(torch.equal(a.view(torch.int16), b.view(torch.int16)) for a, b in zip(*outs))
