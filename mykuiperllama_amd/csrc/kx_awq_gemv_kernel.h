@@ -106,9 +106,8 @@ __global__ __launch_bounds__(WAVES * kWave) void awq_gemv_kernel(
     constexpr bool PRENORM = PRO == kProPreNorm;
     static_assert(!PRENORM || MB == 1, "the pre-reduced norm serves one activation row");
     constexpr int HB = KB / kHeadDim > 0 ? KB / kHeadDim : 1;     // heads in the workgroup's K range
-    constexpr int EPT = kMergeParts * KB / THREADS;               // (part, row) elements a thread merges
-    static_assert(!MERGE || (MB == 1 && KB % kHeadDim == 0 && EPT * THREADS == kMergeParts * KB && HB <= WAVES),
-                  "the attention merge serves one activation row and whole heads");
+    static_assert(!MERGE || (MB == 1 && KB % kHeadDim == 0 && 2 * THREADS == kMergeParts * KB && HB <= WAVES),
+                  "the attention merge serves one activation row and whole heads, two neighbouring rows of a part per thread");
     static_assert(RT % 8 == 0, "a lane reads its activations in 16-byte pieces");
     static_assert(KB <= THREADS, "one staging thread per row of the workgroup's K range");
 
@@ -117,7 +116,7 @@ __global__ __launch_bounds__(WAVES * kWave) void awq_gemv_kernel(
     __shared__ float s_ss[NORM ? MB : 1][WAVES];
     __shared__ __attribute__((aligned(16))) float s_factor[MERGE ? HB : 1][MERGE ? kMergeParts * HOLD : 4];
     __shared__ float s_norm[MERGE ? HB : 1];
-    __shared__ float s_mpart[MERGE ? kMergeParts : 1][MERGE ? KB : 1];
+    __shared__ __attribute__((aligned(8))) float s_mpart[MERGE ? kMergeParts : 1][MERGE ? KB : 1];
 
     // The pointers of the epilogue are fetched with the other kernel arguments: left to itself the compiler loads
     // them where they are first used, a scalar-memory round trip behind the reduction.
@@ -183,26 +182,23 @@ __global__ __launch_bounds__(WAVES * kWave) void awq_gemv_kernel(
     const uint16_t* b_src = has_b ? fi.b : fi.a;  // without a delta the second operand is read and ignored
     uint16_t own_a[MB], own_b[MB], own_gain = 0;
     uint4 row_a[NORM ? MB : 1][NCH], row_b[NORM ? MB : 1][NCH];
-    float held[MERGE ? EPT : 1][MERGE ? HOLD : 1];
+    f32x2 held[MERGE ? HOLD : 1];
     MergeStats<STATS> stats;
+    const int pair_part = tid / (KB / 2), pair_row = 2 * (tid % (KB / 2));
     if constexpr (MERGE) {
-        // element e of the workgroup = (part, row): row of the K range, chunks part, part + 4, ...
+        // the thread's part and two rows of the K range, chunks part, part + 4, ...
+        // (eight-byte loads: the loads of the merge stand in front of the weights'.  us per launch into the residual stream,
+        // one row per load -> two: 4096 -> 4096 of 66 chunks 7.55 -> 7.39, 8192 -> 5120 of 65 14.0 -> 13.7, of 32 11.0 -> 10.75)
         const int G = fi.heads_per_kv;
         const size_t cstride = static_cast<size_t>(G) * kHeadDim;
+        const int rrow = kt * KB + pair_row;
+        const int row_c = rrow < K ? rrow : K - 2;
+        const int hq = row_c / kHeadDim;
+        const float* po = fi.part_out + (static_cast<size_t>(hq / G) * fi.nchunks * G + hq % G) * kHeadDim + row_c % kHeadDim;
 #pragma unroll
-        for (int i = 0; i < EPT; i++) {
-            const int e = tid + i * THREADS;
-            const int part = e / KB;
-            const int rrow = kt * KB + e % KB;
-            const int row_c = rrow < K ? rrow : K - 1;
-            const int hq = row_c / kHeadDim;
-            const float* po = fi.part_out + (static_cast<size_t>(hq / G) * fi.nchunks * G + hq % G) * kHeadDim +
-                              row_c % kHeadDim;
-#pragma unroll
-            for (int j = 0; j < HOLD; j++) {
-                const int c = part + j * kMergeParts;
-                held[i][j] = po[(c < fi.nchunks ? c : fi.nchunks - 1) * cstride];
-            }
+        for (int j = 0; j < HOLD; j++) {
+            const int c = pair_part + j * kMergeParts;
+            held[j] = *reinterpret_cast<const f32x2*>(po + (c < fi.nchunks ? c : fi.nchunks - 1) * cstride);
         }
         // wave w prepares the factors of head w of the K range
         const int wave_id = tid / kWave;
@@ -366,30 +362,22 @@ __global__ __launch_bounds__(WAVES * kWave) void awq_gemv_kernel(
             if (tid % kWave == 0) s_norm[wave_id] = l;
         }
         lds_barrier();
+        // The thread's HOLD factors lie side by side and chunks that do not exist carry factor 0, so
+        // the sum is straight-line code: a test on the chunk count per step had been compiled to a branch
+        // and an LDS read with a full wait per chunk, forty dependent LDS round trips per thread.
+        static_assert(HOLD % 4 == 0, "the factors are read four at a time");
+        const f32x4* f4 = reinterpret_cast<const f32x4*>(&s_factor[pair_row / kHeadDim][pair_part * HOLD]);
+        f32x2 merged = {0.0f, 0.0f};
 #pragma unroll
-        for (int i = 0; i < EPT; i++) {
-            const int e = tid + i * THREADS;
-            const int part = e / KB;
-            const int row = e % KB;
-            // The thread's HOLD factors lie side by side and chunks that do not exist carry factor 0, so
-            // the sum is straight-line code: a test on the chunk count per step had been compiled to a branch
-            // and an LDS read with a full wait per chunk, forty dependent LDS round trips per thread.
-            static_assert(HOLD % 4 == 0, "the factors are read four at a time");
-            const f32x4* f4 = reinterpret_cast<const f32x4*>(&s_factor[row / kHeadDim][part * HOLD]);
-            float f[HOLD];
+        for (int j4 = 0; j4 < HOLD / 4; j4++) {
+            const f32x4 f = f4[j4];
 #pragma unroll
-            for (int j4 = 0; j4 < HOLD / 4; j4++) {
-                const f32x4 v = f4[j4];
-                f[4 * j4] = v.x;
-                f[4 * j4 + 1] = v.y;
-                f[4 * j4 + 2] = v.z;
-                f[4 * j4 + 3] = v.w;
+            for (int j = 0; j < 4; j++) {
+                merged.x = attn_merge_step(merged.x, held[4 * j4 + j].x, f[j]);
+                merged.y = attn_merge_step(merged.y, held[4 * j4 + j].y, f[j]);
             }
-            float acc_m = 0.0f;
-#pragma unroll
-            for (int j = 0; j < HOLD; j++) acc_m = attn_merge_step(acc_m, held[i][j], f[j]);
-            s_mpart[part][row] = acc_m;
         }
+        *reinterpret_cast<f32x2*>(&s_mpart[pair_part][pair_row]) = merged;
         lds_barrier();
         if (tid < KB) {
             const float total = (s_mpart[0][tid] + s_mpart[1][tid]) + (s_mpart[2][tid] + s_mpart[3][tid]);
