@@ -15,6 +15,7 @@ struct AwqPlan {
     bool walks;    // MFMA kernel: a workgroup walks over such a run; otherwise the read-back adds in that order
     bool fine;     // MFMA kernel: the steps of a wave lie in groups of their own
     bool sliced;   // MFMA kernel: all workgroups of a column tile finish it together
+    bool trio;     // MFMA kernel, plain: the form of which three fit a compute unit
     int waves;     // waves per workgroup stacked along K (4, 8 or 16)
     int rt;        // VALU kernel: consecutive rows per lane (8 or 16); MFMA kernel: 32-row steps per wave
     int mb;        // activation rows per workgroup (1, 2, 4 or 8)
@@ -58,6 +59,14 @@ constexpr int kExchangeRows = 8;    // what a K tile's share of the split-K exch
 //            come in rounds, keep the single reader: with shares the early ones would hold the places the late ones need
 //            (gate|up 4096 -> 24576 at M = 16: 19.7 against 21.5 us), and so do their column-tile-fastest order and 256 /
 //            512 rows per workgroup.
+//            Up to three per compute unit where that many of the form fit (kThreePerUnit, four steps, at most sixteen K
+//            tiles).  Behind a norm always: the figures stand there.  A plain launch, M = 6 / 9 / 16, single reader and two per
+//            compute unit -> shares and three: 5120 -> 15360 (600 workgroups, ten K tiles) 17.7 / 19.1 / 20.2 -> 15.1 / 16.1 /
+//            17.6, 8192 -> 10240 (640, sixteen) 17.0 / 20.3 / 21.2 -> 17.5 / 17.8 / 20.0, 4096 -> 24576 (768, eight) 17.7 / 18.3 /
+//            19.3 -> 16.3 / 18.0 / 19.6, 2048 -> 40960 (640, four) 16.7 / 18.1 / 19.2 -> 16.1 / 17.6 / 19.9: nine and more rows
+//            from ten K tiles on, fewer up to fifteen.  At five to eight rows these grids take four steps per wave in
+//            every form, so that all of them add alike: behind SwiGLU 4096 -> 24576 at M = 6 18.1 -> 17.5, into the
+//            residual stream 18.6 -> 17.6 (two steps -> four, single reader).
 //            Unless K is long as well, more than 16 blocks of 512 rows (32 up to eight rows): then the partial sums
 //            outweigh that, and a workgroup walks over as many blocks as bring the grid down to two per compute unit.  us
 //            per launch, single reader -> walk, M = 5 / 8 / 9 / 16: 14336 -> 5120 (28 blocks) 18.4 / 18.8 / 25.0 / 26.5
@@ -78,8 +87,9 @@ constexpr int kExchangeRows = 8;    // what a K tile's share of the split-K exch
 // group size alone, so that the launches of a shape return the same bits (one that does not walk leaves the runs to the
 // read-back, splitk_sum_runs: 14336 -> 5120 behind SwiGLU at M = 16 30.3 us with K tiles in order, 29.9 in runs).
 // `may_walk`: the kernel exists in a form that walks; `produced_x`: its activations are produced on the way in.
+enum LaunchEnds { kPlainEnds, kNormEnds, kOtherEnds };  // a row in and out; normed on the way in; anything else
 inline AwqPlan make_mfma_plan(int M, int K, int N, int group, bool may_walk = true, bool produced_x = false,
-                              bool may_cross_groups = true) {
+                              bool may_cross_groups = true, LaunchEnds ends = kPlainEnds) {
     AwqPlan p;
     p.mfma = true;
     p.fine = false;
@@ -113,7 +123,7 @@ inline AwqPlan make_mfma_plan(int M, int K, int N, int group, bool may_walk = tr
                          (inside_kt > 48 || 8 * p.coltiles * inside_kt > (inside_kt < 20 ? 16 : 11) * kComputeUnits);
     if (crosses) ks = 4;
     else while (!allowed(ks)) ks /= 2;
-    p.sliced = p.walks = false;
+    p.sliced = p.walks = p.trio = false;
     p.run = 1;
     if (M >= 5) {
         int best = 0;  // the longest run that is allowed, or a shorter one that is short enough
@@ -127,6 +137,10 @@ inline AwqPlan make_mfma_plan(int M, int K, int N, int group, bool may_walk = tr
         if (kt == 1 || (kt <= kSliceMaxKTiles && p.coltiles * kt <= 2 * kComputeUnits)) {
             p.sliced = kt > 1;
             ks = best;
+        } else if (best == 4 && allowed(4) && kt <= 16 && p.coltiles * kt <= 3 * kComputeUnits) {
+            ks = 4;
+            p.trio = ends == kPlainEnds && (M >= 9 ? kt >= 10 : kt < 16);
+            p.sliced = p.trio || ends == kNormEnds;
         } else if (allowed(4) && ktiles_with(4) > (M >= 9 ? 16 : 32)) {
             const int blocks = ktiles_with(4);
             int walk = 2;
@@ -148,7 +162,7 @@ inline AwqPlan make_mfma_plan(int M, int K, int N, int group, bool may_walk = tr
 
 inline AwqPlan make_valu_plan(int M, int K, int N, bool allow_long_rows = true, bool allow_12_waves = true) {
     AwqPlan p;
-    p.mfma = p.sliced = p.walks = p.fine = false;
+    p.mfma = p.sliced = p.trio = p.walks = p.fine = false;
     p.run = 1;
     p.coltiles = (N / 8 + kWC - 1) / kWC;
     p.mb = M >= 8 ? 8 : (M >= 4 ? 4 : (M >= 2 ? 2 : 1));
@@ -211,7 +225,7 @@ constexpr int kFixedExchangeRows = 4;
 
 inline AwqPlan make_fixed_plan(int K, int N) {
     AwqPlan p{};
-    p.mfma = p.sliced = p.walks = p.fine = false;
+    p.mfma = p.sliced = p.trio = p.walks = p.fine = false;
     p.run = 1;
     p.coltiles = (N / 8 + kWC - 1) / kWC;
     p.mb = 1;
@@ -354,6 +368,13 @@ void launch_mfma_fused(const AwqPlan& p, const FusedInput& fi, const ResidualTar
         else if (M <= 8) launch_awq_gemv_mfma<4, KS, 8, 1, PRO, EPI, LONE>(KX_MARGS); \
         else launch_awq_gemv_mfma<4, KS, 8, 2, PRO, EPI, LONE>(KX_MARGS);            \
     } while (0)
+    if constexpr (PRO == kProNone && EPI == kEpiStore) {
+        if (p.trio) {
+            if (M <= 8) launch_awq_gemv_mfma<4, 4, 8, 1, PRO, EPI, LONE, false, false, true>(KX_MARGS);
+            else launch_awq_gemv_mfma<4, 4, 8, 2, PRO, EPI, LONE, false, false, true>(KX_MARGS);
+            return;
+        }
+    }
     if constexpr (PRO != kProPreNorm && EPI != kEpiQkRope && !LONE) {
         if (p.walks) {
             if (M <= 8) launch_awq_gemv_mfma<4, 4, 8, 1, PRO, EPI, false, true>(KX_MARGS);
@@ -581,6 +602,17 @@ extern "C" int kx_gemv_awq_bf16_policy(const uint16_t* x, const int32_t* qweight
             return kx::launch_status();
         }
 #undef KX_MFMA_WALK
+#define KX_MFMA_TRIO(LONE)                                                                                                          \
+    do {                                                                                                                            \
+        if (M <= 8) kx::launch_awq_gemv_mfma<4, 4, 8, 1, kx::kProNone, kx::kEpiStore, LONE, false, false, true>(KX_MARGS);          \
+        else kx::launch_awq_gemv_mfma<4, 4, 8, 2, kx::kProNone, kx::kEpiStore, LONE, false, false, true>(KX_MARGS);                 \
+    } while (0)
+        if (p.trio) {
+            if (N % 16) KX_MFMA_TRIO(true);
+            else KX_MFMA_TRIO(false);
+            return kx::launch_status();
+        }
+#undef KX_MFMA_TRIO
 #define KX_MFMA_FINE(LONE)                                                                                          \
     do {                                                                                                             \
         if (M == 1) kx::launch_awq_gemv_mfma<4, 4, 1, 1, kx::kProNone, kx::kEpiStore, LONE, false, true>(KX_MARGS);  \
@@ -651,7 +683,7 @@ extern "C" int kx_gemv_awq_swiglu_bf16(const uint16_t* gate, const uint16_t* up,
     // Several rows go where kx_gemv_awq_bf16 takes them, when gate and up can be read 16 bytes at a time
     if (kx::rows_on_mfma(M, K, N, group_size) && kx::aligned_to(gate, 16) && kx::aligned_to(up, 16) && (act_ld % 8) == 0) {
         const bool lone = N % 16 != 0;
-        const kx::AwqPlan mp = kx::make_mfma_plan(M, K, N, group_size, !lone, true);
+        const kx::AwqPlan mp = kx::make_mfma_plan(M, K, N, group_size, !lone, true, true, kx::kOtherEnds);
         float* partials = nullptr;
         uint32_t* counters = nullptr;
         rc = kx::resolve_workspace(mp, M, N, workspace, workspace_bytes, &partials, &counters);
@@ -981,7 +1013,9 @@ extern "C" int kx_gemv_awq_chain_bf16(const kx_chain_desc* d, const int32_t* qwe
     if (rows > 1) {
         const kx::AwqPlan mp = kx::make_mfma_plan(rows, K, N, group_size,
                                                    d->in_kind != KX_IN_NORM && d->out_kind != KX_OUT_QKV_ROPE,
-                                                   d->in_kind != KX_IN_ROW);
+                                                   d->in_kind != KX_IN_ROW, true,
+                                                   d->out_kind != KX_OUT_ROW || d->in_kind == KX_IN_SWIGLU
+                                                       ? kx::kOtherEnds : (d->in_kind == KX_IN_NORM ? kx::kNormEnds : kx::kPlainEnds));
         float* partials = nullptr;
         uint32_t* counters = nullptr;
         rc = kx::resolve_workspace(mp, rows, N, workspace, workspace_bytes, &partials, &counters);

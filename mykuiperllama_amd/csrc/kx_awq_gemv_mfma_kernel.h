@@ -153,8 +153,20 @@ __device__ __forceinline__ int group_of_step(const MfmaGrid& g, int step) {
 // 17.1, 1024 -> 24576 11.4 / 11.8 -> 11.2 / 11.7.  Two steps take 167 by themselves; held to it, the plain launch spilled 19: spilled
 // -> left alone, groups of 64, 2048 -> 24576 14.7 / 15.9 -> 13.7 / 14.9, 2048 -> 16896 15.2 / 16.9 -> 13.4 / 15.1, 2048 -> 51200 24.3 /
 // 28.2 -> 23.0 / 26.6; grids of up to 512 workgroups alike.
-template <int WAVES, int KS, int MC, int ROUNDS, int PRO = kProNone, int EPI = kEpiStore, bool LONE = false, bool WALK = false, bool FINE = false>
-__global__ __launch_bounds__(WAVES * kWave, KS == 1 && ROUNDS == 2 && EPI == kEpiStore ? 3 : 2) void awq_gemv_mfma_kernel(
+//
+// Four steps per wave at five and more rows, stored: 185 registers leave two to a compute unit, so that a grid of 513 to 768
+// comes in two rounds and cannot finish its tiles together.  With four nibbles' operands at a time and a step's activations read
+// when it comes they fit 168 (what still goes to memory, 32 to 80 bytes a lane, belongs to the single reader's read-back).  Behind
+// a norm every such launch takes this form: us per launch, M = 6 / 9 / 16, two -> three and finishing together, 4096 -> 24576
+// 18.6 / 20.0 / 20.8 -> 16.1 / 18.0 / 18.7, 5120 -> 15360 18.4 / 20.9 / 21.6 -> 15.4 / 16.9 / 17.4, 8192 -> 10240 17.9 / 21.9 / 22.3
+// -> 17.2 / 18.1 / 20.2; two -> three alone, larger grids, M = 6 / 16, 4096 -> 32768 22.8 / 25.7 -> 22.8 / 24.3, 5120 -> 51200 43.8 /
+// 48.2 -> 43.8 / 46.2, and smaller ones, 4096 -> 12288 12.3 / 13.9 -> 12.2 / 13.9.  A plain launch takes it where make_mfma_plan
+// says so (TRIO): larger grids at sixteen rows lose by it, 4096 -> 32768 23.5 -> 26.1.
+template <int KS, int ROWS, int PRO, int EPI, bool WALK, bool FINE, bool TRIO>
+constexpr bool kThreePerUnit = KS == 4 && ROWS >= 8 && EPI == kEpiStore && !WALK && !FINE && (PRO == kProPreNorm || TRIO);
+template <int WAVES, int KS, int MC, int ROUNDS, int PRO = kProNone, int EPI = kEpiStore, bool LONE = false, bool WALK = false, bool FINE = false,
+          bool TRIO = false>
+__global__ __launch_bounds__(WAVES * kWave, ((KS == 1 && ROUNDS == 2 && EPI == kEpiStore) || kThreePerUnit<KS, MC * ROUNDS, PRO, EPI, WALK, FINE, TRIO> ? 3 : 2)) void awq_gemv_mfma_kernel(
     const uint16_t* __restrict__ x, const uint32_t* __restrict__ qweight,
     const uint16_t* __restrict__ scales, const uint32_t* __restrict__ qzeros,
     uint16_t* __restrict__ y, float* __restrict__ partials, uint32_t* __restrict__ counters,
@@ -170,6 +182,8 @@ __global__ __launch_bounds__(WAVES * kWave, KS == 1 && ROUNDS == 2 && EPI == kEp
     static_assert(PRO == kProNone || PRO == kProSwiGLU || PRO == kProPreNorm, "prologues of the matrix-core kernel");
     static_assert(EPI == kEpiStore || EPI == kEpiResidual || EPI == kEpiQkRope, "epilogues of the matrix-core kernel");
     constexpr bool STAGED = PRO != kProNone;
+    constexpr bool THREE = kThreePerUnit<KS, ROWS, PRO, EPI, WALK, FINE, TRIO>;
+    static_assert(!TRIO || (THREE && PRO == kProNone), "plain launches, three to a compute unit");
     // The loads of the next block go out while the waves of this one meet, except at sixteen rows behind a prologue, whose
     // operands do not fit the registers beside the weights and the sums: there the other workgroup of the compute unit
     // has to cover the gap.
@@ -427,7 +441,7 @@ __global__ __launch_bounds__(WAVES * kWave, KS == 1 && ROUNDS == 2 && EPI == kEp
             lds_barrier();
             const int s_row = c < ROWS ? c : ROWS - 1;
 #pragma unroll
-            for (int ks = 0; ks < KS; ks++) {
+            for (int ks = 0; ks < (THREE ? 0 : KS); ks++) {
                 const uint4 got = *reinterpret_cast<const uint4*>(&s_x[s_row][(wave * KS + ks) * kStepRows + 8 * b]);
                 const bool live = c < M;  // rows M .. ROWS-1 and elements past K were staged as zeros
                 xa[ks] = make_uint4(live ? got.x : 0u, live ? got.y : 0u, live ? got.z : 0u, live ? got.w : 0u);
@@ -456,27 +470,51 @@ __global__ __launch_bounds__(WAVES * kWave, KS == 1 && ROUNDS == 2 && EPI == kEp
                 const uint32_t keep = c < M && kblock + wave * WROWS + ks * kStepRows < K ? 0xffffffffu : 0u;
                 xa[ks] = make_uint4(xa[ks].x & keep, xa[ks].y & keep, xa[ks].z & keep, xa[ks].w & keep);
             }
+            if constexpr (STAGED && THREE) {  // the others read all steps' operands at once
+                const uint4 got = *reinterpret_cast<const uint4*>(&s_x[c < ROWS ? c : ROWS - 1][(wave * KS + ks) * kStepRows + 8 * b]);
+                const bool live = c < M;
+                xa[ks] = make_uint4(live ? got.x : 0u, live ? got.y : 0u, live ? got.z : 0u, live ? got.w : 0u);
+            }
             const bf16x8 a_op = as_bf16x8(xa[ks].x, xa[ks].y, xa[ks].z, xa[ks].w);
             xs = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_op, ones, ks == 0 || FINE ? zero4 : xs, 0, 0, 0);
 #pragma unroll
             for (int h = h0; h < h1; h++) {
-                uint32_t bop[8][4];  // [nibble p][row pair]
+                if constexpr (THREE) {  // four nibbles at a time: half the operands in registers
 #pragma unroll
-                for (int rp = 0; rp < 4; rp++) {
-                    const uint32_t wa = w[ks][2 * rp][h];      // row 2rp   -> low half
-                    const uint32_t wb = w[ks][2 * rp + 1][h];  // row 2rp+1 -> high half
-                    const uint32_t lo = __builtin_amdgcn_perm(wb, wa, 0x05040100u);  // nibbles 0..3, both rows
-                    const uint32_t hi = __builtin_amdgcn_perm(wb, wa, 0x07060302u);  // nibbles 4..7
+                    for (int q = 0; q < 8; q += 4) {
+                        uint32_t bop[4][4];  // [nibble][row pair]
 #pragma unroll
-                    for (int p = 0; p < 4; p++) {
-                        bop[p][rp] = code_pair_to_bf16(p == 0 ? lo : lo >> (4 * p), magic);
-                        bop[4 + p][rp] = code_pair_to_bf16(p == 0 ? hi : hi >> (4 * p), magic);
+                        for (int rp = 0; rp < 4; rp++) {
+                            const uint32_t v = __builtin_amdgcn_perm(w[ks][2 * rp + 1][h], w[ks][2 * rp][h], q ? 0x07060302u : 0x05040100u);
+#pragma unroll
+                            for (int p = 0; p < 4; p++) bop[p][rp] = code_pair_to_bf16(p == 0 ? v : v >> (4 * p), magic);
+                        }
+#pragma unroll
+                        for (int p = 0; p < 4; p++) {
+                            acc[h][q + p] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                                a_op, as_bf16x8(bop[p][0], bop[p][1], bop[p][2], bop[p][3]), ks == 0 ? zero4 : acc[h][q + p], 0, 0, 0);
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
                     }
-                }
+                } else {
+                    uint32_t bop[8][4];  // [nibble p][row pair]
 #pragma unroll
-                for (int p = 0; p < 8; p++) {
-                    acc[h][p] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                        a_op, as_bf16x8(bop[p][0], bop[p][1], bop[p][2], bop[p][3]), ks == 0 || FINE ? zero4 : acc[h][p], 0, 0, 0);
+                    for (int rp = 0; rp < 4; rp++) {
+                        const uint32_t wa = w[ks][2 * rp][h];      // row 2rp   -> low half
+                        const uint32_t wb = w[ks][2 * rp + 1][h];  // row 2rp+1 -> high half
+                        const uint32_t lo = __builtin_amdgcn_perm(wb, wa, 0x05040100u);  // nibbles 0..3, both rows
+                        const uint32_t hi = __builtin_amdgcn_perm(wb, wa, 0x07060302u);  // nibbles 4..7
+#pragma unroll
+                        for (int p = 0; p < 4; p++) {
+                            bop[p][rp] = code_pair_to_bf16(p == 0 ? lo : lo >> (4 * p), magic);
+                            bop[4 + p][rp] = code_pair_to_bf16(p == 0 ? hi : hi >> (4 * p), magic);
+                        }
+                    }
+#pragma unroll
+                    for (int p = 0; p < 8; p++) {
+                        acc[h][p] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                            a_op, as_bf16x8(bop[p][0], bop[p][1], bop[p][2], bop[p][3]), ks == 0 || FINE ? zero4 : acc[h][p], 0, 0, 0);
+                    }
                 }
                 if constexpr (FINE && ROWS == 16) {
                     float zoff[8];
@@ -847,7 +885,8 @@ __global__ __launch_bounds__(WAVES * kWave, KS == 1 && ROUNDS == 2 && EPI == kEp
     }
 }
 
-template <int WAVES, int KS, int MC, int ROUNDS, int PRO = kProNone, int EPI = kEpiStore, bool LONE = false, bool WALK = false, bool FINE = false>
+template <int WAVES, int KS, int MC, int ROUNDS, int PRO = kProNone, int EPI = kEpiStore, bool LONE = false, bool WALK = false, bool FINE = false,
+          bool TRIO = false>
 inline void launch_awq_gemv_mfma(const uint16_t* x, const int32_t* qweight, const uint16_t* scales,
                                  const int32_t* qzeros, uint16_t* y, float* partials, uint32_t* counters,
                                  int M, int K, int N, const MfmaGrid& split,
@@ -859,7 +898,7 @@ inline void launch_awq_gemv_mfma(const uint16_t* x, const int32_t* qweight, cons
     dim3 block(WAVES * kWave, 1, 1);
     MfmaGrid ordered = split;
     ordered.order = packed_tile_order(qweight, N, split.coltiles, split.ktiles);
-    hipLaunchKernelGGL((awq_gemv_mfma_kernel<WAVES, KS, MC, ROUNDS, PRO, EPI, LONE, WALK, FINE>), grid, block, 0, stream, x,
+    hipLaunchKernelGGL((awq_gemv_mfma_kernel<WAVES, KS, MC, ROUNDS, PRO, EPI, LONE, WALK, FINE, TRIO>), grid, block, 0, stream, x,
                        reinterpret_cast<const uint32_t*>(qweight), scales,
                        reinterpret_cast<const uint32_t*>(qzeros), y, partials, counters, M, K, N,
                        ordered, fi, res, rope, cache_stride);

@@ -27,7 +27,7 @@ def code_objects(data):
 @pytest.fixture(scope="module")
 def kernels(tmp_path_factory):
     """Template arguments of each awq_gemv_mfma_kernel (waves, steps, rows per round, rounds, prologue, epilogue, odd words,
-    walks, crosses groups) -> its bytes of scratch memory and its vector registers."""
+    walks, crosses groups, plain of which three fit a compute unit) -> its bytes of scratch memory and its vector registers."""
     from mykuiperllama_amd.build import KX_LIB
     if not os.path.exists(READELF):
         pytest.skip("llvm-readelf is not installed")
@@ -66,3 +66,10 @@ def test_two_rows_into_the_residual_stream_leave_room_for_six_workgroups(kernels
     # one step per wave: 512 registers a lane and six waves per SIMD are 80 registers a wave
     few = {args: registers for args, (_, registers) in kernels.items() if args[1:4] == (1, 2, 1) and args[5] == 2 and not args[8]}
     assert few and max(few.values()) <= 80
+
+
+def test_four_steps_behind_a_norm_fit_three_to_a_compute_unit(kernels):
+    # their workgroups wait for each other in grids of up to three per compute unit
+    three = {args: registers for args, (_, registers) in kernels.items()
+             if args[1] == 4 and args[2] * args[3] >= 8 and args[5] == 0 and not args[7] and not args[8] and (args[4] == 5 or args[9])}
+    assert len(three) >= 6 and max(three.values()) <= 168
