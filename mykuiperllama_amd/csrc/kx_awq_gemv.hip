@@ -60,13 +60,13 @@ constexpr int kExchangeRows = 8;    // what a K tile's share of the split-K exch
 //            (gate|up 4096 -> 24576 at M = 16: 19.7 against 21.5 us), and so do their column-tile-fastest order and 256 /
 //            512 rows per workgroup.
 //            Up to three per compute unit where that many of the form fit (kThreePerUnit, four steps, at most sixteen K
-//            tiles).  Behind a norm always: the figures stand there.  A plain launch, M = 6 / 9 / 16, single reader and two per
-//            compute unit -> shares and three: 5120 -> 15360 (600 workgroups, ten K tiles) 17.7 / 19.1 / 20.2 -> 15.1 / 16.1 /
-//            17.6, 8192 -> 10240 (640, sixteen) 17.0 / 20.3 / 21.2 -> 17.5 / 17.8 / 20.0, 4096 -> 24576 (768, eight) 17.7 / 18.3 /
-//            19.3 -> 16.3 / 18.0 / 19.6, 2048 -> 40960 (640, four) 16.7 / 18.1 / 19.2 -> 16.1 / 17.6 / 19.9: nine and more rows
-//            from ten K tiles on, fewer up to fifteen.  At five to eight rows these grids take four steps per wave in
-//            every form, so that all of them add alike: behind SwiGLU 4096 -> 24576 at M = 6 18.1 -> 17.5, into the
-//            residual stream 18.6 -> 17.6 (two steps -> four, single reader).
+//            tiles).  Behind a norm always: the figures stand there.  A plain launch of nine and more rows from ten K tiles on,
+//            M = 9 / 16, single reader and two per compute unit -> shares and three: 5120 -> 15360 (600 workgroups, ten K
+//            tiles) 19.1 / 20.2 -> 16.1 / 17.6, 8192 -> 10240 (640, sixteen) 20.3 / 21.2 -> 17.8 / 20.0; left out 4096 -> 24576
+//            (768, eight) 18.3 / 19.3 -> 18.0 / 19.6, 2048 -> 40960 (640, four) 18.1 / 19.2 -> 17.6 / 19.9, and at six rows 8192 ->
+//            10240 17.0 -> 17.5.  (Five to eight rows with two steps per wave would gain by four and shares, 4096 -> 24576
+//            behind a norm 18.6 -> 16.1, but add their K tiles in another order then: after five layers the logits
+//            of a step are 0.005 apart.)
 //            Unless K is long as well, more than 16 blocks of 512 rows (32 up to eight rows): then the partial sums
 //            outweigh that, and a workgroup walks over as many blocks as bring the grid down to two per compute unit.  us
 //            per launch, single reader -> walk, M = 5 / 8 / 9 / 16: 14336 -> 5120 (28 blocks) 18.4 / 18.8 / 25.0 / 26.5
@@ -137,9 +137,8 @@ inline AwqPlan make_mfma_plan(int M, int K, int N, int group, bool may_walk = tr
         if (kt == 1 || (kt <= kSliceMaxKTiles && p.coltiles * kt <= 2 * kComputeUnits)) {
             p.sliced = kt > 1;
             ks = best;
-        } else if (best == 4 && allowed(4) && kt <= 16 && p.coltiles * kt <= 3 * kComputeUnits) {
-            ks = 4;
-            p.trio = ends == kPlainEnds && (M >= 9 ? kt >= 10 : kt < 16);
+        } else if (ks == 4 && best == 4 && allowed(4) && kt <= 16 && p.coltiles * kt <= 3 * kComputeUnits) {
+            p.trio = ends == kPlainEnds && M >= 9 && kt >= 10;
             p.sliced = p.trio || ends == kNormEnds;
         } else if (allowed(4) && ktiles_with(4) > (M >= 9 ? 16 : 32)) {
             const int blocks = ktiles_with(4);
@@ -370,8 +369,7 @@ void launch_mfma_fused(const AwqPlan& p, const FusedInput& fi, const ResidualTar
     } while (0)
     if constexpr (PRO == kProNone && EPI == kEpiStore) {
         if (p.trio) {
-            if (M <= 8) launch_awq_gemv_mfma<4, 4, 8, 1, PRO, EPI, LONE, false, false, true>(KX_MARGS);
-            else launch_awq_gemv_mfma<4, 4, 8, 2, PRO, EPI, LONE, false, false, true>(KX_MARGS);
+            launch_awq_gemv_mfma<4, 4, 8, 2, PRO, EPI, LONE, false, false, true>(KX_MARGS);
             return;
         }
     }
@@ -602,17 +600,11 @@ extern "C" int kx_gemv_awq_bf16_policy(const uint16_t* x, const int32_t* qweight
             return kx::launch_status();
         }
 #undef KX_MFMA_WALK
-#define KX_MFMA_TRIO(LONE)                                                                                                          \
-    do {                                                                                                                            \
-        if (M <= 8) kx::launch_awq_gemv_mfma<4, 4, 8, 1, kx::kProNone, kx::kEpiStore, LONE, false, false, true>(KX_MARGS);          \
-        else kx::launch_awq_gemv_mfma<4, 4, 8, 2, kx::kProNone, kx::kEpiStore, LONE, false, false, true>(KX_MARGS);                 \
-    } while (0)
         if (p.trio) {
-            if (N % 16) KX_MFMA_TRIO(true);
-            else KX_MFMA_TRIO(false);
+            if (N % 16) kx::launch_awq_gemv_mfma<4, 4, 8, 2, kx::kProNone, kx::kEpiStore, true, false, false, true>(KX_MARGS);
+            else kx::launch_awq_gemv_mfma<4, 4, 8, 2, kx::kProNone, kx::kEpiStore, false, false, false, true>(KX_MARGS);
             return kx::launch_status();
         }
-#undef KX_MFMA_TRIO
 #define KX_MFMA_FINE(LONE)                                                                                          \
     do {                                                                                                             \
         if (M == 1) kx::launch_awq_gemv_mfma<4, 4, 1, 1, kx::kProNone, kx::kEpiStore, LONE, false, true>(KX_MARGS);  \

@@ -156,10 +156,10 @@ __device__ __forceinline__ int group_of_step(const MfmaGrid& g, int step) {
 //
 // Four steps per wave at five and more rows, stored: 185 registers leave two to a compute unit, so that a grid of 513 to 768
 // comes in two rounds and cannot finish its tiles together.  With four nibbles' operands at a time and a step's activations read
-// when it comes they fit 168 (what still goes to memory, 32 to 80 bytes a lane, belongs to the single reader's read-back).  Behind
-// a norm every such launch takes this form: us per launch, M = 6 / 9 / 16, two -> three and finishing together, 4096 -> 24576
-// 18.6 / 20.0 / 20.8 -> 16.1 / 18.0 / 18.7, 5120 -> 15360 18.4 / 20.9 / 21.6 -> 15.4 / 16.9 / 17.4, 8192 -> 10240 17.9 / 21.9 / 22.3
-// -> 17.2 / 18.1 / 20.2; two -> three alone, larger grids, M = 6 / 16, 4096 -> 32768 22.8 / 25.7 -> 22.8 / 24.3, 5120 -> 51200 43.8 /
+// when it comes they fit 168 (what still goes to memory at sixteen rows, 80 bytes a lane, belongs to the single reader's read-back).  Behind
+// a norm every such launch takes this form: us per launch, M = 9 / 16, two -> three and finishing together, 4096 -> 24576 20.0 /
+// 20.8 -> 18.0 / 18.7, 5120 -> 15360 20.9 / 21.6 -> 16.9 / 17.4, 8192 -> 10240 at M = 6 / 9 / 16 17.9 / 21.9 / 22.3 -> 17.2 / 18.1 / 20.2;
+// two -> three alone, larger grids, M = 6 / 16, 4096 -> 32768 22.8 / 25.7 -> 22.8 / 24.3, 5120 -> 51200 43.8 /
 // 48.2 -> 43.8 / 46.2, and smaller ones, 4096 -> 12288 12.3 / 13.9 -> 12.2 / 13.9.  A plain launch takes it where make_mfma_plan
 // says so (TRIO): larger grids at sixteen rows lose by it, 4096 -> 32768 23.5 -> 26.1.
 template <int KS, int ROWS, int PRO, int EPI, bool WALK, bool FINE, bool TRIO>

@@ -1,5 +1,5 @@
-"""Grids of 513 to 768 workgroups with four steps per wave at five and more rows, of which three fit a compute unit in some
-forms: against float64, the same bits in every form of a shape, and when no workgroup waits for the others."""
+"""Grids of 513 to 768 workgroups of four steps per wave at five and more rows, of which three fit a compute unit in some
+forms of nine and more rows: against float64, the same bits in every form of a shape, and when no workgroup waits for the others."""
 import pytest
 
 from tests.test_gpu_rows_same_bits import empty, problem
