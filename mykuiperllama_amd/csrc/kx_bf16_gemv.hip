@@ -198,13 +198,12 @@ __global__ __launch_bounds__(kMfmaWaves * kWave) void bf16_gemv_mfma_kernel(
 // part has UNITS of them or one less.
 // A row of a unit is stored with its 16-byte pieces permuted by the low bits of the row (the lane that loads piece j of
 // row r fetches piece j ^ (r & 7)), so that the sixteen rows that an operand read touches lie in different banks.
-// Two shapes.  Where rows start on memory lines, eight waves and units of 128 elements, 256 bytes of a row, which are two lines.
-// Rows that do not start on lines would have such a piece touch three: four waves and units of 512 elements, nine lines for
-// eight.  us per launch at M = 3 / 8 / 16, eight waves of equal parts of K rounded up to 1024 -> now: rows on lines 151936 x 4096
-// 195 / 202 / 215 -> 194 / 199 / 204, 151936 x 5120 238 / 247 / 263 -> 239 / 242 / 250, 32000 x 768 12.9 / 13.2 / 13.4 -> 10.9 /
-// 11.1 / 11.8; others 144453 x 3144 180 / 192 / 210 -> 160 / 166 / 174, 101754 x 2336 92 / 96 / 106 -> 83 / 86 / 89, 79438 x 1240
-// 48.6 / 50.0 / 53.4 -> 38.8 / 39.6 / 41.7, 69572 x 4688 123 / 126 / 133 -> 110 / 113 / 116 (W alone at the read rate of a large
-// buffer: 173, 216, 6.8; 126, 66, 27, 91).  Cached loads instead of streaming ones lose 10 % on lines and win 2 % off them.
+// Where rows start on memory lines, units of 128 elements, 256 bytes of a row, which are two lines; rows that do not start on
+// lines would have such a piece touch three, and longer units cost them less (launch_held).  us per launch at M = 3 / 8 / 16, eight
+// waves of equal parts of K rounded up to 1024 -> now: rows on lines 151936 x 4096 182 / 189 / 200 -> 180 / 186 / 194, 151936 x 5120
+// 231 / 241 / 254 -> 230 / 233 / 239, 32000 x 768 12.6 / 13.3 / 13.7 -> 10.8 / 11.1 / 11.8; others 144453 x 3144 172 / 182 / 198 -> 137 /
+// 144 / 152, 101754 x 2336 84 / 87 / 101 -> 74 / 75 / 82, 79438 x 1240 46.4 / 47.5 / 51.7 -> 36.9 / 38.4 / 40.1, 69572 x 4688 114 / 120 /
+// 125 -> 104 / 109 / 109 (W alone at the read rate of a large buffer: 173, 216, 6.8; 126, 66, 27, 91).  Cached loads instead of streaming ones lose 10 % on lines and win 2 % off them.
 constexpr int kRingBytes = 131072;
 
 template <int WAVES, int UNIT, int UNITS, int PARTS, bool RUNS>
@@ -392,14 +391,30 @@ int launch_held_parts(const uint16_t* x, const uint16_t* w, uint16_t* y, int M, 
 
 // The fewest parts whose A operands fit the registers and whose last round of blocks is not emptier for it by more than it gains:
 // a barrier for every PARTS-th of the blocks.  us per launch at M = 3, parts of K 8 / 4 / 2 on lines: 32000 x 768 12.0 / 11.6 / 10.9,
-// 60000 x 2048 44.8 / 42.9 / 42.0, 151936 x 4096 198 / 196 / -; 4 / 2 / 1 off lines: 67290 x 912 30.2 / 27.1 / 25.8, 98237 x 1232 49.6 /
-// 47.8 / 46.0, 91208 x 1568 54.1 / 54.3 / 54.7.  Few rounds leave compute units idle: up to four, all waves split K (4764 x 4032 at M = 16
-// 17.6 with four parts, 13.1 with eight).
+// 60000 x 2048 44.8 / 42.9 / 42.0, 151936 x 4096 198 / 196 / -; 4 / 2 / 1 off lines: 67290 x 912 30.2 / 27.1 / 25.8.  Few rounds leave
+// compute units idle: up to four, all waves split K (4764 x 4032 at M = 16 17.6 with four parts, 13.1 with eight).
+// Off lines eight waves that all split K, in units of the length that gives the fullest wave the fewest elements (the longer one of
+// two, with fewer of its pieces across a line), are ahead of four waves and units of 512.  us per launch, four waves -> eight,
+// M = 3 / 14: units of 128 up to K = 1024 4010 x 776 4.06 / 4.45 -> 3.62 / 3.81, 17000 x 904 10.4 / 11.3 -> 9.8 / 10.4, 66000 x 904 27.8 /
+// 29.9 -> 28.1 / 29.6 (left out from 5120 blocks on: 120000 x 904 39.6 / 41.0 -> 47.4 / 47.5); of 256 where they leave fewer than 512
+// 4100 x 1400 5.46 / 6.20 -> 5.10 / 5.75, 120000 x 1400 60.1 / 62.3 -> 57.8 / 57.9, 5500 x 5000 16.6 / 16.8 -> 15.8 / 16.9 (left out past
+// K = 4096 and four rounds: 17000 x 4504 31.4 / 33.2 -> 31.4 / 33.4, 120000 x 4504 177 / 178 -> 185 / 187); of 512 otherwise 4100 x 2200
+// 8.85 / 10.2 -> 6.86 / 8.05, 120000 x 3000 124 / 124 -> 112 / 113, 4100 x 7800 20.4 / 22.9 -> 17.6 / 19.9, 33000 x 7800 89.3 / 93.8 -> 88.6 / 92.8.
 int launch_held(const uint16_t* x, const uint16_t* w, uint16_t* y, int M, int K, int N, hipStream_t s) {
     const bool whole_lines = K % 64 == 0 && reinterpret_cast<uintptr_t>(w) % 128 == 0;
-    const int waves = whole_lines ? 8 : 4;
     const int blocks = (N + 15) / 16;
-    const int least = blocks <= 4 * kComputeUnits ? waves : (whole_lines ? (K <= 2048 ? 2 : (K <= 4096 ? 4 : 8)) : (K <= 1536 ? 1 : 4));
+    if (!whole_lines) {
+        const auto fullest = [&](int unit) { return ((K + unit - 1) / unit + 7) / 8 * unit; };
+        if (K <= 1024) {
+            if (blocks < 20 * kComputeUnits) return launch_held_parts<8, 128, 8>(x, w, y, M, K, N, s);
+        } else if (fullest(256) >= fullest(512)) {
+            return launch_held_parts<8, 512, 8>(x, w, y, M, K, N, s);
+        } else if (K <= 4096 || blocks <= 4 * kComputeUnits) {
+            return launch_held_parts<8, 256, 8>(x, w, y, M, K, N, s);
+        }
+    }
+    const int waves = whole_lines ? 8 : 4;
+    const int least = blocks <= 4 * kComputeUnits ? waves : (whole_lines ? (K <= 2048 ? 2 : (K <= 4096 ? 4 : 8)) : (K <= 1024 ? 1 : 4));
     int parts = waves;
     long best = 0;
     for (int p = waves, weight = 100 + (waves == 8 ? 9 : 6); p >= least; p /= 2, weight -= 3) {

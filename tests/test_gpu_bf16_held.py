@@ -1,5 +1,5 @@
-"""BF16 GEMV of several rows: K at the edges of the units that a wave takes (128 elements where rows start on memory lines, 512
-elsewhere) and of the number of waves that split it, outputs at the edges of runs of four blocks and of a round of 256, against
+"""BF16 GEMV of several rows: K at the edges of the units that a wave takes (128 elements where rows start on memory lines, 128,
+256 or 512 elsewhere) and of the number of waves that split it, outputs at the edges of runs of four blocks and of a round of 256, against
 float64."""
 import pytest
 
@@ -19,7 +19,7 @@ def check(torch, capi, w, K, N, Ms):
         assert ((y.double() - ref).norm() / ref.norm()).item() <= 1e-3, (M, K, N)
 
 
-@pytest.mark.parametrize("K", [16, 64, 128, 192, 504, 520, 896, 1032, 1088, 1536, 1544, 2048, 2056, 4032, 4104, 6144, 6152, 8184])
+@pytest.mark.parametrize("K", [16, 64, 128, 192, 504, 520, 896, 1032, 1088, 1536, 1544, 2048, 2056, 4032, 4088, 4104, 6144, 6152, 8184])
 @pytest.mark.parametrize("N", [4099, 16399])
 def test_units_and_parts(K, N):
     import torch
@@ -38,6 +38,15 @@ def test_rounds_and_runs(K, blocks):
     check(torch, capi, w, K, N, (3, 7))
 
 
+@pytest.mark.parametrize("K,blocks", [(200, 5119), (200, 5120), (1016, 5121), (4360, 1024), (4360, 1025)])
+def test_edges_of_the_forms_off_lines(K, blocks):
+    import torch
+    from mykuiperllama_amd import capi
+    N = 16 * blocks - 7
+    w = torch.randn((N, K), device="cuda").bfloat16()
+    check(torch, capi, w, K, N, (3, 16))
+
+
 def test_weights_off_a_line():
     import torch
     from mykuiperllama_amd import capi
@@ -46,7 +55,7 @@ def test_weights_off_a_line():
     check(torch, capi, flat[8:8 + N * K].view(N, K), K, N, (3, 16))
 
 
-@pytest.mark.parametrize("K", [136, 520, 1000])
+@pytest.mark.parametrize("K", [136, 520, 1000, 1032, 2056, 4104, 8184])
 def test_what_lies_past_a_row_takes_no_part(K):
     """The last unit of a row is read past K's end within W: an infinity there meets no zero."""
     import torch
