@@ -834,9 +834,13 @@ extern "C" int kx_gemv_awq_attn_merge_bf16(const void* attn_workspace, size_t at
     fi.heads_per_kv = n_q_heads / n_kv_heads;
     hipStream_t s = kx::as_stream(stream);
 #define KX_ARGS nullptr, qweight, scales, qzeros, y, partials, counters, 1, K, N, group_size, p.coltiles, p.ktiles, 1, s, fi
-    const bool few = nchunks <= kx::kMergeParts * kx::kMergeHoldShort;
-    if (p.waves == 8 && few) kx::launch_awq_gemv<8, 16, 1, kx::kProAttnMergeShort>(KX_ARGS);
-    else if (p.waves == 8) kx::launch_awq_gemv<8, 16, 1, kx::kProAttnMerge>(KX_ARGS);
+#define KX_MERGE(PRO) \
+    if (p.waves == 8 && nchunks <= kx::kMergeParts * kx::merge_hold(PRO)) kx::launch_awq_gemv<8, 16, 1, PRO>(KX_ARGS)
+    KX_MERGE(kx::kProAttnMerge32);
+    else KX_MERGE(kx::kProAttnMerge48);
+    else KX_MERGE(kx::kProAttnMerge64);
+    else KX_MERGE(kx::kProAttnMerge);
+#undef KX_MERGE
     else kx::launch_awq_gemv<4, 16, 1, kx::kProAttnMerge>(KX_ARGS);  // K = 128: one head
 #undef KX_ARGS
     return kx::launch_status();
@@ -850,7 +854,7 @@ void launch_chain(const AwqPlan& p, const FusedInput& fi, const RopeTarget& rope
                   const uint16_t* x, const int32_t* qweight, const uint16_t* scales, const int32_t* qzeros,
                   uint16_t* y, float* partials, uint32_t* counters, int K, int N, int group, hipStream_t stream) {
 #define KX_ARGS x, qweight, scales, qzeros, y, partials, counters, 1, K, N, group, p.coltiles, p.ktiles, 1, stream, fi, rope, res
-    constexpr bool MERGE = PRO == kProAttnMerge || PRO == kProAttnMergeShort;
+    constexpr bool MERGE = merges_attention(PRO);
     if constexpr (!MERGE) {
         if (p.rt == 32) {
             launch_awq_gemv<8, 32, 1, PRO, EPI>(KX_ARGS);
@@ -1052,7 +1056,9 @@ extern "C" int kx_gemv_awq_chain_bf16(const kx_chain_desc* d, const int32_t* qwe
         case KX_IN_ROW: KX_BY_OUT(kx::kProNone); break;
         case KX_IN_SWIGLU: KX_BY_OUT(kx::kProSwiGLU); break;
         case KX_IN_ATTN:
-            if (fi.nchunks <= kx::kMergeParts * kx::kMergeHoldShort) KX_BY_OUT(kx::kProAttnMergeShort);
+            if (fi.nchunks <= kx::kMergeParts * kx::merge_hold(kx::kProAttnMerge32)) KX_BY_OUT(kx::kProAttnMerge32);
+            else if (fi.nchunks <= kx::kMergeParts * kx::merge_hold(kx::kProAttnMerge48)) KX_BY_OUT(kx::kProAttnMerge48);
+            else if (fi.nchunks <= kx::kMergeParts * kx::merge_hold(kx::kProAttnMerge64)) KX_BY_OUT(kx::kProAttnMerge64);
             else KX_BY_OUT(kx::kProAttnMerge);
             break;
         default: KX_BY_OUT(kx::kProPreNorm); break;

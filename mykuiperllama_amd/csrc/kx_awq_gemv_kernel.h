@@ -99,9 +99,9 @@ __global__ __launch_bounds__(WAVES * kWave) void awq_gemv_kernel(
     constexpr bool STAGED = PRO != kProNone;
     constexpr bool NORM = PRO == kProAddNorm || PRO == kProAddNormLong;
     constexpr int NCH = PRO == kProAddNormLong ? kNormChunks : 1;
-    constexpr bool MERGE = PRO == kProAttnMerge || PRO == kProAttnMergeShort;
-    constexpr int HOLD = PRO == kProAttnMergeShort ? kMergeHoldShort : kMergeHold;
-    constexpr int STATS = PRO == kProAttnMergeShort ? 1 : kMergeStatsPerLane;
+    constexpr bool MERGE = merges_attention(PRO);
+    constexpr int HOLD = merge_hold(PRO);
+    constexpr int STATS = kMergeParts * HOLD <= kWave ? 1 : kMergeStatsPerLane;
     static_assert(kMergeParts * HOLD <= STATS * kWave, "the wave that prepares the factors sees every chunk");
     constexpr bool PRENORM = PRO == kProPreNorm;
     static_assert(!PRENORM || MB == 1, "the pre-reduced norm serves one activation row");

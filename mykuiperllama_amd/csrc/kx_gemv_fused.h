@@ -18,12 +18,19 @@ constexpr int kProAddNorm = 2;  // r = bf16(a + b) (b optional), x = gain * bf16
 constexpr int kProAddNormLong = 3;  // the same for rows of more than eight elements per thread
 constexpr int kProAttnMerge = 4;  // x = the attention output, merged here from the per-chunk results (M = 1)
 constexpr int kProPreNorm = 5;    // x = gain * bf16(a * rsqrt(mean(a^2) + eps)), the sum of squares given per 256 columns
-// The same for up to 32 chunks (2048 positions): a thread's loads go out, ahead of the weights', whatever the number of chunks.
-// us per launch into the residual stream, 80 -> 32 chunks covered: 2048 -> 1024 7.0 -> 5.95, 4096 -> 4096 7.5 -> 6.6, whatever the number of chunks.
-constexpr int kProAttnMergeShort = 6;
+// The same for fewer chunks: a thread's loads go out, ahead of the weights', whatever the number of chunks.  us per launch into the
+// residual stream, 80 -> 32 chunks covered: 2048 -> 1024 7.0 -> 5.95, 4096 -> 4096 7.5 -> 6.6;
+// -> 48 2048 -> 1024 6.74 -> 6.13, 4096 -> 4096 7.33 -> 6.75;
+// -> 64 6.75 -> 6.40 and 7.35 -> 7.08.
+constexpr int kProAttnMerge32 = 6, kProAttnMerge48 = 7, kProAttnMerge64 = 8;
+constexpr bool merges_attention(int pro) {
+    return pro == kProAttnMerge || pro == kProAttnMerge32 || pro == kProAttnMerge48 || pro == kProAttnMerge64;
+}
 constexpr int kNormChunks = 2;  // most 16-byte pieces of a row a thread holds for the sum of squares
 constexpr int kMergeHold = 20;  // per-chunk values a thread holds per element it merges: 80 chunks in four parts
-constexpr int kMergeHoldShort = 8;
+constexpr int merge_hold(int pro) {
+    return pro == kProAttnMerge32 ? 8 : (pro == kProAttnMerge48 ? 12 : (pro == kProAttnMerge64 ? 16 : kMergeHold));
+}
 constexpr int kMergeStatsPerLane = 2;  // chunks per lane of the wave that prepares a head's factors (>= 80 / 64)
 
 struct FusedInput {

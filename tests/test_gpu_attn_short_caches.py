@@ -62,9 +62,10 @@ def test_no_position_to_attend_to():
     assert not out.any()
 
 
-@pytest.mark.parametrize("positions,last", [(64, 63), (300, 5), (2048, 2047), (2049, 2048), (2049, 63), (5120, 5119)])
+@pytest.mark.parametrize("positions,last", [(64, 63), (300, 5), (2048, 2047), (2049, 2048), (2049, 63), (3072, 3071), (3073, 3072), (4096, 4095),
+                                            (4097, 700), (5120, 5119), (6144, 6143), (6145, 6144)])
 def test_merge_on_the_way_into_a_projection(positions, last):
-    """With up to 32 chunks, or more, the projection returns the bits of the merge followed by the projection."""
+    """At the edges of 32, 48 and 64 chunks the projection returns the bits of the merge followed by the projection."""
     torch = pytest.importorskip("torch")
     from mykuiperllama_amd import capi
     n_q, n_kv, N, group = 4, 2, 512, 128
