@@ -67,12 +67,16 @@ class DecodeModel:
         self.max_positions = max_positions
         # Where the attention chunks are merged: in the prologue of the o projection (one launch
         # fewer per layer) when the cache is short enough for it.  Every workgroup of that projection
-        # repeats the merge of its two heads, so it pays while the projection has about one round of
-        # workgroups (Qwen3-8B: 256 of them, 1.5 us per layer faster; Qwen3-32B: 640, 2 us slower
-        # than the separate merge kernel).  The caller can decide otherwise.
+        # repeats the merge of its two heads, so it pays while the projection has one round of workgroups (Qwen3-8B:
+        # 256 of them, 1.1 to 2.3 us per layer faster; Qwen3-32B: 640, 0.7 to 2.7 us slower than the separate merge
+        # kernel) and, up to two, while the heads have few chunks.  us per layer, in the projection / separate, at 1000, 3000
+        # and 5000 positions: 320 workgroups of 40 heads 34.1 / 35.0, 36.8 / 36.7, 39.5 / 38.4, 400 38.6 / 38.8, 40.4 / 40.7,
+        # 43.2 / 42.4, 384 of 64 34.3 / 34.8, 37.4 / 36.2, 40.7 / 38.2.  The caller can decide otherwise.
         fits = max_positions <= capi.FUSED_MERGE_MAX_POSITIONS
         o_workgroups = -(-cfg.hidden // 256) * max(1, cfg.n_q * cfg.head_dim // 256)
-        self.merge_in_o = fits and (o_workgroups <= 512 if merge_in_o is None else bool(merge_in_o))
+        chunks = -(-max_positions // (64 if max_positions <= 5120 else 128))
+        pays = o_workgroups <= 256 or (o_workgroups <= 512 and cfg.n_q * chunks <= 1920)
+        self.merge_in_o = fits and (pays if merge_in_o is None else bool(merge_in_o))
         c = cfg
         gen = torch.Generator(device="cuda")
         gen.manual_seed(seed)
