@@ -147,8 +147,17 @@ constexpr int kMaxGroup = 16;  // query heads per KV head: the rows of one MFMA 
 // 40001 of 40960 (2560 workgroups) 35.7 -> 35.5; one at 15000 of 15500 (976) 16.9 -> 17.1, at 4096 of 4224 (528, first stage
 // alone) 6.38 -> 6.50, at 700 of 1024 (128) 4.03 -> 3.97.
 constexpr int kAsksFrom = 2048;  // workgroups of one sequence: eight for each compute unit
+// HEADS_FIRST: neighbours in the grid are the KV heads of a chunk, which read whole rows together; otherwise the chunks of a head.
+// With 16 or 32 KV heads a head's rows lie 4 or 8 KB apart, and chunks of one head side by side ask the same few memory channels
+// for 256 bytes each: us with the merge, chunks first -> heads first, 32 KV heads, one sequence of 8192 positions 30.4 -> 27.5, of
+// 16384 62.4 -> 46.5, eight of 4096 102 -> 82 (87 before K was read by rows), four of 3500 42.2 -> 38.9; 16, one of 16384 34.7 -> 27.0, two
+// of 4096 0.94 of the time.  Caches of a few hundred positions lose by it (sixteen sequences of 300, 16 / 32 KV heads + 1 / + 3 %), and so
+// do other numbers of heads as often as they gain (of 4224 to 16384 positions 4 KV heads + 3 to - 2 %, 8 + 5 to - 2, 20 + 2 to + 4, 24
+// + 1 to - 1).
+constexpr int kHeadsFirstFrom = 1024;  // positions
+inline bool heads_first(int n_kv, int max_positions) { return n_kv % 16 == 0 && max_positions >= kHeadsFirstFrom; }
 
-template <int CHUNK, bool ASKS>
+template <int CHUNK, bool ASKS, bool HEADS_FIRST>
 __global__ __launch_bounds__(kAttnThreads) void attn_decode_stage1(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k_cache, const uint16_t* __restrict__ v_cache,
     float* __restrict__ part_out, float* __restrict__ part_ml, int n_kv, int G, const int32_t* __restrict__ pos_ptr,
@@ -166,8 +175,8 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_stage1(
     uint32_t(*s_v)[kVRow] = reinterpret_cast<uint32_t(*)[kVRow]>(s_rows);
     uint32_t(*s_k)[kKRow] = reinterpret_cast<uint32_t(*)[kKRow]>(s_rows);
 
-    const int kvh = blockIdx.y;
-    const int chunk = blockIdx.x;
+    const int kvh = HEADS_FIRST ? blockIdx.x : blockIdx.y;
+    const int chunk = HEADS_FIRST ? blockIdx.y : blockIdx.x;
     const int p0 = chunk * CHUNK;
     const int tid = threadIdx.x;
     {
@@ -799,15 +808,22 @@ int attn_decode(const uint16_t* q, const uint16_t* k_cache, const uint16_t* v_ca
     float* part_ml = part_out + static_cast<size_t>(batch) * nchunks * n_q_heads * kx::kHeadDim;
     const float scale = 1.0f / sqrtf(static_cast<float>(kx::kHeadDim));
     hipStream_t s = kx::as_stream(stream);
-    dim3 grid1(nchunks, n_kv_heads, batch);
+    const bool heads = kx::heads_first(n_kv_heads, max_positions);
+    const dim3 grid1(heads ? n_kv_heads : nchunks, heads ? nchunks : n_kv_heads, batch);
     const bool asks = batch > 1 || nchunks * n_kv_heads > kx::kAsksFrom;
-#define KX_STAGE1(CHUNK, ASKS)                                                                                                     \
-    hipLaunchKernelGGL((kx::attn_decode_stage1<CHUNK, ASKS>), grid1, dim3(kx::kAttnThreads), 0, s, q, k_cache, v_cache, part_out, \
-                       part_ml, n_kv_heads, G, pos, nchunks, max_positions, scale, cache_stride)
+#define KX_STAGE1_IN(CHUNK, ASKS, HEADS)                                                                                           \
+    hipLaunchKernelGGL((kx::attn_decode_stage1<CHUNK, ASKS, HEADS>), grid1, dim3(kx::kAttnThreads), 0, s, q, k_cache, v_cache,    \
+                       part_out, part_ml, n_kv_heads, G, pos, nchunks, max_positions, scale, cache_stride)
+#define KX_STAGE1(CHUNK, ASKS)                        \
+    do {                                              \
+        if (heads) KX_STAGE1_IN(CHUNK, ASKS, true);   \
+        else KX_STAGE1_IN(CHUNK, ASKS, false);        \
+    } while (0)
     if (long_chunks && asks) KX_STAGE1(kx::kAttnChunkLong, true);
     else if (long_chunks) KX_STAGE1(kx::kAttnChunkLong, false);
     else if (asks) KX_STAGE1(kx::kAttnChunkShort, true);
     else KX_STAGE1(kx::kAttnChunkShort, false);
+#undef KX_STAGE1_IN
 #undef KX_STAGE1
     if (out) {
         // slots per chunk subset: at least what the first flight of the merge covers

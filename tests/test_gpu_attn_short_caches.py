@@ -1,5 +1,5 @@
 """Attention over caches that are not full: chunks behind the last position, at every form of the first stage (asking for the
-position first or not, chunks of 64 and 128) and of the merge (chunks covered by its first flight)."""
+position first or not, chunks of 64 and 128, chunks or heads side by side) and of the merge (chunks covered by its first flight)."""
 import pytest
 
 pytestmark = pytest.mark.gpu
@@ -16,6 +16,9 @@ def reference(torch, q, k, v, n_q, n_kv, last):
 CASES = [(4, 2, 64, [0, 63]), (4, 2, 200, [0, 62, 63, 64, 127, 128, 199]), (6, 2, 2048, [700, 2047]), (6, 2, 2049, [2048, 64]),
          (6, 2, 3072, [3071, 1]), (6, 2, 3073, [3072, 1000]), (8, 1, 5120, [5119, 5]), (4, 4, 4097, [4096, 4095, 127, 128, 255]),
          (16, 1, 130, [129, 127, 128, 0]),
+         # many KV heads, whose chunks lie side by side in the grid from 1024 positions on
+         (16, 16, 1023, [1022, 5]), (16, 16, 1024, [1023, 0, 64]), (32, 32, 1100, [1099, 63, 64, 700]), (64, 32, 1024, [1000]),
+         (32, 32, 5120, [700]), (48, 48, 5121, [5120]),
          (8, 8, 1000, [999]), (8, 8, 32768, [32767]), (8, 8, 32769, [32768]), (8, 8, 32769, [700]), (8, 8, 32769, [0])]
 
 
@@ -62,13 +65,16 @@ def test_no_position_to_attend_to():
     assert not out.any()
 
 
-@pytest.mark.parametrize("positions,last", [(64, 63), (300, 5), (2048, 2047), (2049, 2048), (2049, 63), (3072, 3071), (3073, 3072), (4096, 4095),
-                                            (4097, 700), (5120, 5119), (6144, 6143), (6145, 6144)])
-def test_merge_on_the_way_into_a_projection(positions, last):
+# 32 KV heads at 5120 positions: a first stage that asks for the position and leaves the chunks behind it unwritten
+@pytest.mark.parametrize("positions,last,n_q,n_kv", [(64, 63, 4, 2), (300, 5, 4, 2), (2048, 2047, 4, 2), (2049, 2048, 4, 2), (2049, 63, 4, 2),
+                                                     (3072, 3071, 4, 2), (3073, 3072, 4, 2), (4096, 4095, 4, 2), (4097, 700, 4, 2),
+                                                     (5120, 5119, 4, 2), (6144, 6143, 4, 2), (6145, 6144, 4, 2),
+                                                     (5120, 63, 32, 32), (5120, 700, 32, 32), (5120, 5119, 32, 32)])
+def test_merge_on_the_way_into_a_projection(positions, last, n_q, n_kv):
     """At the edges of 32, 48 and 64 chunks the projection returns the bits of the merge followed by the projection."""
     torch = pytest.importorskip("torch")
     from mykuiperllama_amd import capi
-    n_q, n_kv, N, group = 4, 2, 512, 128
+    N, group = 512, 128
     K = n_q * 128
     g = torch.Generator(device="cuda")
     g.manual_seed(positions)
