@@ -232,8 +232,9 @@ __global__ __launch_bounds__(WAVES * kWave, ((KS == 1 && ROUNDS == 2 && EPI == k
     const int lane = tid % kWave;
     const int c = lane % 16;  // column slot: word pair c of the tile, MFMA column c
     const int b = lane / 16;  // k block inside the step, D row block
-    // Column tiles run fastest, so neighbours in time are neighbours in N; where workgroups finish a tile together, in
-    // groups of at most eight, so that they start within 8 * ktiles of each other.
+    // By number column tiles run fastest, so neighbours in time are neighbours in N; where workgroups finish a tile together, in
+    // groups of at most eight, so that they start within 8 * ktiles of each other.  By XCD (grid.order) those of a tile lie
+    // anywhere in the grid: grids that finish together are sized to be resident whole, and their wait is bounded.
     Tile tile{static_cast<int>(blockIdx.z * grid.side + blockIdx.x), static_cast<int>(blockIdx.y)};
     const int ktiles = grid.ktiles;
     if (grid.order.run) tile = tile_of_workgroup(grid.order, (blockIdx.z * ktiles + blockIdx.y) * grid.side + blockIdx.x, static_cast<uint32_t>(ktiles));
@@ -897,7 +898,8 @@ inline void launch_awq_gemv_mfma(const uint16_t* x, const int32_t* qweight, cons
     const dim3 grid(split.side, split.ktiles, split.coltiles / split.side);
     dim3 block(WAVES * kWave, 1, 1);
     MfmaGrid ordered = split;
-    ordered.order = packed_tile_order(qweight, N, split.coltiles, split.ktiles);
+    const bool by_number = split.sliced && split.run == 1 && together_by_number(M, KS, split.coltiles, split.ktiles);
+    if (!by_number) ordered.order = packed_tile_order(qweight, N, split.coltiles, split.ktiles);
     hipLaunchKernelGGL((awq_gemv_mfma_kernel<WAVES, KS, MC, ROUNDS, PRO, EPI, LONE, WALK, FINE, TRIO>), grid, block, 0, stream, x,
                        reinterpret_cast<const uint32_t*>(qweight), scales,
                        reinterpret_cast<const uint32_t*>(qzeros), y, partials, counters, M, K, N,

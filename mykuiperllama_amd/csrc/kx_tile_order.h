@@ -77,6 +77,21 @@ inline TileOrder packed_tile_order(const void* qweight, int N, int coltiles, int
     return whole_lines ? TileOrder{} : tile_order_of(static_cast<uint32_t>(coltiles), static_cast<uint32_t>(ktiles));
 }
 
+// Whether workgroups that finish a column tile together (`steps` 32-row steps for each of four waves and one block of K each) keep
+// the order of the numbers all the same.  With a multiple of eight column tiles that order has every column on one XCD, and so the
+// exchange, which grows with the rows, while the shared lines grow with the rows of W that a workgroup reads.  us per launch, by
+// number -> by XCD, M = 16: one step 1024 -> 6072 7.6 -> 8.5, 2048 -> 4056 8.5 -> 9.4; two steps 5312 -> 1920 with groups of 64 behind
+// SwiGLU 9.05 -> 10.2, 2048 -> 8168 9.3 -> 9.8; four steps 6144 -> 4056 (192 workgroups) 10.9 -> 11.3, 4096 -> 8168 (256) 12.6 -> 11.8;
+// M = 9: one step 1024 -> 6072 7.25 -> 7.75, two 2048 -> 6072 8.3 -> 8.4, 2048 -> 8168 8.9 -> 8.9, four 4096 -> 6072 (192) 10.5 -> 10.2;
+// M = 6: one step 1024 -> 8168 7.1 -> 7.4, two 2048 -> 8168 8.3 -> 8.2.
+// With two and four column tiles an XCD's run is few rows of tiles and, unless the K tiles divide by eight, begins inside one:
+// 6144 -> 264 (12 K tiles) at M = 6 / 16 8.3 / 8.8 -> 8.6 / 9.2, 2112 -> 896 with groups of 64 behind SwiGLU at M = 12 (9) 7.65 -> 8.0;
+// 4096 -> 776 (16) at M = 6 / 16 7.5 / 8.1 -> 7.3 / 8.0.
+inline bool together_by_number(int M, int steps, int coltiles, int ktiles) {
+    if (coltiles % static_cast<int>(kXcds) == 0) return 4 * steps < M || coltiles * ktiles <= 12 * M;
+    return (coltiles == 2 || coltiles == 4) && ktiles % static_cast<int>(kXcds) != 0;
+}
+
 }  // namespace kx
 
 #endif  // KX_TILE_ORDER_H

@@ -33,6 +33,17 @@ def test_against_the_oracle(oracle, M, K, N, group):
     assert H.rel_l2(H.bf16_to_f64(bits), ref) <= 1e-3
 
 
+# grids that finish together, on both sides of the rule that keeps the order of the numbers: eight column tiles and more with one,
+# two and four steps and with 12 M workgroups and more, two and four with K tiles that do and do not divide by eight
+@pytest.mark.parametrize("M,K,N", [(16, 4096, 24 * 256), (16, 4608, 24 * 256), (16, 1024, 8 * 256), (9, 4096, 16 * 256), (8, 4096, 16 * 256),
+                                   (5, 1024, 24 * 256), (6, 6144, 512), (6, 4096, 512), (12, 2304, 1024), (12, 2048, 1024), (16, 8192, 8 * 256)])
+def test_few_workgroups_that_finish_together(M, K, N):
+    import torch
+    from mykuiperllama_amd import capi
+    on, off = (run(torch, capi, M, K, N, 128, shift)[1] for shift in (0, 1))
+    assert np.array_equal(on, off)
+
+
 @pytest.mark.parametrize("M", [1, 3, 9])
 def test_weights_off_a_line_return_the_same_bits(M):
     import torch
