@@ -5,7 +5,10 @@
 // accumulator, and the lanes meet in a wave-wide sum at the end.  Rows are contiguous, so every load
 // is a full 1 KiB per wave.  Several rows: matrix cores, the activations held in registers while a workgroup walks over
 // blocks of output rows (third kernel below), or, for K > 8192, sixteen output rows per workgroup (second kernel).
+#include <type_traits>
+
 #include "kx_common.h"
+#include "kx_internal.h"
 
 namespace kx {
 namespace {
@@ -355,40 +358,17 @@ __global__ __launch_bounds__(WAVES * kWave, WAVES / 4) void bf16_gemv_held_kerne
 constexpr int kHeldMostK = 8192;
 constexpr int kComputeUnits = 256;
 
-template <int WAVES, int UNIT, int PARTS, bool RUNS>
-int launch_held_parts(const uint16_t* x, const uint16_t* w, uint16_t* y, int M, int K, int N, hipStream_t s) {
-    constexpr int SIDE = WAVES / PARTS;
-    const int blocks = (N + 15) / 16, sides = (blocks + SIDE - 1) / SIDE;
-    const dim3 grid(sides < kComputeUnits ? sides : kComputeUnits), block(WAVES * kWave);
-#define KX_HELD(U)                                                                                                                   \
-    case U:                                                                                                                          \
-        if constexpr (UNIT * PARTS * (U - 1) < kHeldMostK && (PARTS > 1 || U <= 3)) {                                                \
-            hipLaunchKernelGGL((bf16_gemv_held_kernel<WAVES, UNIT, U, PARTS, RUNS>), grid, block, 0, s, x, w, y, M, K, N, blocks);   \
-        }                                                                                                                            \
-        break
-    switch (((K + UNIT - 1) / UNIT + PARTS - 1) / PARTS) {
-        KX_HELD(1);
-        KX_HELD(2);
-        KX_HELD(3);
-        KX_HELD(4);
-        KX_HELD(5);
-        KX_HELD(6);
-        KX_HELD(7);
-        KX_HELD(8);
-    }
-#undef KX_HELD
-    return launch_status();
-}
+// Which form of the kernel a launch takes.
+struct HeldForm {
+    int waves, unit, parts;
+    int units;  // of the fullest part
+    bool runs;
+};
 
 // Runs of four blocks pay with the rows of y that are written and are lost among long rows of W: us per launch, one by one -> in
 // runs, M = 16 151936 x 4096 214 -> 204, 151936 x 5120 266 -> 250, 144453 x 3144 184 -> 174; M = 8 151936 x 4096 203 -> 199; M = 3
 // 144453 x 3144 160 -> 162; 40000 x 8192 at M = 8 / 16 110 / 114 -> 115 / 118.
-template <int WAVES, int UNIT, int PARTS>
-int launch_held_parts(const uint16_t* x, const uint16_t* w, uint16_t* y, int M, int K, int N, hipStream_t s) {
-    if (M >= 6 && K <= 6144) return launch_held_parts<WAVES, UNIT, PARTS, true>(x, w, y, M, K, N, s);
-    return launch_held_parts<WAVES, UNIT, PARTS, false>(x, w, y, M, K, N, s);
-}
-
+//
 // The fewest parts whose A operands fit the registers and whose last round of blocks is not emptier for it by more than it gains:
 // a barrier for every PARTS-th of the blocks.  us per launch at M = 3, parts of K 8 / 4 / 2 on lines: 32000 x 768 12.0 / 11.6 / 10.9,
 // 60000 x 2048 44.8 / 42.9 / 42.0, 151936 x 4096 198 / 196 / -; 4 / 2 / 1 off lines: 67290 x 912 30.2 / 27.1 / 25.8.  Few rounds leave
@@ -400,21 +380,22 @@ int launch_held_parts(const uint16_t* x, const uint16_t* w, uint16_t* y, int M, 
 // 4100 x 1400 5.46 / 6.20 -> 5.10 / 5.75, 120000 x 1400 60.1 / 62.3 -> 57.8 / 57.9, 5500 x 5000 16.6 / 16.8 -> 15.8 / 16.9 (left out past
 // K = 4096 and four rounds: 17000 x 4504 31.4 / 33.2 -> 31.4 / 33.4, 120000 x 4504 177 / 178 -> 185 / 187); of 512 otherwise 4100 x 2200
 // 8.85 / 10.2 -> 6.86 / 8.05, 120000 x 3000 124 / 124 -> 112 / 113, 4100 x 7800 20.4 / 22.9 -> 17.6 / 19.9, 33000 x 7800 89.3 / 93.8 -> 88.6 / 92.8.
-int launch_held(const uint16_t* x, const uint16_t* w, uint16_t* y, int M, int K, int N, hipStream_t s) {
-    const bool whole_lines = K % 64 == 0 && reinterpret_cast<uintptr_t>(w) % 128 == 0;
+HeldForm held_form(bool whole_lines, int M, int K, int N) {
     const int blocks = (N + 15) / 16;
+    const auto fullest = [&](int unit, int parts) { return ((K + unit - 1) / unit + parts - 1) / parts; };
+    const auto form = [&](int waves, int unit, int parts) { return HeldForm{waves, unit, parts, fullest(unit, parts), M >= 6 && K <= 6144}; };
     if (!whole_lines) {
-        const auto fullest = [&](int unit) { return ((K + unit - 1) / unit + 7) / 8 * unit; };
         if (K <= 1024) {
-            if (blocks < 20 * kComputeUnits) return launch_held_parts<8, 128, 8>(x, w, y, M, K, N, s);
-        } else if (fullest(256) >= fullest(512)) {
-            return launch_held_parts<8, 512, 8>(x, w, y, M, K, N, s);
+            if (blocks < 20 * kComputeUnits) return form(8, 128, 8);
+        } else if (256 * fullest(256, 8) >= 512 * fullest(512, 8)) {
+            return form(8, 512, 8);
         } else if (K <= 4096 || blocks <= 4 * kComputeUnits) {
-            return launch_held_parts<8, 256, 8>(x, w, y, M, K, N, s);
+            return form(8, 256, 8);
         }
     }
     const int waves = whole_lines ? 8 : 4;
-    const int least = blocks <= 4 * kComputeUnits ? waves : (whole_lines ? (K <= 2048 ? 2 : (K <= 4096 ? 4 : 8)) : (K <= 1024 ? 1 : 4));
+    int least = K <= 1024 ? 1 : 4;
+    if (whole_lines) least = blocks <= 4 * kComputeUnits ? waves : (K <= 2048 ? 2 : (K <= 4096 ? 4 : 8));
     int parts = waves;
     long best = 0;
     for (int p = waves, weight = 100 + (waves == 8 ? 9 : 6); p >= least; p /= 2, weight -= 3) {
@@ -426,18 +407,51 @@ int launch_held(const uint16_t* x, const uint16_t* w, uint16_t* y, int M, int K,
             parts = p;
         }
     }
-    if (whole_lines) {
-        if (parts == 8) return launch_held_parts<8, 128, 8>(x, w, y, M, K, N, s);
-        if (parts == 4) return launch_held_parts<8, 128, 4>(x, w, y, M, K, N, s);
-        return launch_held_parts<8, 128, 2>(x, w, y, M, K, N, s);
-    }
-    if (parts == 4) return launch_held_parts<4, 512, 4>(x, w, y, M, K, N, s);
-    if (parts == 2) return launch_held_parts<4, 512, 2>(x, w, y, M, K, N, s);
-    return launch_held_parts<4, 512, 1>(x, w, y, M, K, N, s);
+    return form(waves, whole_lines ? 128 : 512, parts);
+}
+
+// Launches `form` if it is one of these; UNITS are the numbers of units that the rule above gives with the others, and no
+// more are compiled.
+template <int WAVES, int UNIT, int PARTS, bool RUNS, int... UNITS>
+bool launch_held_of(const HeldForm& form, const uint16_t* x, const uint16_t* w, uint16_t* y, int M, int K, int N, hipStream_t s) {
+    if (form.waves != WAVES || form.unit != UNIT || form.parts != PARTS || form.runs != RUNS) return false;
+    constexpr int SIDE = WAVES / PARTS;
+    const int blocks = (N + 15) / 16, sides = (blocks + SIDE - 1) / SIDE;
+    const dim3 grid(sides < kComputeUnits ? sides : kComputeUnits), block(WAVES * kWave);
+    const auto launch = [&](auto units) {
+        constexpr int U = decltype(units)::value;
+        if (form.units != U) return false;
+        hipLaunchKernelGGL((bf16_gemv_held_kernel<WAVES, UNIT, U, PARTS, RUNS>), grid, block, 0, s, x, w, y, M, K, N, blocks);
+        return true;
+    };
+    return (launch(std::integral_constant<int, UNITS>{}) || ...);
+}
+
+int launch_held(const uint16_t* x, const uint16_t* w, uint16_t* y, int M, int K, int N, hipStream_t s) {
+    const bool whole_lines = K % 64 == 0 && reinterpret_cast<uintptr_t>(w) % 128 == 0;
+    const HeldForm form = held_form(whole_lines, M, K, N);
+#define KX_HELD(WAVES, UNIT, PARTS, RUNS, ...) launch_held_of<WAVES, UNIT, PARTS, RUNS, __VA_ARGS__>(form, x, w, y, M, K, N, s)
+    const bool launched =
+        KX_HELD(8, 128, 8, false, 1, 2, 3, 4, 5, 6, 7, 8) || KX_HELD(8, 128, 8, true, 1, 2, 3, 4, 5, 6) ||
+        KX_HELD(8, 128, 4, false, 1, 2, 3, 4, 5, 6, 7, 8) || KX_HELD(8, 128, 4, true, 1, 2, 3, 4, 5, 6, 7, 8) ||
+        KX_HELD(8, 128, 2, false, 1, 2, 3, 4, 5, 6, 7, 8) || KX_HELD(8, 128, 2, true, 1, 2, 3, 4, 5, 6, 7, 8) ||
+        KX_HELD(8, 256, 8, false, 1, 3) || KX_HELD(8, 256, 8, true, 1, 3) || KX_HELD(8, 512, 8, false, 1, 2) || KX_HELD(8, 512, 8, true, 1) ||
+        KX_HELD(4, 512, 4, false, 1, 3) || KX_HELD(4, 512, 4, true, 1, 3) || KX_HELD(4, 512, 2, false, 1) || KX_HELD(4, 512, 2, true, 1) ||
+        KX_HELD(4, 512, 1, false, 1, 2) || KX_HELD(4, 512, 1, true, 1, 2);
+#undef KX_HELD
+    return launched ? launch_status() : KX_ERR_BAD_SHAPE;
 }
 
 }  // namespace
 }  // namespace kx
+
+extern "C" int kx_bf16_held_form(int32_t whole_lines, int32_t M, int32_t K, int32_t N, int32_t* form) {
+    if (!form || M < 2 || M > KX_MAX_BATCH || K < 8 || K % 8 != 0 || K > kx::kHeldMostK || N < 1) return 0;
+    const kx::HeldForm f = kx::held_form(whole_lines != 0, M, K, N);
+    const int32_t fields[5] = {f.waves, f.unit, f.units, f.parts, f.runs};
+    for (int i = 0; i < 5; i++) form[i] = fields[i];
+    return 1;
+}
 
 extern "C" int kx_gemv_bf16(const uint16_t* x, const uint16_t* w, uint16_t* y, int32_t M, int32_t K,
                             int32_t N, void* workspace, size_t workspace_bytes, void* stream) {

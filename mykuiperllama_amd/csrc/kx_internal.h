@@ -69,6 +69,11 @@ int kx_decode_step_bf16(const kx_step_desc* desc, const kx_step_layer* layers, v
  * 1, or 0 where such a grid is too small or too large for it and a workgroup takes the tile of its own number. */
 int kx_shared_line_tile(int32_t coltiles, int32_t ktiles, int32_t id, int32_t* ct, int32_t* kt);
 
+/* The form of csrc/kx_bf16_gemv.hip's kernel for two to sixteen rows and K <= 8192 that a launch takes, by whether every row of W
+ * starts on a memory line: waves, elements of K per unit, units of a wave, waves that split K, runs of four blocks (0 or 1).
+ * Returns 1, or 0 for sizes that the kernel does not take. */
+int kx_bf16_held_form(int32_t whole_lines, int32_t M, int32_t K, int32_t N, int32_t* form);
+
 /* Bytes of a kx_step_desc and of a kx_step_layer as the library was compiled: a binding that mirrors them compares. */
 size_t kx_step_desc_bytes(void);
 size_t kx_step_layer_bytes(void);
