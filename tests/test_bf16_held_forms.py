@@ -1,10 +1,12 @@
-"""Which form of the BF16 kernel of several rows a launch takes: the library holds the forms that the rule gives and no others."""
+"""Which form of the BF16 kernel of several rows a launch takes: the library holds the forms that the rule gives and no others, and
+the tests on the GPU run each of them."""
 import ctypes
 import re
 
 import pytest
 
 from mykuiperllama_amd.build import KX_LIB
+from tests.test_gpu_bf16_held import FORMS
 
 # a block and its neighbours where the rule looks at their number, and numbers between
 BLOCKS = sorted({1, 255, 256, 257, 1023, 1024, 1025, 5119, 5120, 5121, *range(1026, 12000, 97)})
@@ -28,6 +30,12 @@ def test_the_library_holds_what_the_rule_gives(reached):
     with open(KX_LIB, "rb") as f:
         names = re.findall(rb"bf16_gemv_held_kernelILi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)ELb(\d)E", f.read())
     assert {tuple(int(n) for n in name) for name in names} == reached
+
+
+def test_the_tests_on_the_gpu_run_every_form(reached):
+    lib = ctypes.CDLL(KX_LIB)
+    assert all(K % 64 == 0 for K, _, on_lines in FORMS if on_lines)
+    assert {form(lib, on_lines, M, K, 16 * blocks - 5) for K, blocks, on_lines in FORMS for M in (3, 16)} == reached
 
 
 def test_sizes_that_the_kernel_does_not_take():

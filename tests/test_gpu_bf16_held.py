@@ -47,6 +47,26 @@ def test_edges_of_the_forms_off_lines(K, blocks):
     check(torch, capi, w, K, N, (3, 16))
 
 
+# every form of the kernel (test_bf16_held_forms.py holds this list to it): K, blocks, and whether W starts on a memory line.
+# Eight, four and two of eight waves to a block, one to eight units each, the last block beside nothing; off lines two and one of four
+FORMS = ([(K, 300, True) for K in (1088, 2112, 3072, 3136, 5120, 5184, 7168, 8128, 8192)] +
+         [(K, 1285, True) for K in (64, 512, 704, 1024, 1088, 1472, 2048, 2112, 2560, 3008, 3520, 4096)] +
+         [(1984, 3500, True)] +
+         [(K, 2000, True) for K in (64, 256, 448, 704, 768, 1024, 1280, 1536, 1728, 2048)] + [(768, 1999, True), (704, 1803, True)] +
+         [(K, 300, False) for K in (64, 1216, 2816, 4096, 5056, 6400)] +
+         [(4608, 1025, False), (6080, 1029, False), (904, 5120, False), (200, 5120, False), (904, 7499, False), (904, 7500, False), (896, 7500, False),
+          (1024, 5121, False)])
+
+
+@pytest.mark.parametrize("K,blocks,on_lines", FORMS)
+def test_every_form(K, blocks, on_lines):
+    import torch
+    from mykuiperllama_amd import capi
+    N, shift = 16 * blocks - 5, 0 if on_lines else 8
+    flat = torch.randn(N * K + shift, device="cuda").bfloat16()
+    check(torch, capi, flat[shift:].view(N, K), K, N, (3, 16))
+
+
 def test_weights_off_a_line():
     import torch
     from mykuiperllama_amd import capi
