@@ -86,7 +86,13 @@ __device__ __forceinline__ float dot2_bf16(uint32_t a, uint32_t b, float c) {
     return __builtin_amdgcn_fdot2_f32_bf16(va, vb, c, false);
 }
 
-template <int WAVES, int RT, int MB, int PRO, int EPI>
+// ORDERED: a workgroup takes its tile by the order that is handed over, if there is one.  One-row launches that need none have a
+// form without the test, which stands in front of the first load.  us per launch, with the test -> without: plain 1024 -> 2048 3.386 ->
+// 3.370, 2048 -> 1024 3.463 -> 3.446, 12288 -> 4096 7.77 -> 7.71; behind a norm 1024 -> 2048 4.659 -> 4.630, 4096 -> 4096 5.284 -> 5.242,
+// 12288 -> 4096 9.62 -> 9.57; behind SwiGLU into the residual stream 8192 -> 5120 8.79 -> 8.68; behind the attention merge of 16 chunks
+// 4096 -> 4096 6.53 -> 6.43; with a rotary epilogue 4096 -> 6144 7.47 -> 7.36.  (The arguments fetched ahead of the test and the
+// ordered branch out of line give none of it back.)
+template <int WAVES, int RT, int MB, int PRO, int EPI, bool ORDERED>
 __global__ __launch_bounds__(WAVES * kWave) void awq_gemv_kernel(
     const uint16_t* __restrict__ x, const uint32_t* __restrict__ qweight,
     const uint16_t* __restrict__ scales, const uint32_t* __restrict__ qzeros,
@@ -123,11 +129,10 @@ __global__ __launch_bounds__(WAVES * kWave) void awq_gemv_kernel(
     asm volatile("" ::"s"(y), "s"(partials), "s"(counters));
     const int tid = threadIdx.x;
     // grid = (column tiles, K tiles, activation-row tiles): x runs fastest, so workgroups that start together read
-    // neighbouring 128-byte pieces of the same rows, and no division stands in front of the first load
+    // neighbouring 128-byte pieces of the same rows, and no division stands in front of the first load (ORDERED: a multiplication
+    // in its place)
     Tile tile{static_cast<int>(blockIdx.x), static_cast<int>(blockIdx.y)};
-    // (Rotary launches have whole tiles, which share lines only where W itself lies off one: without the test 4096 -> 6144 7.47 ->
-    // 7.36 us.)
-    if constexpr (EPI != kEpiQkRope) {
+    if constexpr (ORDERED) {
         if (order.run) tile = tile_of_workgroup(order, static_cast<uint32_t>(tile.kt * coltiles + tile.ct), static_cast<uint32_t>(ktiles));
     }
     const int ct = tile.ct;
@@ -665,10 +670,17 @@ inline void launch_awq_gemv(const uint16_t* x, const int32_t* qweight, const uin
     for (int sh = 0; sh < 31; sh++) {
         if ((1 << sh) == group) group_shift = sh;
     }
-    hipLaunchKernelGGL((awq_gemv_kernel<WAVES, RT, MB, PRO, EPI>), grid, block, 0, stream, x,
-                       reinterpret_cast<const uint32_t*>(qweight), scales,
-                       reinterpret_cast<const uint32_t*>(qzeros), y, partials, counters, M, K, N,
-                       group, group_shift, coltiles, ktiles, packed_tile_order(qweight, N, coltiles, ktiles), fi, rope, res);
+    const TileOrder order = packed_tile_order(qweight, N, coltiles, ktiles);
+    const auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, block, 0, stream, x, reinterpret_cast<const uint32_t*>(qweight), scales,
+                           reinterpret_cast<const uint32_t*>(qzeros), y, partials, counters, M, K, N, group, group_shift,
+                           coltiles, ktiles, order, fi, rope, res);
+    };
+    // Rotary launches have whole tiles, which share lines only where W itself lies off one.
+    if constexpr (EPI != kEpiQkRope) {
+        if (MB > 1 || order.run) return launch(awq_gemv_kernel<WAVES, RT, MB, PRO, EPI, true>);
+    }
+    if constexpr (MB == 1 || EPI == kEpiQkRope) launch(awq_gemv_kernel<WAVES, RT, MB, PRO, EPI, false>);
 }
 
 }  // namespace kx
