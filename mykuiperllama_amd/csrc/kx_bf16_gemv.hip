@@ -365,25 +365,34 @@ struct HeldForm {
     bool runs;
 };
 
-// Runs of four blocks pay with the rows of y that are written and are lost among long rows of W: us per launch, one by one -> in
-// runs, M = 16 151936 x 4096 214 -> 204, 151936 x 5120 266 -> 250, 144453 x 3144 184 -> 174; M = 8 151936 x 4096 203 -> 199; M = 3
-// 144453 x 3144 160 -> 162; 40000 x 8192 at M = 8 / 16 110 / 114 -> 115 / 118.
+// Runs of four blocks pay with the rows of y that are written and the rounds of blocks, and cost a little with few of either.  Time in
+// runs over one by one, M = 3 / 5 / 8 / 16, at 6, 12, 16 and 37 rounds: K = 3072 1.03 / 1.03 / 1.02 / 1.01, 1.04 / 1.03 / 1.02 / 1.00, 1.03 / 1.02 /
+// 1.00 / 0.98 and 1.02 / 1.00 / 0.97 / 0.93; 6144 1.06 / 1.05 / 1.04 / 1.03, 1.03 / 1.02 / 1.00 / 0.99, 1.02 / 0.98 / 0.99 / 0.98 and 1.01 / 0.98 / 0.97 /
+// 0.95; 3592 alike.  Rows of 4 KB, where the blocks of a round ask the same memory channels, gain from few rounds on (K = 2048 at four:
+// 0.93 / 0.94 / 0.93 / 0.92).  Past K = 6144 they are lost (40000 x 8192 at M = 8 / 16 110 / 114 us -> 115 / 118); four waves gain 1 to 2 % from
+// eight rows on and lose nothing before.
 //
-// The fewest parts whose A operands fit the registers and whose last round of blocks is not emptier for it by more than it gains:
-// a barrier for every PARTS-th of the blocks.  us per launch at M = 3, parts of K 8 / 4 / 2 on lines: 32000 x 768 12.0 / 11.6 / 10.9,
-// 60000 x 2048 44.8 / 42.9 / 42.0, 151936 x 4096 198 / 196 / -; 4 / 2 / 1 off lines: 67290 x 912 30.2 / 27.1 / 25.8.  Few rounds leave
-// compute units idle: up to four, all waves split K (4764 x 4032 at M = 16 17.6 with four parts, 13.1 with eight).
+// On lines the fewest parts whose A operands fit the registers and whose last round of blocks is not emptier for it by more than it
+// gains, a barrier for every PARTS-th of the blocks: time with two parts over four, M = 3 / 8 / 16, at 8 and 16 rounds, K = 1024 1.00 / 1.02 / 1.05
+// and 0.95 / 0.97 / 0.98, 1280 0.96 / 1.00 / 1.04 and 0.96 / 0.98 / 1.00, 1536 1.02 / 1.06 / 1.08 and 1.01 / 1.02 / 1.04; four over eight 2048 0.94 /
+// 0.95 / 1.00 and 0.93 / 0.95 / 0.98, 2560 0.99 / 0.98 / 1.02 and 0.97 / 0.98 / 1.00, 3072 1.02 / 1.03 / 1.05 and 1.00 / 1.01 / 1.05, 4096 1.01 / 1.03 /
+// 1.02 and 0.99 / 1.01 / 1.02, at 37 rounds 0.96 / 1.02 / 1.03.  Few rounds leave
+// compute units idle: up to four, all waves split K (4764 x 4032 at M = 16 17.6 us with four parts, 13.1 with eight).
 // Off lines eight waves that all split K, in units of the length that gives the fullest wave the fewest elements (the longer one of
 // two, with fewer of its pieces across a line), are ahead of four waves and units of 512.  us per launch, four waves -> eight,
 // M = 3 / 14: units of 128 up to K = 1024 4010 x 776 4.06 / 4.45 -> 3.62 / 3.81, 17000 x 904 10.4 / 11.3 -> 9.8 / 10.4, 66000 x 904 27.8 /
-// 29.9 -> 28.1 / 29.6 (left out from 5120 blocks on: 120000 x 904 39.6 / 41.0 -> 47.4 / 47.5); of 256 where they leave fewer than 512
+// 29.9 -> 28.1 / 29.6 (left out from 5120 blocks on: 120000 x 904 39.6 / 41.0 -> 47.4 / 47.5, there four, two or one part: 67290 x 912 at M = 3
+// 30.2 / 27.1 / 25.8); of 256 where they leave fewer than 512
 // 4100 x 1400 5.46 / 6.20 -> 5.10 / 5.75, 120000 x 1400 60.1 / 62.3 -> 57.8 / 57.9, 5500 x 5000 16.6 / 16.8 -> 15.8 / 16.9 (left out past
 // K = 4096 and four rounds: 17000 x 4504 31.4 / 33.2 -> 31.4 / 33.4, 120000 x 4504 177 / 178 -> 185 / 187); of 512 otherwise 4100 x 2200
 // 8.85 / 10.2 -> 6.86 / 8.05, 120000 x 3000 124 / 124 -> 112 / 113, 4100 x 7800 20.4 / 22.9 -> 17.6 / 19.9, 33000 x 7800 89.3 / 93.8 -> 88.6 / 92.8.
 HeldForm held_form(bool whole_lines, int M, int K, int N) {
     const int blocks = (N + 15) / 16;
     const auto fullest = [&](int unit, int parts) { return ((K + unit - 1) / unit + parts - 1) / parts; };
-    const auto form = [&](int waves, int unit, int parts) { return HeldForm{waves, unit, parts, fullest(unit, parts), M >= 6 && K <= 6144}; };
+    const auto form = [&](int waves, int unit, int parts) {
+        const bool many = waves == 4 || (whole_lines && K == 2048) ? M >= 6 : M >= 5 && static_cast<long>(M) * blocks >= 150 * kComputeUnits;
+        return HeldForm{waves, unit, parts, fullest(unit, parts), K <= 6144 && many};
+    };
     if (!whole_lines) {
         if (K <= 1024) {
             if (blocks < 20 * kComputeUnits) return form(8, 128, 8);
@@ -395,7 +404,10 @@ HeldForm held_form(bool whole_lines, int M, int K, int N) {
     }
     const int waves = whole_lines ? 8 : 4;
     int least = K <= 1024 ? 1 : 4;
-    if (whole_lines) least = blocks <= 4 * kComputeUnits ? waves : (K <= 2048 ? 2 : (K <= 4096 ? 4 : 8));
+    if (whole_lines) {
+        const bool four = K <= 2560 || (K <= 4096 && M <= 4 && blocks > 15 * kComputeUnits);
+        least = blocks <= 4 * kComputeUnits ? waves : (K <= 1280 ? 2 : (four ? 4 : 8));
+    }
     int parts = waves;
     long best = 0;
     for (int p = waves, weight = 100 + (waves == 8 ? 9 : 6); p >= least; p /= 2, weight -= 3) {
@@ -408,6 +420,22 @@ HeldForm held_form(bool whole_lines, int M, int K, int N) {
         }
     }
     return form(waves, whole_lines ? 128 : 512, parts);
+}
+
+// Two rows share the vector kernel's loads well enough where N is small, its sweeps of 128 pieces fit a short row, or the held
+// kernel's last round of blocks would be nearly empty.  us, vector -> held: 47090 x 776 17.2 -> 16.6, 53553 x 1176 33.5 -> 28.2, 101754 x
+// 2336 96.7 -> 82.8, 46389 x 3912 71.6 -> 64.7, 69572 x 4688 122 -> 110, 151936 x 4096 195 -> 193, 17672 x 7064 53.4 -> 50.8; what the line
+// leaves out: 32000 x 1024 13.2 -> 13.8, 28732 x 2696 31.7 -> 32.9, 83762 x 896 29.4 -> 29.4, 4361 x 1080 5.1 -> 5.7, 5573 x 3736 11.0 -> 12.7.
+// Held over vector by rounds, 1.6 / 2.0 / 2.05 / 2.15 / 2.3 / 2.6 / 3.03 / 3.2 / 4.03 / 4.6: K = 3072 1.03 / 0.97 / 1.11 / 1.08 / 1.01 / 1.00 / 1.07 /
+// 1.03 / 1.03 / 0.97, 4096 0.93 / 0.93 / 1.04 / 1.02 / 0.98 / 0.92 / 0.99 / 0.98 / 0.98 / 0.91, 5000 1.00 / 0.97 / 1.11 / 1.09 / 1.03 / 0.97 / 1.06 / 1.04 /
+// 1.04 / 0.95; 768, a sweep for the vector kernel, 0.96 / 0.91 / 1.10 / 1.09 / 1.08 / 1.05 / 1.00 / 1.00 / 1.08 / 1.02, at 5.9 0.96.
+bool takes_held(int M, int K, int N) {
+    if (M == 1 || K > kHeldMostK) return false;
+    if (M >= 3) return true;
+    const int pieces = K / 8, swept = (pieces + 127) / 128 * 128;
+    const long blocks = (static_cast<long>(N) + 15) / 16, rounds = (blocks + kComputeUnits - 1) / kComputeUnits;
+    const int least_full = K < 1024 && rounds >= 3 && rounds <= 6 ? 92 : 77;  // percent of the rounds that blocks have to fill
+    return N >= 6500 && (K >= 3072 || 5 * swept >= 6 * pieces) && 100 * blocks >= least_full * rounds * kComputeUnits;
 }
 
 // Launches `form` if it is one of these; UNITS are the numbers of units that the rule above gives with the others, and no
@@ -433,9 +461,9 @@ int launch_held(const uint16_t* x, const uint16_t* w, uint16_t* y, int M, int K,
 #define KX_HELD(WAVES, UNIT, PARTS, RUNS, ...) launch_held_of<WAVES, UNIT, PARTS, RUNS, __VA_ARGS__>(form, x, w, y, M, K, N, s)
     const bool launched =
         KX_HELD(8, 128, 8, false, 1, 2, 3, 4, 5, 6, 7, 8) || KX_HELD(8, 128, 8, true, 1, 2, 3, 4, 5, 6) ||
-        KX_HELD(8, 128, 4, false, 1, 2, 3, 4, 5, 6, 7, 8) || KX_HELD(8, 128, 4, true, 1, 2, 3, 4, 5, 6, 7, 8) ||
-        KX_HELD(8, 128, 2, false, 1, 2, 3, 4, 5, 6, 7, 8) || KX_HELD(8, 128, 2, true, 1, 2, 3, 4, 5, 6, 7, 8) ||
-        KX_HELD(8, 256, 8, false, 1, 3) || KX_HELD(8, 256, 8, true, 1, 3) || KX_HELD(8, 512, 8, false, 1, 2) || KX_HELD(8, 512, 8, true, 1) ||
+        KX_HELD(8, 128, 4, false, 1, 2, 3, 4, 5, 6, 7, 8) || KX_HELD(8, 128, 4, true, 1, 2, 3, 4, 5) ||
+        KX_HELD(8, 128, 2, false, 1, 2, 3, 4, 5) || KX_HELD(8, 128, 2, true, 1, 2, 3, 4, 5) ||
+        KX_HELD(8, 256, 8, false, 1, 3) || KX_HELD(8, 256, 8, true, 1) || KX_HELD(8, 512, 8, false, 1, 2) || KX_HELD(8, 512, 8, true, 1) ||
         KX_HELD(4, 512, 4, false, 1, 3) || KX_HELD(4, 512, 4, true, 1, 3) || KX_HELD(4, 512, 2, false, 1) || KX_HELD(4, 512, 2, true, 1) ||
         KX_HELD(4, 512, 1, false, 1, 2) || KX_HELD(4, 512, 1, true, 1, 2);
 #undef KX_HELD
@@ -446,7 +474,7 @@ int launch_held(const uint16_t* x, const uint16_t* w, uint16_t* y, int M, int K,
 }  // namespace kx
 
 extern "C" int kx_bf16_held_form(int32_t whole_lines, int32_t M, int32_t K, int32_t N, int32_t* form) {
-    if (!form || M < 2 || M > KX_MAX_BATCH || K < 8 || K % 8 != 0 || K > kx::kHeldMostK || N < 1) return 0;
+    if (!form || M < 1 || M > KX_MAX_BATCH || K < 8 || K % 8 != 0 || N < 1 || !kx::takes_held(M, K, N)) return 0;
     const kx::HeldForm f = kx::held_form(whole_lines != 0, M, K, N);
     const int32_t fields[5] = {f.waves, f.unit, f.units, f.parts, f.runs};
     for (int i = 0; i < 5; i++) form[i] = fields[i];
@@ -464,13 +492,7 @@ extern "C" int kx_gemv_bf16(const uint16_t* x, const uint16_t* w, uint16_t* y, i
         return KX_ERR_ALIGNMENT;
     }
     hipStream_t s = kx::as_stream(stream);
-    // Two rows share the vector kernel's loads well enough where N is small or its sweeps of 128 pieces fit a short row.  us, vector
-    // -> held: 47090 x 776 17.2 -> 16.6, 53553 x 1176 33.5 -> 28.2, 101754 x 2336 96.7 -> 82.8, 46389 x 3912 71.6 -> 64.7, 69572 x 4688
-    // 122 -> 110, 151936 x 4096 195 -> 193, 17672 x 7064 53.4 -> 50.8; what the line leaves out: 32000 x 1024 13.2 -> 13.8, 28732 x 2696
-    // 31.7 -> 32.9, 83762 x 896 29.4 -> 29.4, 4361 x 1080 5.1 -> 5.7, 5573 x 3736 11.0 -> 12.7.
-    const int pieces = K / 8, swept = (pieces + 127) / 128 * 128;
-    const bool two_rows = M == 2 && N >= 6500 && (K >= 3072 || 5 * swept >= 6 * pieces);
-    if ((M >= 3 || two_rows) && K <= kx::kHeldMostK) return kx::launch_held(x, w, y, M, K, N, s);
+    if (kx::takes_held(M, K, N)) return kx::launch_held(x, w, y, M, K, N, s);
     if (M >= 3) {
         // K > 8192: the activations of a wave's part do not fit its registers
         if (M <= 8) {

@@ -71,7 +71,7 @@ int kx_shared_line_tile(int32_t coltiles, int32_t ktiles, int32_t id, int32_t* c
 
 /* The form of csrc/kx_bf16_gemv.hip's kernel for two to sixteen rows and K <= 8192 that a launch takes, by whether every row of W
  * starts on a memory line: waves, elements of K per unit, units of a wave, waves that split K, runs of four blocks (0 or 1).
- * Returns 1, or 0 for sizes that the kernel does not take. */
+ * Returns 1, or 0 for sizes that the kernel does not take (among them two rows where the kernel for one and two is faster). */
 int kx_bf16_held_form(int32_t whole_lines, int32_t M, int32_t K, int32_t N, int32_t* form);
 
 /* Bytes of a kx_step_desc and of a kx_step_layer as the library was compiled: a binding that mirrors them compares. */

@@ -48,12 +48,15 @@ def test_edges_of_the_forms_off_lines(K, blocks):
 
 
 # every form of the kernel (test_bf16_held_forms.py holds this list to it): K, blocks, and whether W starts on a memory line.
-# Eight, four and two of eight waves to a block, one to eight units each, the last block beside nothing; off lines two and one of four
-FORMS = ([(K, 300, True) for K in (1088, 2112, 3072, 3136, 5120, 5184, 7168, 8128, 8192)] +
-         [(K, 1285, True) for K in (64, 512, 704, 1024, 1088, 1472, 2048, 2112, 2560, 3008, 3520, 4096)] +
-         [(1984, 3500, True)] +
-         [(K, 2000, True) for K in (64, 256, 448, 704, 768, 1024, 1280, 1536, 1728, 2048)] + [(768, 1999, True), (704, 1803, True)] +
-         [(K, 300, False) for K in (64, 1216, 2816, 4096, 5056, 6400)] +
+# Eight, four and two of eight waves to a block, one to eight units each, one by one and in runs, the last block beside nothing;
+# off lines all of eight waves, four, two and one of four
+FORMS = ([(K, 300, True) for K in (64, 1088, 2048, 2112, 3072, 3136, 5120, 5184, 7168, 8128, 8192)] +
+         [(K, 2600, True) for K in (2112, 3136, 5056, 6144)] + [(1024, 2601, True)] +
+         [(K, 1301, True) for K in (64, 512, 704, 1024, 1088, 1472, 2048, 2112, 2560)] +
+         [(K, 2401, True) for K in (64, 512, 576, 1024, 1088, 1472, 2112, 2560)] + [(K, 3850, True) for K in (2624, 3520, 4096)] +
+         [(K, 1803, True) for K in (64, 256, 448, 704, 768, 1024, 1088, 1280)] +
+         [(K, 2825, True) for K in (64, 320, 576, 768, 832, 1024, 1088, 1280)] + [(768, 1999, True), (768, 2000, True)] +
+         [(K, 300, False) for K in (64, 1216, 2816, 4096, 5056, 6400)] + [(K, 2401, False) for K in (1032, 2056, 2816)] +
          [(4608, 1025, False), (6080, 1029, False), (904, 5120, False), (200, 5120, False), (904, 7499, False), (904, 7500, False), (896, 7500, False),
           (1024, 5121, False)])
 
