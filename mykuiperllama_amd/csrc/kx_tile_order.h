@@ -87,8 +87,12 @@ inline TileOrder packed_tile_order(const void* qweight, int N, int coltiles, int
 // With two and four column tiles an XCD's run is few rows of tiles and, unless the K tiles divide by eight, begins inside one:
 // 6144 -> 264 (12 K tiles) at M = 6 / 16 8.3 / 8.8 -> 8.6 / 9.2, 2112 -> 896 with groups of 64 behind SwiGLU at M = 12 (9) 7.65 -> 8.0;
 // 4096 -> 776 (16) at M = 6 / 16 7.5 / 8.1 -> 7.3 / 8.0.
-inline bool together_by_number(int M, int steps, int coltiles, int ktiles) {
+// Where every other row starts on a line, half as many lines are shared, which four column tiles do not make up for: 2048 -> 896 with
+// groups of 64 (eight) at M = 6 / 16 6.40 / 6.97 -> 6.64 / 7.21, 6144 -> 896 (24) at M = 9 / 16 8.41 / 8.56 -> 8.83 / 9.00; left out 12288 ->
+// 896 (24, with groups of 64 48) at M = 6 9.46 -> 9.06 (9.69 -> 9.02) and at M = 9 with groups of 64 10.36 -> 9.98 (at M = 16 10.9 -> 12.0).
+inline bool together_by_number(int M, int steps, int N, int coltiles, int ktiles) {
     if (coltiles % static_cast<int>(kXcds) == 0) return 4 * steps < M || coltiles * ktiles <= 12 * M;
+    if (coltiles == 4 && N % kTileCols == kTileCols / 2 && (M > 12 || ktiles <= (M > 8 ? 24 : 16))) return true;
     return (coltiles == 2 || coltiles == 4) && ktiles % static_cast<int>(kXcds) != 0;
 }
 
