@@ -156,8 +156,9 @@ __device__ __forceinline__ int group_of_step(const MfmaGrid& g, int step) {
 //
 // Four steps per wave at five and more rows, stored: 185 registers leave two to a compute unit, so that a grid of 513 to 768
 // comes in two rounds and cannot finish its tiles together.  With four nibbles' operands at a time and a step's activations read
-// when it comes they fit 168 (what still goes to memory at sixteen rows, 80 bytes a lane, belongs to the single reader's read-back).  Behind
-// a norm every such launch takes this form: us per launch, M = 9 / 16, two -> three and finishing together, 4096 -> 24576 20.0 /
+// when it comes they fit 168 (what still goes to memory at sixteen rows behind a norm, 80 bytes a lane, belongs to the single
+// reader's read-back; the plain form, which has none, keeps all but two words).
+// Behind a norm every such launch takes this form: us per launch, M = 9 / 16, two -> three and finishing together, 4096 -> 24576 20.0 /
 // 20.8 -> 18.0 / 18.7, 5120 -> 15360 20.9 / 21.6 -> 16.9 / 17.4, 8192 -> 10240 at M = 6 / 9 / 16 17.9 / 21.9 / 22.3 -> 17.2 / 18.1 / 20.2;
 // two -> three alone, larger grids, M = 6 / 16, 4096 -> 32768 22.8 / 25.7 -> 22.8 / 24.3, 5120 -> 51200 43.8 /
 // 48.2 -> 43.8 / 46.2, and smaller ones, 4096 -> 12288 12.3 / 13.9 -> 12.2 / 13.9.  A plain launch takes it where make_mfma_plan
@@ -852,7 +853,7 @@ __global__ __launch_bounds__(WAVES * kWave, ((KS == 1 && ROUNDS == 2 && EPI == k
             }
         }
         if constexpr (ROWS >= 8) {
-            if (grid.sliced) {
+            if (TRIO || grid.sliced) {  // every TRIO plan is
                 splitk_exchange_sliced<ROWS>(M, N, ct, kt, ktiles, partials, counters, s_word, grid.wait_ticks, request,
                                              finish);
                 return;
