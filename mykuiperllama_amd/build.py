@@ -74,7 +74,7 @@ def build_kuiper():
                   glob.glob(os.path.join(KUIPER, "source", "**", "*.hip"), recursive=True))
     if not srcs:
         return None
-    inc = ["-I", INCLUDE, "-I", os.path.join(KUIPER, "include"), "-I", os.path.join(KUIPER, "source", "op")]
+    inc = ["-I", INCLUDE, "-I", CSRC, "-I", os.path.join(KUIPER, "include"), "-I", os.path.join(KUIPER, "source", "op")]
     _run([HIPCC] + DEVICE_FLAGS + COMMON + ["-shared"] + inc + srcs +
          ["-L", LIB_DIR, "-lkx_hip", "-Wl,-rpath,$ORIGIN", "-o", KUIPER_LIB])
     _run([HIPCC, "--offload-arch=gfx950"] + COMMON + inc + [os.path.join(KUIPER, "app", "safetensors_dump.cpp")] +
@@ -106,7 +106,7 @@ def build_kuiper_asan():
     os.makedirs(LIB_DIR, exist_ok=True)
     obj_dir = os.path.join(LIB_DIR, "obj_asan")
     os.makedirs(obj_dir, exist_ok=True)
-    inc = ["-I", INCLUDE, "-I", os.path.join(KUIPER, "include"), "-I", os.path.join(KUIPER, "source", "op"),
+    inc = ["-I", INCLUDE, "-I", CSRC, "-I", os.path.join(KUIPER, "include"), "-I", os.path.join(KUIPER, "source", "op"),
            "-I", TESTS_CPP]
     asan = ["-O1", "-g", "-std=c++17", "-Xarch_host", "-fsanitize=address", "-Xarch_host", "-fno-omit-frame-pointer"]
     srcs = sorted(glob.glob(os.path.join(KUIPER, "source", "**", "*.cpp"), recursive=True) +

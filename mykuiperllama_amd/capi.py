@@ -61,6 +61,7 @@ SIGNATURES = {
 INTERNAL_SIGNATURES = {
     "kx_gemv_awq_bf16_policy": (ctypes.c_int, [_P, _P, _P, _P, _P, _I32, _I32, _I32, _I32, _P, _SZ, _P, _I32]),
     "kx_decode_step_bf16": (ctypes.c_int, [_P, _P, _P]),
+    "kx_step_merges_in_o": (ctypes.c_int, [_I32, _I32, _I32]),
     "kx_step_desc_bytes": (_SZ, []),
     "kx_step_layer_bytes": (_SZ, []),
 }

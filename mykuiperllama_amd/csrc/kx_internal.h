@@ -65,6 +65,10 @@ typedef struct kx_step_desc {
 
 int kx_decode_step_bf16(const kx_step_desc* desc, const kx_step_layer* layers, void* stream);
 
+/* Where a step of one sequence merges the chunks of the attention: 1 on the way into the o projection, 0 in a launch of its own,
+ * which is then the faster, -1 in a launch of its own because the cache has more chunks than the projection merges. */
+int kx_step_merges_in_o(int32_t hidden, int32_t n_q_heads, int32_t max_positions);
+
 /* Column tile and K tile of workgroup `id` of a grid whose neighbouring column tiles share memory lines (csrc/kx_tile_order.h):
  * 1, or 0 where such a grid is too small or too large for it and a workgroup takes the tile of its own number. */
 int kx_shared_line_tile(int32_t coltiles, int32_t ktiles, int32_t id, int32_t* ct, int32_t* kt);

@@ -16,7 +16,7 @@ packed tensors of the separate projections are concatenated along N when the wei
 into the next RMSNorm, and by default (`fused=True`) both ride in the prologue of the GEMV that
 consumes the normalised row, as does SwiGLU in front of the down projection, and the per-head
 norm, rotation and cache append ride in the epilogue of the q/k/v GEMV, and the o projection
-merges the chunks of the attention itself (contexts up to 5120 positions): five launches per
+merges the chunks of the attention itself (caches of up to 10240 positions): five launches per
 layer instead of ten.  The residual stream then alternates between two buffers, because a fused
 launch reads the whole incoming row in every workgroup while it writes the updated one.
 Every launch goes to torch's current stream, so a step can be captured in a HIP graph; token and
@@ -65,18 +65,10 @@ class DecodeModel:
         self.torch = torch
         self.cfg = cfg
         self.max_positions = max_positions
-        # Where the attention chunks are merged: in the prologue of the o projection (one launch
-        # fewer per layer) when the cache is short enough for it.  Every workgroup of that projection
-        # repeats the merge of its two heads, so it pays while the projection has one round of workgroups (Qwen3-8B:
-        # 256 of them, 1.1 to 2.3 us per layer faster; Qwen3-32B: 640, 0.7 to 2.7 us slower than the separate merge
-        # kernel) and, up to two, while the heads have few chunks.  us per layer, in the projection / separate, at 1000, 3000
-        # and 5000 positions: 320 workgroups of 40 heads 34.1 / 35.0, 36.8 / 36.7, 39.5 / 38.4, 400 38.6 / 38.8, 40.4 / 40.7,
-        # 43.2 / 42.4, 384 of 64 34.3 / 34.8, 37.4 / 36.2, 40.7 / 38.2.  The caller can decide otherwise.
-        fits = max_positions <= capi.FUSED_MERGE_MAX_POSITIONS
-        o_workgroups = -(-cfg.hidden // 256) * max(1, cfg.n_q * cfg.head_dim // 256)
-        chunks = -(-max_positions // (64 if max_positions <= 5120 else 128))
-        pays = o_workgroups <= 256 or (o_workgroups <= 512 and cfg.n_q * chunks <= 1920)
-        self.merge_in_o = fits and (pays if merge_in_o is None else bool(merge_in_o))
+        # Where the attention chunks are merged: in the prologue of the o projection (one launch fewer per layer) when the
+        # cache is short enough for it and it is the faster way, or as the caller decides.
+        rule = capi.load().kx_step_merges_in_o(cfg.hidden, cfg.n_q, max_positions)
+        self.merge_in_o = rule >= 0 and bool(rule if merge_in_o is None else merge_in_o)
         c = cfg
         gen = torch.Generator(device="cuda")
         gen.manual_seed(seed)

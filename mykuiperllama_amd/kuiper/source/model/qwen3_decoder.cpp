@@ -11,16 +11,13 @@
 #include "kernel/hip/matmul_kernel.h"
 #include "kernel/kernel_interface.h"
 #include "kx_hip.h"
+#include "kx_internal.h"
 #include "random_fill.h"
 
 namespace model {
 namespace {
 
-constexpr int32_t kTileColumns = 256;          // columns per sum of squares that a residual launch leaves
-constexpr int32_t kMergeInOMaxPositions = 10240;  // longest context the o projection can merge itself
-constexpr int32_t kMergeInOWorkgroups = 256;      // up to here the o projection always merges
-constexpr int32_t kMergeInOMaxWorkgroups = 512;   // beyond this the separate merge launch is cheaper, between the two where
-constexpr int32_t kMergeInOMaxHeadChunks = 1920;  // there are more chunks than this, all heads together
+constexpr int32_t kTileColumns = 256;  // columns per sum of squares that a residual launch leaves
 
 std::string layer_prefix(int32_t i) { return "model.layers." + std::to_string(i) + "."; }
 
@@ -109,17 +106,7 @@ Qwen3Decoder::Qwen3Decoder(const Qwen3Config& config, int32_t max_positions, Dec
     stream_ = std::make_shared<kernel::CudaConfig>();
     stream_->create();
 
-    // The o projection merges the attention chunks itself while it has one round of workgroups, or up to two and few
-    // chunks; with more, every one of them repeating the merge of its heads costs more than the launch it saves (us per
-    // layer, in the projection / separate, at 1000, 3000 and 5000 positions: 320 workgroups of 40 heads 34.1 / 35.0, 36.8 / 36.7,
-    // 39.5 / 38.4, 384 of 64 34.3 / 34.8, 37.4 / 36.2, 40.7 / 38.2).
-    const int32_t o_workgroups =
-        ((c.hidden + kTileColumns - 1) / kTileColumns) * std::max(1, c.n_q_heads * c.head_dim / kTileColumns);
-    const int32_t chunk = max_positions <= 5120 ? 64 : 128;  // positions of a chunk of the first attention stage
-    const int64_t head_chunks = static_cast<int64_t>(c.n_q_heads) * ((max_positions + chunk - 1) / chunk);
-    merge_in_o_ = max_positions <= kMergeInOMaxPositions &&
-                  (o_workgroups <= kMergeInOWorkgroups ||
-                   (o_workgroups <= kMergeInOMaxWorkgroups && head_chunks <= kMergeInOMaxHeadChunks));
+    merge_in_o_ = kx_step_merges_in_o(c.hidden, c.n_q_heads, max_positions) == 1;
 
     const base::DataType bf16 = base::DataType::DataTypeBf16;
     layers_.resize(static_cast<size_t>(c.layers));
