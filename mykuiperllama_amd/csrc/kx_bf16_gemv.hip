@@ -196,13 +196,14 @@ __global__ __launch_bounds__(kMfmaWaves * kWave) void bf16_gemv_mfma_kernel(
 // straight from memory asks for 64 bytes of sixteen rows at a time, which the memory system answers at three quarters of its
 // rate.  Here the A operands of a wave's part of K stay in registers for the life of the workgroup, and W goes through LDS: a
 // unit is UNIT elements of the block's sixteen rows, loaded straight into the wave's own ring, so that no barrier and no
-// register stands between the stream and the MFMAs and 128 KB per compute unit are in flight.  The waves of a block meet in
-// LDS, two buffers in turn, one barrier per block that leaves loads alone.  K is cut into whole units, as evenly as they go: a
-// part has UNITS of them or one less.
+// register stands between the stream and the MFMAs and 128 KB per compute unit are in flight.  (Eight waves and units of 512
+// leave a wave one slot: there it reads its unit into registers, 64 of them, before it asks for the next, and only the other waves'
+// units are in flight meanwhile.)  The waves of a block meet in LDS, two buffers in turn, one barrier per block that leaves loads
+// alone.  K is cut into whole units, as evenly as they go: a part has UNITS of them or one less.
 // A row of a unit is stored with its 16-byte pieces permuted by the low bits of the row (the lane that loads piece j of
 // row r fetches piece j ^ (r & 7)), so that the sixteen rows that an operand read touches lie in different banks.
 // Where rows start on memory lines, units of 128 elements, 256 bytes of a row, which are two lines; rows that do not start on
-// lines would have such a piece touch three, and longer units cost them less (launch_held).  us per launch at M = 3 / 8 / 16, eight
+// lines would have such a piece touch three, and longer units cost them less (held_form).  us per launch at M = 3 / 8 / 16, eight
 // waves of equal parts of K rounded up to 1024 -> now: rows on lines 151936 x 4096 182 / 189 / 200 -> 180 / 186 / 194, 151936 x 5120
 // 231 / 241 / 254 -> 230 / 233 / 239, 32000 x 768 12.6 / 13.3 / 13.7 -> 10.8 / 11.1 / 11.8; others 144453 x 3144 172 / 182 / 198 -> 137 /
 // 144 / 152, 101754 x 2336 84 / 87 / 101 -> 74 / 75 / 82, 79438 x 1240 46.4 / 47.5 / 51.7 -> 36.9 / 38.4 / 40.1, 69572 x 4688 114 / 120 /

@@ -1,4 +1,4 @@
-"""BF16 GEMV at several activation rows: lengths of K at the edges of a wave's part (1024 elements per unit), output
+"""BF16 GEMV at several activation rows: lengths of K at the edges of the units and parts it is cut into and of 8192, output
 counts at the edges of a block of sixteen and of one block per compute unit, against fp64."""
 import pytest
 
