@@ -280,11 +280,7 @@ inline MfmaGrid mfma_grid(const AwqPlan& p, int group) {
     MfmaGrid g{};
     g.coltiles = p.coltiles;
     g.ktiles = p.ktiles;
-    g.side = p.coltiles;
-    if (p.sliced) {  // the widest group that divides the tiles: no workgroup without a tile, no test for one
-        g.side = kTileGroup;
-        while (p.coltiles % g.side != 0) g.side--;
-    }
+    g.side = p.sliced ? tile_group(p.coltiles) : p.coltiles;
     g.sliced = p.sliced;
     g.run = p.run;
     g.wait_ticks = kSliceWaitTicks;
@@ -469,6 +465,10 @@ extern "C" int kx_shared_line_tile(int32_t coltiles, int32_t ktiles, int32_t id,
     *ct = tile.ct;
     *kt = tile.kt;
     return 1;
+}
+
+extern "C" int kx_tiles_by_number(int32_t M, int32_t steps, int32_t N, int32_t coltiles, int32_t ktiles, int32_t together) {
+    return together && kx::together_by_number(M, steps, N, coltiles, ktiles);
 }
 
 extern "C" int kx_workspace_init(void* workspace, size_t workspace_bytes, void* stream) {

@@ -43,7 +43,6 @@
 namespace kx {
 
 constexpr int kStepRows = 32;  // rows of K per MFMA step
-constexpr int kTileGroup = 8;  // most column tiles whose workgroups start side by side when they finish together
 
 // Column (0..7) inside a word -> nibble that holds it (inverse of order_of).
 __host__ __device__ constexpr int nibble_of(int col) {

@@ -73,6 +73,10 @@ int kx_step_merges_in_o(int32_t hidden, int32_t n_q_heads, int32_t max_positions
  * 1, or 0 where such a grid is too small or too large for it and a workgroup takes the tile of its own number. */
 int kx_shared_line_tile(int32_t coltiles, int32_t ktiles, int32_t id, int32_t* ct, int32_t* kt);
 
+/* Whether a matrix-core launch whose column tiles share memory lines has its workgroups take the tiles of their own numbers all the
+ * same: rows, 32-row steps per wave, output columns, the grid, and whether its workgroups finish a column tile together. */
+int kx_tiles_by_number(int32_t M, int32_t steps, int32_t N, int32_t coltiles, int32_t ktiles, int32_t together);
+
 /* The form of csrc/kx_bf16_gemv.hip's kernel for two to sixteen rows and K <= 8192 that a launch takes, by whether every row of W
  * starts on a memory line: waves, elements of K per unit, units of a wave, waves that split K, runs of four blocks (0 or 1).
  * Returns 1, or 0 for sizes that the kernel does not take (among them two rows where the kernel for one and two is faster). */

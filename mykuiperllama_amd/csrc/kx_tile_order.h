@@ -7,6 +7,14 @@
 namespace kx {
 
 constexpr int kTileCols = 256;  // output columns per column tile: 128 bytes of a packed row
+constexpr int kTileGroup = 8;   // most column tiles whose workgroups start side by side when they finish together
+
+// The widest such group that divides the column tiles: no workgroup without a tile, no test for one.
+inline int tile_group(int coltiles) {
+    int side = kTileGroup;
+    while (coltiles % side != 0) side--;
+    return side;
+}
 
 // Which tile of a (column tiles x K tiles) grid a workgroup takes when neighbouring column tiles are to run on one XCD.
 // Workgroups go to the eight XCDs in turn; the tiles, counted in groups of kTilesSideBySide columns with the columns of a
@@ -90,9 +98,22 @@ inline TileOrder packed_tile_order(const void* qweight, int N, int coltiles, int
 // Where every other row starts on a line, half as many lines are shared, which four column tiles do not make up for: 2048 -> 896 with
 // groups of 64 (eight) at M = 6 / 16 6.40 / 6.97 -> 6.64 / 7.21, 6144 -> 896 (24) at M = 9 / 16 8.41 / 8.56 -> 8.83 / 9.00; left out 12288 ->
 // 896 (24, with groups of 64 48) at M = 6 9.46 -> 9.06 (9.69 -> 9.02) and at M = 9 with groups of 64 10.36 -> 9.98 (at M = 16 10.9 -> 12.0).
+// More column tiles on such half lines lose by it as long as there is at most one workgroup per compute unit and few K tiles for the rows,
+// those in groups of eight most, those in other even groups, whose columns lie on two or four XCDs, with one and two steps; odd groups
+// have a column on all XCDs either way.  Groups of eight, four steps 15232 -> 1920 (240 workgroups, 30 K tiles) behind SwiGLU at M = 16
+// 12.8 -> 13.4, 7680 -> 3968 (240, 15) at M = 15 11.8 -> 12.2; two 3328 -> 3968 (208, 13) at M = 7 7.8 -> 8.2, 1792 -> 8064 (224, 7)
+// behind a norm at M = 8 7.6 -> 8.0; left out 14592 -> 1920 (232, 29) at M = 11 0.98 of the time, 4352 -> 3968 (272, 17) at M = 5 0.92.  Groups
+// of six 3968 -> 2944 (192, 16) behind a norm at M = 10 8.8 -> 9.2, 3328 -> 1408 (78, 13) behind SwiGLU at M = 11 8.2 -> 8.4; left out
+// 5632 -> 1408 (132, 22) at M = 7 0.95, 2048 -> 13696 (432, 8) at M = 10 0.985, four steps 1.00 up to K tiles for 2 M, then 0.95.
 inline bool together_by_number(int M, int steps, int N, int coltiles, int ktiles) {
-    if (coltiles % static_cast<int>(kXcds) == 0) return 4 * steps < M || coltiles * ktiles <= 12 * M;
-    if (coltiles == 4 && N % kTileCols == kTileCols / 2 && (M > 12 || ktiles <= (M > 8 ? 24 : 16))) return true;
+    const int workgroups = coltiles * ktiles, side = tile_group(coltiles);
+    const bool half_lines = N % kTileCols == kTileCols / 2;
+    if (half_lines && workgroups <= 256 && coltiles > 4) {
+        if (side == static_cast<int>(kXcds) && (steps == 4 ? 5 * ktiles <= 12 * M : ktiles <= 3 * M)) return true;
+        if (side % 2 == 0 && steps <= 2 && ktiles <= 2 * M) return true;
+    }
+    if (coltiles % static_cast<int>(kXcds) == 0) return 4 * steps < M || workgroups <= 12 * M;
+    if (coltiles == 4 && half_lines && (M > 12 || ktiles <= (M > 8 ? 24 : 16))) return true;
     return (coltiles == 2 || coltiles == 4) && ktiles % static_cast<int>(kXcds) != 0;
 }
 

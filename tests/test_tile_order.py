@@ -37,3 +37,18 @@ def test_every_tile_is_taken_once(coltiles):
 
 def test_grids_past_the_reach_of_the_divisions_keep_their_numbers():
     assert not ctypes.CDLL(KX_LIB).kx_shared_line_tile(2048, 2000, 5, ctypes.byref(ctypes.c_int32()), ctypes.byref(ctypes.c_int32()))
+
+
+# rows, steps per wave, N, K tiles -> whether the grid keeps the order of its numbers
+@pytest.mark.parametrize("M,steps,N,ktiles,by_number", [
+    # half lines, groups of eight column tiles: up to 256 workgroups, by K tiles for the rows
+    (16, 4, 1920, 32, 1), (16, 4, 1920, 33, 0), (11, 4, 1920, 26, 1), (11, 4, 1920, 29, 0), (8, 2, 3968, 12, 1), (5, 2, 3968, 17, 0), (7, 2, 1920, 20, 1),
+    (7, 2, 1920, 25, 0), (8, 2, 8064, 7, 1), (5, 2, 8064, 9, 0),
+    # other even groups: one and two steps
+    (10, 2, 2944, 16, 1), (10, 4, 2944, 16, 0), (11, 2, 1408, 22, 1), (11, 2, 1408, 23, 0), (7, 2, 1408, 22, 0), (10, 2, 13696, 8, 0),
+    # odd groups, and rows on quarters of lines
+    (11, 2, 1664, 13, 0), (8, 2, 3904, 17, 0),
+    # as before: eight and more by rows and workgroups, two and four by K tiles
+    (16, 2, 8128, 9, 1), (16, 4, 4056, 12, 1), (16, 4, 8168, 8, 0), (6, 1, 264, 12, 1), (6, 1, 264, 16, 0)])
+def test_which_grids_that_finish_together_keep_their_numbers(M, steps, N, ktiles, by_number):
+    assert ctypes.CDLL(KX_LIB).kx_tiles_by_number(M, steps, N, -(-N // 256), ktiles, 1) == by_number
