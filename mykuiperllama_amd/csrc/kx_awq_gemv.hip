@@ -468,7 +468,7 @@ extern "C" int kx_shared_line_tile(int32_t coltiles, int32_t ktiles, int32_t id,
 }
 
 extern "C" int kx_tiles_by_number(int32_t M, int32_t steps, int32_t N, int32_t coltiles, int32_t ktiles, int32_t together) {
-    return together && kx::together_by_number(M, steps, N, coltiles, ktiles);
+    return together ? kx::together_by_number(M, steps, N, coltiles, ktiles) : kx::alone_by_number(M, steps, coltiles, ktiles);
 }
 
 extern "C" int kx_workspace_init(void* workspace, size_t workspace_bytes, void* stream) {

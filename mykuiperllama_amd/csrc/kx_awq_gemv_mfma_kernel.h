@@ -898,7 +898,8 @@ inline void launch_awq_gemv_mfma(const uint16_t* x, const int32_t* qweight, cons
     const dim3 grid(split.side, split.ktiles, split.coltiles / split.side);
     dim3 block(WAVES * kWave, 1, 1);
     MfmaGrid ordered = split;
-    const bool by_number = split.sliced && split.run == 1 && together_by_number(M, KS, N, split.coltiles, split.ktiles);
+    const bool by_number = split.sliced ? split.run == 1 && together_by_number(M, KS, N, split.coltiles, split.ktiles)
+                                        : alone_by_number(M, KS, split.coltiles, split.ktiles);
     if (!by_number) ordered.order = packed_tile_order(qweight, N, split.coltiles, split.ktiles);
     hipLaunchKernelGGL((awq_gemv_mfma_kernel<WAVES, KS, MC, ROUNDS, PRO, EPI, LONE, WALK, FINE, TRIO>), grid, block, 0, stream, x,
                        reinterpret_cast<const uint32_t*>(qweight), scales,

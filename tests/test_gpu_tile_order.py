@@ -34,15 +34,25 @@ def test_against_the_oracle(oracle, M, K, N, group):
 
 
 # grids that finish together, on both sides of the rule that keeps the order of the numbers: eight column tiles and more with one,
-# two and four steps and with 12 M workgroups and more, two and four with K tiles that do and do not divide by eight, four
-# whose rows start on half lines
+# two and four steps and with 12 M workgroups and more, two and four with K tiles that do and do not divide by eight, four,
+# six, twelve and sixteen whose rows start on half lines
 @pytest.mark.parametrize("M,K,N", [(16, 4096, 24 * 256), (16, 4608, 24 * 256), (16, 1024, 8 * 256), (9, 4096, 16 * 256), (8, 4096, 16 * 256),
                                    (5, 1024, 24 * 256), (6, 6144, 512), (6, 4096, 512), (12, 2304, 1024), (12, 2048, 1024), (16, 8192, 8 * 256),
-                                   (6, 2048, 896), (6, 12288, 896), (9, 12288, 896), (6, 6144, 896)])
+                                   (6, 2048, 896), (6, 12288, 896), (9, 12288, 896), (6, 6144, 896), (15, 7680, 3968), (7, 3328, 3968),
+                                   (5, 4352, 3968), (10, 3968, 2944), (7, 5632, 1408)])
 def test_few_workgroups_that_finish_together(M, K, N):
     import torch
     from mykuiperllama_amd import capi
     on, off = (run(torch, capi, M, K, N, 128, shift)[1] for shift in (0, 1))
+    assert np.array_equal(on, off)
+
+
+# grids of more than two workgroups per compute unit, which one workgroup reads back, on both sides of that rule (steps across groups)
+@pytest.mark.parametrize("M,K,N", [(9, 22528, 12 * 256), (9, 23552, 12 * 256), (8, 24576, 12 * 256), (8, 16384, 17 * 256), (10, 16384, 17 * 256)])
+def test_grids_with_one_reader(M, K, N):
+    import torch
+    from mykuiperllama_amd import capi
+    on, off = (run(torch, capi, M, K, N, 64, shift)[1] for shift in (0, 1))
     assert np.array_equal(on, off)
 
 

@@ -52,3 +52,14 @@ def test_grids_past_the_reach_of_the_divisions_keep_their_numbers():
     (16, 2, 8128, 9, 1), (16, 4, 4056, 12, 1), (16, 4, 8168, 8, 0), (6, 1, 264, 12, 1), (6, 1, 264, 16, 0)])
 def test_which_grids_that_finish_together_keep_their_numbers(M, steps, N, ktiles, by_number):
     assert ctypes.CDLL(KX_LIB).kx_tiles_by_number(M, steps, N, -(-N // 256), ktiles, 1) == by_number
+
+
+@pytest.mark.parametrize("M,steps,coltiles,ktiles,by_number", [
+    # nine and more rows: a grid just past two workgroups per compute unit, or runs that begin on the same columns
+    (16, 4, 12, 44, 1), (9, 4, 16, 34, 1), (9, 4, 16, 32, 0), (10, 4, 57, 9, 1), (10, 4, 55, 10, 0), (10, 4, 19, 32, 1), (10, 4, 19, 33, 0), (16, 4, 31, 48, 1),
+    (16, 4, 32, 24, 1), (16, 4, 33, 24, 0), (16, 2, 19, 32, 0),
+    # five to eight: many K tiles and a little more than two per compute unit
+    (8, 4, 12, 48, 1), (5, 4, 15, 36, 1), (8, 4, 16, 40, 0), (8, 4, 19, 32, 0), (8, 4, 14, 42, 0),
+    (4, 4, 12, 48, 0)])
+def test_which_grids_with_one_reader_keep_their_numbers(M, steps, coltiles, ktiles, by_number):
+    assert ctypes.CDLL(KX_LIB).kx_tiles_by_number(M, steps, 256 * coltiles - 128, coltiles, ktiles, 0) == by_number
