@@ -204,10 +204,10 @@ __global__ __launch_bounds__(kMfmaWaves * kWave) void bf16_gemv_mfma_kernel(
 // row r fetches piece j ^ (r & 7)), so that the sixteen rows that an operand read touches lie in different banks.
 // Where rows start on memory lines, units of 128 elements, 256 bytes of a row, which are two lines; rows that do not start on
 // lines would have such a piece touch three, and longer units cost them less (held_form).  us per launch at M = 3 / 8 / 16, eight
-// waves of equal parts of K rounded up to 1024 -> now: rows on lines 151936 x 4096 182 / 189 / 200 -> 180 / 186 / 194, 151936 x 5120
-// 231 / 241 / 254 -> 230 / 233 / 239, 32000 x 768 12.6 / 13.3 / 13.7 -> 10.8 / 11.1 / 11.8; others 144453 x 3144 172 / 182 / 198 -> 137 /
-// 144 / 152, 101754 x 2336 84 / 87 / 101 -> 74 / 75 / 82, 79438 x 1240 46.4 / 47.5 / 51.7 -> 36.9 / 38.4 / 40.1, 69572 x 4688 114 / 120 /
-// 125 -> 104 / 109 / 109 (W alone at the read rate of a large buffer: 173, 216, 6.8; 126, 66, 27, 91).  Cached loads instead of streaming ones lose 10 % on lines and win 2 % off them.
+// waves of equal parts of K rounded up to 1024 -> now: rows on lines 151936 x 4096 181 / 187 / 202 -> 180 / 182 / 189, 151936 x 5120
+// 222 / 235 / 252 -> 221 / 224 / 233, 32000 x 768 12.3 / 12.6 / 12.9 -> 10.4 / 10.6 / 11.3; others 144453 x 3144 165 / 178 / 194 -> 136 /
+// 139 / 150, 101754 x 2336 84 / 88 / 98 -> 74 / 75 / 79, 79438 x 1240 44.5 / 45.9 / 49.9 -> 35.8 / 37.2 / 38.2, 69572 x 4688 114 / 118 /
+// 125 -> 103 / 106 / 109 (W alone at the read rate of a large buffer: 173, 216, 6.8; 126, 66, 27, 91).  Cached loads instead of streaming ones lose 10 % on lines and win 2 % off them.
 constexpr int kRingBytes = 131072;
 
 template <int WAVES, int UNIT, int UNITS, int PARTS, bool RUNS>
