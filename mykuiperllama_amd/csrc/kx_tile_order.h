@@ -122,8 +122,8 @@ inline bool together_by_number(int M, int steps, int N, int coltiles, int ktiles
 // round is all but empty, the columns that are left for the end are the same on every XCD.  us per launch, by number -> by XCD, groups
 // of 64 and 32: 22464 -> 2944 (528 workgroups, 44 K tiles) at M = 16 31.6 -> 38.5, 16256 -> 4736 (608, 32) at M = 10 27.2 -> 31.0, 20480 -> 3712
 // (600, 40) behind SwiGLU at M = 10 32.5 -> 38.4, 24128 -> 6016 (1152, 48) at M = 16 42.3 -> 47.3, 24448 -> 2944 (576, 48) at M = 8 23.6 ->
-// 25.7; with other numbers of K tiles, of those at nine and more rows 0.93 to 1.04 of the time by number past 544 workgroups, with more
-// column tiles than lie side by side 0.92 to 1.06, 0.96 on average; up to eight rows 0.92 to 1.05, 0.95.
+// 25.7.  What the rule leaves out, time by XCD over by number: past 544 workgroups at nine and more rows, other numbers of K tiles 0.93 to
+// 1.04, more column tiles than lie side by side 0.92 to 1.06, 0.96 on average; up to eight rows 0.92 to 1.05, 0.95.
 inline bool alone_by_number(int M, int steps, int coltiles, int ktiles) {
     const int workgroups = coltiles * ktiles;
     if (M < 5 || steps != 4 || workgroups <= 512) return false;
